@@ -1,74 +1,34 @@
-// Small dense solve x = lhs^{-1} rhs on one workgroup (1024 lanes), the
-// reference's LUsolver_v1_KeeplhsMat (src/DLSsolvers.c:106-208):
-// Crout factorisation with unit-diagonal U and no pivoting, forward then
-// backward substitution.  gfx950.
+// Small dense solve x = lhs^{-1} rhs, the reference's LUsolver_v1_KeeplhsMat
+// (src/DLSsolvers.c:106-208): Crout factorisation with unit-diagonal U and no
+// pivoting, forward then backward substitution.  gfx950.
 //
-// Factorisation: right-looking, one barrier-separated step per pivot; every
-// element sees the same operations in the same order as in the reference's
-// loops, so the factor is bit-identical.  For N <= 128 the matrix is held in
-// registers (4 x 4 elements per lane of a 32 x 32 lane grid) and the factor is
-// then kept in LDS (128 KiB of the 160 KiB); larger N work in a global
-// scratch block.
+// Every element of the factor and of y = L^{-1} rhs receives its subtractions
+// a - l u (product and difference rounded separately) in ascending order of
+// the pivot, with the reciprocal pivot applied last, as in the reference's
+// loops, so both are the reference's bits however the work is divided.  The
+// backward substitution of mode FAST is column-oriented (descending pivot);
+// mode REFERENCE keeps the reference's ascending sums.
 //
-// Forward substitution runs column-oriented (for q: finalise row q, broadcast
-// it through LDS, update the rows below).  Each y[i][c] still receives its
-// subtractions in ascending q and the reciprocal scaling last, as in the
-// reference's row-oriented loop, so it is bit-identical too.  The right-hand
-// side is held in registers, JMAX rows per lane.
-//
-// Backward substitution: the reference subtracts x[q] u_iq in ascending q,
-// which makes each row wait for all later rows; mode REFERENCE keeps that
-// order (one sequential chain per column, x in LDS, U from the scratch copy).
-// Mode FAST runs it column-oriented (descending q).
-//
-// With the factor in LDS it is stored column-major with an odd stride
-// (element (r, c) at c (N + 1) + r), so the reads of a factor column by
-// consecutive rows are consecutive words, and fast-order substitutions run
-// wave-local: every right-hand-side column is solved by the lanes of one
-// wave, which pass finished rows to each other by readlane or lane shuffle,
-// with no barrier (lu_subst_wave).
+// N <= 128: one workgroup factors (lu_factor_body), panels of 8 pivots in
+// the registers of a few waves, the trailing matrix in the registers of all
+// 16; up to 32 right-hand sides ride along as further columns, so the forward
+// substitution costs no step of its own.  N > 128: blocks of 128, a factor
+// kernel, triangular solves and products per block, each over many CUs.
 #include <math.h>
+
+#include <type_traits>
 
 #include "kcommon.hpp"
 
 namespace {
 
 constexpr int LU_T = 1024;
-constexpr int JMAX = 16;
-
-// right-hand-side columns per substitution pass: the register block (JMAX
-// rows per lane) must cover N, and without the LDS factor the reference pass
-// keeps N x kc in LDS; 0 when N is out of range
-__host__ __device__ inline int lu_columns(int N, int k, bool in_lds)
-{
-    int kc = k < N ? k : N;
-    if ((long)N * kc > (long)LU_T * JMAX)
-        kc = (int)((long)LU_T * JMAX / N);
-    if (!in_lds && (long)N * kc > 8192)
-        kc = 8192 / N;
-    if (kc < 1 || (LU_T / kc) * JMAX < N)
-        return 0;
-    return kc;
-}
-
-// dynamic LDS of a solve: factor (N x (N + 1)), broadcast rows (2 x kc),
-// pivot row/column (2 x 2 x 128), 2 reciprocal pivots, N reciprocal diagonal
-// entries; without the LDS factor an N x kc block instead of the factor
-__host__ __device__ inline size_t lu_lds_bytes(int N, int k, bool in_lds)
-{
-    const int kc = lu_columns(N, k, in_lds);
-    if (in_lds)
-        return ((size_t)N * (N + 1) + 2 * (size_t)kc + 512 + 2 + N) * sizeof(double);
-    return ((size_t)N * kc + 2 * (size_t)kc + N) * sizeof(double);
-}
-
-// position of factor element (r, c): column-major with stride N + 1 in LDS,
-// row-major in the global scratch block
-template <bool IN_LDS>
-__device__ __forceinline__ long fidx(int N, int r, int c)
-{
-    return IN_LDS ? (long)c * (N + 1) + r : (long)r * N + c;
-}
+constexpr int LU_B = 128;      // rows of a diagonal block
+constexpr int LU_P = 8;        // pivots of a panel
+constexpr int LU_PS = 10;      // LDS row stride of a panel: 20 words, so 16 lanes' 16-byte
+                               // reads of consecutive rows cover all 64 banks
+constexpr int LU_K = 32;       // right-hand sides that ride along with a factorisation
+constexpr int TRI_W = 8;       // waves of a triangular-solve workgroup
 
 // v of lane src (src the same on every lane of the wave)
 __device__ __forceinline__ double readlane_f64(double v, int src)
@@ -79,409 +39,692 @@ __device__ __forceinline__ double readlane_f64(double v, int src)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// v of lane src of this lane's group of LPC lanes
-template <int LPC>
-__device__ __forceinline__ double group_bcast(double v, int src)
-{
-    if constexpr (LPC == 64)
-        return readlane_f64(v, src);
-    else
-        return __shfl(v, src, LPC);
-}
+// ---- substitutions of one vector by one wave -------------------------------------
+//
+// Lane l holds entries l (y0) and 64 + l (y1) of a vector of nb <= 128.  Step q
+// finishes entry q, hands it to the wave by readlane, and the other entries
+// subtract its multiple.  T(q) points to the multipliers of step q (entry i at
+// T(q)[i]; entries outside the triangle are read and not used).  A wave issues
+// one FP64 instruction about every 8.5 cycles and an LDS read waits for 64 or
+// more, so the multipliers of the next 4 steps are read while the current 4
+// run.
 
-// Fast-order forward and backward substitutions with the factor in LDS
-// (a: column-major, stride N + 1; dinv: reciprocal diagonal of L), N <= 128.
-// Right-hand-side column `col` is solved by LPC lanes of one wave (64 / LPC
-// columns per wave, 1024 / LPC per pass); lane lc holds rows lc + LPC r in
-// registers.  Row q is finished by its lane and handed to the others of the
-// group (readlane, or a lane shuffle for LPC < 64), which update their rows:
-// ascending q for L y = rhs with the reciprocal pivot applied last, then
-// descending q for U x = y (unit U).  Each element receives exactly the
-// operations of the barrier-per-step form, in the same order, so the result
-// is the same bits; nothing is shared between waves, so no barrier is needed.
-// Columns cbase + w WC + l / LPC, then + cstride, ... (w = the wave in the
-// workgroup); the single-workgroup solve passes 0 and the columns its waves
-// cover per pass.
-template <int LPC>
-__device__ __forceinline__ void lu_subst_wave(int N, const double *__restrict__ a,
-                                              const double *__restrict__ dinv, int k,
-                                              const double *__restrict__ rhs,
-                                              double *__restrict__ x, int cbase = 0,
-                                              int cstride = (LU_T / 64) * (64 / LPC))
+// ascending: entry i > q subtracts y_q T(q)[i]; with SCALE entry q is first
+// multiplied by its reciprocal pivot (d0, d1: those of this lane's entries)
+template <bool SCALE, typename F>
+__device__ __forceinline__ void tri_forward(int nb, F T, double d0, double d1, double &y0,
+                                            double &y1)
 {
-    constexpr int RPL = 128 / LPC;  // rows per lane
-    constexpr int WC = 64 / LPC;    // columns per wave
-    const int R = N + 1;
-    const int t = threadIdx.x, w = t >> 6, l = t & 63;
-    const int lc = l % LPC;
-    for (int c0 = cbase; c0 < k; c0 += cstride) {
-        const int col = c0 + w * WC + l / LPC;
-        const bool has = col < k;
-        double y[RPL];
+    const int l = threadIdx.x & 63;
+    const int n0 = nb < 64 ? nb : 64;
+    const bool two = nb > 64;
+    double a[2][4], b[2][4];
+    auto load = [&](int s, int q0, bool lo) {
 #pragma unroll
-        for (int r = 0; r < RPL; r++) {
-            const int i = lc + LPC * r;
-            y[r] = (has && i < N) ? rhs[(long)i * k + col] : 0.0;
+        for (int u = 0; u < 4; u++) {
+            const double *t = T(q0 + u < nb ? q0 + u : nb - 1);
+            a[s][u] = lo ? t[l] : 0.0;
+            b[s][u] = two ? t[64 + l] : 0.0;
         }
+    };
+    auto steps0 = [&](int s, int q0) {
 #pragma unroll
-        for (int rq = 0; rq < RPL; rq++) {
+        for (int u = 0; u < 4; u++) {
+            const int q = q0 + u;
+            if (q < n0) {
+                const double yd = SCALE ? mul_rn(y0, d0) : y0;
+                const double yq = readlane_f64(yd, q);
+                const double w = sub_rn(y0, mul_rn(yq, a[s][u]));
+                y0 = l > q ? w : (SCALE && l == q ? yd : y0);
+                if (two)
+                    y1 = sub_rn(y1, mul_rn(yq, b[s][u]));
+            }
+        }
+    };
+    auto steps1 = [&](int s, int q0) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int q = q0 + u;
+            if (q < nb) {
+                const double yd = SCALE ? mul_rn(y1, d1) : y1;
+                const double yq = readlane_f64(yd, q - 64);
+                const double w = sub_rn(y1, mul_rn(yq, b[s][u]));
+                y1 = l > q - 64 ? w : (SCALE && l == q - 64 ? yd : y1);
+            }
+        }
+    };
+    load(0, 0, true);
 #pragma unroll 1
-            for (int lq = 0; lq < LPC; lq++) {
-                const int q = lq + LPC * rq;
-                if (q >= N)
-                    break;
-                if (lc == lq)
-                    y[rq] = mul_rn(y[rq], dinv[q]);
-                const double yq = group_bcast<LPC>(y[rq], lq);
-                const double *Lq = a + (long)q * R;
-#pragma unroll
-                for (int r = rq; r < RPL; r++) {
-                    const int i = lc + LPC * r;
-                    if (i > q && i < N)
-                        y[r] = sub_rn(y[r], mul_rn(yq, Lq[i]));
-                }
-            }
-        }
-#pragma unroll
-        for (int rq = RPL - 1; rq >= 0; rq--) {
+    for (int q0 = 0; q0 < n0; q0 += 8) {
+        load(1, q0 + 4, true);
+        __builtin_amdgcn_sched_barrier(0);
+        steps0(0, q0);
+        load(0, q0 + 8, true);
+        __builtin_amdgcn_sched_barrier(0);
+        steps0(1, q0 + 4);
+    }
+    if (!two)
+        return;
+    load(0, 64, false);
 #pragma unroll 1
-            for (int lq = LPC - 1; lq >= 0; lq--) {
-                const int q = lq + LPC * rq;
-                if (q >= N)
-                    continue;
-                const double xq = group_bcast<LPC>(y[rq], lq);
-                const double *Uq = a + (long)q * R;
-#pragma unroll
-                for (int r = 0; r <= rq; r++) {
-                    const int i = lc + LPC * r;
-                    if (i < q)
-                        y[r] = sub_rn(y[r], mul_rn(xq, Uq[i]));
-                }
-            }
-        }
-        if (has) {
-#pragma unroll
-            for (int r = 0; r < RPL; r++) {
-                const int i = lc + LPC * r;
-                if (i < N)
-                    x[(long)i * k + col] = y[r];
-            }
-        }
+    for (int q0 = 64; q0 < nb; q0 += 8) {
+        load(1, q0 + 4, false);
+        __builtin_amdgcn_sched_barrier(0);
+        steps1(0, q0);
+        load(0, q0 + 8, false);
+        __builtin_amdgcn_sched_barrier(0);
+        steps1(1, q0 + 4);
     }
 }
 
-// The solve of one system by one workgroup of LU_T lanes; lds is the dynamic
-// LDS block (lu_lds_bytes).  Shared by the single-system kernel and the
-// batched one.
-template <bool IN_LDS>
-__device__ __forceinline__ void lu_solve_body(int N, const double *__restrict__ lhs, int k,
-                                              const double *__restrict__ rhs,
-                                              double *__restrict__ x, double *__restrict__ gw,
-                                              int *flag, int mode, int kc, int reuse, double *lds)
+// descending, unit diagonal: entry i < q subtracts y_q T(q)[i]
+template <typename F>
+__device__ __forceinline__ void tri_backward(int nb, F T, double &y0, double &y1)
 {
-    double *a = IN_LDS ? lds : gw;
-    double *rowbuf = IN_LDS ? lds + (long)N * (N + 1) : lds;
-    double *xs = IN_LDS ? lds : lds + 2 * kc;
-    const int t = threadIdx.x;
-
-    // ---- factorisation (or the factor left in gw by the previous call)
-    int bad = 0;
-    if (reuse) {
-        if (IN_LDS) {
-            for (long e = t; e < (long)N * N; e += LU_T)
-                a[fidx<true>(N, (int)(e / N), (int)(e % N))] = gw[e];
+    const int l = threadIdx.x & 63;
+    const int n0 = nb < 64 ? nb : 64;
+    double a[2][4], b[2][4];
+    auto load = [&](int s, int q0, bool hi) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const double *t = T(q0 - u > 0 ? q0 - u : 0);
+            a[s][u] = t[l];
+            b[s][u] = hi ? t[64 + l] : 0.0;
         }
-        __syncthreads();
-    } else if (IN_LDS) {
-        // N <= 128: a 32 x 32 lane grid, lane (tr, tc) owns a[tr + 32 i][tc + 32 j]
-        // in registers.  Step p: the owners of row p and of column p publish them
-        // (double-buffered, one barrier per step); every lane scales the row by
-        // the reciprocal pivot itself (same bits as the row owner) and updates
-        // its elements.  Per element: the reference's operations, in its order.
-        const int tr = t >> 5, tc = t & 31;
-        double v[4][4];
+    };
+    auto steps1 = [&](int s, int q0) {
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int r = tr + 32 * i, c = tc + 32 * j;
-                v[i][j] = (r < N && c < N) ? lhs[(long)r * N + c] : 0.0;
+        for (int u = 0; u < 4; u++) {
+            const int q = q0 - u;
+            if (q >= 64) {
+                const double yq = readlane_f64(y1, q - 64);
+                const double w = sub_rn(y1, mul_rn(yq, b[s][u]));
+                y1 = l < q - 64 ? w : y1;
+                y0 = sub_rn(y0, mul_rn(yq, a[s][u]));
             }
-        double *ub = lds + (long)N * (N + 1) + 2 * kc;  // 2 x 128: unscaled row p
-        double *lb = ub + 256;                     // 2 x 128: column p
-        double *ib = lb + 256;                     // 2: reciprocal pivot
-        // pivot p = 32 ip + pr: ip is a compile-time index into the register block
+        }
+    };
+    auto steps0 = [&](int s, int q0) {
 #pragma unroll
-        for (int ip = 0; ip < 4; ip++) {
-            for (int pr = 0; pr < 32; pr++) {
-                const int p = ip * 32 + pr;
-                if (p >= N)
-                    break;
-                const int off = (p & 1) * 128;
-                if (tr == pr && tc == pr)
-                    ib[p & 1] = 1.0 / v[ip][ip];
-                if (tr == pr) {
+        for (int u = 0; u < 4; u++) {
+            const int q = q0 - u;
+            if (q > 0) {
+                const double yq = readlane_f64(y0, q);
+                const double w = sub_rn(y0, mul_rn(yq, a[s][u]));
+                y0 = l < q ? w : y0;
+            }
+        }
+    };
+    if (nb > 64) {
+        load(0, nb - 1, true);
+#pragma unroll 1
+        for (int q0 = nb - 1; q0 >= 64; q0 -= 8) {
+            load(1, q0 - 4, true);
+            __builtin_amdgcn_sched_barrier(0);
+            steps1(0, q0);
+            load(0, q0 - 8, true);
+            __builtin_amdgcn_sched_barrier(0);
+            steps1(1, q0 - 4);
+        }
+    }
+    load(0, n0 - 1, false);
+#pragma unroll 1
+    for (int q0 = n0 - 1; q0 > 0; q0 -= 8) {
+        load(1, q0 - 4, false);
+        __builtin_amdgcn_sched_barrier(0);
+        steps0(0, q0);
+        load(0, q0 - 8, false);
+        __builtin_amdgcn_sched_barrier(0);
+        steps0(1, q0 - 4);
+    }
+}
+
+// ---- factorisation of up to 128 rows ----------------------------------------------
+
+// columns of U above the diagonal, packed: column q at q (q - 1) / 2
+__host__ __device__ inline int upk(int q) { return q * (q - 1) / 2; }
+
+// dynamic LDS (doubles) of lu_factor_body: the column panel (128 rows), the row
+// panel (128 columns and LU_K right-hand sides), and with `back` the packed U
+// and the right-hand sides after the forward substitution
+__host__ __device__ inline int lu_factor_lds(int N, int k, bool back)
+{
+    const int pan = LU_PS * (2 * LU_B + LU_K);
+    return back ? pan + upk(N) + 2 * LU_B + k * (N + 1) + LU_B : pan;
+}
+
+// Factor the N x N block at lhs (row stride ldl) into gw (row stride ldg; lhs
+// may be gw), N <= 128, with k <= LU_K right-hand sides: y = L^{-1} rhs, and
+// with back also x = U^{-1} y in mode FAST's order; written to x (N x k).
+//
+// Lane (tr, tc) of a 32 x 32 grid keeps elements (tr + 32 i, tc + 32 j) and
+// right-hand side tc of rows tr + 32 i in registers.  Per panel of 8 pivots:
+//   1. the panel's columns (all rows below) and rows (all columns to the right,
+//      the right-hand sides among them) lie in LDS.  A row wave holds the 8
+//      panel rows and 56 rows below, one row of the panel's 8 columns a lane;
+//      a column wave the 8 panel columns and 56 columns to the right, one
+//      column of the panel's 8 rows a lane.  Each factors the 8 x 8 diagonal
+//      block for itself, passing pivots between lanes by readlane, so l and u
+//      of the whole panel are ready without a barrier inside it;
+//   2. every lane applies the 8 rank-1 updates to its elements, in order, and
+//      the owners of the next panel put it into LDS.
+// Two barriers per 8 pivots.  What bounds it is the chain of pivots: one
+// reciprocal, one product and one subtraction each, about 200 cycles; a barrier
+// and a broadcast through LDS for every pivot had taken 1870.
+__device__ __forceinline__ void lu_factor_body(int N, const double *lhs, long ldl, double *gw,
+                                               long ldg, int k, const double *__restrict__ rhs,
+                                               double *__restrict__ x, int *flag, bool back,
+                                               double *lds)
+{
+    double *cp = lds;                            // column panel: row r at cp + r LU_PS
+    double *rp = lds + LU_PS * LU_B;             // row panel: column c at rp + c LU_PS
+    double *U = lds + LU_PS * (2 * LU_B + LU_K); // packed U
+    double *ys = U + upk(N) + 2 * LU_B;          // right-hand side c at ys + c (N + 1)
+    const int t = threadIdx.x, tr = t >> 5, tc = t & 31;
+    const int wave = t >> 6, lane = t & 63;
+    double v[4][4], vr[4];
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const int c = tc + 32 * j;
-                        if (c >= p && c < N)
-                            ub[off + c] = v[ip][j];
-                    }
+    for (int i = 0; i < 4; i++) {
+        const int r = tr + 32 * i;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int c = tc + 32 * j;
+            v[i][j] = (r < N && c < N) ? lhs[(long)r * ldl + c] : (r == c ? 1.0 : 0.0);
+        }
+        vr[i] = (r < N && tc < k) ? rhs[(long)r * k + tc] : 0.0;
+    }
+    auto publish = [&](auto I, int q0) {
+        constexpr int ip = decltype(I)::value;
+        const int dr = tr - q0, dc = tc - q0;
+        if (dr >= 0 && dr < LU_P) {
+#pragma unroll
+            for (int j = ip; j < 4; j++)
+                rp[(tc + 32 * j) * LU_PS + dr] = v[ip][j];
+            if (k > 0)
+                rp[(LU_B + tc) * LU_PS + dr] = vr[ip];
+        }
+        if (dc >= 0 && dc < LU_P) {
+#pragma unroll
+            for (int i = ip; i < 4; i++)
+                cp[(tr + 32 * i) * LU_PS + dc] = v[i][ip];
+        }
+    };
+    // elements above or left of the next panel are final and stored: they take
+    // part here only because leaving them out would cost a test, and are not
+    // read again
+    auto update = [&](auto I) {
+        constexpr int ip = decltype(I)::value;
+#pragma unroll 1
+        for (int p = 0; p < LU_P; p += 2) {
+            double2 l[4];
+#pragma unroll
+            for (int i = ip; i < 4; i++)
+                l[i] = *(const double2 *)(cp + (tr + 32 * i) * LU_PS + p);
+#pragma unroll
+            for (int j = ip; j < 4; j++) {
+                const double2 u = *(const double2 *)(rp + (tc + 32 * j) * LU_PS + p);
+#pragma unroll
+                for (int i = ip; i < 4; i++) {
+                    v[i][j] = sub_rn(v[i][j], mul_rn(l[i].x, u.x));
+                    v[i][j] = sub_rn(v[i][j], mul_rn(l[i].y, u.y));
                 }
-                if (tc == pr) {
+            }
+            if (k > 0) {
+                const double2 u = *(const double2 *)(rp + (LU_B + tc) * LU_PS + p);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int r = tr + 32 * i;
-                        if (r > p && r < N)
-                            lb[off + r] = v[i][ip];
-                    }
+                for (int i = ip; i < 4; i++) {
+                    vr[i] = sub_rn(vr[i], mul_rn(l[i].x, u.x));
+                    vr[i] = sub_rn(vr[i], mul_rn(l[i].y, u.y));
                 }
-                __syncthreads();
-                const double piv = ub[off + p];
-                if (!(piv != 0.0 && isfinite(piv)))
+            }
+        }
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    publish(I0{}, 0);
+    __syncthreads();
+#pragma unroll 1
+    for (int P0 = 0; P0 < N; P0 += LU_P) {
+        const int P1 = P0 + LU_P;
+        // ---- 1: the panel
+        const int below = N - P1 > 0 ? N - P1 : 0;
+        const int nrw = below > 0 ? (below + 55) / 56 : 1;
+        const int ncw = (below + k + 55) / 56;
+        if (wave < nrw) {
+            const int r = lane < LU_P ? P0 + lane : P1 + wave * 56 + lane - LU_P;
+            const bool in = r < N;
+            double w[LU_P];
+#pragma unroll
+            for (int j = 0; j < LU_P; j++)
+                w[j] = cp[(r < LU_B ? r : 0) * LU_PS + j];
+            int bad = 0;
+#pragma unroll
+            for (int p = 0; p < LU_P; p++) {
+                const double piv = readlane_f64(w[p], p);
+                if (P0 + p < N && !(piv != 0.0 && isfinite(piv)))
                     bad = 1;
-                const double inv = ib[p & 1];
-                double u[4];
+                const double inv = 1.0 / piv;
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int c = tc + 32 * j;
-                    u[j] = (c > p && c < N) ? mul_rn(ub[off + c], inv) : 0.0;
+                for (int j = p + 1; j < LU_P; j++) {
+                    const double u = mul_rn(readlane_f64(w[j], p), inv);
+                    const double d = sub_rn(w[j], mul_rn(w[p], u));
+                    w[j] = lane > p ? d : (lane == p ? u : w[j]);
                 }
+            }
+            if (in && (lane >= LU_P || wave == 0)) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int r = tr + 32 * i;
-                    if (i == ip && tr == pr) {
-#pragma unroll
-                        for (int j = 0; j < 4; j++)
-                            if (tc + 32 * j > p && tc + 32 * j < N)
-                                v[i][j] = u[j];
-                    } else if (r > p && r < N) {
-                        const double l = lb[off + r];
-#pragma unroll
-                        for (int j = 0; j < 4; j++)
-                            if (tc + 32 * j > p && tc + 32 * j < N)
-                                v[i][j] = sub_rn(v[i][j], mul_rn(l, u[j]));
+                for (int j = 0; j < LU_P; j++) {
+                    if (lane >= LU_P)
+                        cp[r * LU_PS + j] = w[j];
+                    if (P0 + j < N) {
+                        gw[(long)r * ldg + P0 + j] = w[j];
+                        if (back && lane < j)
+                            U[upk(P0 + j) + r] = w[j];
                     }
                 }
             }
-        }
+            if (wave == 0 && lane == 0 && bad)
+                *flag = 1;
+        } else if (wave < nrw + ncw) {
+            // column: the panel's own, one to the right, or a right-hand side
+            const int e = (wave - nrw) * 56 + lane - LU_P;
+            const int c = lane < LU_P ? P0 + lane : (e < below ? P1 + e : LU_B + e - below);
+            const bool rh = lane >= LU_P && e >= below;
+            const bool in = lane >= LU_P && e < below + k;
+            double w[LU_P];
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+            for (int i = 0; i < LU_P; i++)
+                w[i] = rp[(in || lane < LU_P ? c : 0) * LU_PS + i];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int r = tr + 32 * i, c = tc + 32 * j;
-                if (r < N && c < N) {
-                    a[fidx<true>(N, r, c)] = v[i][j];
-                    gw[(long)r * N + c] = v[i][j];
+            for (int p = 0; p < LU_P; p++) {
+                const double inv = 1.0 / readlane_f64(w[p], p);
+                const double u = mul_rn(w[p], inv);
+                w[p] = lane > p ? u : w[p];
+#pragma unroll
+                for (int i = p + 1; i < LU_P; i++) {
+                    const double l = readlane_f64(w[i], p);
+                    const double d = sub_rn(w[i], mul_rn(l, u));
+                    w[i] = lane > p ? d : w[i];
                 }
             }
-        __syncthreads();
-    } else {
-        for (long e = t; e < (long)N * N; e += LU_T)
-            a[e] = lhs[e];
-        __syncthreads();
-        for (int p = 0; p < N; p++) {
-            const double piv = a[(long)p * N + p];
-            if (!(piv != 0.0 && isfinite(piv)))
-                bad = 1;
-            const double inv = 1.0 / piv;
-            for (int c = p + 1 + t; c < N; c += LU_T)
-                a[(long)p * N + c] = mul_rn(a[(long)p * N + c], inv);
-            __syncthreads();
-            const int w = N - p - 1;
-            // rows p+1.., one row per lane group of 64, columns strided by 64
-            for (int r = p + 1 + (t >> 6); r < N; r += LU_T / 64) {
-                const double l = a[(long)r * N + p];
-                for (int c = p + 1 + (t & 63); c < N; c += 64)
-                    a[(long)r * N + c] = sub_rn(a[(long)r * N + c], mul_rn(l, a[(long)p * N + c]));
-            }
-            (void)w;
-            __syncthreads();
-        }
-    }
-    if (t == 0 && bad)
-        *flag = 1;
-    // reciprocal diagonal of L for the forward pass (the reference's 1.0 / L_ii)
-    double *dinv = IN_LDS ? lds + (long)N * (N + 1) + 2 * kc + 512 + 2
-                          : rowbuf + 2 * kc + (long)N * kc;
-    for (int q = t; q < N; q += LU_T)
-        dinv[q] = 1.0 / a[fidx<IN_LDS>(N, q, q)];
-    __syncthreads();
-
-    if constexpr (IN_LDS) {
-        if (mode == CACG_MODE_FAST) {
-            if (k <= 16)
-                lu_subst_wave<64>(N, a, dinv, k, rhs, x);
-            else if (k <= 32)
-                lu_subst_wave<32>(N, a, dinv, k, rhs, x);
-            else if (k <= 64)
-                lu_subst_wave<16>(N, a, dinv, k, rhs, x);
-            else
-                lu_subst_wave<8>(N, a, dinv, k, rhs, x);
-            return;
-        }
-    }
-
-    // ---- substitutions, kc columns at a time
-    for (int c0 = 0; c0 < k; c0 += kc) {
-        const int kw = (k - c0) < kc ? (k - c0) : kc;
-        const int G = LU_T / kw;
-        const int cl = t % kw, g = t / kw;
-        const bool own = g < G;
-        if (IN_LDS && mode == CACG_MODE_REFERENCE && c0 > 0) {
-            // the previous chunk's backward pass reused the factor's LDS
-            for (long e = t; e < (long)N * N; e += LU_T)
-                a[fidx<true>(N, (int)(e / N), (int)(e % N))] = gw[e];
-            __syncthreads();
-        }
-        double y[JMAX];
+            if (in) {
 #pragma unroll
-        for (int j = 0; j < JMAX; j++) {
-            const int i = g + G * j;
-            y[j] = (own && i < N) ? rhs[(long)i * k + c0 + cl] : 0.0;
-        }
-        // forward: L y = rhs.  Row q = gq + G jq is owned by lane group gq as its
-        // register y[jq]; jq is a compile-time index.
-#pragma unroll
-        for (int jq = 0; jq < JMAX; jq++) {
-            for (int gq = 0; gq < G; gq++) {
-                const int q = gq + G * jq;
-                if (q >= N)
-                    break;
-                double *rb = rowbuf + (q & 1) * kc;
-                if (own && g == gq) {
-                    y[jq] = mul_rn(y[jq], dinv[q]);
-                    rb[cl] = y[jq];
-                }
-                __syncthreads();
-                if (own) {
-                    const double yq = rb[cl];
-#pragma unroll
-                    for (int j = jq; j < JMAX; j++) {
-                        const int i = g + G * j;
-                        if ((j > jq || g > gq) && i < N)
-                            y[j] = sub_rn(y[j], mul_rn(yq, a[fidx<IN_LDS>(N, i, q)]));
-                    }
-                }
-            }
-        }
-        if (mode == CACG_MODE_REFERENCE) {
-            __syncthreads();  // all reads of the factor's LDS done before xs overwrites it
-#pragma unroll
-            for (int j = 0; j < JMAX; j++) {
-                const int i = g + G * j;
-                if (own && i < N)
-                    xs[(long)i * kw + cl] = y[j];
-            }
-            __syncthreads();
-            if (t < kw) {
-                for (int i = N - 2; i >= 0; i--) {
-                    double xi = xs[(long)i * kw + t];
-                    const double *u = gw + (long)i * N;
-                    int q = i + 1;
-                    for (; q + 4 <= N; q += 4) {
-                        const double u0 = u[q], u1 = u[q + 1], u2 = u[q + 2], u3 = u[q + 3];
-                        xi = sub_rn(xi, mul_rn(xs[(long)q * kw + t], u0));
-                        xi = sub_rn(xi, mul_rn(xs[(long)(q + 1) * kw + t], u1));
-                        xi = sub_rn(xi, mul_rn(xs[(long)(q + 2) * kw + t], u2));
-                        xi = sub_rn(xi, mul_rn(xs[(long)(q + 3) * kw + t], u3));
-                    }
-                    for (; q < N; q++)
-                        xi = sub_rn(xi, mul_rn(xs[(long)q * kw + t], u[q]));
-                    xs[(long)i * kw + t] = xi;
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < JMAX; j++) {
-                const int i = g + G * j;
-                if (own && i < N)
-                    x[(long)i * k + c0 + cl] = xs[(long)i * kw + cl];
-            }
-            __syncthreads();
-        } else {
-            __syncthreads();  // the forward pass's last broadcast row is read before reuse
-#pragma unroll
-            for (int jq = JMAX - 1; jq >= 0; jq--) {
-                for (int gq = G - 1; gq >= 0; gq--) {
-                    const int q = gq + G * jq;
-                    if (q >= N)
+                for (int i = 0; i < LU_P; i++) {
+                    const int r = P0 + i;
+                    rp[c * LU_PS + i] = w[i];
+                    if (r >= N)
                         continue;
-                    double *rb = rowbuf + (q & 1) * kc;
-                    if (own && g == gq)
-                        rb[cl] = y[jq];
-                    __syncthreads();
-                    if (own) {
-                        const double xq = rb[cl];
-#pragma unroll
-                        for (int j = 0; j <= jq; j++) {
-                            const int i = g + G * j;
-                            if (j < jq || g < gq)
-                                y[j] = sub_rn(y[j], mul_rn(xq, a[fidx<IN_LDS>(N, i, q)]));
-                        }
+                    if (rh) {
+                        if (back)
+                            ys[(c - LU_B) * (N + 1) + r] = w[i];
+                        else
+                            x[(long)r * k + c - LU_B] = w[i];
+                    } else {
+                        gw[(long)r * ldg + c] = w[i];
+                        if (back)
+                            U[upk(c) + r] = w[i];
                     }
                 }
             }
-#pragma unroll
-            for (int j = 0; j < JMAX; j++) {
-                const int i = g + G * j;
-                if (own && i < N)
-                    x[(long)i * k + c0 + cl] = y[j];
-            }
-            __syncthreads();
         }
+        __syncthreads();
+        if (P1 >= N)
+            break;
+        // ---- 2: the trailing elements
+        switch (P0 / 32) {
+        case 0: update(I0{}); break;
+        case 1: update(I1{}); break;
+        case 2: update(I2{}); break;
+        default: update(I3{}); break;
+        }
+        __syncthreads();   // the panel has been read: the next one may be written
+        switch (P1 / 32) {
+        case 0: publish(I0{}, P1 % 32); break;
+        case 1: publish(I1{}, P1 % 32); break;
+        case 2: publish(I2{}, P1 % 32); break;
+        default: publish(I3{}, P1 % 32); break;
+        }
+        __syncthreads();
+    }
+    if (!back)
+        return;
+    __syncthreads();
+    for (int c = wave; c < k; c += LU_T / 64) {
+        double *y = ys + c * (N + 1);
+        double y0 = y[lane < N ? lane : 0], y1 = y[64 + lane < N ? 64 + lane : 0];
+        tri_backward(N, [&](int q) { return (const double *)(U + upk(q)); }, y0, y1);
+        if (lane < N)
+            x[(long)lane * k + c] = y0;
+        if (64 + lane < N)
+            x[(long)(64 + lane) * k + c] = y1;
     }
 }
 
-template <bool IN_LDS>
-__global__ __launch_bounds__(LU_T) void lu_solve_kernel(int N, const double *__restrict__ lhs, int k,
-                                                        const double *__restrict__ rhs,
-                                                        double *__restrict__ x,
-                                                        double *__restrict__ gw, int *flag,
-                                                        int mode, int kc, int reuse)
+__global__ __launch_bounds__(LU_T) void lu_factor_kernel(int N, const double *lhs, long ldl,
+                                                         double *gw, long ldg, int k,
+                                                         const double *__restrict__ rhs,
+                                                         double *__restrict__ x, int *flag,
+                                                         int back)
 {
     extern __shared__ double lds[];
-    lu_solve_body<IN_LDS>(N, lhs, k, rhs, x, gw, flag, mode, kc, reuse, lds);
+    lu_factor_body(N, lhs, ldl, gw, ldg, k, rhs, x, flag, back != 0, lds);
 }
 
-// The fast-order solve with a kept factor (N <= 128), spread over workgroups of
-// LU_SUB_W waves: wave w of workgroup b solves column LU_SUB_W b + w (64 lanes,
-// 2 rows each), with its own LDS copy of the factor (gw, N x N row-major).
-// The single-workgroup solve ran every column on one CU, whose LDS served the
-// factor to all of them step after step (~106 us for 128 columns); per element
-// the operations are those of lu_subst_wave in its order, so the bits are the
-// same whichever lanes and workgroup solve a column.
-constexpr int LU_SUB_W = 4;
-__global__ __launch_bounds__(LU_SUB_W * 64) void lu_subst_multi_kernel(int N,
-                                                                      const double *__restrict__ gw,
-                                                                      int k,
-                                                                      const double *__restrict__ rhs,
-                                                                      double *__restrict__ x)
+// ---- triangular solves with a kept factor block -----------------------------------
+
+// A set of vectors: entry i of vector v at in / out + v vs + i es
+struct TriSet {
+    const double *in;
+    double *out;
+    long vs, es;
+    int count;
+    int kind;
+};
+enum { TRI_FORWARD = 1, TRI_BACKWARD = 2, TRI_UT = 4 };
+
+__host__ __device__ inline int tri_lds(int nb) { return (nb + 1) * (nb + 1) + LU_B; }
+
+// Vectors first .. of a set, one per wave and step, by the nb x nb factor block at
+// F (row stride ldf): kind FORWARD: L y = v; FORWARD | BACKWARD: then U x = y
+// (descending pivots); BACKWARD alone: U x = v; UT: y U = v (rows of L left of
+// the block: ascending pivots, unit diagonal).  The block is copied to LDS
+// first, column by column (UT: row by row) with the odd stride nb + 1, so the
+// multipliers of a step lie in consecutive words.
+__device__ __forceinline__ void tri_body(int nb, const double *F, long ldf, const TriSet &s,
+                                         int first, int step, double *lds)
+{
+    const int t = threadIdx.x, R = nb + 1;
+    const int w = t >> 6, l = t & 63;
+    const bool ut = s.kind == TRI_UT;
+    // a wave copies rows w, w + TRI_W, ...: 64 columns a load, 8 rows in flight
+    for (int r0 = w; r0 < nb; r0 += 8 * TRI_W) {
+        double f[8][2];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int r = r0 + u * TRI_W;
+            const double *p = F + (long)(r < nb ? r : 0) * ldf;
+            f[u][0] = l < nb ? p[l] : 0.0;
+            f[u][1] = 64 + l < nb ? p[64 + l] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int r = r0 + u * TRI_W;
+            if (r >= nb)
+                continue;
+            if (l < nb)
+                lds[ut ? r * R + l : l * R + r] = f[u][0];
+            if (64 + l < nb)
+                lds[ut ? r * R + 64 + l : (64 + l) * R + r] = f[u][1];
+        }
+    }
+    __syncthreads();
+    const int i0 = l < nb ? l : 0, i1 = 64 + l < nb ? 64 + l : 0;
+    const double d0 = 1.0 / lds[i0 * R + i0], d1 = 1.0 / lds[i1 * R + i1];
+    auto T = [&](int q) { return (const double *)(lds + q * R); };
+    for (int v = first + w; v < s.count; v += step) {
+        const double *p = s.in + v * s.vs;
+        double y0 = p[i0 * s.es], y1 = p[i1 * s.es];
+        if (ut)
+            tri_forward<false>(nb, T, d0, d1, y0, y1);
+        else if (s.kind & TRI_FORWARD)
+            tri_forward<true>(nb, T, d0, d1, y0, y1);
+        if (s.kind & TRI_BACKWARD)
+            tri_backward(nb, T, y0, y1);
+        double *o = s.out + v * s.vs;
+        if (l < nb)
+            o[i0 * s.es] = y0;
+        if (64 + l < nb)
+            o[i1 * s.es] = y1;
+    }
+}
+
+// workgroups of a set: TRI_W vectors each
+__host__ __device__ inline int tri_groups(int count) { return (count + TRI_W - 1) / TRI_W; }
+
+__global__ __launch_bounds__(TRI_W * 64) void lu_tri_kernel(int nb, const double *F, long ldf,
+                                                            TriSet s0, TriSet s1, TriSet s2)
 {
     extern __shared__ double lds[];
-    double *a = lds;                          // N x N, column-major, stride N + 1
-    double *dinv = lds + (long)N * (N + 1);   // reciprocal diagonal
-    for (long e = threadIdx.x; e < (long)N * N; e += LU_SUB_W * 64)
-        a[fidx<true>(N, (int)(e / N), (int)(e % N))] = gw[e];
-    __syncthreads();
-    for (int q = threadIdx.x; q < N; q += LU_SUB_W * 64)
-        dinv[q] = 1.0 / a[fidx<true>(N, q, q)];
-    __syncthreads();
-    lu_subst_wave<64>(N, a, dinv, k, rhs, x, LU_SUB_W * blockIdx.x, LU_SUB_W * gridDim.x);
+    int g = blockIdx.x;
+    if (g < tri_groups(s0.count)) {
+        tri_body(nb, F, ldf, s0, g * TRI_W, s0.count, lds);
+    } else if ((g -= tri_groups(s0.count)) < tri_groups(s1.count)) {
+        tri_body(nb, F, ldf, s1, g * TRI_W, s1.count, lds);
+    } else {
+        g -= tri_groups(s1.count);
+        tri_body(nb, F, ldf, s2, g * TRI_W, s2.count, lds);
+    }
 }
 
-// batched: workgroup b solves system items[b].x (N = sm <= 128, factor in LDS);
-// which 0: beta = QtAQ^{-1} QtAS with the factor kept from the last alpha solve,
-// which 1: alpha = QtAQ^{-1} QtR, factoring QtAQ
-__global__ __launch_bounds__(LU_T) void lu_batch_kernel(const cacg_bsys *__restrict__ sys,
-                                                        const int2 *__restrict__ items, int which)
+// ---- block products ---------------------------------------------------------------
+
+// out = in - A B for an M x K block, A M x nb and B nb x K, nb <= 128: each
+// element subtracts its products one after the other, q ascending (or, `desc`,
+// descending), rounded separately.  A workgroup takes 32 x 32 elements, 2 x 2 a
+// lane, its 32 rows of A and 32 columns of B in LDS.
+struct MulSet {
+    const double *A, *B, *in;
+    double *out;
+    long lda, ldb, ldi, ldo;
+    int M, K;
+};
+
+__global__ __launch_bounds__(256) void lu_mul_kernel(int nb, MulSet s0, MulSet s1, int g0,
+                                                     int desc)
+{
+    __shared__ double sa[LU_B][33], sb[LU_B][33];
+    const MulSet &s = (int)blockIdx.x < g0 ? s0 : s1;
+    const int g = (int)blockIdx.x < g0 ? blockIdx.x : blockIdx.x - g0;
+    const int gk = (s.K + 31) / 32;
+    const int r0 = g / gk * 32, c0 = g % gk * 32;
+    const int t = threadIdx.x;
+    for (int e = t; e < 32 * nb; e += 256) {
+        const int r = e / nb, q = e % nb;
+        sa[q][r] = r0 + r < s.M ? s.A[(long)(r0 + r) * s.lda + q] : 0.0;
+    }
+    for (int e = t; e < 32 * nb; e += 256) {
+        const int q = e / 32, c = e % 32;
+        sb[q][c] = c0 + c < s.K ? s.B[(long)q * s.ldb + c0 + c] : 0.0;
+    }
+    const int tr = t / 16, tc = t % 16;
+    double v[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int r = r0 + tr + 16 * i, c = c0 + tc + 16 * j;
+            v[i][j] = r < s.M && c < s.K ? s.in[(long)r * s.ldi + c] : 0.0;
+        }
+    __syncthreads();
+#pragma unroll 4
+    for (int e = 0; e < nb; e++) {
+        const int q = desc ? nb - 1 - e : e;
+        const double a0 = sa[q][tr], a1 = sa[q][tr + 16], b0 = sb[q][tc], b1 = sb[q][tc + 16];
+        v[0][0] = sub_rn(v[0][0], mul_rn(a0, b0));
+        v[0][1] = sub_rn(v[0][1], mul_rn(a0, b1));
+        v[1][0] = sub_rn(v[1][0], mul_rn(a1, b0));
+        v[1][1] = sub_rn(v[1][1], mul_rn(a1, b1));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int r = r0 + tr + 16 * i, c = c0 + tc + 16 * j;
+            if (r < s.M && c < s.K)
+                s.out[(long)r * s.ldo + c] = v[i][j];
+        }
+}
+
+__global__ __launch_bounds__(256) void lu_copy_kernel(long count, const double *__restrict__ src,
+                                                      double *__restrict__ dst)
+{
+    for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < count; e += (long)gridDim.x * 256)
+        dst[e] = src[e];
+}
+
+// ---- the reference's backward substitution ------------------------------------------
+
+// x_i = y_i - sum of x_q u_iq, q = i + 1, i + 2, ... subtracted in that order: row
+// i can only start once x_{i+1} is known, so a column is one chain of
+// N (N - 1) / 2 dependent subtractions.  One wave per workgroup, a lane per
+// column (cw of them); the columns lie in LDS, entry q of lane c at c S + q with S
+// even and S / 2 odd, so two entries come with one 16-byte read; u_iq is the same
+// for all lanes (scalar loads).  In place on x.
+__global__ __launch_bounds__(64) void lu_back_ref_kernel(int N, const double *__restrict__ gw,
+                                                         int k, double *__restrict__ x, int cw)
+{
+    extern __shared__ double xs[];
+    const int S = (N + 1) / 2 * 2 + ((N + 1) / 2 % 2 == 0 ? 2 : 0);
+    const int c0 = blockIdx.x * cw, t = threadIdx.x;
+    const int kw = k - c0 < cw ? k - c0 : cw;
+    for (long e = t; e < (long)N * kw; e += 64)
+        xs[e % kw * S + e / kw] = x[e / kw * k + c0 + e % kw];
+    __syncthreads();
+    const int c = t < kw ? t : 0;
+    double *col = xs + (long)c * S;
+    for (int i = N - 2; i >= 0; i--) {
+        const double *u = gw + (long)i * N;
+        double xi = col[i];
+        int q = i + 1;
+        if (q & 1) {
+            xi = sub_rn(xi, mul_rn(col[q], u[q]));
+            q++;
+        }
+        for (; q + 16 <= N; q += 16) {
+            double2 w[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                w[e] = *(const double2 *)(col + q + 2 * e);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                xi = sub_rn(xi, mul_rn(w[e].x, u[q + 2 * e]));
+                xi = sub_rn(xi, mul_rn(w[e].y, u[q + 2 * e + 1]));
+            }
+        }
+        for (; q < N; q++)
+            xi = sub_rn(xi, mul_rn(col[q], u[q]));
+        if (t < kw)
+            col[i] = xi;
+    }
+    __syncthreads();
+    for (long e = t; e < (long)N * kw; e += 64)
+        x[e / kw * k + c0 + e % kw] = xs[e % kw * S + e / kw];
+}
+
+// ---- batched ------------------------------------------------------------------------
+
+// workgroup b factors system items[b].x (N = sm <= 128, m <= 32): alpha = QtAQ^{-1} QtR
+__global__ __launch_bounds__(LU_T) void lu_batch_alpha_kernel(const cacg_bsys *__restrict__ sys,
+                                                              const int2 *__restrict__ items)
 {
     extern __shared__ double lds[];
     const cacg_bsys &d = sys[items[blockIdx.x].x];
-    const int N = d.sm, k = which == 0 ? d.sm : d.m;
-    const int kc = lu_columns(N, k, true);
-    lu_solve_body<true>(N, d.QtAQ, k, which == 0 ? d.QtAS : d.QtR, which == 0 ? d.beta : d.alpha,
-                        d.lu, d.flag, CACG_MODE_FAST, kc, which == 0 ? 1 : 0, lds);
+    lu_factor_body(d.sm, d.QtAQ, d.sm, d.lu, d.sm, d.m, d.QtR, d.alpha, d.flag, true, lds);
+}
+
+// beta = QtAQ^{-1} QtAS with the factor kept from the last alpha solve; workgroup
+// (b, y) takes columns TRI_W y .., in steps of TRI_W gridDim.y
+__global__ __launch_bounds__(TRI_W * 64) void lu_batch_beta_kernel(
+    const cacg_bsys *__restrict__ sys, const int2 *__restrict__ items)
+{
+    extern __shared__ double lds[];
+    const cacg_bsys &d = sys[items[blockIdx.x].x];
+    if ((int)blockIdx.y * TRI_W >= d.sm)
+        return;
+    const TriSet s = {d.QtAS, d.beta, 1, d.sm, d.sm, TRI_FORWARD | TRI_BACKWARD};
+    tri_body(d.sm, d.lu, d.sm, s, blockIdx.y * TRI_W, TRI_W * gridDim.y, lds);
+}
+
+int launch_factor(int N, const double *lhs, long ldl, double *gw, long ldg, int k,
+                  const double *rhs, double *x, int *flag, int back, hipStream_t st)
+{
+    const size_t shm = (size_t)lu_factor_lds(N, k, back != 0) * sizeof(double);
+    cacg_allow_lds(lu_factor_kernel, shm);
+    hipLaunchKernelGGL(lu_factor_kernel, dim3(1), dim3(LU_T), shm, st, N, lhs, ldl, gw, ldg, k,
+                       rhs, x, flag, back);
+    CACG_LAUNCH_CHECK();
+    return 0;
+}
+
+const TriSet TRI_NONE = {nullptr, nullptr, 0, 0, 0, 0};
+
+int launch_tri(int nb, const double *F, long ldf, const TriSet &a, const TriSet &b,
+               const TriSet &c, hipStream_t st)
+{
+    const int G = tri_groups(a.count) + tri_groups(b.count) + tri_groups(c.count);
+    if (G == 0)
+        return 0;
+    const size_t shm = (size_t)tri_lds(nb) * sizeof(double);
+    cacg_allow_lds(lu_tri_kernel, shm);
+    hipLaunchKernelGGL(lu_tri_kernel, dim3(G), dim3(TRI_W * 64), shm, st, nb, F, ldf, a, b, c);
+    CACG_LAUNCH_CHECK();
+    return 0;
+}
+
+int launch_mul(int nb, const MulSet &a, const MulSet &b, int desc, hipStream_t st)
+{
+    const int ga = (a.M + 31) / 32 * ((a.K + 31) / 32), gb = (b.M + 31) / 32 * ((b.K + 31) / 32);
+    if (ga + gb == 0)
+        return 0;
+    hipLaunchKernelGGL(lu_mul_kernel, dim3(ga + gb), dim3(256), 0, st, nb, a, b, ga, desc);
+    CACG_LAUNCH_CHECK();
+    return 0;
+}
+
+#define LU_TRY(call)                                                                              \
+    do {                                                                                          \
+        const int rc_ = (call);                                                                   \
+        if (rc_)                                                                                  \
+            return rc_;                                                                           \
+    } while (0)
+
+// N > 128 in blocks of 128.  Right-looking, so each element receives its
+// subtractions in ascending order of the pivot, block after block.  `factor`:
+// factor first, the right-hand sides (fewer columns of the same steps) along
+// with it; else the factor is in gw.  In x afterwards: y = L^{-1} rhs for a
+// reference-order backward pass (`back` false), or x.
+int lu_blocked(int N, int k, const double *rhs, double *x, double *gw, int *flag, bool factor,
+               bool back, hipStream_t st)
+{
+    for (int p = 0; p < N; p += LU_B) {
+        const int nb = N - p < LU_B ? N - p : LU_B, rest = N - p - nb, e = p + nb;
+        double *F = gw + (long)p * N + p;
+        // the first block's right-hand side rows come from rhs, later ones have
+        // been updated into x
+        const double *in = p == 0 ? rhs : x + (long)p * k;
+        double *xp = x + (long)p * k;
+        // the last block's backward pass follows its forward pass
+        const int kind = TRI_FORWARD | (back && rest == 0 ? TRI_BACKWARD : 0);
+        if (factor)
+            LU_TRY(launch_factor(nb, F, N, F, N, 0, nullptr, nullptr, flag, 0, st));
+        const TriSet y = {in, xp, 1, k, k, kind};
+        const TriSet u = {gw + (long)p * N + e, gw + (long)p * N + e, 1, N, rest, TRI_FORWARD};
+        const TriSet l = {gw + (long)e * N + p, gw + (long)e * N + p, N, 1, rest, TRI_UT};
+        LU_TRY(launch_tri(nb, F, N, y, factor ? u : TRI_NONE, factor ? l : TRI_NONE, st));
+        if (rest == 0)
+            break;
+        double *L = gw + (long)e * N + p, *A = gw + (long)e * N + e;
+        const double *rin = p == 0 ? rhs + (long)e * k : x + (long)e * k;
+        const MulSet ry = {L, xp, rin, x + (long)e * k, N, k, k, k, rest, k};
+        MulSet ra = {L, gw + (long)p * N + e, A, A, N, N, N, N, rest, rest};
+        if (!factor)
+            ra.M = ra.K = 0;
+        LU_TRY(launch_mul(nb, ry, ra, 0, st));
+    }
+    if (!back)
+        return 0;
+    for (int p = (N - 1) / LU_B * LU_B; p > 0; p -= LU_B) {
+        // x above block p subtracts U(:, block) x(block), then the block above it
+        const int nb = N - p < LU_B ? N - p : LU_B;
+        const MulSet up = {gw + p, x + (long)p * k, x, x, N, k, k, k, p, k};
+        LU_TRY(launch_mul(nb, up, MulSet{}, 1, st));
+        const int q = p - LU_B;
+        const TriSet b = {x + (long)q * k, x + (long)q * k, 1, k, k, TRI_BACKWARD};
+        LU_TRY(launch_tri(LU_B, gw + (long)q * N + q, N, b, TRI_NONE, TRI_NONE, st));
+    }
+    return 0;
 }
 
 }  // namespace
@@ -493,9 +736,17 @@ extern "C" int cacg_k_lu_batch(const cacg_bsys *d_sys, const int2 *d_items, int 
         return 0;
     if (max_sm <= 0 || max_sm > 128 || (which != 0 && which != 1))
         return (int)hipErrorInvalidValue;
-    const size_t shm = lu_lds_bytes(max_sm, max_sm, true);
-    cacg_allow_lds(lu_batch_kernel, shm);
-    hipLaunchKernelGGL(lu_batch_kernel, dim3(count), dim3(LU_T), shm, st, d_sys, d_items, which);
+    if (which == 1) {
+        const size_t shm = (size_t)lu_factor_lds(max_sm, LU_K, true) * sizeof(double);
+        cacg_allow_lds(lu_batch_alpha_kernel, shm);
+        hipLaunchKernelGGL(lu_batch_alpha_kernel, dim3(count), dim3(LU_T), shm, st, d_sys,
+                           d_items);
+    } else {
+        const size_t shm = (size_t)tri_lds(max_sm) * sizeof(double);
+        cacg_allow_lds(lu_batch_beta_kernel, shm);
+        hipLaunchKernelGGL(lu_batch_beta_kernel, dim3(count, (max_sm + 15) / 16),
+                           dim3(TRI_W * 64), shm, st, d_sys, d_items);
+    }
     CACG_LAUNCH_CHECK();
     return 0;
 }
@@ -504,30 +755,37 @@ extern "C" int cacg_k_lu_solve(int N, const double *lhs, int k, const double *rh
                                double *d_work, int *d_flag, int mode, int reuse_factor,
                                hipStream_t st)
 {
-    if (N <= 0 || k <= 0)
+    if (N <= 0 || k <= 0 || N > 16384)
         return (int)hipErrorInvalidValue;
-    const bool in_lds = (long)N * N <= 128L * 128L;
-    const int kc = lu_columns(N, k, in_lds);
-    if (kc < 1)
-        return (int)hipErrorInvalidValue;  // N > 16384 is out of range
-    if (in_lds && mode == CACG_MODE_FAST && reuse_factor) {
-        // the kept factor: one column per wave over as many workgroups as it takes
-        const size_t sub = ((size_t)N * (N + 1) + N) * sizeof(double);
-        const int G = (k + LU_SUB_W - 1) / LU_SUB_W;
-        cacg_allow_lds(lu_subst_multi_kernel, sub);
-        hipLaunchKernelGGL(lu_subst_multi_kernel, dim3(G), dim3(LU_SUB_W * 64), sub, st, N, d_work,
-                           k, rhs, x);
-        CACG_LAUNCH_CHECK();
-        return 0;
+    const bool fast = mode == CACG_MODE_FAST;
+    const bool factor = !reuse_factor;
+    if (N <= LU_B) {
+        const bool along = factor && k <= LU_K;   // the right-hand sides with the factorisation
+        if (factor)
+            LU_TRY(launch_factor(N, lhs, N, d_work, N, along ? k : 0, rhs, x, d_flag,
+                                 along && fast, st));
+        if (!along) {
+            const TriSet s = {rhs, x, 1, k, k, TRI_FORWARD | (fast ? TRI_BACKWARD : 0)};
+            LU_TRY(launch_tri(N, d_work, N, s, TRI_NONE, TRI_NONE, st));
+        }
+    } else {
+        if (factor) {
+            hipLaunchKernelGGL(lu_copy_kernel, dim3(cacg_grid((long)N * N, 256, 1024)), dim3(256),
+                               0, st, (long)N * N, lhs, d_work);
+            CACG_LAUNCH_CHECK();
+        }
+        LU_TRY(lu_blocked(N, k, rhs, x, d_work, d_flag, factor, fast, st));
     }
-    const size_t shm = lu_lds_bytes(N, k, in_lds);
-    cacg_allow_lds(in_lds ? lu_solve_kernel<true> : lu_solve_kernel<false>, shm);
-    if (in_lds)
-        hipLaunchKernelGGL(lu_solve_kernel<true>, dim3(1), dim3(LU_T), shm, st, N, lhs, k, rhs, x,
-                           d_work, d_flag, mode, kc, reuse_factor);
-    else
-        hipLaunchKernelGGL(lu_solve_kernel<false>, dim3(1), dim3(LU_T), shm, st, N, lhs, k, rhs, x,
-                           d_work, d_flag, mode, kc, reuse_factor);
-    CACG_LAUNCH_CHECK();
+    if (!fast) {
+        // columns per workgroup: 16, fewer where N x 16 doubles exceed 128 KiB
+        const int S = N + 3;
+        int cw = 16384 / S;
+        cw = cw > 16 ? 16 : cw < 1 ? 1 : cw;
+        const size_t shm = (size_t)cw * S * sizeof(double);
+        cacg_allow_lds(lu_back_ref_kernel, shm);
+        hipLaunchKernelGGL(lu_back_ref_kernel, dim3((k + cw - 1) / cw), dim3(64), shm, st, N,
+                           d_work, k, x, cw);
+        CACG_LAUNCH_CHECK();
+    }
     return 0;
 }
