@@ -52,6 +52,25 @@ __device__ __forceinline__ void load_row(const T *p, double *out)
     }
 }
 
+// the first `have` of K consecutive values of a row, zeros after them; VEC 2:
+// 16-byte loads (p 16-byte aligned, `have` even)
+template <typename T, int K, int VEC>
+__device__ __forceinline__ void load_row_part(const T *p, int have, double *out)
+{
+#pragma unroll
+    for (int u = 0; u < K; u += VEC) {
+        if constexpr (VEC == 2) {
+            double2 w = {0.0, 0.0};
+            if (u < have)
+                w = *reinterpret_cast<const double2 *>(p + u);
+            out[u] = w.x;
+            out[u + 1] = w.y;
+        } else {
+            out[u] = u < have ? (double)p[u] : 0.0;
+        }
+    }
+}
+
 // ---- reference order ----------------------------------------------------------
 
 // RPT > 1 (sm divides 256): a thread updates RPT rows of one column, rows
@@ -753,6 +772,157 @@ __global__ __launch_bounds__(256) void xrupdate_mfma_kernel(int n, int m, const 
     }
 }
 
+// Q = S - Qin beta for any width sm <= SM (SM the next multiple of 16): the
+// scheme of qupdate_mfma_kernel with beta zero-padded to SM x SM in LDS and the
+// operand rows zero-padded in registers.  Qin (row stride ldi) may be Q itself:
+// a wave has read its 16 rows before it writes them.  S may be null (zero).
+// VEC 2: sm and ldi even, Qin 16-byte aligned (16-byte loads).
+// Bound by memory: three blocks of n sm values, and at n = 250,047, sm = 60 the
+// MFMAs take a fifth of that time.  Before, these widths took the
+// reference-order kernel, whose every product reads LDS twice.
+template <typename TS, int SM, int VEC>
+__global__ __launch_bounds__(256) void qupdate_pad_kernel(int n, int sm, const TS *__restrict__ S,
+                                                          const double *Qin, long ldi, double *Q,
+                                                          const double *__restrict__ beta)
+{
+    constexpr int KQ = SM / 4, NTL = SM / 16;
+    extern __shared__ double bl[];
+    for (int e = threadIdx.x; e < SM * SM; e += 256) {
+        const int k = e / SM, c = e % SM;
+        bl[e] = k < sm && c < sm ? beta[k * sm + c] : 0.0;
+    }
+    __syncthreads();
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int lg = lane >> 4, lc = lane & 15;
+    const int have = sm - lg * KQ;
+    const int ntiles = (n + 15) / 16, nw = gridDim.x * 4;
+    const int wid = xcd_remap(blockIdx.x, gridDim.x) * 4 + wave;
+    const int per = (ntiles + nw - 1) / nw;
+    const int tb = wid * per, te = tb + per < ntiles ? tb + per : ntiles;
+    double av[KQ];
+    auto load = [&](int tile) {
+        const long row = (long)tile * 16 + lc;
+        load_row_part<double, KQ, VEC>(Qin + (row < n ? row : n - 1) * ldi + lg * KQ, have, av);
+    };
+    if (tb < te)
+        load(tb);
+    for (int tile = tb; tile < te; tile++) {
+        const long i0 = (long)tile * 16;
+        TS sv[NTL][4];
+#pragma unroll
+        for (int j = 0; j < NTL; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const long i = i0 + lg + 4 * r;
+                const int c = j * 16 + lc;
+                sv[j][r] = S && i < n && c < sm ? S[i * sm + c] : (TS)0;
+            }
+#pragma unroll
+        for (int j = 0; j < NTL; j++) {
+            asm volatile("" ::: "memory");   // each tile's beta reads after the last one's MFMAs
+            const double *bcol = bl + (lg * KQ) * SM + j * 16 + lc;
+            const dbl4 acc = mfma_chain_lds<KQ>(av, bcol, SM, dbl4{0.0, 0.0, 0.0, 0.0});
+            const int c = j * 16 + lc;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const long i = i0 + lg + 4 * r;
+                if (i < n && c < sm)
+                    Q[i * sm + c] = (double)sv[j][r] - acc[r];
+            }
+        }
+        if (tile + 1 < te)
+            load(tile + 1);
+    }
+}
+
+// X += Q alpha, R -= AQ alpha and the column norms of the new R for any width
+// sm <= SM, as xrupdate_mfma_kernel with zero-padded operands
+template <int SM, int NTM, int VEC>
+__global__ __launch_bounds__(256) void xrupdate_pad_kernel(int n, int sm, int m,
+                                                           const double *__restrict__ Q,
+                                                           const double *__restrict__ AQ,
+                                                           const double *__restrict__ alpha,
+                                                           double *__restrict__ X,
+                                                           double *__restrict__ R,
+                                                           double *__restrict__ part)
+{
+    constexpr int KQ = SM / 4;
+    __shared__ double red[4][64][NTM];
+    __shared__ double s_alf[SM][16 * NTM];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int lg = lane >> 4, lc = lane & 15;
+    for (int e = threadIdx.x; e < SM * 16 * NTM; e += 256) {
+        const int k = e / (16 * NTM), c = e % (16 * NTM);
+        s_alf[k][c] = k < sm && c < m ? alpha[(long)k * m + c] : 0.0;
+    }
+    __syncthreads();
+    const int have = sm - lg * KQ;
+    double nrm[NTM];
+#pragma unroll
+    for (int j = 0; j < NTM; j++)
+        nrm[j] = 0.0;
+    const int nw = gridDim.x * 4;
+    const int wid = xcd_remap(blockIdx.x, gridDim.x) * 4 + wave;
+    const int ntiles = (n + 15) / 16;
+    const int per = (ntiles + nw - 1) / nw;
+    const int tb = wid * per, te = tb + per < ntiles ? tb + per : ntiles;
+    for (int tile = tb; tile < te; tile++) {
+        asm volatile("" ::: "memory");   // alpha is read again for every tile
+        const long i0 = (long)tile * 16;
+        const long row = i0 + lc < n ? i0 + lc : (long)n - 1;
+        double av[KQ], aq[KQ];
+        load_row_part<double, KQ, VEC>(Q + row * sm + lg * KQ, have, av);
+        load_row_part<double, KQ, VEC>(AQ + row * sm + lg * KQ, have, aq);
+        double xo[NTM][4], ro[NTM][4];
+#pragma unroll
+        for (int j = 0; j < NTM; j++) {
+            const int c = j * 16 + lc;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const long i = i0 + lg + 4 * r;
+                const bool in = c < m && i < n;
+                xo[j][r] = in ? X[i * m + c] : 0.0;
+                ro[j][r] = in ? R[i * m + c] : 0.0;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NTM; j++) {
+            dbl4 ax = {0.0, 0.0, 0.0, 0.0}, ar = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int tt = 0; tt < KQ; tt++) {
+                const double b = s_alf[lg * KQ + tt][j * 16 + lc];
+                ax = mfma16x16x4(av[tt], b, ax);
+                ar = mfma16x16x4(aq[tt], b, ar);
+            }
+            const int c = j * 16 + lc;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const long i = i0 + lg + 4 * r;
+                if (c < m && i < n) {
+                    X[i * m + c] = xo[j][r] + ax[r];
+                    const double rn = ro[j][r] - ar[r];
+                    R[i * m + c] = rn;
+                    nrm[j] += rn * rn;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NTM; j++)
+        red[wave][lane][j] = nrm[j];
+    __syncthreads();
+    if (threadIdx.x < NTM * 16) {
+        const int j = threadIdx.x / 16, l = threadIdx.x % 16;
+        const int c = j * 16 + l;
+        double acc = 0.0;
+        for (int w = 0; w < 4; w++)
+            for (int g = 0; g < 4; g++)
+                acc += red[w][g * 16 + l][j];
+        if (c < m)
+            part[(long)blockIdx.x * m + c] = acc;
+    }
+}
+
 // per-block partial column norms of a row-major n x m block (fast order)
 __global__ __launch_bounds__(256) void colnorm2_part_kernel(int n, int m, const double *__restrict__ R,
                                                            double *__restrict__ part)
@@ -844,6 +1014,68 @@ int launch_xrupdate_mfma(int n, int m, const T *Q, const T *AQ, const double *al
     return 0;
 }
 
+// workgroups of qupdate_pad_kernel: as many as are resident at once (4 waves each; LDS
+// holds beta once per workgroup)
+template <typename TS, int SM>
+int launch_qupdate_pad(int n, int sm, const TS *S, const double *Qin, long ldi, double *Q,
+                       const double *beta, hipStream_t st)
+{
+    const size_t shm = (size_t)SM * SM * sizeof(double);
+    const int ntiles = (n + 15) / 16;
+    const int perCU = SM <= 64 ? 4 : SM <= 96 ? 2 : 1;
+    int G = (ntiles + 3) / 4;
+    if (G > 256 * perCU)
+        G = 256 * perCU;
+    if (G >= 8)
+        G &= ~7;
+    if (sm % 2 == 0 && ldi % 2 == 0 && (uintptr_t)Qin % 16 == 0) {
+        cacg_allow_lds(qupdate_pad_kernel<TS, SM, 2>, shm);
+        hipLaunchKernelGGL((qupdate_pad_kernel<TS, SM, 2>), dim3(G), dim3(256), shm, st, n, sm, S,
+                           Qin, ldi, Q, beta);
+    } else {
+        cacg_allow_lds(qupdate_pad_kernel<TS, SM, 1>, shm);
+        hipLaunchKernelGGL((qupdate_pad_kernel<TS, SM, 1>), dim3(G), dim3(256), shm, st, n, sm, S,
+                           Qin, ldi, Q, beta);
+    }
+    CACG_LAUNCH_CHECK();
+    return 0;
+}
+
+template <typename TS>
+int qupdate_pad(int n, int sm, const TS *S, const double *Qin, long ldi, double *Q,
+                const double *beta, hipStream_t st)
+{
+    switch ((sm + 15) / 16) {
+    case 1: return launch_qupdate_pad<TS, 16>(n, sm, S, Qin, ldi, Q, beta, st);
+    case 2: return launch_qupdate_pad<TS, 32>(n, sm, S, Qin, ldi, Q, beta, st);
+    case 3: return launch_qupdate_pad<TS, 48>(n, sm, S, Qin, ldi, Q, beta, st);
+    case 4: return launch_qupdate_pad<TS, 64>(n, sm, S, Qin, ldi, Q, beta, st);
+    case 5: return launch_qupdate_pad<TS, 80>(n, sm, S, Qin, ldi, Q, beta, st);
+    case 6: return launch_qupdate_pad<TS, 96>(n, sm, S, Qin, ldi, Q, beta, st);
+    case 7: return launch_qupdate_pad<TS, 112>(n, sm, S, Qin, ldi, Q, beta, st);
+    case 8: return launch_qupdate_pad<TS, 128>(n, sm, S, Qin, ldi, Q, beta, st);
+    default: return (int)hipErrorInvalidValue;
+    }
+}
+
+template <int SM, int NTM>
+int launch_xrupdate_pad(int n, int sm, int m, const double *Q, const double *AQ,
+                        const double *alpha, double *X, double *R, double *d_norm2, double *work,
+                        hipStream_t st)
+{
+    if (sm % 2 == 0 && ((uintptr_t)Q | (uintptr_t)AQ) % 16 == 0)
+        hipLaunchKernelGGL((xrupdate_pad_kernel<SM, NTM, 2>), dim3(XR_BLOCKS), dim3(256), 0, st, n,
+                           sm, m, Q, AQ, alpha, X, R, work);
+    else
+        hipLaunchKernelGGL((xrupdate_pad_kernel<SM, NTM, 1>), dim3(XR_BLOCKS), dim3(256), 0, st, n,
+                           sm, m, Q, AQ, alpha, X, R, work);
+    CACG_LAUNCH_CHECK();
+    hipLaunchKernelGGL(colnorm2_final_kernel, dim3(m), dim3(256), 0, st, work, XR_BLOCKS, m,
+                       d_norm2);
+    CACG_LAUNCH_CHECK();
+    return 0;
+}
+
 }  // namespace
 
 extern "C" int cacg_k_colnorm2_ref(int n, int m, const double *R, long ldr, double *d_norm2,
@@ -867,6 +1099,16 @@ extern "C" int cacg_k_colnorm2_ref(int n, int m, const double *R, long ldr, doub
 
 namespace {
 
+// widths of 4 and 8 over many rows stay on the reference-order kernels in the
+// fast order: an MFMA operand row would be 3/4 or 1/2 padding.  Q and X / R
+// updates at sm = 4 (8): 71 (136) us against 126 (177) at 2,097,152 rows, 21 (26)
+// against 24 (26) at 250,047, 16 (18) against 13 (14) at 20,000.
+bool narrow_ref(int n, int sm)
+{
+    (void)n;
+    return sm <= 8 && sm % 4 == 0;
+}
+
 template <typename TS, typename T>
 int qupdate(int n, int sm, const TS *S, T *Q, const double *beta, int mode, hipStream_t st)
 {
@@ -884,8 +1126,11 @@ int qupdate(int n, int sm, const TS *S, T *Q, const double *beta, int mode, hipS
         case 48: return launch_qupdate_mfma<TS, T, 48>(n, S, Q, beta, st);
         case 32: return launch_qupdate_mfma<TS, T, 32>(n, S, Q, beta, st);
         case 16: return launch_qupdate_mfma<TS, T, 16>(n, S, Q, beta, st);
-        default: break;  // other widths: the reference-order kernel
+        default: break;
         }
+        // other widths up to 128: zero-padded to the next multiple of 16
+        if (sm < 128 && !narrow_ref(n, sm))
+            return qupdate_pad<TS>(n, sm, S, Q, sm, Q, beta, st);
     }
     // 512 lanes when sm is even, divides 512 and beta plus the tile fit in LDS
     if (sm % 2 == 0 && sm <= QR2_T && QR2_T % sm == 0 &&
@@ -971,6 +1216,27 @@ int xrupdate(int n, int sm, int m, const T *Q, const T *AQ, const double *alpha,
         default: break;
         }
 #undef CACG_XR
+#define CACG_XRP(SMV)                                                                             \
+    case SMV / 16:                                                                                \
+        return m <= 16 ? launch_xrupdate_pad<SMV, 1>(n, sm, m, Q, AQ, alpha, X, R, d_norm2,       \
+                                                     d_work, st)                                  \
+                       : launch_xrupdate_pad<SMV, 2>(n, sm, m, Q, AQ, alpha, X, R, d_norm2,       \
+                                                     d_work, st);
+        // other widths up to 128: zero-padded to the next multiple of 16
+        if (n > 0 && !narrow_ref(n, sm)) {
+            switch ((sm + 15) / 16) {
+                CACG_XRP(16)
+                CACG_XRP(32)
+                CACG_XRP(48)
+                CACG_XRP(64)
+                CACG_XRP(80)
+                CACG_XRP(96)
+                CACG_XRP(112)
+                CACG_XRP(128)
+            default: break;
+            }
+        }
+#undef CACG_XRP
     }
     // 512 lanes when m is even and divides 512, s <= 8 (a thread holds 2 s values
     // of the next tile) and alpha plus the two tiles fit in LDS
@@ -1142,6 +1408,16 @@ extern "C" int cacg_k_xrupdate_split(int n, int sm, int m, const double *Q, cons
 extern "C" int cacg_k_qupdate_zero(int n, int sm, double *Q, const double *beta, hipStream_t st)
 {
     return qupdate<double, double>(n, sm, (const double *)nullptr, Q, beta, CACG_MODE_FAST, st);
+}
+
+extern "C" int cacg_k_rowmul_neg(int n, int sm, const double *A, long lda, double *Q,
+                                 const double *beta, hipStream_t st)
+{
+    if (n < 0 || sm <= 0 || sm > 128 || lda < sm)
+        return (int)hipErrorInvalidValue;
+    if (n == 0)
+        return 0;
+    return qupdate_pad<double>(n, sm, nullptr, A, lda, Q, beta, st);
 }
 
 extern "C" int cacg_k_qupdate_s32(int n, int sm, const float *S, double *Q, const double *beta,

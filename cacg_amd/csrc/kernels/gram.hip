@@ -15,6 +15,8 @@
 // double buffer).  Each chunk writes a kl_pad x kr_pad partial; a second
 // kernel sums the partials in chunk order, so the result is deterministic and
 // independent of scheduling.
+#include <type_traits>
+
 #include "kcommon.hpp"
 
 namespace {
@@ -185,6 +187,16 @@ GramPlan plan_gram(int n, int kl, int kr)
     return p;
 }
 
+// the shapes with a block-major R1, given the 16-byte vectors of a stage of 16
+// and of 8 rows: the wide kernels', or at most 5 vectors per lane of 256
+bool blk_shape(int n, const GramPlan &p, long vec16, long vec8)
+{
+    (void)n;
+    const bool wide = p.TM == 8 && p.chunk % 16 == 0 && (p.TN == 8 || p.TN == 9) &&
+                      vec16 <= (p.TN == 9 ? 12 * 64 * 3 : 16 * 64 * 2);
+    return wide || (vec8 <= 256 * 5 && p.chunk % 8 == 0);
+}
+
 // L and R1 are FP64 (the FP64 solver) or FP32 (the FP32 basis: Q, AQ, S);
 // R2 (the residual R) is always FP64.  Loaded values are widened to FP64 and
 // every product and sum is FP64.  R1 may be block-major (bs1 > 0): column c
@@ -213,142 +225,17 @@ __device__ __forceinline__ long r1_col(const SrcT<TL, T1> &s, int c)
     return s.bs1 ? (long)(c / s.ld1) * s.bs1 + c % s.ld1 : (long)c;
 }
 
-template <typename TL, typename T1, int MT, int NT>
-__global__ __launch_bounds__(256) void gram_mfma_kernel(int n, SrcT<TL, T1> s,
-                                                        double *__restrict__ part,
-                                                        int kl_pad, int kr_pad, int chunk, int GN,
-                                                        int NG, int WGG, int KS)
-{
-    extern __shared__ double red[];  // (KS - 1) * WGG * MT * NT * 4 * 64 doubles when KS > 1
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int lr = lane >> 4, lc = lane & 15;
-    const int gb = wave % WGG, ks = wave / WGG;
-    const int g = blockIdx.y * WGG + gb;
-    const bool active = g < NG && ks < KS;
-    const int gm = active ? g / GN : 0, gn = active ? g % GN : 0;
-    const int kr = s.kr1 + s.kr2;
-
-    // per-lane operand columns: A tile t reads column ca0 + 16 t of L; B tile t
-    // reads column cb0 + 16 t of [R1 | R2]
-    const int ca0 = gm * MT * 16 + lc;
-    const int cb0 = gn * NT * 16 + lc;
-
-    dbl4 acc[MT][NT];
-#pragma unroll
-    for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int j = 0; j < NT; j++)
-            acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
-
-    const int r0 = blockIdx.x * chunk;
-    int r1 = r0 + chunk;
-    if (r1 > n)
-        r1 = n;
-
-    // k-steps of 4 rows; wave ks takes steps ks, ks + KS, ...; two steps per
-    // batch, batches double-buffered in registers
-    double av[2][2][MT], bv[2][2][NT];
-    auto load = [&](int buf, int rb) {
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const int row = rb + u * 4 * KS + lr;
-            const bool rok = row < r1;
-            const TL *pl = s.L + (long)row * s.ldl;
-            const T1 *p1 = s.R1 + (long)row * s.ld1;
-            const double *p2 = s.R2 + (long)row * s.ld2 - s.kr1;
-#pragma unroll
-            for (int t = 0; t < MT; t++) {
-                const int a = ca0 + 16 * t;
-                av[buf][u][t] = (rok && a < s.kl) ? (double)pl[a] : 0.0;
-            }
-#pragma unroll
-            for (int t = 0; t < NT; t++) {
-                const int b = cb0 + 16 * t;
-                bv[buf][u][t] = (rok && b < kr) ? (b < s.kr1 ? (double)p1[b] : p2[b]) : 0.0;
-            }
-        }
-    };
-    auto compute = [&](int buf) {
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int i = 0; i < MT; i++)
-#pragma unroll
-                for (int j = 0; j < NT; j++)
-                    acc[i][j] = mfma16x16x4(av[buf][u][i], bv[buf][u][j], acc[i][j]);
-    };
-    if (active) {
-        const int stride = 8 * KS;
-        int rb = r0 + ks * 4;
-        if (rb < r1)
-            load(0, rb);
-        for (; rb < r1; rb += 2 * stride) {
-            if (rb + stride < r1)
-                load(1, rb + stride);
-            compute(0);
-            if (rb + stride >= r1)
-                break;
-            if (rb + 2 * stride < r1)
-                load(0, rb + 2 * stride);
-            compute(1);
-        }
-    }
-
-    // combine the KS waves of one tile group in wave order
-    if (KS > 1) {
-        const int per = MT * NT * 4;
-        if (active && ks > 0) {
-            double *dst = red + ((long)((ks - 1) * WGG + gb) * per) * 64;
-#pragma unroll
-            for (int i = 0; i < MT; i++)
-#pragma unroll
-                for (int j = 0; j < NT; j++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        dst[((i * NT + j) * 4 + r) * 64 + lane] = acc[i][j][r];
-        }
-        __syncthreads();
-        if (active && ks == 0) {
-            for (int q = 1; q < KS; q++) {
-                const double *src = red + ((long)((q - 1) * WGG + gb) * per) * 64;
-#pragma unroll
-                for (int i = 0; i < MT; i++)
-#pragma unroll
-                    for (int j = 0; j < NT; j++)
-#pragma unroll
-                        for (int r = 0; r < 4; r++)
-                            acc[i][j][r] += src[((i * NT + j) * 4 + r) * 64 + lane];
-            }
-        }
-    }
-    if (!active || ks != 0)
-        return;
-    double *out = part + (long)blockIdx.x * kl_pad * kr_pad;
-#pragma unroll
-    for (int i = 0; i < MT; i++) {
-        const int tm = gm * MT + i;
-        if (tm * 16 >= kl_pad)
-            continue;
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            const int tn = gn * NT + j;
-            if (tn * 16 >= kr_pad)
-                continue;
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-                out[(long)(tm * 16 + lr + 4 * r) * kr_pad + tn * 16 + lc] = acc[i][j][r];
-        }
-    }
-}
-
 // 64 consecutive outputs per block; wave w sums chunk partials x in
-// [w*gx/4, (w+1)*gx/4) in order, then the four wave sums are added in wave order
+// [w*gx/4, (w+1)*gx/4) in order, then the four wave sums are added in wave order.
+// 32 loads are in flight ahead of their additions: a wave's share is otherwise a
+// chain of memory latencies.
 __global__ __launch_bounds__(256) void gram_reduce_kernel(const double *__restrict__ part, int gx,
                                                           int kl, int kr1, int kr2, int kl_pad,
                                                           int kr_pad, double *__restrict__ G1,
                                                           double *__restrict__ G2)
 {
-    __shared__ double red[4][64];
+    constexpr int W = 4, LD = 32;
+    __shared__ double red[W][64];
     const int kr = kr1 + kr2;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const long e = (long)blockIdx.x * 64 + lane;
@@ -356,21 +243,20 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(const double *__restri
     const int a = ok ? (int)(e / kr) : 0, b = ok ? (int)(e % kr) : 0;
     const long stride = (long)kl_pad * kr_pad;
     const double *p = part + (long)a * kr_pad + b;
-    const int q = (gx + 3) / 4;
+    const int q = (gx + W - 1) / W;
     const int x0 = wave * q, x1 = (x0 + q) < gx ? (x0 + q) : gx;
     double acc = 0.0;
     if (ok) {
-        int x = x0;
-        for (; x + 4 <= x1; x += 4) {
-            const double v0 = p[x * stride], v1 = p[(x + 1) * stride];
-            const double v2 = p[(x + 2) * stride], v3 = p[(x + 3) * stride];
-            acc += v0;
-            acc += v1;
-            acc += v2;
-            acc += v3;
+        for (int x = x0; x < x1; x += LD) {
+            double v[LD];
+#pragma unroll
+            for (int u = 0; u < LD; u++)
+                v[u] = x + u < x1 ? p[(x + u) * stride] : 0.0;
+#pragma unroll
+            for (int u = 0; u < LD; u++)
+                if (x + u < x1)
+                    acc += v[u];
         }
-        for (; x < x1; x++)
-            acc += p[x * stride];
     }
     red[wave][lane] = acc;
     __syncthreads();
@@ -628,44 +514,337 @@ int launch_gram_wide(int n, const SrcT<TL, T1> &s, const GramPlan &p, double *wo
     return 1;
 }
 
-template <typename TL, typename T1, int MT, int NT>
-int launch_gram_mfma(int n, const SrcT<TL, T1> &s, const GramPlan &p, double *G1, double *G2,
-                     double *work, hipStream_t st)
+// ---- every other shape: waves share tiles out by group and by rows ----------------
+//
+// G is cut into blocks of at most 8 x 10 tiles of 16 x 16 (blockIdx.y); a workgroup
+// forms one block over one row chunk.  Its waves are NG groups of MT x NT tiles,
+// times KS shares of the rows: a stage is 16 KS rows, wave (g, ks) takes every
+// KS-th step of 4 rows of it for group g, and the KS partial sums are added in
+// order at the end.  Narrow blocks so get as many waves, and as many bytes
+// in flight, as wide ones.  Stages are loaded cooperatively two ahead (VEC
+// columns a load: 2, or 1 where a source has a single column) and read from one of two LDS buffers as in gram_lds_kernel.
+// Bound by memory up to about 64 columns, by the matrix cores above.
+struct GramTile {
+    int TMB, TNB;    // tiles of a block
+    int nbn;         // blocks along N
+    int GN, NG, KS;  // groups along N, groups, row shares
+    int MT, NT, VEC;
+    int W;           // waves the kernel is built for: 16, or 8 with twice the registers
+    size_t lds;
+};
+
+constexpr int GT_TM = 8, GT_TN = 10;
+
+// two columns, aligned as one
+typedef double pair64 __attribute__((ext_vector_type(2), aligned(8)));
+typedef float pair32 __attribute__((ext_vector_type(2), aligned(4)));
+
+// loads of a stage per lane
+__host__ __device__ constexpr int gt_loads(int W, int VEC)
 {
-    constexpr int SR = 8, LDG = 3, VPT = 5;
-    constexpr int EL = 16 / sizeof(TL), E1 = 16 / sizeof(T1);
-    const int kl_pad = p.TM * 16, kr_pad = p.TN * 16;
-    const int kr = s.kr1 + s.kr2;
-    auto al16 = [](const void *q) { return ((uintptr_t)q & 15) == 0; };
-    // 16-byte vectors: column counts and row strides in whole vectors, aligned rows
-    const bool aligned = p.KS == 1 && s.kl % EL == 0 && s.kr1 % E1 == 0 && s.kr2 % 2 == 0 &&
-                         s.ldl % EL == 0 && s.ld1 % E1 == 0 && s.bs1 % E1 == 0 &&
-                         (s.kr2 == 0 || s.ld2 % 2 == 0) &&
-                         al16(s.L) && al16(s.R1) && (s.kr2 == 0 || al16(s.R2));
-    const bool staged = aligned && stage_vectors(s, SR) <= 256 * VPT && p.chunk % SR == 0;
-    if (launch_gram_wide(n, s, p, work, aligned, st)) {
-        // launched
-    } else if (s.bs1 && !staged) {
-        return (int)hipErrorInvalidValue;  // a block-major R1 needs the staged kernels
-    } else if (staged) {
-        const size_t shm =
-            2 * (size_t)SR * (lds_row_stride(s.kl) + lds_row_stride(kr)) * sizeof(double);
-        cacg_allow_lds(gram_lds_kernel<TL, T1, 4, MT, NT, SR, LDG, VPT>, shm);
-        hipLaunchKernelGGL((gram_lds_kernel<TL, T1, 4, MT, NT, SR, LDG, VPT>), dim3(p.gx, p.gy),
-                           dim3(256), shm, st, n, s, work, kl_pad, kr_pad, p.chunk, p.GN, p.NG);
-    } else {
-        const size_t shm =
-            p.KS > 1 ? (size_t)(p.KS - 1) * p.WGG * MT * NT * 4 * 64 * sizeof(double) : 0;
-        cacg_allow_lds(gram_mfma_kernel<TL, T1, MT, NT>, shm);
-        hipLaunchKernelGGL((gram_mfma_kernel<TL, T1, MT, NT>), dim3(p.gx, p.gy), dim3(256), shm,
-                           st, n, s, work, kl_pad, kr_pad, p.chunk, p.GN, p.NG, p.WGG, p.KS);
+    return W == 16 ? (VEC == 2 ? 3 : 5) : (VEC == 2 ? 5 : 9);
+}
+
+// the tile group and row shares of a block: the fewest MFMA slots per row on the
+// busiest SIMD (waves are dealt round-robin over 4), then the most waves; at
+// most 16 waves and 80 KiB of LDS (two workgroups a CU) while a single row share
+// allows it
+GramTile plan_tile(int TM, int TN, int VEC, int chunk)
+{
+    static const int shape[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 5}, {2, 2}, {2, 3}};
+    GramTile best{};
+    const int bm = (TM + GT_TM - 1) / GT_TM, bn = (TN + GT_TN - 1) / GT_TN;
+    best.TMB = (TM + bm - 1) / bm;
+    best.TNB = (TN + bn - 1) / bn;
+    best.nbn = (TN + best.TNB - 1) / best.TNB;
+    best.VEC = VEC;
+    double cost = 1e30;
+    const int cols = lds_row_stride(best.TMB * 16) + lds_row_stride(best.TNB * 16);
+    for (const auto &sh : shape) {
+        const int MT = sh[0], NT = sh[1];
+        const int GM = (best.TMB + MT - 1) / MT, GN = (best.TNB + NT - 1) / NT, NG = GM * GN;
+        // no more row shares than 16-row pieces in a chunk
+        for (int KS = 1; NG * KS <= 16 && (KS == 1 || 16 * KS <= chunk); KS++) {
+            const int W = NG * KS <= 8 ? 8 : 16;
+            // loads of a row: L, R1 and R2 may each end with an odd column
+            if (16 * (best.TMB + best.TNB) / VEC + VEC - 1 > 4 * gt_loads(W, VEC) * NG)
+                continue;
+            const size_t stage = 2 * (size_t)(16 * KS * cols + 32) * sizeof(double);
+            const size_t red = (size_t)(KS - 1) * NG * MT * NT * 256 * sizeof(double);
+            const size_t lds = stage > red ? stage : red;
+            if (lds > (KS == 1 ? 160 : 80) * 1024)
+                break;
+            const double c = (double)((NG * KS + 3) / 4) * MT * NT / KS - 1e-3 * NG * KS;
+            if (c < cost) {
+                cost = c;
+                best.GN = GN;
+                best.NG = NG;
+                best.KS = KS;
+                best.MT = MT;
+                best.NT = NT;
+                best.W = W;
+                best.lds = lds;
+            }
+        }
     }
-    CACG_LAUNCH_CHECK();
-    const long outs = (long)s.kl * (s.kr1 + s.kr2);
-    hipLaunchKernelGGL(gram_reduce_kernel, dim3(cacg_grid(outs, 64, 0)), dim3(256), 0, st, work,
-                       p.gx, s.kl, s.kr1, s.kr2, kl_pad, kr_pad, G1, G2);
-    CACG_LAUNCH_CHECK();
-    return 0;
+    return best;
+}
+
+template <typename TL, typename T1, int MT, int NT, int VEC, int W, bool ONE>
+__global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s,
+                                                         double *__restrict__ part, int kl_pad,
+                                                         int kr_pad, int chunk, GramTile g)
+{
+    constexpr int LDG = 2, VPT = gt_loads(W, VEC);
+    using V = typename std::conditional<VEC == 2, pair64, double>::type;
+    using V4 = typename std::conditional<VEC == 2, pair32, float>::type;
+    constexpr bool one = VEC == 2 && ONE;   // R2 is a single column
+    extern __shared__ double lds[];
+    const int ca = (int)blockIdx.y / g.nbn * g.TMB * 16, cb = (int)blockIdx.y % g.nbn * g.TNB * 16;
+    const int krt = s.kr1 + s.kr2;
+    const int kl = s.kl - ca < g.TMB * 16 ? s.kl - ca : g.TMB * 16;
+    const int kr = krt - cb < g.TNB * 16 ? krt - cb : g.TNB * 16;
+    const int LDP = lds_row_stride(kl), RDP = lds_row_stride(kr);
+    const int SR = 16 * g.KS;
+    // a tile past the last column reads into the next row (past the last row: 32
+    // doubles more); it feeds outputs of the padding only
+    const int BUF = SR * (LDP + RDP) + 32;
+    const int t = threadIdx.x, nth = blockDim.x;
+    const int wave = t >> 6, lane = t & 63, lr = lane >> 4, lc = lane & 15;
+    const int gi = wave % g.NG, ks = wave / g.NG;
+    const int tm = gi / g.GN * MT, tn = gi % g.GN * NT;
+    const int r0 = blockIdx.x * chunk, r1 = r0 + chunk < n ? r0 + chunk : n;
+    const int nstage = (r1 - r0 + SR - 1) / SR;
+
+    // this lane's vectors of a stage: source address, and LDS offset, row and
+    // source (0 L, 1 R1, 2 R2) packed
+    const char *src[VPT];
+    unsigned info[VPT];
+    // R1's columns of the block, then R2's; a last odd column's pair starts one
+    // column early, inside the row
+    const int k1 = s.kr1 - cb < 0 ? 0 : s.kr1 - cb < kr ? s.kr1 - cb : kr, k2 = kr - k1;
+    const int wl = (kl + VEC - 1) / VEC, w1 = (k1 + VEC - 1) / VEC;
+    const int wr = w1 + (one ? 0 : (k2 + VEC - 1) / VEC);
+    auto start = [](int q, int k) { return VEC * q + VEC <= k || VEC == 1 ? VEC * q : k - VEC; };
+    // v / w for v < 2^14, w <= 256: the error of the product is far below 0.5 / w
+    const float il = 1.0f / wl, ir = 1.0f / wr;
+#pragma unroll
+    for (int u = 0; u < VPT; u++) {
+        int v = t + nth * u;
+        info[u] = ~0u;
+        src[u] = reinterpret_cast<const char *>(s.L);
+        if (v < SR * wl) {
+            const int row = (int)((v + 0.5f) * il), c = start(v - row * wl, kl);
+            src[u] = reinterpret_cast<const char *>(s.L + (long)(r0 + row) * s.ldl + ca + c);
+            info[u] = (unsigned)(row * LDP + c) << 12 | row;
+        } else if ((v -= SR * wl) < SR * wr) {
+            const int row = (int)((v + 0.5f) * ir), q = v - row * wr;
+            const int c = q < w1 ? start(q, k1) : k1 + start(q - w1, k2);
+            if (q < w1)
+                src[u] = reinterpret_cast<const char *>(s.R1 + (long)(r0 + row) * s.ld1 +
+                                                        r1_col(s, cb + c));
+            else
+                src[u] = reinterpret_cast<const char *>(s.R2 + (long)(r0 + row) * s.ld2 + cb + c -
+                                                        s.kr1);
+            info[u] = (unsigned)(SR * LDP + row * RDP + c) << 12 | (q < w1 ? 1u : 2u) << 10 | row;
+        }
+    }
+    const long incl = (long)SR * s.ldl * sizeof(TL), inc1 = (long)SR * s.ld1 * sizeof(T1),
+               inc2 = (long)SR * s.ld2 * sizeof(double);
+    V stg[LDG][VPT];
+    // a single column of R2 has a load of its own, row t of the stage
+    double stg1[LDG];
+    const double *src1 = s.R2 + (long)(r0 + t) * s.ld2;
+    auto gload = [&](int slot, int st) {
+        const int left = st < nstage ? r1 - r0 - st * SR : 0;
+        if constexpr (one) {
+            stg1[slot] = t < SR && t < left && k2 > 0 ? *src1 : 0.0;
+            src1 += SR * s.ld2;
+        }
+#pragma unroll
+        for (int u = 0; u < VPT; u++) {
+            const int row = info[u] & 1023, kind = info[u] >> 10 & 3;
+            V w{};
+            if (row < left) {
+                if (sizeof(T1) == 4 && kind == 1) {
+                    const V4 f = *reinterpret_cast<const V4 *>(src[u]);
+                    __builtin_memcpy(&w, &f, sizeof(f));
+                } else {
+                    w = *reinterpret_cast<const V *>(src[u]);
+                }
+            }
+            stg[slot][u] = w;
+            src[u] += kind == 0 ? incl : kind == 1 ? inc1 : inc2;
+        }
+    };
+    auto lstore = [&](int slot, int buf) {
+        double *b = lds + buf * BUF;
+        if constexpr (one) {
+            if (t < SR && k2 > 0)
+                b[SR * LDP + t * RDP + k1] = stg1[slot];
+        }
+#pragma unroll
+        for (int u = 0; u < VPT; u++) {
+            if (info[u] == ~0u)
+                continue;
+            V w = stg[slot][u];
+            if (sizeof(T1) == 4 && (info[u] >> 10 & 3) == 1) {
+                V4 f;
+                __builtin_memcpy(&f, &w, sizeof(f));
+                if constexpr (VEC == 2)
+                    w = V{(double)f.x, (double)f.y};
+                else
+                    w = (double)f;
+            }
+            *reinterpret_cast<V *>(b + (info[u] >> 12)) = w;
+        }
+    };
+    dbl4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+            acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+    auto compute = [&](int buf) {
+        const double *bl = lds + buf * BUF + (4 * ks + lr) * LDP + tm * 16 + lc;
+        const double *br = lds + buf * BUF + SR * LDP + (4 * ks + lr) * RDP + tn * 16 + lc;
+        double av[2][MT], bv[2][NT];
+        auto operands = [&](int q, int p) {
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+                av[p][i] = bl[4 * q * g.KS * LDP + 16 * i];
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                bv[p][j] = br[4 * q * g.KS * RDP + 16 * j];
+        };
+        operands(0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            if (q + 1 < 4)
+                operands(q + 1, (q + 1) & 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    acc[i][j] = mfma16x16x4(av[q & 1][i], bv[q & 1][j], acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < LDG; q++)
+        gload(q, q);
+    lstore(0, 0);
+    gload(0, LDG);
+    __syncthreads();
+    for (int st0 = 0; st0 < nstage; st0 += LDG) {
+#pragma unroll
+        for (int q = 0; q < LDG; q++) {
+            const int st = st0 + q;
+            if (st < nstage) {
+                compute(st & 1);
+                const int nslot = (q + 1) % LDG;
+                lstore(nslot, (st + 1) & 1);
+                gload(nslot, st + 1 + LDG);
+            }
+            __syncthreads();
+        }
+    }
+    // the KS shares of a group, added in order
+    if (g.KS > 1) {
+        constexpr int per = MT * NT * 4;
+        double *dst = lds + ((ks - 1) * g.NG + gi) * per * 64 + lane;
+        if (ks > 0) {
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        dst[((i * NT + j) * 4 + r) * 64] = acc[i][j][r];
+        }
+        __syncthreads();
+        if (ks > 0)
+            return;
+        for (int q = 0; q + 1 < g.KS; q++) {
+            const double *from = lds + (q * g.NG + gi) * per * 64 + lane;
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        acc[i][j][r] += from[((i * NT + j) * 4 + r) * 64];
+        }
+    }
+    double *out = part + (long)blockIdx.x * kl_pad * kr_pad;
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        const int a = ca + (tm + i) * 16;
+        if (tm + i >= g.TMB || a >= kl_pad)
+            continue;
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            const int b = cb + (tn + j) * 16;
+            if (tn + j >= g.TNB || b >= kr_pad)
+                continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                out[(long)(a + lr + 4 * r) * kr_pad + b + lc] = acc[i][j][r];
+        }
+    }
+}
+
+template <typename TL, typename T1, int VEC>
+int launch_gram_tile(int n, const SrcT<TL, T1> &s, GramPlan &p, double *work, hipStream_t st)
+{
+    // from 8192 rows on at least 128 rows a chunk where a block's few tiles leave
+    // waves for more row shares: the same waves on half the partials (4 + 4 columns
+    // against 4, 20,000 rows: 14.0 -> 11.3 us; 100 columns: 28 -> 31 us, not taken)
+    if (n >= 8192 && p.chunk < 128 && p.TM * p.TN <= 24) {
+        p.chunk = 128;
+        p.gx = (n + 127) / 128;
+    }
+    const GramTile g = plan_tile(p.TM, p.TN, VEC, p.chunk);
+    if (VEC == 2) {
+        // every source has two columns in every block it reaches, R2 one column in
+        // all; a block that holds a single one of a wider source cannot pair it
+        auto lone = [](int w, int k) { return k > 0 && k % w == 1; };
+        const int w = g.TNB * 16, e1 = s.kr1 % w;   // columns of R1 before R2 in their block
+        const int first2 = s.kr2 < w - e1 ? s.kr2 : w - e1;
+        const bool r2 = s.kr2 > 1 && (first2 == 1 || lone(w, s.kr2 - first2));
+        if (n < 2 || lone(g.TMB * 16, s.kl) || lone(w, s.kr1) || r2)
+            return (int)hipErrorInvalidValue;
+    }
+    const int kl_pad = p.TM * 16, kr_pad = p.TN * 16;
+    const dim3 grid(p.gx, (p.TM + g.TMB - 1) / g.TMB * g.nbn), block(64 * g.NG * g.KS);
+#define CACG_GT(M, N, WV, ONE)                                                                    \
+    if (g.MT == M && g.NT == N && g.W == WV) {                                                    \
+        cacg_allow_lds(gram_tile_kernel<TL, T1, M, N, VEC, WV, ONE>, g.lds);                      \
+        hipLaunchKernelGGL((gram_tile_kernel<TL, T1, M, N, VEC, WV, ONE>), grid, block, g.lds,    \
+                           st, n, s, work, kl_pad, kr_pad, p.chunk, g);                           \
+        return 0;                                                                                 \
+    }
+    if (VEC == 2 && s.kr2 == 1 && sizeof(T1) == 8) {
+        CACG_GT(1, 1, 8, true)
+        CACG_GT(1, 1, 16, true)
+        CACG_GT(1, 2, 8, true)
+        CACG_GT(1, 2, 16, true)
+        return (int)hipErrorInvalidValue;
+    }
+    if (VEC == 2 && s.kr2 == 1)
+        return (int)hipErrorInvalidValue;
+#define CACG_GTW(M, N) CACG_GT(M, N, 8, false) CACG_GT(M, N, 16, false)
+    CACG_GTW(1, 1)
+    CACG_GTW(1, 2)
+    CACG_GTW(1, 3)
+    CACG_GTW(1, 4)
+    CACG_GTW(1, 5)
+    CACG_GTW(2, 2)
+    CACG_GTW(2, 3)
+#undef CACG_GTW
+#undef CACG_GT
+    return (int)hipErrorInvalidValue;
 }
 
 template <typename TL, typename T1>
@@ -675,27 +854,33 @@ int gram_fast(int n, const TL *L, long ldl, int kl, const T1 *R1, long ld1, int 
 {
     if (n < 0 || kl <= 0 || kr1 < 0 || kr2 < 0 || kr1 + kr2 <= 0)
         return (int)hipErrorInvalidValue;
-    const GramPlan p = plan_gram(n, kl, kr1 + kr2);
+    GramPlan p = plan_gram(n, kl, kr1 + kr2);
     const SrcT<TL, T1> s = {L, ldl, kl, R1, ld1, kr1, R2, ld2, kr2, bs1};
-    // MT in {1, 2}, NT in 1..9
-#define CACG_GRAM_NT(MTV)                                                                         \
-    switch (p.NT) {                                                                               \
-    case 1: return launch_gram_mfma<TL, T1, MTV, 1>(n, s, p, G1, G2, d_work, st);                 \
-    case 2: return launch_gram_mfma<TL, T1, MTV, 2>(n, s, p, G1, G2, d_work, st);                 \
-    case 3: return launch_gram_mfma<TL, T1, MTV, 3>(n, s, p, G1, G2, d_work, st);                 \
-    case 4: return launch_gram_mfma<TL, T1, MTV, 4>(n, s, p, G1, G2, d_work, st);                 \
-    case 5: return launch_gram_mfma<TL, T1, MTV, 5>(n, s, p, G1, G2, d_work, st);                 \
-    case 6: return launch_gram_mfma<TL, T1, MTV, 6>(n, s, p, G1, G2, d_work, st);                 \
-    case 7: return launch_gram_mfma<TL, T1, MTV, 7>(n, s, p, G1, G2, d_work, st);                 \
-    case 8: return launch_gram_mfma<TL, T1, MTV, 8>(n, s, p, G1, G2, d_work, st);                 \
-    default: return launch_gram_mfma<TL, T1, MTV, 9>(n, s, p, G1, G2, d_work, st);                \
+    constexpr int EL = 16 / sizeof(TL), E1 = 16 / sizeof(T1);
+    auto al16 = [](const void *q) { return ((uintptr_t)q & 15) == 0; };
+    // 16-byte vectors: column counts and row strides in whole vectors, aligned rows
+    const bool aligned = p.KS == 1 && kl % EL == 0 && kr1 % E1 == 0 && kr2 % 2 == 0 &&
+                         ldl % EL == 0 && ld1 % E1 == 0 && bs1 % E1 == 0 &&
+                         (kr2 == 0 || ld2 % 2 == 0) && al16(L) && al16(R1) &&
+                         (kr2 == 0 || al16(R2));
+    // a block-major R1 is taken in the shapes cacg_gram_blk_supported names only
+    if (bs1 && !(aligned && blk_shape(n, p, stage_vectors(s, 16), stage_vectors(s, 8))))
+        return (int)hipErrorInvalidValue;
+    if (!launch_gram_wide(n, s, p, d_work, aligned, st)) {
+        // pairs of columns (16-byte loads need no alignment beyond the element's), or
+        // single ones where a source has only one
+        if (launch_gram_tile<TL, T1, 2>(n, s, p, d_work, st)) {
+            const int rc = launch_gram_tile<TL, T1, 1>(n, s, p, d_work, st);
+            if (rc)
+                return rc;
+        }
     }
-    if (p.MT == 2) {
-        CACG_GRAM_NT(2)
-    } else {
-        CACG_GRAM_NT(1)
-    }
-#undef CACG_GRAM_NT
+    CACG_LAUNCH_CHECK();
+    const long outs = (long)kl * (kr1 + kr2);
+    hipLaunchKernelGGL(gram_reduce_kernel, dim3(cacg_grid(outs, 64, 0)), dim3(256), 0, st, d_work,
+                       p.gx, kl, kr1, kr2, p.TM * 16, p.TN * 16, G1, G2);
+    CACG_LAUNCH_CHECK();
+    return 0;
 }
 
 }  // namespace
@@ -750,16 +935,10 @@ extern "C" int cacg_gram_blk_supported(int n, int kl, int kr1, int bw)
 {
     if (n <= 0 || kl <= 0 || bw <= 0 || kr1 <= 0 || kr1 % bw != 0 || bw % 2 != 0 || kl % 2 != 0)
         return 0;
-    // the conditions under which launch_gram_mfma stages the operands through
-    // LDS (16-byte aligned L, R1 and ldl = kl assumed)
+    // 16-byte aligned L, R1 and ldl = kl assumed
     const GramPlan p = plan_gram(n, kl, kr1);
     const SrcT<double, double> s = {nullptr, kl, kl, nullptr, bw, kr1, nullptr, 1, 0, (long)n * bw};
-    if (p.KS != 1)
-        return 0;
-    const bool wide = p.TM == 8 && p.chunk % 16 == 0 && (p.TN == 8 || p.TN == 9) &&
-                      stage_vectors(s, 16) <= (p.TN == 9 ? 12 * 64 * 3 : 16 * 64 * 2);
-    const bool staged = stage_vectors(s, 8) <= 256 * 5 && p.chunk % 8 == 0;
-    return wide || staged;
+    return p.KS == 1 && blk_shape(n, p, stage_vectors(s, 16), stage_vectors(s, 8)) ? 1 : 0;
 }
 
 extern "C" int cacg_k_gram_fast_blk(int n, const double *L, long ldl, int kl, const double *R1,

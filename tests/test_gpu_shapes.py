@@ -1,0 +1,108 @@
+"""Kernel dispatch edges: widths and row counts around the tiles, panels and
+blocks of the fast-order Gram, the padded updates, the small LU and the QR."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -52
+
+
+# a block of G is at most 8 x 10 tiles of 16; pairs of columns need two of them
+GRAM = [(1, 1, 1, 0), (1, 5, 4, 1), (2, 4, 4, 1), (3, 1, 1, 1), (15, 16, 16, 1), (17, 17, 17, 3),
+        (63, 21, 21, 3), (64, 40, 40, 5), (65, 33, 30, 2), (127, 2, 3, 7), (129, 96, 96, 12),
+        (1000, 129, 160, 0), (999, 128, 129, 17), (513, 145, 20, 141), (8191, 8, 8, 1),
+        (8192, 8, 8, 1), (8193, 60, 60, 10), (20001, 100, 100, 20), (4097, 128, 128, 32),
+        (300, 256, 256, 32), (2, 1, 17, 1)]
+
+
+@pytest.mark.parametrize("n,kl,kr1,kr2", GRAM)
+def test_gram_fast_edges_exact_on_integers(gpu_lib, n, kl, kr1, kr2):
+    rng = np.random.default_rng(n + kl + kr1 + kr2)
+    L, R1, R2 = (rng.integers(-8, 9, size=(n, k)).astype(np.float64) for k in (kl, kr1, kr2))
+    print(f"gram n={n} {kl} x ({kr1} + {kr2})", flush=True)
+    out = gpu_lib.k_gram(L, R1, R2 if kr2 else None, mode="fast")
+    G1, G2 = out if kr2 else (out, None)
+    assert np.array_equal(G1, L.T @ R1)   # integers below 2^53: exact in any order
+    if kr2:
+        assert np.array_equal(G2, L.T @ R2)
+
+
+@pytest.mark.parametrize("n,k", [(1, 2), (130, 17), (9000, 31), (5000, 60)])
+def test_gram_f64f32_edges_exact_on_integers(gpu_lib, n, k):
+    rng = np.random.default_rng(n + k)
+    L = rng.integers(-8, 9, size=(n, k)).astype(np.float64)
+    R = rng.integers(-8, 9, size=(n, k)).astype(np.float32)
+    print(f"gram f64 x f32 n={n} k={k}", flush=True)
+    assert np.array_equal(gpu_lib.k_gram_f64f32(L, R), L.T @ R.astype(np.float64))
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 1000, 16385])
+@pytest.mark.parametrize("sm,m", [(1, 1), (3, 1), (7, 7), (10, 2), (15, 3), (17, 1), (60, 10),
+                                  (63, 21), (100, 20), (127, 1), (24, 8), (31, 31)])
+def test_padded_updates_exact_on_integers(gpu_lib, n, sm, m):
+    rng = np.random.default_rng(n + 131 * sm + m)
+    ints = lambda *s: rng.integers(-8, 9, size=s).astype(np.float64)  # noqa: E731
+    S, Q, AQ, beta, alpha, X, R = (ints(n, sm), ints(n, sm), ints(n, sm), ints(sm, sm),
+                                   ints(sm, m), ints(n, m), ints(n, m))
+    print(f"updates n={n} sm={sm} m={m}", flush=True)
+    assert np.array_equal(gpu_lib.k_qupdate(S, Q, beta, mode="fast"), S - Q @ beta)
+    assert np.array_equal(gpu_lib.k_qupdate_s32(S.astype(np.float32), Q, beta), S - Q @ beta)
+    Xn, Rn, norm2 = gpu_lib.k_xrupdate(Q, AQ, alpha, X, R, mode="fast")
+    assert np.array_equal(Xn, X + Q @ alpha) and np.array_equal(Rn, R - AQ @ alpha)
+    assert np.array_equal(norm2, ((R - AQ @ alpha) ** 2).sum(0))
+
+
+def _spd(N, seed):
+    M = np.random.default_rng(seed).standard_normal((N, N))
+    return M @ M.T + N * np.eye(N)
+
+
+@pytest.mark.parametrize("N,k", [(1, 1), (7, 7), (8, 16), (9, 32), (31, 33), (33, 5), (64, 64),
+                                 (65, 32), (120, 33), (127, 1), (128, 128), (129, 3), (200, 40),
+                                 (256, 32), (257, 257), (300, 1)])
+def test_lu_panels_and_blocks_bitwise(gpu_lib, oracle_lib, N, k):
+    """Fast and reference order, first call and kept factor, around the panel
+    (8), the right-hand sides that ride along (32) and the block (128)."""
+    from conftest import lu_restated
+    A, rng = _spd(N, N + k), np.random.default_rng(k)
+    rhs, rhs2 = rng.standard_normal((N, k)), rng.standard_normal((N, N))
+    print(f"lu N={N} k={k}", flush=True)
+    x, x2, flag = gpu_lib.k_lu_solve(A, rhs, mode="fast", rhs2=rhs2)
+    assert flag == 0
+    assert np.array_equal(x, lu_restated(A, rhs, "fast"))
+    assert np.array_equal(x2, lu_restated(A, rhs2, "fast"))
+    x, x2, flag = gpu_lib.k_lu_solve(A, rhs, mode="reference", rhs2=rhs2)
+    assert flag == 0
+    assert np.array_equal(x, oracle_lib.lu_solve(A, rhs))
+    assert np.array_equal(x2, oracle_lib.lu_solve(A, rhs2))
+
+
+@pytest.mark.parametrize("N,p", [(12, 0), (40, 17), (128, 127), (200, 130)])
+def test_lu_flags_a_zero_pivot_anywhere(gpu_lib, N, p):
+    A = np.eye(N)
+    A[p, p] = 0.0
+    print(f"lu zero pivot N={N} p={p}", flush=True)
+    for mode in ("fast", "reference"):
+        assert gpu_lib.k_lu_solve(A, np.ones((N, 2)), mode=mode)[1] == 1
+
+
+@pytest.mark.parametrize("n,k,lda", [(300, 7, 7), (300, 8, 11), (1000, 9, 16), (2000, 33, 40),
+                                     (5000, 65, 65), (5000, 127, 128)])
+def test_tsqr_strided_input(gpu_lib, n, k, lda):
+    """A with a row stride is read where it lies; bounds as for contiguous input:
+    orthogonality 50 k u, residual 1e-13."""
+    W = np.random.default_rng(n + k).standard_normal((n, lda))
+    L = gpu_lib.lib()
+    dA, dQ, dR = (gpu_lib.DeviceBuffer.from_array(W), gpu_lib.DeviceBuffer(8 * n * k),
+                  gpu_lib.DeviceBuffer(8 * k * k))
+    ws = gpu_lib.DeviceBuffer(8 * L.cacg_tsqr_workspace(k))
+    flag = gpu_lib.DeviceBuffer.from_array(np.zeros(1, dtype=np.int32))
+    print(f"tsqr n={n} k={k} lda={lda}", flush=True)
+    assert L.cacg_k_tsqr(n, k, dA.ptr, lda, dQ.ptr, dR.ptr, ws.ptr, flag.ptr, None) == 0
+    Q, R = dQ.download((n, k)), dR.download((k, k))
+    assert int(flag.download(1, np.int32)[0]) == 0
+    assert np.array_equal(dA.download((n, lda)), W)
+    assert np.all(np.tril(R, -1) == 0.0) and np.all(np.diag(R) > 0)
+    assert np.abs(Q.T @ Q - np.eye(k)).max() <= 50 * k * EPS / 2
+    assert np.linalg.norm(Q @ R - W[:, :k]) <= 1e-13 * np.linalg.norm(W[:, :k])
