@@ -21,16 +21,38 @@
 
 namespace {
 
-// One workgroup per 8 x 8 block of G: lane l of wave 0 keeps the chain of
-// G[a0 + l / 8][b0 + l % 8], sequential in the row index (the reference's
-// summation, bit for bit), so the kernel takes n steps of one product and one
-// dependent sum whatever the grid.  Waves 1-3 meanwhile stage the block's
-// columns of the next GREF_ROWS rows (8 values of L and 8 of [R1 | R2] a row,
-// columns past the last clamped to it) into the other of two LDS buffers, so
-// a stage costs the chain one barrier instead of a global latency, and the
-// chain lanes read their two operands 16 rows ahead of the sums.
-constexpr int GREF_ROWS = 256;                          // rows per stage (two 32 KiB buffers)
-constexpr int GREF_J = (GREF_ROWS * 16 + 191) / 192;    // values per loader lane and stage
+// One workgroup per NJ x 16 block of G; every entry's sum is one chain in row
+// order (the reference's summation, bit for bit), so the kernel takes n steps
+// whatever the grid and what counts is the length of a step.  A wave issues an
+// FP64 instruction about every 8.5 cycles, dependent or not, so the chain
+// lanes (64 entries a wave) do nothing but add and the other waves form the
+// products: lane l of a producer holds column b0 + l % 16 of RL adjacent rows,
+// the columns of L lie RL x NJ to 16 lanes, and v_fmac_f64 takes L's value from
+// its lane by DPP (row_newbcast; product + 0 rounds as the product does).  Two
+// rows' products go to LDS with one 16-byte write, which a chain lane takes
+// with one 16-byte read, a batch ahead of its sums.  Producer lanes load GREF_D
+// stages ahead into registers; a stage ends with a barrier that waits for LDS
+// alone, so loads stay in flight, and the chain lanes cross it with a batch in
+// registers.  With one chain wave, wave 4 does nothing else than the barriers:
+// it shares the chain's SIMD, and a producer there costs the chain 6%.
+// 262,144 rows, 128 x 144: 3.77 -> 1.86 ms (7.1 ns a row), 128 x 128 3.4 -> 1.63
+// ms; the chain alone takes 3.7 ns a row, the producers alone 5.3 (products
+// through LDS and, with every CU at work, 13 TB/s out of the L2s).  Slower:
+// chain waves of 16 or 32 lanes (2.99, 2.53 ms), 9 producers, loads 2 or 8
+// stages ahead (the same).
+constexpr int GREF_D = 4;
+
+template <int NJ>
+struct GrefShape {
+    static constexpr int CW = NJ > 4 ? 2 : 1;                     // chain waves: 0 .. CW - 1
+    static constexpr int PW = 6;                                  // producer waves
+    static constexpr int RL = NJ > 5 ? 2 : NJ > 2 ? 4 : 8;        // rows per producer lane and stage
+    static constexpr int ROWS = 4 * PW * RL;                      // rows a stage: 48, 96 or 192
+    static constexpr int NB = RL == 8 ? 12 : 6, BP = ROWS / NB / 2;   // batches a stage, row pairs each
+    static constexpr int BUF = ROWS * NJ * 8;                     // double2 per buffer
+    static constexpr int JP = NJ > 4 ? 8 : NJ > 2 ? 4 : 2;        // lanes per row of L
+    static constexpr int RA = 16 / JP, NA = RL / RA;              // rows per load of L, loads
+};
 
 struct GrefSrc {
     const double *L;
@@ -44,96 +66,209 @@ struct GrefSrc {
     int kr2;
 };
 
-__global__ __launch_bounds__(256) void gram_ref_kernel(int n, GrefSrc s, int nbb,
+// a of lanes L0 .. L0 + 3 (or L0 alone) of each 16, times b.  s_nop: a DPP read
+// comes two wait states after the write of its register.
+template <int L0>
+__device__ __forceinline__ void bcast_mul4(double *p, double a, double b)
+{
+    p[0] = p[1] = p[2] = p[3] = 0.0;
+#define CACG_BM(r, l) "v_fmac_f64_dpp %" #r ", %4, %5 row_newbcast:%" #l " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" CACG_BM(0, 6) CACG_BM(1, 7) CACG_BM(2, 8) CACG_BM(3, 9)
+        : "+&v"(p[0]), "+&v"(p[1]), "+&v"(p[2]), "+&v"(p[3])
+        : "v"(a), "v"(b), "n"(L0), "n"(L0 + 1), "n"(L0 + 2), "n"(L0 + 3));
+#undef CACG_BM
+}
+template <int L0>
+__device__ __forceinline__ double bcast_mul(double a, double b)
+{
+    double p = 0.0;
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+        : "+&v"(p)
+        : "v"(a), "v"(b), "n"(L0));
+    return p;
+}
+template <int L0, int NJ>
+__device__ __forceinline__ void bcast_row(double *p, double a, double b)
+{
+    if constexpr (NJ >= 4) {
+        bcast_mul4<L0>(p, a, b);
+        if constexpr (NJ > 4)
+            bcast_row<L0 + 4, NJ - 4>(p + 4, a, b);
+    } else {
+        p[0] = bcast_mul<L0>(a, b);
+        if constexpr (NJ > 1)
+            bcast_row<L0 + 1, NJ - 1>(p + 1, a, b);
+    }
+}
+
+// the LDS accesses of every wave before it are done, loads from memory may be
+// in flight
+__device__ __forceinline__ void lds_barrier()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// products of row pair U / 2, U / 2 + 1, .. of a lane's RL rows
+template <int NJ, int U = 0>
+__device__ __forceinline__ void gref_products(double2 *out, const double *va, const double *vb)
+{
+    using SH = GrefShape<NJ>;
+    double x[NJ], y[NJ];
+    bcast_row<U % SH::RA * SH::JP, NJ>(x, va[U / SH::RA], vb[U]);
+    bcast_row<(U + 1) % SH::RA * SH::JP, NJ>(y, va[(U + 1) / SH::RA], vb[U + 1]);
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+        out[U / 2 * NJ * 16 + j * 16] = make_double2(x[j], y[j]);
+    if constexpr (U + 2 < SH::RL)
+        gref_products<NJ, U + 2>(out, va, vb);
+}
+
+template <int NJ>
+__global__ __launch_bounds__(512) void gram_ref_kernel(int n, GrefSrc s, int nbb,
                                                        double *__restrict__ G1,
                                                        double *__restrict__ G2)
 {
-    __shared__ double stg[2][GREF_ROWS * 16];   // row r: L values 0..7, R values 8..15
-    const int t = threadIdx.x;
-    const int a0 = (blockIdx.x / nbb) * 8, b0 = (blockIdx.x % nbb) * 8;
+    using SH = GrefShape<NJ>;
+    constexpr int CH = NJ * 16;   // chains
+    extern __shared__ double2 gref_lds[];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    // an XCD's workgroups take consecutive blocks, so they share columns of L
+    const int q8 = gridDim.x >> 3, r8 = gridDim.x & 7, xcd = blockIdx.x & 7;
+    const int id = xcd * q8 + (xcd < r8 ? xcd : r8) + (blockIdx.x >> 3);
+    const int a0 = id / nbb * NJ, b0 = id % nbb * 16;
     const int kr = s.kr1 + s.kr2;
-    const long nst = ((long)n + GREF_ROWS - 1) / GREF_ROWS;
-    // loader lanes: stage st into buffer st & 1, all loads before the stores
-    auto produce = [&](long st) {
-        double *buf = stg[st & 1];
-        const long i0 = st * GREF_ROWS;
-        const int cnt = (n - i0 < GREF_ROWS ? (int)(n - i0) : GREF_ROWS) * 16;
-        const int tp = t - 64;
-        double v[GREF_J];
-#pragma unroll
-        for (int j = 0; j < GREF_J; j++) {
-            const int e = tp + 192 * j;
-            // rows and columns past the last are clamped to it (never summed)
-            const long i = i0 + (e >> 4) < n ? i0 + (e >> 4) : (long)n - 1;
-            const int q = e & 15, qb = q < 8 ? 0 : q - 8;
-            const int a = a0 + q < s.kl ? a0 + q : s.kl - 1;
-            const int bb = b0 + qb < kr ? b0 + qb : kr - 1;
-            const double *pr = bb < s.kr1 ? s.R1 + i * s.ld1 + bb : s.R2 + i * s.ld2 + (bb - s.kr1);
-            const double *p = q < 8 ? s.L + i * s.ldl + a : pr;
-            v[j] = e < cnt ? *p : 0.0;
+    const int nst = (int)(((unsigned)n + SH::ROWS - 1) / SH::ROWS);
+    if (w >= SH::CW) {
+        // with one chain wave, wave 4 (which shares its SIMD) only keeps the barriers
+        const int wp = SH::CW == 2 ? w - 2 : w < 4 ? w - 1 : w == 4 ? -1 : w - 2;
+        if (wp < 0) {
+            for (int st = 0; st <= nst; st++)
+                lds_barrier();
+            return;
         }
+        const int c = lane & 15;
+        // columns past the last are clamped to it (their sums are not stored)
+        const int a = min(a0 + min(c % SH::JP, NJ - 1), s.kl - 1), b = min(b0 + c, kr - 1);
+        const long la = s.ldl, lb = b < s.kr1 ? s.ld1 : s.ld2;
+        const unsigned r0 = (wp * 4 + (lane >> 4)) * SH::RL;   // first of the lane's rows of a stage
+        unsigned il = r0, ip = r0;                             // of the next load, the next products
+        const unsigned ra = c / SH::JP;
+        const double *pa = s.L + a, *pb = b < s.kr1 ? s.R1 + b : s.R2 + (b - s.kr1);
+        const double *const ea = pa + (n - 1L) * la, *const eb = pb + (n - 1L) * lb;
+        pa += (r0 + ra) * la;
+        pb += r0 * lb;
+        double va[GREF_D][SH::NA], vb[GREF_D][SH::RL];
+        // EDGE: rows past the last may come; the last row is read again and zero
+        // products formed, which change no sum (no chain is ever -0)
+        auto load = [&](auto edge, int d) {
 #pragma unroll
-        for (int j = 0; j < GREF_J; j++) {
-            const int e = tp + 192 * j;
-            if (e < cnt)
-                buf[e] = v[j];
-        }
-    };
-    if (t >= 64 && nst > 0)
-        produce(0);
-    __syncthreads();
-    const int ai = t >> 3, bi = t & 7;
-    double acc = 0.0;
-    for (long st = 0; st < nst; st++) {
-        if (t >= 64) {
-            if (st + 1 < nst)
-                produce(st + 1);
-        } else {
-            const double *buf = stg[st & 1];
-            const long i0 = st * GREF_ROWS;
-            const int rows = n - i0 < GREF_ROWS ? (int)(n - i0) : GREF_ROWS;
-            int r = 0;
-            if (rows >= 32) {
-                double la[16], ra[16], lb[16], rb[16];
-#pragma unroll
-                for (int u = 0; u < 16; u++) {
-                    la[u] = buf[u * 16 + ai];
-                    ra[u] = buf[u * 16 + 8 + bi];
-                }
-                for (; r + 32 <= rows; r += 32) {
-#pragma unroll
-                    for (int u = 0; u < 16; u++) {
-                        lb[u] = buf[(r + 16 + u) * 16 + ai];
-                        rb[u] = buf[(r + 16 + u) * 16 + 8 + bi];
-                    }
-#pragma unroll
-                    for (int u = 0; u < 16; u++)
-                        acc = add_rn(acc, mul_rn(la[u], ra[u]));
-                    if (r + 64 <= rows) {
-#pragma unroll
-                        for (int u = 0; u < 16; u++) {
-                            la[u] = buf[(r + 32 + u) * 16 + ai];
-                            ra[u] = buf[(r + 32 + u) * 16 + 8 + bi];
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < 16; u++)
-                        acc = add_rn(acc, mul_rn(lb[u], rb[u]));
-                }
+            for (int k = 0; k < SH::NA; k++) {
+                const double *q = pa + k * SH::RA * la;
+                va[d][k] = *(!edge || il + ra + k * SH::RA < (unsigned)n ? q : ea);
             }
-            for (; r < rows; r++)
-                acc = add_rn(acc, mul_rn(buf[r * 16 + ai], buf[r * 16 + 8 + bi]));
+#pragma unroll
+            for (int u = 0; u < SH::RL; u++) {
+                const double *q = pb + u * lb;
+                vb[d][u] = *(!edge || il + u < (unsigned)n ? q : eb);
+            }
+            pa += SH::ROWS * la;
+            pb += SH::ROWS * lb;
+            il += SH::ROWS;
+        };
+        double2 *const out = gref_lds + (r0 >> 1) * CH + c;
+        auto produce = [&](auto edge, int buf, int d) {
+            if constexpr (edge) {
+                double xa[SH::NA], xb[SH::RL];
+#pragma unroll
+                for (int k = 0; k < SH::NA; k++)
+                    xa[k] = ip + ra + k * SH::RA < (unsigned)n ? va[d][k] : 0.0;
+#pragma unroll
+                for (int u = 0; u < SH::RL; u++)
+                    xb[u] = ip + u < (unsigned)n ? vb[d][u] : 0.0;
+                gref_products<NJ>(out + buf * SH::BUF, xa, xb);
+            } else {
+                gref_products<NJ>(out + buf * SH::BUF, va[d], vb[d]);
+            }
+            ip += SH::ROWS;
+        };
+        // stage st + 1 while stage st is summed; the last turn forms a stage that
+        // nothing reads
+        auto stage = [&](auto edge, int d) {
+            produce(edge, (d + 1) & 1, (d + 1) % GREF_D);
+            load(edge, (d + 1) % GREF_D);
+            lds_barrier();
+        };
+#pragma unroll
+        for (int d = 0; d < GREF_D; d++) {
+            load(std::true_type(), d);
+            __builtin_amdgcn_sched_barrier(0);   // in this order: waits count loads
         }
-        __syncthreads();
+        produce(std::true_type(), 0, 0);
+        load(std::true_type(), 0);
+        lds_barrier();
+        const int inner = n / SH::ROWS - 2 * GREF_D - 1;   // loads reach stage st + 2 D
+        int st = 0;
+        for (; st <= inner; st += GREF_D) {
+#pragma unroll
+            for (int d = 0; d < GREF_D; d++)
+                stage(std::false_type(), d);
+        }
+        for (; st < nst; st += GREF_D) {
+#pragma unroll
+            for (int d = 0; d < GREF_D; d++)
+                if (st + d < nst)
+                    stage(std::true_type(), d);
+        }
+        return;
     }
-    if (t < 64) {
-        const int a = a0 + ai, b = b0 + bi;
-        if (a < s.kl) {
-            if (b < s.kr1)
-                G1[(long)a * s.kr1 + b] = acc;
-            else if (b < kr)
-                G2[(long)a * s.kr2 + (b - s.kr1)] = acc;
+    __builtin_amdgcn_s_setprio(3);
+    const int ch = w * 64 + lane;
+    if (ch >= CH)
+        return;
+    const double2 *const col = gref_lds + ch;
+    const double2 *p = col;
+    double2 x[SH::BP], y[SH::BP];
+    double acc = 0.0;
+    auto read = [&](double2 *v, int b) {
+#pragma unroll
+        for (int u = 0; u < SH::BP; u++)
+            v[u] = p[(b * SH::BP + u) * CH];
+        __builtin_amdgcn_sched_barrier(0);   // ahead of the sums, and no further
+    };
+    auto sum = [&](const double2 *v) {
+#pragma unroll
+        for (int u = 0; u < SH::BP; u++) {
+            acc = add_rn(acc, v[u].x);
+            acc = add_rn(acc, v[u].y);
         }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    lds_barrier();
+    read(x, 0);
+    for (int st = 0; st < nst; st++) {
+#pragma unroll
+        for (int b = 1; b < SH::NB; b += 2) {
+            read(y, b);
+            sum(x);
+            if (b + 1 == SH::NB) {
+                lds_barrier();
+                p = col + ((st + 1) & 1) * SH::BUF;
+                read(x, 0);
+            } else {
+                read(x, b + 1);
+            }
+            sum(y);
+        }
+    }
+    const int a = a0 + (ch >> 4), b = b0 + (ch & 15);
+    if (a < s.kl) {
+        if (b < s.kr1)
+            G1[(long)a * s.kr1 + b] = acc;
+        else if (b < kr)
+            G2[(long)a * s.kr2 + (b - s.kr1)] = acc;
     }
 }
 
@@ -885,6 +1020,22 @@ int gram_fast(int n, const TL *L, long ldl, int kl, const T1 *R1, long ld1, int 
 
 }  // namespace
 
+namespace {
+
+template <int NJ>
+int launch_gram_ref(int n, const GrefSrc &s, long blocks, int nbb, double *G1, double *G2,
+                    hipStream_t st)
+{
+    constexpr size_t lds = 2 * GrefShape<NJ>::BUF * sizeof(double2);
+    cacg_allow_lds(gram_ref_kernel<NJ>, lds);
+    hipLaunchKernelGGL(gram_ref_kernel<NJ>, dim3((unsigned)blocks), dim3(512), lds, st, n, s, nbb,
+                       G1, G2);
+    CACG_LAUNCH_CHECK();
+    return 0;
+}
+
+}  // namespace
+
 extern "C" int cacg_k_gram_ref(int n, const double *L, long ldl, int kl, const double *R1, long ld1,
                                int kr1, const double *R2, long ld2, int kr2, double *G1,
                                double *G2, hipStream_t st)
@@ -901,12 +1052,20 @@ extern "C" int cacg_k_gram_ref(int n, const double *L, long ldl, int kl, const d
         return rc;
     }
     const int kr = kr1 + kr2;
-    const int nab = (kl + 7) / 8, nbb = (kr + 7) / 8;
     const GrefSrc s = {L, ldl, kl, R1, ld1, kr1, R2, ld2, kr2};
-    hipLaunchKernelGGL(gram_ref_kernel, dim3((unsigned)(nab * nbb)), dim3(256), 0, st, n, s, nbb,
-                       G1, G2);
-    CACG_LAUNCH_CHECK();
-    return 0;
+    // the narrowest block whose grid gives no CU a second workgroup: 262,144 rows
+    // take 1.06, 1.24, 1.47, 1.86 ms with NJ = 1, 2, 4, 5
+    const int nbb = (kr + 15) / 16;
+    const auto blocks = [&](int nj) { return (long)((kl + nj - 1) / nj) * nbb; };
+#define CACG_GREF(nj)                                                                             \
+    if (blocks(nj) <= 256)                                                                        \
+    return launch_gram_ref<nj>(n, s, blocks(nj), nbb, G1, G2, st)
+    CACG_GREF(1);
+    CACG_GREF(2);
+    CACG_GREF(4);
+    CACG_GREF(5);
+#undef CACG_GREF
+    return launch_gram_ref<8>(n, s, blocks(8), nbb, G1, G2, st);
 }
 
 extern "C" long cacg_gram_workspace(int kl, int kr)

@@ -106,3 +106,32 @@ def test_tsqr_strided_input(gpu_lib, n, k, lda):
     assert np.all(np.tril(R, -1) == 0.0) and np.all(np.diag(R) > 0)
     assert np.abs(Q.T @ Q - np.eye(k)).max() <= 50 * k * EPS / 2
     assert np.linalg.norm(Q @ R - W[:, :k]) <= 1e-13 * np.linalg.norm(W[:, :k])
+
+
+# blocks of 1, 2, 4, 5 and 8 columns of L by the size of G; stages of 192, 96 or 48 rows, the
+# last 8 or so of them checked row by row
+GREF = [(1, 1, 1, 0), (191, 3, 3, 2), (192, 16, 15, 1), (193, 17, 33, 3), (1728, 20, 16, 4),
+        (1727, 60, 60, 10), (1921, 33, 128, 16), (96, 128, 128, 0), (863, 112, 112, 14),
+        (865, 127, 128, 0), (97, 128, 128, 16), (960, 125, 126, 18), (49, 160, 160, 20),
+        (431, 161, 150, 17), (433, 168, 168, 1)]
+
+
+@pytest.mark.parametrize("n,kl,kr1,kr2", GREF)
+def test_gram_reference_edges_bitwise(gpu_lib, oracle_lib, n, kl, kr1, kr2):
+    rng = np.random.default_rng(n + kl + kr1 + kr2)
+    L, R1, R2 = (rng.standard_normal((n, k)) for k in (kl, kr1, kr2))
+    print(f"reference gram n={n} {kl} x ({kr1} + {kr2})", flush=True)
+    out = gpu_lib.k_gram(L, R1, R2 if kr2 else None, mode="reference")
+    G1, G2 = out if kr2 else (out, None)
+    assert np.array_equal(G1, oracle_lib.gram(L, R1))
+    if kr2:
+        assert np.array_equal(G2, oracle_lib.gram(L, R2))
+
+
+@pytest.mark.parametrize("n,m,ld", [(15, 4, 4), (16, 5, 7), (17, 3, 3), (511, 6, 6), (512, 16, 16),
+                                    (513, 7, 9), (1025, 9, 9)])
+def test_colnorm2_reference_edges_bitwise(gpu_lib, oracle_lib, n, m, ld):
+    R = np.random.default_rng(n + m).standard_normal((n, m))
+    print(f"reference column norms n={n} m={m} ld={ld}", flush=True)
+    want = np.array([oracle_lib.col_norm2sq(R, c) for c in range(m)])
+    assert np.array_equal(gpu_lib.k_colnorm2_ref(R, ld), want)
