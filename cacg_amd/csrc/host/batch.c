@@ -72,7 +72,7 @@ typedef struct {
     long k;
     long o_it, n_it, o_fr, n_fr;
     long o_qc[9][2], n_qc[9][2], o_xc[9][2][2], n_xc[9][2][2];
-    long o_gc[2][25], n_gc[2][25];
+    long o_g[2], n_g[2], g_groups[2];
     long o_b0, n_b0, o_lu[2][2], n_lu[2][2], o_b1, n_b1, o_all, n_all, o_sys, n_sys;
     int s, f32, max_sm, pad_;
 } wlists;
@@ -704,19 +704,6 @@ static int retire(cacg_batch *b, breq *r, int status, const double *norm2)
     return arena_free(b, r->off, r->bytes);
 }
 
-/* MFMA tile class of a system's Gram (cacg_kb_gram_class): 1 and (tm, tn) when
- * tm = ceil(sm / 16) is 1 .. 8 and tn = ceil(kr / 16) is in tm .. tm + 2 */
-static int gram_class(const cacg_bsys *d, int which, int *tm, int *tn)
-{
-    const int kr = d->sm + (which ? d->m : 0);
-    const int a = (d->sm + 15) / 16, c = (kr + 15) / 16;
-    if (a < 1 || a > 8 || c < a || c > a + 2)
-        return 0;
-    *tm = a;
-    *tn = c;
-    return 1;
-}
-
 /* append {slot, 0 .. count - 1} */
 static long put_range(int2 *it, long k, int slot, int count)
 {
@@ -728,20 +715,15 @@ static long put_range(int2 *it, long k, int slot, int count)
     return k;
 }
 
-/* the Gram partials of every listed system (one MFMA launch per tile class),
- * then the chunk-ordered sums */
-static int gram_phase(cacg_batch *b, const int2 *di, const long *o, const long *cnt,
-                      const int2 *blocks, long nblocks, int which, int f32)
+/* the Gram partials of every listed system, then the chunk-ordered sums */
+static int gram_phase(cacg_batch *b, const wlists *L, int which)
 {
-    hipStream_t st = b->st;
-    int rc = cnt[0] > 0 ? (int)hipErrorInvalidValue : 0;   /* no class: not admissible */
-    for (int c = 1; c < 25 && rc == 0; c++) {
-        const int tm = 1 + (c - 1) / 3, tn = tm + (c - 1) % 3;
-        rc = cacg_kb_gram_class(b->d_sys, di + o[c], (int)cnt[c], which, f32, tm, tn, st);
-    }
-    if (rc == 0)
-        rc = cacg_kb_gram_reduce(b->d_sys, blocks, (int)nblocks, which, st);
-    return rc;
+    const int2 *di = b->d_items;
+    const int rc = cacg_kb_gram(b->d_sys, di + L->o_g[which], (int)L->n_g[which],
+                                (int)L->g_groups[which], which, L->f32, b->st);
+    return rc ? rc
+              : cacg_kb_gram_reduce(b->d_sys, di + (which ? L->o_b1 : L->o_b0),
+                                    (int)(which ? L->n_b1 : L->n_b0), which, b->st);
 }
 
 /* one outer iteration of a solo system with the single-system kernels (fast
@@ -889,7 +871,7 @@ static int batched_launches(cacg_batch *b, const wlists *L)
                 KCHK(cacg_kb_basis(b->d_sys, di + L->o_it, (int)L->n_it, j, f32, st));
         }
         KCHK(cacg_kb_q_from_s(b->d_sys, di + L->o_fr, (int)L->n_fr, f32, st));
-        KCHK(gram_phase(b, di, L->o_gc[0], L->n_gc[0], di + L->o_b0, L->n_b0, 0, f32));
+        KCHK(gram_phase(b, L, 0));
         KCHK(cacg_k_lu_batch(b->d_sys, di + L->o_lu[0][0], (int)L->n_lu[0][0], 0, 64, st));
         KCHK(cacg_k_lu_batch(b->d_sys, di + L->o_lu[0][1], (int)L->n_lu[0][1], 0, L->max_sm, st));
         for (int c = 1; c <= 8; c++)
@@ -897,7 +879,7 @@ static int batched_launches(cacg_batch *b, const wlists *L)
                 KCHK(cacg_kb_qupdate_class(b->d_sys, di + L->o_qc[c][ex], (int)L->n_qc[c][ex],
                                            16 * c, ex, f32, st));
         KCHK(cacg_kb_aq(b->d_sys, di + L->o_it, (int)L->n_it, st));
-        KCHK(gram_phase(b, di, L->o_gc[1], L->n_gc[1], di + L->o_b1, L->n_b1, 1, f32));
+        KCHK(gram_phase(b, L, 1));
         KCHK(cacg_k_lu_batch(b->d_sys, di + L->o_lu[1][0], (int)L->n_lu[1][0], 1, 64, st));
         KCHK(cacg_k_lu_batch(b->d_sys, di + L->o_lu[1][1], (int)L->n_lu[1][1], 1, L->max_sm, st));
         for (int c = 1; c <= 8; c++)
@@ -1168,23 +1150,22 @@ static int step_locked(cacg_batch *b, cacg_batch_stats *stats)
                 wl.n_xc[c][ex][h] = k - wl.o_xc[c][ex][h];
             }
         }
-    /* Gram chunks per tile class: [which][1 + 3 (tm - 1) + tn - tm]; [which][0] stays empty
-     * (every admissible system has a class) */
-    for (int w = 0; w < 2; w++)
-        for (int c = 0; c < 25; c++) {
-            wl.o_gc[w][c] = k;
+    /* Gram chunks, the widest systems (the longest workgroups) first */
+    for (int w = 0; w < 2; w++) {
+        wl.o_g[w] = k;
+        for (int c = 8; c >= 1; c--)
             FOR_BATCHED(i) {
-                const breq *r = b->slot[i];
-                if (!BATCHED(i) || !r->joined || (w == 0 && r->fresh))
+                const cacg_bsys *d = &b->h_sys[i];
+                if (!BATCHED(i) || !b->slot[i]->joined || (w == 0 && b->slot[i]->fresh) ||
+                    (d->sm + 15) / 16 != c)
                     continue;
-                int tm = 0, tn = 0, cls = 0;
-                if (gram_class(&b->h_sys[i], w, &tm, &tn))
-                    cls = 1 + 3 * (tm - 1) + (tn - tm);
-                if (cls == c)
-                    k = put_range(it, k, i, b->h_sys[i].nchunk);
+                const int g = cacg_bgram_groups(d->sm, d->sm + (w ? d->m : 0));
+                if (g > wl.g_groups[w])
+                    wl.g_groups[w] = g;
+                k = put_range(it, k, i, d->nchunk);
             }
-            wl.n_gc[w][c] = k - wl.o_gc[w][c];
-        }
+        wl.n_g[w] = k - wl.o_g[w];
+    }
     wl.o_b0 = k;
     FOR_BATCHED(i)
         if (BATCHED(i) && b->slot[i]->joined && !b->slot[i]->fresh) {

@@ -269,236 +269,177 @@ __global__ __launch_bounds__(256) void baq_kernel(const cacg_bsys *__restrict__ 
     }
 }
 
-// LDS row stride of k doubles: 16 mod 32, so a wave's operand read (4 rows x
-// 16 doubles) falls on disjoint halves of the 64 banks
-constexpr int bstride(int k)
-{
-    return k + (48 - k % 32) % 32;
-}
+// ---- Gram partials ------------------------------------------------------------------
 
-// waves of the Gram kernel of tile class TM
-constexpr int gram_waves(int TM)
-{
-    return TM >= 4 ? 8 : 4;
-}
-
-// rows per stage of the Gram kernel: the narrow classes do little work per
-// row, so their stages are longer (fewer load round trips and barriers; the
-// rows are still taken in order)
-constexpr int gram_stage(int TM)
-{
-    return TM <= 2 ? 64 : 16;
-}
-
-// MFMA Gram partial of one 2048-row chunk for systems with TM = ceil(sm / 16)
-// row tiles and TN = ceil(kr / 16) column tiles (columns past sm and kr are
-// zeros in LDS and are not written); WHICH 0: Q^T A S = AQ^T S, 1: Q^T [AQ | R].
-// NW waves split the TM x TN tiles into GMG x GNG groups of MT x NT tiles.
-// Stages of GS rows of L and of [R1 | R2] are loaded with 16-byte vectors
-// where a row's width allows (single elements otherwise) into registers one
-// stage ahead, stored to one of two LDS buffers and read as MFMA operands
-// (contraction index = row).  Per tile the k-steps run in row order from
-// zero (rows past the chunk are zeros), so the partial depends on the system
+// A round lists a few hundred chunks of 2048 rows at most, so the chip is filled
+// by splitting a chunk's output tiles, not its rows, over waves: a wave owns one
+// 16 x 16 tile (systems of up to BG_SMALL tiles) or 2 x 2 of them and feeds the
+// MFMAs straight from global memory, lane l loading L and [R1 | R2] at row
+// l / 16 of each step of 4 and its own columns, BG_D steps ahead in registers.
+// No LDS, no barrier; the rows that the 4 waves of a workgroup share come from
+// L1, and grid.x is a multiple of 8, so a chunk's workgroups (grid.y) share an
+// L2.  One launch serves every width.  Per tile the k-steps run in row order
+// from zero (rows past the chunk are zeros), so a partial depends on the system
 // alone.
-template <typename TB, int TM, int TN, int WHICH>
-__global__ __launch_bounds__(gram_waves(TM) * 64) void bgram_mfma_kernel(
-    const cacg_bsys *__restrict__ sys, const int2 *__restrict__ items)
+constexpr int BG_SMALL = CACG_BGRAM_SMALL;
+
+template <int MT, int NT>
+struct BgDepth {   // steps in flight: about 2000 to 3000 cycles of MFMAs
+    static constexpr int D = MT * NT == 1 ? 32 : MT * NT == 2 ? 20 : 12;
+};
+
+template <typename T1, int MT, int NT>
+__device__ __forceinline__ void bgram_tiles(const double *const *pa0, long sa, const T1 *const *pb0,
+                                            const long *sb, int rows, double *gp, int sm, int kr,
+                                            int a0, int b0)
 {
-    constexpr int NW = gram_waves(TM), NTH = NW * 64, GS = gram_stage(TM);
-    constexpr int GMG = TM < NW ? TM : NW, GNG = NW / GMG;
-    constexpr int MT = (TM + GMG - 1) / GMG, NT = (TN + GNG - 1) / GNG;
-    constexpr int KL = TM * 16, KR = TN * 16, LP = bstride(KL), RP = bstride(KR);
-    constexpr int BUF = GS * (LP + RP);
-    // register slots per lane and stage: L and R1 up to GS x KL elements, R2 up
-    // to GS x 32, one element or one 16-byte vector each
-    constexpr int SLL = (GS * KL + NTH - 1) / NTH, SL2 = (GS * MM + NTH - 1) / NTH;
-    using T1 = typename std::conditional<WHICH == 1, double, TB>::type;
-    extern __shared__ double lds[];
-    const int2 it = items[blockIdx.x];
-    const cacg_bsys &d = sys[it.x];
-    const int n = d.n, m = d.m, sm = d.sm;
-    const int kr = sm + (WHICH ? m : 0);
-    const double *L = WHICH ? d.Q : d.AQ;
-    const T1 *R1 = WHICH ? reinterpret_cast<const T1 *>(d.AQ) : reinterpret_cast<const T1 *>(d.S);
-    const int c0 = it.y * GR, c1 = (c0 + GR) < n ? (c0 + GR) : n;
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, lr = lane >> 4, lc = lane & 15;
-    const int gm = wave % GMG, gn = wave / GMG;
-    const bool active = gn < GNG;
-
-    // element widths of one load: 2 doubles / 4 floats where the row width
-    // (and so every row start) allows 16-byte alignment
-    constexpr int V1 = 16 / (int)sizeof(T1);
-    const int wl = sm % 2 == 0 ? 2 : 1, w1 = sm % V1 == 0 ? V1 : 1;
-    const int w2 = m % 2 == 0 ? 2 : 1;
-    const int nl = sm / wl, n1 = sm / w1, n2 = WHICH ? m / w2 : 0;
-    int lrow[SLL], lcol[SLL], r1row[SLL], r1col[SLL], r2row[SL2], r2col[SL2];
-#pragma unroll
-    for (int u = 0; u < SLL; u++) {
-        const int v = t + NTH * u;
-        lrow[u] = v < GS * nl ? v / nl : -1;
-        lcol[u] = v < GS * nl ? (v % nl) * wl : 0;
-        r1row[u] = v < GS * n1 ? v / n1 : -1;
-        r1col[u] = v < GS * n1 ? (v % n1) * w1 : 0;
-    }
-#pragma unroll
-    for (int u = 0; u < SL2; u++) {
-        const int v = t + NTH * u;
-        r2row[u] = v < GS * n2 ? v / n2 : -1;
-        r2col[u] = v < GS * n2 ? (v % n2) * w2 : 0;
-    }
-    using V1T = typename std::conditional<sizeof(T1) == 4, float4, double2>::type;
-    double2 gl[SLL], g2[SL2];
-    V1T g1[SLL];
-    auto gload = [&](int rb) {
-#pragma unroll
-        for (int u = 0; u < SLL; u++) {
-            const long i = rb + lrow[u];
-            gl[u] = double2{0.0, 0.0};
-            if (lrow[u] >= 0 && i < c1) {
-                const double *p = L + i * sm + lcol[u];
-                if (wl == 2)
-                    gl[u] = *reinterpret_cast<const double2 *>(p);
-                else
-                    gl[u] = double2{p[0], 0.0};
-            }
-            const long i1 = rb + r1row[u];
-            if constexpr (sizeof(T1) == 4)
-                g1[u] = float4{0.f, 0.f, 0.f, 0.f};
-            else
-                g1[u] = double2{0.0, 0.0};
-            if (r1row[u] >= 0 && i1 < c1) {
-                const T1 *p = R1 + i1 * sm + r1col[u];
-                if (w1 == V1)
-                    g1[u] = *reinterpret_cast<const V1T *>(p);
-                else if constexpr (sizeof(T1) == 4)
-                    g1[u] = float4{p[0], 0.f, 0.f, 0.f};
-                else
-                    g1[u] = double2{p[0], 0.0};
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < SL2; u++) {
-            const long i = rb + r2row[u];
-            g2[u] = double2{0.0, 0.0};
-            if (r2row[u] >= 0 && i < c1) {
-                const double *p = d.R + i * m + r2col[u];
-                if (w2 == 2)
-                    g2[u] = *reinterpret_cast<const double2 *>(p);
-                else
-                    g2[u] = double2{p[0], 0.0};
-            }
-        }
-    };
-    auto lstore = [&](int buf) {
-        double *Ls = lds + buf * BUF, *Rs = Ls + GS * LP;
-#pragma unroll
-        for (int u = 0; u < SLL; u++) {
-            if (lrow[u] >= 0) {
-                Ls[lrow[u] * LP + lcol[u]] = gl[u].x;
-                if (wl == 2)
-                    Ls[lrow[u] * LP + lcol[u] + 1] = gl[u].y;
-            }
-            if (r1row[u] >= 0) {
-                double *q = Rs + r1row[u] * RP + r1col[u];
-                if constexpr (sizeof(T1) == 4) {
-                    q[0] = (double)g1[u].x;
-                    if (w1 == 4) {
-                        q[1] = (double)g1[u].y;
-                        q[2] = (double)g1[u].z;
-                        q[3] = (double)g1[u].w;
-                    }
-                } else {
-                    q[0] = g1[u].x;
-                    if (w1 == 2)
-                        q[1] = g1[u].y;
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < SL2; u++) {
-            if (r2row[u] >= 0) {
-                double *q = Rs + r2row[u] * RP + sm + r2col[u];
-                q[0] = g2[u].x;
-                if (w2 == 2)
-                    q[1] = g2[u].y;
-            }
-        }
-    };
-
-    // the padding columns (past sm in L, past kr in R) stay zero in both buffers
-    for (int e = t; e < 2 * GS; e += NTH) {
-        double *Ls = lds + (e / GS) * BUF, *Rs = Ls + GS * LP;
-        const int r = e % GS;
-        for (int c = sm; c < KL; c++)
-            Ls[r * LP + c] = 0.0;
-        for (int c = kr; c < KR; c++)
-            Rs[r * RP + c] = 0.0;
-    }
+    constexpr int D = BgDepth<MT, NT>::D;
+    const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15;
+    const double *pa[MT], *ea[MT];
+    const T1 *pb[NT], *eb[NT];
+    double va[D][MT];
+    T1 vb[D][NT];
     dbl4 acc[MT][NT];
+    // rows past the last: the last row is read again and zeros are multiplied
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        ea[i] = pa0[i] + (rows - 1L) * sa;
+        pa[i] = pa0[i] + lr * sa;
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+            acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+    }
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        eb[j] = pb0[j] + (rows - 1L) * sb[j];
+        pb[j] = pb0[j] + lr * sb[j];
+    }
+    int il = lr, im = lr;   // row of the next load, of the next step
+    auto load = [&](auto edge, int d) {
+        const bool in = !edge || il < rows;
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            va[d][i] = *(in ? pa[i] : ea[i]);
+            pa[i] += 4 * sa;
+        }
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            vb[d][j] = *(in ? pb[j] : eb[j]);
+            pb[j] += 4 * sb[j];
+        }
+        il += 4;
+    };
+    auto step = [&](auto edge, int d) {
+        const bool in = !edge || im < rows;
+        double x[MT], y[NT];
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+            x[i] = in ? va[d][i] : 0.0;
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+            y[j] = in ? (double)vb[d][j] : 0.0;
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                acc[i][j] = mfma16x16x4(x[i], y[j], acc[i][j]);
+        im += 4;
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+        load(std::true_type(), d);
+        __builtin_amdgcn_sched_barrier(0);   // in this order: waits count loads
+    }
+    const int nk = (rows + 3) / 4, full = rows / 4;
+    int k = 0;
+    for (; k + 2 * D <= full; k += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            step(std::false_type(), d);
+            load(std::false_type(), d);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    for (; k < nk; k += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++)
+            if (k + d < nk) {
+                step(std::true_type(), d);
+                load(std::true_type(), d);
+            }
+    }
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
         for (int j = 0; j < NT; j++)
-            acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
-    const int nst = (c1 - c0 + GS - 1) / GS;
-    gload(c0);
-    lstore(0);
-    if (nst > 1)
-        gload(c0 + GS);
-    __syncthreads();
-    for (int stg = 0; stg < nst; stg++) {
-        const int cur = stg & 1;
-        if (active) {
-            const double *Ls = lds + cur * BUF, *Rs = Ls + GS * LP;
-#pragma unroll
-            for (int ks = 0; ks < GS / 4; ks++) {
-                const int row = ks * 4 + lr;
-                double av[MT], bv[NT];
-#pragma unroll
-                for (int i = 0; i < MT; i++) {
-                    const int a = (gm * MT + i) * 16 + lc;
-                    av[i] = a < KL ? Ls[row * LP + a] : 0.0;
-                }
-#pragma unroll
-                for (int j = 0; j < NT; j++) {
-                    const int b = (gn * NT + j) * 16 + lc;
-                    bv[j] = b < KR ? Rs[row * RP + b] : 0.0;
-                }
-#pragma unroll
-                for (int i = 0; i < MT; i++)
-#pragma unroll
-                    for (int j = 0; j < NT; j++)
-                        acc[i][j] = mfma16x16x4(av[i], bv[j], acc[i][j]);
-            }
-        }
-        if (stg + 1 < nst) {
-            lstore(cur ^ 1);
-            if (stg + 2 < nst)
-                gload(c0 + (stg + 2) * GS);
-        }
-        __syncthreads();
-    }
-    if (!active)
-        return;
-    double *gp = d.gpart + (long)it.y * sm * kr;
-#pragma unroll
-    for (int i = 0; i < MT; i++) {
-        const int tm = gm * MT + i;
-        if (tm >= TM)
-            continue;
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            const int tn = gn * NT + j;
-            if (tn >= TN)
-                continue;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int a = tm * 16 + lr + 4 * r, b = tn * 16 + lc;
+                const int a = a0 + i * 16 + lr + 4 * r, b = b0 + j * 16 + lc;
                 if (a < sm && b < kr)
                     gp[(long)a * kr + b] = acc[i][j][r];
             }
+}
+
+// WHICH 0: Q^T A S = AQ^T S, 1: Q^T [AQ | R]
+template <typename TB, int WHICH>
+__global__ __launch_bounds__(256) void bgram_kernel(const cacg_bsys *__restrict__ sys,
+                                                    const int2 *__restrict__ items, int count)
+{
+    using T1 = typename std::conditional<WHICH == 1, double, TB>::type;
+    if ((int)blockIdx.x >= count)
+        return;
+    const int2 it = items[blockIdx.x];
+    const cacg_bsys &d = sys[it.x];
+    const int m = d.m, sm = d.sm, kr = sm + (WHICH ? m : 0);
+    const int tm = (sm + 15) / 16, tn = (kr + 15) / 16;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int ti, tj, mt = 1, nt = 1;   // the wave's first tile and how many
+    if (tm * tn <= BG_SMALL) {
+        const int tile = blockIdx.y * 4 + w;
+        ti = tile / tn;
+        tj = tile - ti * tn;
+    } else {
+        const int gn = (tn + 3) / 4, g = blockIdx.y / gn;
+        ti = g * 4 + (w >> 1) * 2;
+        tj = (blockIdx.y - g * gn) * 4 + (w & 1) * 2;
+        mt = tm - ti >= 2 ? 2 : 1;
+        nt = tn - tj >= 2 ? 2 : 1;
+    }
+    if (ti >= tm || tj >= tn)
+        return;
+    const int lc = threadIdx.x & 15;
+    const long c0 = (long)it.y * GR;
+    const int rows = d.n - c0 < GR ? (int)(d.n - c0) : GR;
+    // columns past the last are clamped to it (their sums are not stored)
+    const double *L = (WHICH ? d.Q : d.AQ) + c0 * sm;
+    const T1 *R1 = (WHICH ? reinterpret_cast<const T1 *>(d.AQ) : reinterpret_cast<const T1 *>(d.S)) +
+                   c0 * sm;
+    const double *pa[2];
+    const T1 *pb[2];
+    long sb[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int a = min((ti + u) * 16 + lc, sm - 1), b = min((tj + u) * 16 + lc, kr - 1);
+        pa[u] = L + a;
+        pb[u] = R1 + b;
+        sb[u] = sm;
+        if constexpr (WHICH == 1) {
+            if (b >= sm) {
+                pb[u] = d.R + c0 * m + (b - sm);
+                sb[u] = m;
+            }
         }
     }
+    double *gp = d.gpart + (long)it.y * sm * kr;
+    const int a0 = ti * 16, b0 = tj * 16;
+    if (mt == 1 && nt == 1)
+        bgram_tiles<T1, 1, 1>(pa, sm, pb, sb, rows, gp, sm, kr, a0, b0);
+    else if (mt == 1)
+        bgram_tiles<T1, 1, 2>(pa, sm, pb, sb, rows, gp, sm, kr, a0, b0);
+    else if (nt == 1)
+        bgram_tiles<T1, 2, 1>(pa, sm, pb, sb, rows, gp, sm, kr, a0, b0);
+    else
+        bgram_tiles<T1, 2, 2>(pa, sm, pb, sb, rows, gp, sm, kr, a0, b0);
 }
 
 // chunk-ordered sum of the partials, 256 result entries per workgroup
@@ -526,8 +467,22 @@ __global__ __launch_bounds__(256) void bgram_reduce_kernel(const cacg_bsys *__re
         d.QtR[(long)a * m + (b - sm)] = acc;
 }
 
+// rows [c0, c1) of chunk `chunk` that part blockIdx.y of gridDim.y takes, whole
+// multiples of `unit`; empty past the last.  Rows are independent in the
+// updates: the split changes no bit, so it follows the launch.
+struct part_rows {
+    int c0, c1;
+    __device__ __forceinline__ part_rows(int chunk, int n, int unit)
+    {
+        const int len = (GR / unit + (int)gridDim.y - 1) / (int)gridDim.y * unit;
+        const int e = chunk * GR + GR < n ? chunk * GR + GR : n;
+        c0 = chunk * GR + (int)blockIdx.y * len;
+        c1 = c0 + len < e ? c0 + len : e;
+    }
+};
+
 // Q = S - Q beta with FP64 MFMA for systems with 16 (SM / 16 - 1) < sm <= SM:
-// one 2048-row chunk per 512-lane workgroup, beta in LDS (zero-padded to
+// a part of a 2048-row chunk per 512-lane workgroup, beta in LDS (zero-padded to
 // SM x SM), each wave takes 16-row tiles of the chunk; the contraction index
 // is permuted across the lane groups (group g supplies k = g SM/4 + t at step
 // t), so each lane's A operand is SM/4 contiguous values of one row (16-byte
@@ -552,7 +507,8 @@ __global__ __launch_bounds__(512) void bqupdate_mfma_kernel(const cacg_bsys *__r
     double *Q = d.Q;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int lg = lane >> 4, lc = lane & 15;
-    const int c0 = it.y * GR, c1 = (c0 + GR) < n ? (c0 + GR) : n;
+    const part_rows pr(it.y, n, 128);
+    const int c0 = pr.c0, c1 = pr.c1;
     for (int i0 = c0 + wave * 16; i0 < c1; i0 += 8 * 16) {
         const long arow = i0 + lc;
         double av[KQ];
@@ -596,7 +552,7 @@ __global__ __launch_bounds__(512) void bqupdate_mfma_kernel(const cacg_bsys *__r
 }
 
 // X += Q alpha with FP64 MFMA for systems with 16 (SM / 16 - 1) < sm <= SM:
-// one 2048-row chunk per 256-lane workgroup, alpha (sm x m, m <= 16 NTM) in
+// a part of a 2048-row chunk per 256-lane workgroup, alpha (sm x m, m <= 16 NTM) in
 // registers in the K-permuted order of the A operand (zeros past sm), 16-row
 // tiles per wave; 16-byte Q loads when sm == SM (EXACT).
 template <int SM, int NTM, bool EXACT>
@@ -619,7 +575,8 @@ __global__ __launch_bounds__(256) void bxupdate_mfma_kernel(const cacg_bsys *__r
             alf[j][t] = (c < m && k < sm) ? d.alpha[(long)k * m + c] : 0.0;
         }
     }
-    const int c0 = it.y * GR, c1 = (c0 + GR) < n ? (c0 + GR) : n;
+    const part_rows pr(it.y, n, 64);
+    const int c0 = pr.c0, c1 = pr.c1;
     for (int i0 = c0 + wave * 16; i0 < c1; i0 += 4 * 16) {
         const long arow = i0 + lc;
         double av[KQ];
@@ -750,62 +707,28 @@ extern "C" int cacg_kb_aq(const cacg_bsys *d_sys, const int2 *d_tiles, int count
     return 0;
 }
 
-namespace {
-template <typename TB, int TM, int TN, int WHICH>
-void launch_bgram(const cacg_bsys *d_sys, const int2 *d_chunks, int nchunks, hipStream_t st)
+extern "C" int cacg_bgram_groups(int sm, int kr)
 {
-    constexpr int NW = gram_waves(TM);
-    const size_t shm =
-        2 * (size_t)gram_stage(TM) * (bstride(TM * 16) + bstride(TN * 16)) * sizeof(double);
-    cacg_allow_lds(bgram_mfma_kernel<TB, TM, TN, WHICH>, shm);
-    hipLaunchKernelGGL((bgram_mfma_kernel<TB, TM, TN, WHICH>), dim3(nchunks), dim3(NW * 64), shm,
-                       st, d_sys, d_chunks);
+    const int tm = (sm + 15) / 16, tn = (kr + 15) / 16;
+    return tm * tn <= BG_SMALL ? (tm * tn + 3) / 4 : ((tm + 3) / 4) * ((tn + 3) / 4);
 }
 
-template <typename TB, int TM>
-int launch_gram_class(const cacg_bsys *d_sys, const int2 *d_chunks, int nchunks, int which, int tn,
-                      hipStream_t st)
-{
-    // which 0: kr = sm (TN = TM); which 1: kr = sm + m, m <= 32 (TN - TM in 0..2)
-    if (which == 0 && tn == TM)
-        launch_bgram<TB, TM, TM, 0>(d_sys, d_chunks, nchunks, st);
-    else if (which == 1 && tn == TM)
-        launch_bgram<TB, TM, TM, 1>(d_sys, d_chunks, nchunks, st);
-    else if (which == 1 && tn == TM + 1)
-        launch_bgram<TB, TM, TM + 1, 1>(d_sys, d_chunks, nchunks, st);
-    else if (which == 1 && tn == TM + 2)
-        launch_bgram<TB, TM, TM + 2, 1>(d_sys, d_chunks, nchunks, st);
-    else
-        return (int)hipErrorInvalidValue;
-    CACG_LAUNCH_CHECK();
-    return 0;
-}
-}  // namespace
-
-extern "C" int cacg_kb_gram_class(const cacg_bsys *d_sys, const int2 *d_chunks, int nchunks,
-                                  int which, int f32, int tm, int tn, hipStream_t st)
+extern "C" int cacg_kb_gram(const cacg_bsys *d_sys, const int2 *d_chunks, int nchunks, int groups,
+                            int which, int f32, hipStream_t st)
 {
     if (nchunks <= 0)
         return 0;
-    if (which != 0 && which != 1)
+    if ((which != 0 && which != 1) || groups < 1 || groups > 65535)
         return (int)hipErrorInvalidValue;
-#define CACG_GCLASS(TMV)                                                                          \
-    case TMV:                                                                                     \
-        return f32 ? launch_gram_class<float, TMV>(d_sys, d_chunks, nchunks, which, tn, st)      \
-                   : launch_gram_class<double, TMV>(d_sys, d_chunks, nchunks, which, tn, st);
-    switch (tm) {
-        CACG_GCLASS(1)
-        CACG_GCLASS(2)
-        CACG_GCLASS(3)
-        CACG_GCLASS(4)
-        CACG_GCLASS(5)
-        CACG_GCLASS(6)
-        CACG_GCLASS(7)
-        CACG_GCLASS(8)
-    default:
-        return (int)hipErrorInvalidValue;
-    }
-#undef CACG_GCLASS
+    const dim3 grid((nchunks + 7) / 8 * 8, groups);
+    if (which == 1)
+        hipLaunchKernelGGL((bgram_kernel<double, 1>), grid, dim3(256), 0, st, d_sys, d_chunks, nchunks);
+    else if (f32)
+        hipLaunchKernelGGL((bgram_kernel<float, 0>), grid, dim3(256), 0, st, d_sys, d_chunks, nchunks);
+    else
+        hipLaunchKernelGGL((bgram_kernel<double, 0>), grid, dim3(256), 0, st, d_sys, d_chunks, nchunks);
+    CACG_LAUNCH_CHECK();
+    return 0;
 }
 
 extern "C" int cacg_kb_gram_reduce(const cacg_bsys *d_sys, const int2 *d_blocks, int nblocks,
@@ -819,16 +742,25 @@ extern "C" int cacg_kb_gram_reduce(const cacg_bsys *d_sys, const int2 *d_blocks,
     return 0;
 }
 
+// parts per chunk that bring `count` chunks to at most about `want` workgroups
+static int chunk_parts(int count, int want, int most)
+{
+    const int p = want / count;
+    return p < 1 ? 1 : p > most ? most : p;
+}
+
 extern "C" int cacg_kb_qupdate_class(const cacg_bsys *d_sys, const int2 *d_chunks, int count,
                                      int smp, int exact, int f32, hipStream_t st)
 {
     if (count <= 0)
         return 0;
     const size_t shm = (size_t)smp * smp * sizeof(double);
+    // parts: one workgroup per CU where beta takes its LDS, more where it does not
+    const int parts = chunk_parts(count, shm > 81920 ? 256 : 512, 16);
 #define CACG_QLAUNCH(TBV, SMV, EX)                                                                \
     do {                                                                                          \
         cacg_allow_lds(bqupdate_mfma_kernel<TBV, SMV, EX>, shm);                                  \
-        hipLaunchKernelGGL((bqupdate_mfma_kernel<TBV, SMV, EX>), dim3(count), dim3(512), shm, st, \
+        hipLaunchKernelGGL((bqupdate_mfma_kernel<TBV, SMV, EX>), dim3(count, parts), dim3(512), shm, st, \
                            d_sys, d_chunks);                                                      \
     } while (0)
 #define CACG_QCLASS(SMV)                                                                          \
@@ -870,8 +802,9 @@ extern "C" int cacg_kb_xupdate_class(const cacg_bsys *d_sys, const int2 *d_chunk
         return 0;
     if (m < 1 || m > 32)
         return (int)hipErrorInvalidValue;
+    const int parts = chunk_parts(count, 1024, 32);
 #define CACG_XLAUNCH(SMV, NT, EX)                                                                 \
-    hipLaunchKernelGGL((bxupdate_mfma_kernel<SMV, NT, EX>), dim3(count), dim3(256), 0, st, d_sys, \
+    hipLaunchKernelGGL((bxupdate_mfma_kernel<SMV, NT, EX>), dim3(count, parts), dim3(256), 0, st, d_sys, \
                        d_chunks)
 #define CACG_XCLASS(SMV)                                                                          \
     case SMV:                                                                                     \

@@ -274,14 +274,16 @@ int cacg_kb_q_from_s(const cacg_bsys *d_sys, const int2 *d_tiles, int count, int
                      hipStream_t st);
 /* AQ = A Q (FP64) */
 int cacg_kb_aq(const cacg_bsys *d_sys, const int2 *d_tiles, int count, hipStream_t st);
-/* Gram partials per 2048-row chunk with FP64 MFMA for the systems of one tile
- * class, tm = ceil(sm / 16) in 1 .. 8 and tn = ceil(kr / 16) in tm .. tm + 2,
- * kr = sm (which 0: QtAS = AQ^T S) or sm + m (which 1: [QtAQ | QtR] =
- * Q^T [AQ | R]); then the chunk-ordered sums by cacg_kb_gram_reduce ({slot,
- * 256-entry block} items).  Every admissible system (m <= 32, sm <= 128) is
- * in some class. */
-int cacg_kb_gram_class(const cacg_bsys *d_sys, const int2 *d_chunks, int nchunks, int which,
-                       int f32, int tm, int tn, hipStream_t st);
+/* Gram partials per 2048-row chunk with FP64 MFMA of every listed system:
+ * QtAS = AQ^T S (which 0, kr = sm) or [QtAQ | QtR] = Q^T [AQ | R] (which 1, kr =
+ * sm + m); then the chunk-ordered sums by cacg_kb_gram_reduce ({slot, 256-entry
+ * block} items).  `groups` workgroups share a chunk's 16 x 16 output tiles: at
+ * least cacg_bgram_groups(sm, kr) of every listed system.  Systems of up to
+ * CACG_BGRAM_SMALL tiles give each wave one. */
+#define CACG_BGRAM_SMALL 6
+int cacg_bgram_groups(int sm, int kr);
+int cacg_kb_gram(const cacg_bsys *d_sys, const int2 *d_chunks, int nchunks, int groups, int which,
+                 int f32, hipStream_t st);
 int cacg_kb_gram_reduce(const cacg_bsys *d_sys, const int2 *d_blocks, int nblocks, int which,
                         hipStream_t st);
 /* which 0: beta = QtAQ^{-1} QtAS (factor from the last which-1 call); which 1:

@@ -1,6 +1,8 @@
 """Kernel dispatch edges: widths and row counts around the tiles, panels and
 blocks of the fast-order Gram, the padded updates, the small LU and the QR."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -135,3 +137,53 @@ def test_colnorm2_reference_edges_bitwise(gpu_lib, oracle_lib, n, m, ld):
     print(f"reference column norms n={n} m={m} ld={ld}", flush=True)
     want = np.array([oracle_lib.col_norm2sq(R, c) for c in range(m)])
     assert np.array_equal(gpu_lib.k_colnorm2_ref(R, ld), want)
+
+
+class BSys(ctypes.Structure):
+    _fields_ = ([(f, ctypes.c_int) for f in ("n", "m", "sm", "ntile", "nchunk", "pad_")] +
+                [(f, ctypes.c_void_p) for f in ("rowptr", "col", "val", "val32", "B", "X", "R", "S",
+                                                "Q", "AQ", "QtAQ", "QtAS", "beta", "lu", "QtR",
+                                                "alpha", "gpart", "npart", "norm2", "flag")] +
+                [(f, ctypes.c_double) for f in ("sa", "sb")])
+
+
+# (n, m, sm) of systems that share a launch: one tile to 8 x 10, chunks of 1 to 2048 rows, steps
+# in flight 12 to 32
+BGRAM = [[(1, 1, 1)], [(127, 1, 4), (2048, 2, 8), (2049, 17, 17), (95, 32, 128)],
+         [(6000, 3, 9), (4097, 5, 20), (255, 8, 32), (2175, 10, 40)],
+         [(2047, 16, 64), (130, 32, 96), (2303, 30, 120), (383, 7, 112)], [(5000, 32, 128)]]
+
+
+@pytest.mark.parametrize("f32", [0, 1])
+@pytest.mark.parametrize("systems", BGRAM)
+def test_batched_gram_exact_on_integers(gpu_lib, systems, f32):
+    lib, D, rng = gpu_lib.lib(), gpu_lib.DeviceBuffer.from_array, np.random.default_rng(len(systems))
+    print(f"batched gram {systems} f32={f32}", flush=True)
+    descs, host, keep = (BSys * len(systems))(), [], []
+    for d, (n, m, sm) in zip(descs, systems):
+        Q, AQ, S = (rng.integers(-8, 9, size=(n, sm)).astype(np.float64) for _ in range(3))
+        R = rng.integers(-8, 9, size=(n, m)).astype(np.float64)
+        d.n, d.m, d.sm, d.ntile, d.nchunk = n, m, sm, (n + 63) // 64, (n + 2047) // 2048
+        bufs = dict(Q=D(Q), AQ=D(AQ), S=D(S.astype(np.float32) if f32 else S), R=D(R),
+                    gpart=D(np.full(d.nchunk * sm * (sm + m), np.nan)),
+                    QtAQ=D(np.full((sm, sm), np.nan)), QtAS=D(np.full((sm, sm), np.nan)),
+                    QtR=D(np.full((sm, m), np.nan)))
+        for f, b in bufs.items():
+            setattr(d, f, b.ptr)
+        host.append((Q, AQ, S, R))
+        keep.append(bufs)
+    dsys = D(np.frombuffer(bytes(descs), dtype=np.uint8))
+    for which in (0, 1):
+        kr = [sm + (m if which else 0) for _, m, sm in systems]
+        chunks = [(i, c) for i, d in enumerate(descs) for c in range(d.nchunk)]
+        blocks = [(i, e) for i, (_, _, sm) in enumerate(systems) for e in range((sm * kr[i] + 255) // 256)]
+        groups = max(lib.cacg_bgram_groups(sm, k) for (_, _, sm), k in zip(systems, kr))
+        dc, db = (D(np.array(v, dtype=np.int32)) for v in (chunks, blocks))
+        assert lib.cacg_kb_gram(dsys.ptr, dc.ptr, len(chunks), groups, which, f32, None) == 0
+        assert lib.cacg_kb_gram_reduce(dsys.ptr, db.ptr, len(blocks), which, None) == 0
+        for (n, m, sm), (Q, AQ, S, R), b in zip(systems, host, keep):
+            if which == 0:
+                assert np.array_equal(b["QtAS"].download((sm, sm)), AQ.T @ S)
+            else:
+                assert np.array_equal(b["QtAQ"].download((sm, sm)), Q.T @ AQ)
+                assert np.array_equal(b["QtR"].download((sm, m)), Q.T @ R)
