@@ -84,8 +84,8 @@ typedef struct {
  * are the solve's own (a schedule changes no bit), so tuning costs no extra
  * work; the candidates are those of the single-system solver's offline tuner. */
 static const cacg_spmm_sched CAND[] = {
-    {0, 0, 0},       {4096, 0, 0},    {8192, 0, 0},    {0, 1024, 0},   {0, 2048, 0},
-    {0, 4096, 0},    {4096, 2048, 0}, {8192, 4096, 0}, {16384, 512, 4}, {32768, 512, 4}};
+    {0, 0, 0},       {4096, 0, 0},    {8192, 0, 0},    {0, 2048, 0},    {4096, 2048, 0},
+    {8192, 4096, 0}, {768, 2048, 0},  {1024, 1024, 0}, {16384, 512, 4}, {32768, 512, 4}};
 #define NCAND ((int)(sizeof(CAND) / sizeof(CAND[0])))
 
 typedef struct {

@@ -680,9 +680,8 @@ static unsigned long long pattern_key(long n, const long *row_start, const long 
 static int tune_spmm(cacg_solver *sv, int blk)
 {
     static const cacg_spmm_sched cand[] = {
-        {0, 0, 0},       {4096, 0, 0},    {8192, 0, 0},       {0, 1024, 0},
-        {0, 2048, 0},    {0, 4096, 0},    {4096, 2048, 0},    {8192, 4096, 0},
-        {16384, 512, 4}, {32768, 512, 4}};
+        {0, 0, 0},       {4096, 0, 0},    {8192, 0, 0},   {0, 2048, 0},    {4096, 2048, 0},
+        {8192, 4096, 0}, {768, 2048, 0},  {1024, 1024, 0}, {16384, 512, 4}, {32768, 512, 4}};
     const int nc = (int)(sizeof(cand) / sizeof(cand[0]));
     sv->tuned = 1;
     if (sv->n < TUNE_MIN_ROWS)

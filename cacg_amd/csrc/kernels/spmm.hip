@@ -3,7 +3,8 @@
 //
 // Scheduling: vector-per-row.  A row is served by LPR consecutive lanes, each
 // lane owning VW contiguous output columns (VW = 4 when k is a multiple of 4
-// and x is 16-byte aligned with an even leading dimension, else 1), so the
+// and x is 16-byte aligned with an even leading dimension, 2 when k is even
+// and x allows pairs, else 1), so the
 // gather of x(col, :) is one contiguous k*8-byte segment per nonzero read
 // with 16-byte loads, and the lanes of a row read the same (col, val) pair
 // (an LDS broadcast).  Each output is summed in CSR order from 0, product and
@@ -45,14 +46,34 @@
 namespace {
 
 
-// VW consecutive elements of T from a 16-byte aligned address (VW = 4) or
-// one element (VW = 1)
+// VW consecutive elements of T from a 16-byte aligned address (VW = 4), two
+// from one aligned to both (VW = 2), or one element (VW = 1)
 template <typename T, int VW>
 struct vecld;
 template <typename T>
 struct vecld<T, 1> {
     T v[1];
     __device__ __forceinline__ void load(const T *p) { v[0] = *p; }
+};
+template <>
+struct vecld<double, 2> {
+    double v[2];
+    __device__ __forceinline__ void load(const double *p)
+    {
+        const double2 a = *reinterpret_cast<const double2 *>(p);
+        v[0] = a.x;
+        v[1] = a.y;
+    }
+};
+template <>
+struct vecld<float, 2> {
+    float v[2];
+    __device__ __forceinline__ void load(const float *p)
+    {
+        const float2 a = *reinterpret_cast<const float2 *>(p);
+        v[0] = a.x;
+        v[1] = a.y;
+    }
 };
 template <>
 struct vecld<double, 4> {
@@ -523,9 +544,28 @@ __global__ __launch_bounds__(LR_T) void spmm_long_kernel(
     }
 }
 
-// Launch shape (measured on the 128^3 Laplacian, k = 16 and k = 128): narrow
-// rows (LPR <= 8) one row per lane group and 32 workgroups per CU; wide rows
-// two rows per lane group and 16 workgroups per CU.
+// Launch shape: narrow rows (LPR <= 8) one row per lane group, wide rows two,
+// and, unless the schedule names a grid, 32 and 16 workgroups per CU in bands.
+// A grid of more workgroups than run at once sweeps a band with gaps (the first
+// ones walk it to its end before the rest start), so the rows a front gathers
+// lie further apart.  For blocks that outgrow the 256 MB behind the L2s the
+// default is therefore as many workgroups as stay resident, in chunks: 3 per CU
+// and 2048 rows up to 16 columns (from 16 MB, where the order of the front starts
+// to count), 4 per CU and 1024 rows above 64 columns.  In between neither order
+// wins everywhere, and rows of very different lengths (a long-row list) need
+// the spare workgroups to balance.  128^3 Laplacian: k = 16 242 -> 224 us, k =
+// 128 1517 -> 1336 us (a copy of the same bytes takes 200 and 900); 96^3: 107 ->
+// 101, 673 -> 583; 1024^2: 109 -> 103, 667 -> 598; 64^3: 34 -> 33, 166 -> 147.
+inline cacg_spmm_sched default_sched(long n, int k, int lpr, int vw, bool ragged)
+{
+    const long bytes = n * (long)k * 8;
+    if (!ragged && vw == 4 && lpr <= 4 && bytes >= 16L << 20)
+        return {768, 2048, 0};
+    if (!ragged && vw == 4 && k > 64 && bytes >= 256L << 20)
+        return {1024, 1024, 0};
+    return {0, 0, 0};
+}
+
 template <typename TV, typename TX, typename TY, int LPR, int VW>
 int launch_spmm(int n, const int *rowptr, const int *col, const TV *val, int k, const TX *x,
                 long ldx, TY *y, long ldy, int epi, double a, double b, const TY *p1, long ld1,
@@ -534,7 +574,10 @@ int launch_spmm(int n, const int *rowptr, const int *col, const TV *val, int k, 
 {
     constexpr int RPG = LPR >= 16 ? 2 : 1;
     constexpr int TR = (256 / LPR) * RPG;
-    const int gmax = sc && sc->grid > 0 ? sc->grid : (LPR >= 16 ? 4096 : 8192);
+    const cacg_spmm_sched def = default_sched(n, k, LPR, VW, n_long > 0);
+    if (!sc || (sc->grid == 0 && sc->chunk_rows == 0))
+        sc = &def;
+    const int gmax = sc->grid > 0 ? sc->grid : (LPR >= 16 ? 4096 : 8192);
     const int ntiles = (n + TR - 1) / TR;
     // a multiple of 8 so every XCD gets the same number of workgroups
     int G = ntiles < gmax ? ntiles : gmax;
@@ -542,7 +585,7 @@ int launch_spmm(int n, const int *rowptr, const int *col, const TV *val, int k, 
         G &= ~7;
     // chunk order: chunk_rows rounded to whole tiles
     int P = 0, Q = 1;
-    if (sc && sc->chunk_rows > 0) {
+    if (sc->chunk_rows > 0) {
         P = sc->chunk_rows >= TR ? sc->chunk_rows / TR : 1;
         Q = sc->passes > 1 ? sc->passes : 1;
     }
@@ -636,6 +679,23 @@ int dispatch_spmm(int n, const int *rowptr, const int *col, const TV *val, int k
         if (q > 1)
             return launch_spmm<TV, TX, TY, 2, 4>(CACG_SPMM_ARGS);
         return launch_spmm<TV, TX, TY, 1, 4>(CACG_SPMM_ARGS);
+    }
+    // pairs of columns: a row of 10 takes 8 lanes and 16-byte gathers instead of
+    // 16 lanes and 8-byte ones
+    const bool vec2 = k % 2 == 0 && ((uintptr_t)x & (2 * sizeof(TX) - 1)) == 0 && ldx % 2 == 0;
+    if (vec2) {
+        const int q = k / 2;
+        if (q > 16)
+            return launch_spmm<TV, TX, TY, 32, 2>(CACG_SPMM_ARGS);
+        if (q > 8)
+            return launch_spmm<TV, TX, TY, 16, 2>(CACG_SPMM_ARGS);
+        if (q > 4)
+            return launch_spmm<TV, TX, TY, 8, 2>(CACG_SPMM_ARGS);
+        if (q > 2)
+            return launch_spmm<TV, TX, TY, 4, 2>(CACG_SPMM_ARGS);
+        if (q > 1)
+            return launch_spmm<TV, TX, TY, 2, 2>(CACG_SPMM_ARGS);
+        return launch_spmm<TV, TX, TY, 1, 2>(CACG_SPMM_ARGS);
     }
     if (k > 32)
         return launch_spmm<TV, TX, TY, 64, 1>(CACG_SPMM_ARGS);

@@ -6,6 +6,8 @@ import ctypes
 import numpy as np
 import pytest
 
+from cacg_amd import problems as P
+
 pytestmark = pytest.mark.gpu
 EPS = 2.0 ** -52
 
@@ -187,3 +189,34 @@ def test_batched_gram_exact_on_integers(gpu_lib, systems, f32):
             else:
                 assert np.array_equal(b["QtAQ"].download((sm, sm)), Q.T @ AQ)
                 assert np.array_equal(b["QtR"].download((sm, m)), Q.T @ R)
+
+
+@pytest.mark.parametrize("k", [2, 6, 10, 14, 18, 22, 30, 34, 66, 130])
+def test_spmm_column_pairs_bitwise(gpu_lib, oracle_lib, k):
+    """Even widths that are no multiple of 4 (two columns a lane), every epilogue; the FP32 forms
+    against the row split, which sums the same products in the same order."""
+    A = P.random_spd_like(P.laplacian_3d(9), seed=5)
+    X, p1, p2 = (P.rhs_normal(A.n, k, sd) for sd in (1, 2, 3))
+    print(f"spmm pairs k={k}", flush=True)
+    AX, a, b = oracle_lib.spmm(A, X), 0.37, -0.21
+    assert np.array_equal(gpu_lib.k_spmm(A, X), AX)
+    assert np.array_equal(gpu_lib.k_spmm(A, X, "cheb", a, b, p1=p1, p2=p2), (a * AX + b * p1) - p2)
+    assert np.array_equal(gpu_lib.k_spmm(A, X, "resid", p1=p1), p1 - AX)
+    S1, S0 = gpu_lib.k_spmm(A, X, "cheb1", a, b, want_copy0=True)
+    assert np.array_equal(S0, X) and np.array_equal(S1, a * AX + b * X)
+    X32, q1, q2 = (v.astype(np.float32) for v in (X, p1, p2))
+    for epi, kw in (("none", {}), ("cheb", dict(p1=q1, p2=q2))):
+        want = gpu_lib.k_spmm_f32(A, X32, epi, 0.5, -0.25, long_min=1, **kw)
+        assert np.array_equal(gpu_lib.k_spmm_f32(A, X32, epi, 0.5, -0.25, long_min=0, **kw), want)
+    for w, g in zip(gpu_lib.k_cheb1_f32(A, X, 0.5, -0.25, long_min=1),
+                    gpu_lib.k_cheb1_f32(A, X, 0.5, -0.25, long_min=0)):
+        assert np.array_equal(g, w)
+
+
+@pytest.mark.parametrize("edge,k", [(96, 3), (73, 12), (96, 16), (69, 104)])
+def test_spmm_default_order_gives_the_same_bits(gpu_lib, edge, k):
+    """Blocks just past the sizes from which the default order is chunks over a resident grid."""
+    A = P.laplacian_3d(edge)
+    X = P.rhs_uniform(A.n, k, 3)
+    print(f"spmm default order {edge}^3 k={k}", flush=True)
+    assert np.array_equal(gpu_lib.k_spmm(A, X), gpu_lib.k_spmm(A, X, sched=(4096, 0, 0)))
