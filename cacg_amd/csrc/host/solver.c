@@ -62,6 +62,8 @@ struct cacg_solver {
     double *d_QtAQ, *d_QtAS, *d_QtR, *d_alpha, *d_beta;
     double *d_norm2, *d_bounds, *d_gwork, *d_gram_work, *d_xr_work, *d_lu_work;
     int *d_flag;
+    int direct;      /* the kernels write an iteration's norms and the flag to h_pin themselves */
+    hipEvent_t norms_ev;   /* an iteration's norms are in h_pin */
     double *h_pin;   /* pinned: [0, m) column norms^2, [m, 2m) ||B(:,c)||^2, [2m, 2m+2) bounds, then the flag */
     /* SpMM schedules of the basis steps and of A Q, picked by timing on the
      * first solve (tuned = 1) */
@@ -315,7 +317,7 @@ int cacg_solver_destroy(cacg_solver *sv)
     void *ptrs[] = {sv->d_rowptr, sv->d_col,   sv->d_val,   sv->d_R,       sv->d_S,
                     sv->d_Q,      sv->d_AQ,    sv->d_QtAQ,  sv->d_QtAS,    sv->d_QtR,
                     sv->d_alpha,  sv->d_beta,  sv->d_norm2, sv->d_bounds,  sv->d_gwork,
-                    sv->d_gram_work, sv->d_xr_work, sv->d_lu_work, sv->d_flag,
+                    sv->d_gram_work, sv->d_xr_work, sv->d_lu_work,
                     sv->f_val,    sv->f_S,     sv->d_lz_work, sv->d_lz_ab, sv->d_long_rows};
     for (size_t i = 0; i < sizeof(ptrs) / sizeof(ptrs[0]); i++)
         if (ptrs[i])
@@ -326,6 +328,8 @@ int cacg_solver_destroy(cacg_solver *sv)
     for (int i = 0; i < 2; i++)
         if (sv->tev[i])
             hipEventDestroy(sv->tev[i]);
+    if (sv->norms_ev)
+        hipEventDestroy(sv->norms_ev);
     if (sv->st)
         hipStreamDestroy(sv->st);
     if (sv->h_pin)
@@ -401,15 +405,24 @@ int cacg_solver_create(cacg_solver **out, long n, const long *row_start, const l
         cacg_solver_destroy(sv);
         return CACG_ENOMEM;
     }
+    sv->direct = 1;
+    sv->d_flag = (int *)(sv->h_pin + 2 * m + 2);
     if (hipStreamCreate(&sv->st) != hipSuccess) {
         cacg_solver_destroy(sv);
         return CACG_EDEVICE;
     }
+    /* the phase marks order nothing with the host: without a system fence they cost
+     * a small solve 5 us an iteration less (of 27) */
     for (int i = 0; i < MAXEV; i++)
-        if (hipEventCreate(&sv->ev[i]) != hipSuccess) {
+        if (hipEventCreateWithFlags(&sv->ev[i], hipEventDisableSystemFence) != hipSuccess) {
             cacg_solver_destroy(sv);
             return CACG_EDEVICE;
         }
+    if (hipEventCreateWithFlags(&sv->norms_ev, hipEventDisableTiming) != hipSuccess) {
+        sv->norms_ev = NULL;
+        cacg_solver_destroy(sv);
+        return CACG_EDEVICE;
+    }
     for (int i = 0; i < 2; i++)
         if (hipEventCreate(&sv->tev[i]) != hipSuccess) {
             cacg_solver_destroy(sv);
@@ -445,7 +458,6 @@ int cacg_solver_create(cacg_solver **out, long n, const long *row_start, const l
     rc |= dalloc(sv, (void **)&sv->d_gram_work, gram_ws * (long)sizeof(double));
     rc |= dalloc(sv, (void **)&sv->d_xr_work, cacg_xrupdate_workspace((int)m) * (long)sizeof(double));
     rc |= dalloc(sv, (void **)&sv->d_lu_work, sm * sm * (long)sizeof(double));
-    rc |= dalloc(sv, (void **)&sv->d_flag, (long)sizeof(int));
     if (sv->opts.bounds == CACG_BOUNDS_LANCZOS) {
         int k = sv->opts.lanczos_steps > 0 ? sv->opts.lanczos_steps : 20;
         if (k > n)
@@ -562,11 +574,13 @@ static void mark(cacg_solver *sv, int phase_done)
     sv->nev++;
 }
 
-static void harvest(cacg_solver *sv, cacg_report *rep)
+/* book the phases between the first `upto` marks; the last of them stays as the
+ * start of the next, the later ones (not reached by the device yet) move up */
+static void harvest_upto(cacg_solver *sv, cacg_report *rep, int upto)
 {
-    if (sv->noev)
+    if (sv->noev || upto <= 0)
         return;
-    for (int i = 1; i < sv->nev; i++) {
+    for (int i = 1; i < upto; i++) {
         float ms = 0.f;
         if (hipEventElapsedTime(&ms, sv->ev[i - 1], sv->ev[i]) == hipSuccess && rep) {
             const int ph = sv->ev_phase[i];
@@ -575,14 +589,17 @@ static void harvest(cacg_solver *sv, cacg_report *rep)
             rep->seconds += ms * 1e-3;
         }
     }
-    if (sv->nev > 0) {
-        hipEvent_t last = sv->ev[sv->nev - 1];
-        sv->ev[sv->nev - 1] = sv->ev[0];
-        sv->ev[0] = last;
-        sv->ev_phase[0] = sv->ev_phase[sv->nev - 1];
-        sv->nev = 1;
+    const int last = upto - 1, keep = sv->nev - last;
+    for (int j = 0; j < keep && last > 0; j++) {
+        hipEvent_t e = sv->ev[j];
+        sv->ev[j] = sv->ev[last + j];
+        sv->ev[last + j] = e;
+        sv->ev_phase[j] = sv->ev_phase[last + j];
     }
+    sv->nev = keep;
 }
+
+static void harvest(cacg_solver *sv, cacg_report *rep) { harvest_upto(sv, rep, sv->nev); }
 
 /* ---- the solve ------------------------------------------------------------------ */
 
@@ -776,6 +793,44 @@ static int interval_finish(cacg_solver *sv, const double g[2], double iv[2])
     return CACG_OK;
 }
 
+/* where the kernels leave an iteration's column norms, and the copies that bring
+ * them and the flag to the host when that is device memory */
+static double *norms_out(cacg_solver *sv) { return sv->direct ? sv->h_pin : sv->d_norm2; }
+
+static int norms_back(cacg_solver *sv, double *h_norm2, int *h_flag)
+{
+    if (sv->direct)
+        return 0;
+    const int rc = (int)hipMemcpyAsync(h_norm2, sv->d_norm2, sizeof(double) * (size_t)sv->m,
+                                       hipMemcpyDeviceToHost, sv->st);
+    return rc ? rc
+              : (int)hipMemcpyAsync(h_flag, sv->d_flag, sizeof(int), hipMemcpyDeviceToHost, sv->st);
+}
+
+/* the basis S_0 .. S_{s-1} of the residual: block j at SB + j bo, rows lb apart
+ * (src/common.c:182-256) */
+static int basis_enqueue(cacg_solver *sv, double *SB, long bo, long lb, double sa, double sb)
+{
+    const int n = (int)sv->n, m = (int)sv->m, s = (int)sv->s;
+    hipStream_t st = sv->st;
+    int rc = 0;
+    if (s == 1) {
+        rc = (int)hipMemcpyAsync(SB, sv->d_R, sizeof(double) * (size_t)n * m,
+                                 hipMemcpyDeviceToDevice, st);
+    } else {
+        rc = cacg_k_spmm_x(&sv->A, m, sv->d_R, m, SB + bo, lb, CACG_EPI_CHEB1, sa, sb, NULL, 0, NULL,
+                           0, SB, lb, &sv->sch_basis, st);
+        mark(sv, CACG_PHASE_BASIS1);
+        for (int j = 2; j < s && rc == 0; j++)
+            rc = cacg_k_spmm_x(&sv->A, m, SB + (j - 1) * bo, lb, SB + j * bo, lb, CACG_EPI_CHEB,
+                               2.0 * sa, 2.0 * sb, SB + (j - 1) * bo, lb, SB + (j - 2) * bo, lb,
+                               NULL, 0, &sv->sch_basis, st);
+    }
+    if (s != 2)
+        mark(sv, s == 1 ? CACG_PHASE_BASIS1 : CACG_PHASE_BASIS);
+    return rc;
+}
+
 #define SCHK(call)                                                                               \
     do {                                                                                         \
         int e_ = (int)(call);                                                                    \
@@ -806,6 +861,9 @@ int cacg_solver_solve_device(cacg_solver *sv, const double *d_B, double *d_X, ca
     const int blk = split && m % 4 == 0 && s >= 2 && !sv->basis_rows &&
                     cacg_gram_blk_supported(n, sm, sm, m);
     const long bs = (long)n * m;
+    /* fast order, small s m: Gram sums and the solve after them in one launch
+     * (their time is booked as the Gram's) */
+    const int small = mode == CACG_MODE_FAST && !blk && cacg_gram_solve_supported(sm, m);
     hipStream_t st = sv->st;
     double *h_norm2 = sv->h_pin, *h_bnorm2 = sv->h_pin + m, *h_bounds = sv->h_pin + 2 * m;
     int *h_flag = (int *)(sv->h_pin + 2 * m + 2);
@@ -859,38 +917,38 @@ int cacg_solver_solve_device(cacg_solver *sv, const double *d_B, double *d_X, ca
     /* src/bcbcgKernel.c:113-115 */
     const double sa = 2.0 / (iv[1] - iv[0]);
     const double sb = -(iv[1] + iv[0]) / (iv[1] - iv[0]);
-    const double sa2 = 2.0 * sa, sb2 = 2.0 * sb;
+    /* small blocks: the host needs longer to see the norms and launch again than a
+     * basis takes, so the next iteration's basis goes out before it waits for
+     * them (it reads R and writes S only; after the last iteration it is not
+     * used).  2^20 elements: a basis of about 10 us a step, the wait about 20 us;
+     * 16,384 x 1, s = 4: 11.9 -> 9.9 ms a solve together with the norms written
+     * to the host by the kernels and the cheaper marks */
+    const int ahead = sv->direct && s >= 2 && (long)n * m <= 1L << 20;
+    int have = 0;   /* this iteration's basis is already enqueued */
 
     for (it = 0; it < o->maxiter; it++) {
-        mark(sv, CACG_PHASE_OTHER);
-        /* Chebyshev basis (src/common.c:182-256): block j at SB + j * bo, rows
-         * lb apart; the first iteration's basis is its Q */
+        /* block j of the basis at SB + j * bo, rows lb apart; the first
+         * iteration's basis is its Q */
         const int bm = blk && it > 0;
-        double *SB = it == 0 ? Q : S;
-        const long bo = bm ? bs : m, lb = bm ? m : sm;
-        if (s == 1) {
-            SCHK(hipMemcpyAsync(SB, sv->d_R, sizeof(double) * (size_t)n * m, hipMemcpyDeviceToDevice, st));
-        } else {
-            SCHK(cacg_k_spmm_x(&sv->A, m, sv->d_R, m, SB + bo, lb, CACG_EPI_CHEB1, sa, sb, NULL, 0,
-                               NULL, 0, SB, lb, &sv->sch_basis, st));
-            mark(sv, CACG_PHASE_BASIS1);
-            for (int j = 2; j < s; j++)
-                SCHK(cacg_k_spmm_x(&sv->A, m, SB + (j - 1) * bo, lb, SB + j * bo, lb,
-                                   CACG_EPI_CHEB, sa2, sb2, SB + (j - 1) * bo, lb,
-                                   SB + (j - 2) * bo, lb, NULL, 0, &sv->sch_basis, st));
+        if (!have) {
+            mark(sv, CACG_PHASE_OTHER);
+            SCHK(basis_enqueue(sv, it == 0 ? Q : S, bm ? bs : m, bm ? m : sm, sa, sb));
         }
-        if (s != 2)
-            mark(sv, s == 1 ? CACG_PHASE_BASIS1 : CACG_PHASE_BASIS);
+        have = 0;
         if (it > 0) {
-            if (bm)
+            if (small)
+                SCHK(cacg_k_gram_beta(n, sm, sv->d_AQ, S, NULL, sv->d_QtAS, sv->d_beta,
+                                      sv->d_lu_work, sv->d_gram_work, st));
+            else if (bm)
                 SCHK(cacg_k_gram_fast_blk(n, sv->d_AQ, sm, sm, S, m, bs, sm, sv->d_QtAS,
                                           sv->d_gram_work, st));
             else
                 SCHK(gram(sv, mode, sv->d_AQ, S, sm, sm, NULL, 0, 0, sv->d_QtAS, NULL));
             mark(sv, CACG_PHASE_GRAM_AS);
             /* Q^T A Q of the previous iteration: its factor is still in d_lu_work */
-            SCHK(cacg_k_lu_solve(sm, sv->d_QtAQ, sm, sv->d_QtAS, sv->d_beta, sv->d_lu_work,
-                                 sv->d_flag, mode, 1, st));
+            if (!small)
+                SCHK(cacg_k_lu_solve(sm, sv->d_QtAQ, sm, sv->d_QtAS, sv->d_beta, sv->d_lu_work,
+                                     sv->d_flag, mode, 1, st));
             mark(sv, CACG_PHASE_SOLVE);
             if (split && bm) /* X += Q alpha of the previous iteration, then Q = S - Q beta */
                 SCHK(cacg_k_qxupdate_blk(n, sm, m, S, bs, Q, sv->d_beta, sv->d_alpha, d_X, st));
@@ -903,22 +961,36 @@ int cacg_solver_solve_device(cacg_solver *sv, const double *d_B, double *d_X, ca
         SCHK(cacg_k_spmm_x(&sv->A, sm, Q, sm, sv->d_AQ, sm, CACG_EPI_NONE, 0.0, 0.0, NULL, 0, NULL,
                            0, NULL, 0, &sv->sch_aq, st));
         mark(sv, CACG_PHASE_AQ);
-        SCHK(gram(sv, mode, Q, sv->d_AQ, sm, sm, sv->d_R, m, m, sv->d_QtAQ, sv->d_QtR));
+        if (small)
+            SCHK(cacg_k_gram_alpha(n, sm, m, Q, sv->d_AQ, sv->d_R, sv->d_QtAQ, sv->d_QtR,
+                                   sv->d_alpha, sv->d_lu_work, sv->d_flag, sv->d_gram_work, st));
+        else
+            SCHK(gram(sv, mode, Q, sv->d_AQ, sm, sm, sv->d_R, m, m, sv->d_QtAQ, sv->d_QtR));
         mark(sv, CACG_PHASE_GRAM);
-        SCHK(cacg_k_lu_solve(sm, sv->d_QtAQ, m, sv->d_QtR, sv->d_alpha, sv->d_lu_work, sv->d_flag,
-                             mode, 0, st));
+        if (!small)
+            SCHK(cacg_k_lu_solve(sm, sv->d_QtAQ, m, sv->d_QtR, sv->d_alpha, sv->d_lu_work,
+                                 sv->d_flag, mode, 0, st));
         mark(sv, CACG_PHASE_SOLVE);
         if (split) /* R and its norms now; X with the next Q update */
             SCHK(cacg_k_xrupdate_split(n, sm, m, NULL, sv->d_AQ, sv->d_alpha, NULL, sv->d_R,
-                                       sv->d_norm2, sv->d_xr_work, 2, st));
+                                       norms_out(sv), sv->d_xr_work, 2, st));
         else
-            SCHK(cacg_k_xrupdate(n, sm, m, Q, sv->d_AQ, sv->d_alpha, d_X, sv->d_R, sv->d_norm2,
+            SCHK(cacg_k_xrupdate(n, sm, m, Q, sv->d_AQ, sv->d_alpha, d_X, sv->d_R, norms_out(sv),
                                  sv->d_xr_work, mode, st));
         mark(sv, CACG_PHASE_XRUPDATE);
-        SCHK(hipMemcpyAsync(h_norm2, sv->d_norm2, sizeof(double) * m, hipMemcpyDeviceToHost, st));
-        SCHK(hipMemcpyAsync(h_flag, sv->d_flag, sizeof(int), hipMemcpyDeviceToHost, st));
-        SCHK(hipStreamSynchronize(st));
-        harvest(sv, rep);
+        SCHK(norms_back(sv, h_norm2, h_flag));
+        if (ahead && it + 1 < o->maxiter) {
+            const int upto = sv->nev;
+            SCHK(hipEventRecord(sv->norms_ev, st));
+            mark(sv, CACG_PHASE_OTHER);
+            SCHK(basis_enqueue(sv, S, blk ? bs : m, blk ? m : sm, sa, sb));
+            have = 1;
+            SCHK(hipEventSynchronize(sv->norms_ev));
+            harvest_upto(sv, rep, upto);
+        } else {
+            SCHK(hipStreamSynchronize(st));
+            harvest(sv, rep);
+        }
 
         int done = 1, finite = 1;
         for (int c = 0; c < m; c++) {
@@ -947,10 +1019,10 @@ int cacg_solver_solve_device(cacg_solver *sv, const double *d_B, double *d_X, ca
             break;
         }
     }
-    if (split && it > 0) { /* the last iteration's X += Q alpha */
+    if (split && it > 0) /* the last iteration's X += Q alpha */
         SCHK(cacg_k_xrupdate_split(n, sm, m, Q, NULL, sv->d_alpha, d_X, NULL, NULL, NULL, 1, st));
+    if ((split && it > 0) || have)
         SCHK(hipStreamSynchronize(st));
-    }
 out:
     /* leave the two basis-sized buffers in allocation roles for the next solve */
     sv->d_S = S;
@@ -1165,10 +1237,10 @@ int cacg_solver_solve_bcg_device(cacg_solver *sv, const double *d_B, double *d_X
         mark(sv, CACG_PHASE_GRAM);
         SCHK(cacg_k_lu_solve(m, PtAP, m, RtR, alpha, sv->d_lu_work, sv->d_flag, mode, 0, st));
         mark(sv, CACG_PHASE_SOLVE);
-        SCHK(cacg_k_xrupdate(n, m, m, P, AP, alpha, d_X, R, sv->d_norm2, sv->d_xr_work, mode, st));
+        SCHK(cacg_k_xrupdate(n, m, m, P, AP, alpha, d_X, R, norms_out(sv), sv->d_xr_work, mode,
+                             st));
         mark(sv, CACG_PHASE_XRUPDATE);
-        SCHK(hipMemcpyAsync(h_norm2, sv->d_norm2, sizeof(double) * m, hipMemcpyDeviceToHost, st));
-        SCHK(hipMemcpyAsync(h_flag, sv->d_flag, sizeof(int), hipMemcpyDeviceToHost, st));
+        SCHK(norms_back(sv, h_norm2, h_flag));
         SCHK(hipStreamSynchronize(st));
         harvest(sv, rep);
 
@@ -1303,6 +1375,7 @@ static int solve_refine(cacg_solver *sv, const double *d_B, double *d_X, cacg_re
     /* X += Q alpha deferred into the next Q update (split) and flushed wherever X
      * is read: before a true residual and at the end */
     const int split = cacg_k_split_supported(sm, m);
+    const int small = cacg_gram_solve_supported(sm, m);   /* as in cacg_solver_solve_device */
     int xpend = 0;
     /* opts.fp32_basis_below > 0: the basis is built in FP64 (d_S, the FP64
      * matrix) until the true residual is below it in every column, in FP32 from
@@ -1399,10 +1472,15 @@ static int solve_refine(cacg_solver *sv, const double *d_B, double *d_X, cacg_re
                     SCHK(cacg_k_cvt_f32_f64((long)n * sm, S, Q, st));
                 fresh = 0;
             } else if (use64) {
-                SCHK(cacg_k_gram_fast(n, AQ, sm, sm, sv->d_S, sm, sm, NULL, 0, 0, sv->d_QtAS, NULL,
-                                      sv->d_gram_work, st));
+                if (small)
+                    SCHK(cacg_k_gram_beta(n, sm, AQ, sv->d_S, NULL, sv->d_QtAS, sv->d_beta,
+                                          sv->d_lu_work, sv->d_gram_work, st));
+                else
+                    SCHK(cacg_k_gram_fast(n, AQ, sm, sm, sv->d_S, sm, sm, NULL, 0, 0, sv->d_QtAS,
+                                          NULL, sv->d_gram_work, st));
                 mark(sv, CACG_PHASE_GRAM_AS);
-                SCHK(cacg_k_lu_solve(sm, sv->d_QtAQ, sm, sv->d_QtAS, sv->d_beta, sv->d_lu_work,
+                if (!small)
+                    SCHK(cacg_k_lu_solve(sm, sv->d_QtAQ, sm, sv->d_QtAS, sv->d_beta, sv->d_lu_work,
                                      sv->d_flag, CACG_MODE_FAST, 1, st));
                 mark(sv, CACG_PHASE_SOLVE);
                 if (xpend)
@@ -1411,10 +1489,15 @@ static int solve_refine(cacg_solver *sv, const double *d_B, double *d_X, cacg_re
                     SCHK(cacg_k_qupdate(n, sm, sv->d_S, Q, sv->d_beta, CACG_MODE_FAST, st));
                 xpend = 0;
             } else {
-                SCHK(cacg_k_gram_fast_f64f32(n, AQ, sm, sm, S, sm, sm, NULL, 0, 0, sv->d_QtAS, NULL,
-                                             sv->d_gram_work, st));
+                if (small)
+                    SCHK(cacg_k_gram_beta(n, sm, AQ, NULL, S, sv->d_QtAS, sv->d_beta,
+                                          sv->d_lu_work, sv->d_gram_work, st));
+                else
+                    SCHK(cacg_k_gram_fast_f64f32(n, AQ, sm, sm, S, sm, sm, NULL, 0, 0, sv->d_QtAS,
+                                                 NULL, sv->d_gram_work, st));
                 mark(sv, CACG_PHASE_GRAM_AS);
-                SCHK(cacg_k_lu_solve(sm, sv->d_QtAQ, sm, sv->d_QtAS, sv->d_beta, sv->d_lu_work,
+                if (!small)
+                    SCHK(cacg_k_lu_solve(sm, sv->d_QtAQ, sm, sv->d_QtAS, sv->d_beta, sv->d_lu_work,
                                      sv->d_flag, CACG_MODE_FAST, 1, st));
                 mark(sv, CACG_PHASE_SOLVE);
                 if (xpend)
@@ -1427,23 +1510,27 @@ static int solve_refine(cacg_solver *sv, const double *d_B, double *d_X, cacg_re
             SCHK(cacg_k_spmm_x(&sv->A, sm, Q, sm, AQ, sm, CACG_EPI_NONE, 0.0, 0.0, NULL, 0, NULL,
                                0, NULL, 0, &sv->sch_aq, st));
             mark(sv, CACG_PHASE_AQ);
-            SCHK(cacg_k_gram_fast(n, Q, sm, sm, AQ, sm, sm, sv->d_R, m, m, sv->d_QtAQ, sv->d_QtR,
-                                  sv->d_gram_work, st));
+            if (small)
+                SCHK(cacg_k_gram_alpha(n, sm, m, Q, AQ, sv->d_R, sv->d_QtAQ, sv->d_QtR, sv->d_alpha,
+                                       sv->d_lu_work, sv->d_flag, sv->d_gram_work, st));
+            else
+                SCHK(cacg_k_gram_fast(n, Q, sm, sm, AQ, sm, sm, sv->d_R, m, m, sv->d_QtAQ,
+                                      sv->d_QtR, sv->d_gram_work, st));
             mark(sv, CACG_PHASE_GRAM);
-            SCHK(cacg_k_lu_solve(sm, sv->d_QtAQ, m, sv->d_QtR, sv->d_alpha, sv->d_lu_work,
+            if (!small)
+                SCHK(cacg_k_lu_solve(sm, sv->d_QtAQ, m, sv->d_QtR, sv->d_alpha, sv->d_lu_work,
                                  sv->d_flag, CACG_MODE_FAST, 0, st));
             mark(sv, CACG_PHASE_SOLVE);
             if (split) {
                 SCHK(cacg_k_xrupdate_split(n, sm, m, NULL, AQ, sv->d_alpha, NULL, sv->d_R,
-                                           sv->d_norm2, sv->d_xr_work, 2, st));
+                                           norms_out(sv), sv->d_xr_work, 2, st));
                 xpend = 1;
             } else {
-                SCHK(cacg_k_xrupdate(n, sm, m, Q, AQ, sv->d_alpha, d_X, sv->d_R, sv->d_norm2,
+                SCHK(cacg_k_xrupdate(n, sm, m, Q, AQ, sv->d_alpha, d_X, sv->d_R, norms_out(sv),
                                      sv->d_xr_work, CACG_MODE_FAST, st));
             }
             mark(sv, CACG_PHASE_XRUPDATE);
-            SCHK(hipMemcpyAsync(h_norm2, sv->d_norm2, sizeof(double) * m, hipMemcpyDeviceToHost, st));
-            SCHK(hipMemcpyAsync(h_flag, sv->d_flag, sizeof(int), hipMemcpyDeviceToHost, st));
+            SCHK(norms_back(sv, h_norm2, h_flag));
             SCHK(hipStreamSynchronize(st));
             harvest(sv, rep);
             int reached = 1;

@@ -404,6 +404,105 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(const double *__restri
     }
 }
 
+// The same sums for a small G (kl, k <= 8) and the solve that follows it, in one
+// workgroup: up to 8 x 8 the two launches cost more than their work (16 x 16: 12.6 us in one
+// workgroup, as much as the two).
+// G1 (kl x kr1) and G2 (kl x kr2) are written as above.  factor: x = G1^{-1} G2 (kr1 =
+// kl, k = kr2), the factor of G1 kept in lu; otherwise x = (the G1 in lu)^{-1} G1 (k =
+// kr1).  Every element receives the same operations in the same order as in
+// lu_factor_body and the substitutions of lu.hip: subtractions in ascending order
+// of the pivot, the reciprocal pivot last, the backward substitution by
+// descending pivot.  Thread (i, j) of 8 x 16 keeps element j of row i: columns
+// 0 .. kl - 1 the matrix, 8 .. 8 + k - 1 the right-hand sides.
+// 16,384 rows, sm = 4, m = 1: reduce and solve 3.4 + 4.7 us and a launch -> 4.0 us.
+constexpr int GS_N = 8;
+
+__global__ __launch_bounds__(1024) void gram_solve_kernel(const double *__restrict__ part, int gx,
+                                                          int kl, int kr1, int kr2, int kl_pad,
+                                                          int kr_pad, double *__restrict__ G1,
+                                                          double *__restrict__ G2,
+                                                          double *__restrict__ lu,
+                                                          double *__restrict__ x, int *flag,
+                                                          int factor)
+{
+    constexpr int W = 4, LD = 32;
+    __shared__ double red[4 * W][64];
+    __shared__ double M[GS_N][2 * GS_N + 1];
+    const int kr = kr1 + kr2, t = threadIdx.x;
+    const int wave = t >> 6, lane = t & 63;
+    const int grp = wave / W, wq = wave % W;   // 64 entries to 4 waves, 4 such groups
+    if (!factor && t < kl * kl)
+        M[t / kl][t % kl] = lu[t];
+    for (int e0 = 0; e0 < kl * kr; e0 += 4 * 64) {
+        const int e = e0 + grp * 64 + lane;
+        const bool ok = e < kl * kr;
+        const int a = ok ? e / kr : 0, b = ok ? e % kr : 0;
+        const long stride = (long)kl_pad * kr_pad;
+        const double *p = part + (long)a * kr_pad + b;
+        const int q = (gx + W - 1) / W;
+        const int x0 = wq * q, x1 = (x0 + q) < gx ? (x0 + q) : gx;
+        double acc = 0.0;
+        if (ok) {
+            for (int c = x0; c < x1; c += LD) {
+                double v[LD];
+#pragma unroll
+                for (int u = 0; u < LD; u++)
+                    v[u] = c + u < x1 ? p[(c + u) * stride] : 0.0;
+#pragma unroll
+                for (int u = 0; u < LD; u++)
+                    if (c + u < x1)
+                        acc += v[u];
+            }
+        }
+        red[wave][lane] = acc;
+        __syncthreads();
+        if (wq == 0 && ok) {
+            const double sum =
+                ((red[wave][lane] + red[wave + 1][lane]) + red[wave + 2][lane]) + red[wave + 3][lane];
+            if (b < kr1) {
+                G1[(long)a * kr1 + b] = sum;
+                M[a][factor ? b : GS_N + b] = sum;
+            } else {
+                G2[(long)a * kr2 + (b - kr1)] = sum;
+                M[a][GS_N + b - kr1] = sum;
+            }
+        }
+        __syncthreads();
+    }
+    const int i = t / (2 * GS_N), j = t % (2 * GS_N), k = factor ? kr2 : kr1;
+    const bool in = i < kl && (j < GS_N ? j < kl : j - GS_N < k);
+    const bool rhs = j >= GS_N;
+    double v = in ? M[i][j] : 0.0;
+    for (int p = 0; p < kl; p++) {
+        // every lane its own: u = M[p][j] / pivot, then M[i][j] -= M[i][p] u
+        const double piv = M[p][p], inv = 1.0 / piv;
+        const bool col = in && (rhs || (factor && j > p));
+        const double u = col ? mul_rn(M[p][j], inv) : 0.0;
+        if (col && i == p)
+            v = u;
+        else if (col && i > p)
+            v = sub_rn(v, mul_rn(M[i][p], u));
+        if (t == 0 && factor && !(piv != 0.0 && isfinite(piv)))
+            *flag = 1;
+        __syncthreads();
+        if (col && i >= p)
+            M[i][j] = v;
+        __syncthreads();
+    }
+    if (factor && in && !rhs)
+        lu[i * kl + j] = v;
+    for (int q = kl - 1; q > 0; q--) {
+        if (in && rhs && i < q) {
+            v = sub_rn(v, mul_rn(M[q][j], M[i][q]));
+            if (i == q - 1)
+                M[i][j] = v;
+        }
+        __syncthreads();
+    }
+    if (in && rhs)
+        x[(long)i * k + j - GS_N] = v;
+}
+
 // LDS-staged variant for the large case (even column counts, 16-byte aligned
 // rows).  A stage is SR rows of L and of [R1 | R2]; the NW * 64 lanes load it
 // cooperatively with 16-byte loads, LDG stages ahead, holding the data in
@@ -982,10 +1081,15 @@ int launch_gram_tile(int n, const SrcT<TL, T1> &s, GramPlan &p, double *work, hi
     return (int)hipErrorInvalidValue;
 }
 
+struct GramSolve {
+    double *lu, *x;
+    int *flag, factor;
+};
+
 template <typename TL, typename T1>
 int gram_fast(int n, const TL *L, long ldl, int kl, const T1 *R1, long ld1, int kr1,
               const double *R2, long ld2, int kr2, double *G1, double *G2, double *d_work,
-              hipStream_t st, long bs1 = 0)
+              hipStream_t st, long bs1 = 0, const GramSolve *sol = nullptr)
 {
     if (n < 0 || kl <= 0 || kr1 < 0 || kr2 < 0 || kr1 + kr2 <= 0)
         return (int)hipErrorInvalidValue;
@@ -1011,6 +1115,12 @@ int gram_fast(int n, const TL *L, long ldl, int kl, const T1 *R1, long ld1, int 
         }
     }
     CACG_LAUNCH_CHECK();
+    if (sol) {
+        hipLaunchKernelGGL(gram_solve_kernel, dim3(1), dim3(1024), 0, st, d_work, p.gx, kl, kr1, kr2,
+                           p.TM * 16, p.TN * 16, G1, G2, sol->lu, sol->x, sol->flag, sol->factor);
+        CACG_LAUNCH_CHECK();
+        return 0;
+    }
     const long outs = (long)kl * (kr1 + kr2);
     hipLaunchKernelGGL(gram_reduce_kernel, dim3(cacg_grid(outs, 64, 0)), dim3(256), 0, st, d_work,
                        p.gx, kl, kr1, kr2, p.TM * 16, p.TN * 16, G1, G2);
@@ -1108,6 +1218,36 @@ extern "C" int cacg_k_gram_fast_blk(int n, const double *L, long ldl, int kl, co
         return (int)hipErrorInvalidValue;
     return gram_fast<double, double>(n, L, ldl, kl, R1, bw, kr1, nullptr, 1, 0, G1, nullptr,
                                      d_work, st, bs);
+}
+
+extern "C" int cacg_gram_solve_supported(int sm, int m)
+{
+    return sm >= 1 && sm <= GS_N && m >= 1 && m <= GS_N;
+}
+
+extern "C" int cacg_k_gram_alpha(int n, int sm, int m, const double *Q, const double *AQ,
+                                 const double *R, double *QtAQ, double *QtR, double *alpha,
+                                 double *lu, int *d_flag, double *d_work, hipStream_t st)
+{
+    if (n <= 0 || !cacg_gram_solve_supported(sm, m))
+        return (int)hipErrorInvalidValue;
+    const GramSolve sol = {lu, alpha, d_flag, 1};
+    return gram_fast<double, double>(n, Q, sm, sm, AQ, sm, sm, R, m, m, QtAQ, QtR, d_work, st, 0,
+                                     &sol);
+}
+
+extern "C" int cacg_k_gram_beta(int n, int sm, const double *AQ, const double *S, const float *S32,
+                                double *QtAS, double *beta, double *lu, double *d_work,
+                                hipStream_t st)
+{
+    if (n <= 0 || !cacg_gram_solve_supported(sm, 1))
+        return (int)hipErrorInvalidValue;
+    const GramSolve sol = {lu, beta, nullptr, 0};
+    if (S32)
+        return gram_fast<double, float>(n, AQ, sm, sm, S32, sm, sm, nullptr, 1, 0, QtAS, nullptr,
+                                        d_work, st, 0, &sol);
+    return gram_fast<double, double>(n, AQ, sm, sm, S, sm, sm, nullptr, 1, 0, QtAS, nullptr, d_work,
+                                     st, 0, &sol);
 }
 
 extern "C" int cacg_k_gram_fast_f64f32(int n, const double *L, long ldl, int kl, const float *R1,

@@ -95,8 +95,8 @@ int cacg_k_cheb1_f32(const cacg_scsr *A, int k, const double *r, long ldr, float
  * chunk_rows > 0; 0 or 1: one): each XCD sweeps its chunks in that many passes,
  * pass h taking its chunks h, h + passes, ... (a narrow column of the grid,
  * plane by plane; taken for k > 32, ignored for k = 4..32, whose kernel
- * sweeps one pass).  The _x forms take one (NULL: the defaults); the forms
- * above use the defaults. */
+ * sweeps one pass).  The _x forms take one (NULL or all zeros: the default for
+ * the block's size); the forms above use the default. */
 typedef struct {
     int grid;
     int chunk_rows;
@@ -138,6 +138,17 @@ int cacg_k_gram_fast(int n, const double *L, long ldl, int kl, const double *R1,
  * cacg_k_gram_fast on the row-major copy. */
 int cacg_k_gram_fast_blk(int n, const double *L, long ldl, int kl, const double *R1, int bw,
                          long bs, int kr1, double *G1, double *d_work, hipStream_t st);
+/* Fast order with the small solve in the same launch as the chunk sums, for sm, m
+ * of at most 8 (cacg_gram_solve_supported), same bits as the calls they stand for:
+ * cacg_k_gram_alpha is cacg_k_gram_fast (QtAQ, QtR) and cacg_k_lu_solve (alpha, the
+ * factor kept in lu); cacg_k_gram_beta is cacg_k_gram_fast (QtAS, S FP64, or S32
+ * when not NULL) and cacg_k_lu_solve on the kept factor (beta). */
+int cacg_gram_solve_supported(int sm, int m);
+int cacg_k_gram_alpha(int n, int sm, int m, const double *Q, const double *AQ, const double *R,
+                      double *QtAQ, double *QtR, double *alpha, double *lu, int *d_flag,
+                      double *d_work, hipStream_t st);
+int cacg_k_gram_beta(int n, int sm, const double *AQ, const double *S, const float *S32,
+                     double *QtAS, double *beta, double *lu, double *d_work, hipStream_t st);
 /* 1 when cacg_k_gram_fast_blk takes this shape (ldl = kl, bs = n bw, 16-byte
  * aligned L and R1), else 0 */
 int cacg_gram_blk_supported(int n, int kl, int kr1, int bw);

@@ -220,3 +220,46 @@ def test_spmm_default_order_gives_the_same_bits(gpu_lib, edge, k):
     X = P.rhs_uniform(A.n, k, 3)
     print(f"spmm default order {edge}^3 k={k}", flush=True)
     assert np.array_equal(gpu_lib.k_spmm(A, X), gpu_lib.k_spmm(A, X, sched=(4096, 0, 0)))
+
+
+@pytest.mark.parametrize("n,sm,m", [(1, 1, 1), (300, 4, 1), (16384, 4, 1), (5000, 6, 2), (2000, 8, 8),
+                                    (4097, 7, 3), (700, 5, 5), (20001, 8, 4), (333, 3, 8)])
+def test_gram_with_solve_gives_the_bits_of_the_two_calls(gpu_lib, n, sm, m):
+    lib, D, rng = gpu_lib.lib(), gpu_lib.DeviceBuffer.from_array, np.random.default_rng(n + sm)
+    B = gpu_lib.DeviceBuffer
+    Q, S = rng.standard_normal((n, sm)), rng.standard_normal((n, sm))
+    R, AQ = rng.standard_normal((n, m)), Q * 2.0 + 0.1 * rng.standard_normal((n, sm))
+    dQ, dAQ, dS, dS32, dR = D(Q), D(AQ), D(S), D(S.astype(np.float32)), D(R)
+    ws = B(8 * lib.cacg_gram_workspace(sm, sm + m))
+    print(f"gram + solve n={n} sm={sm} m={m}", flush=True)
+    got, want = ({k: B(8 * sz) for k, sz in (("g1", sm * sm), ("g2", sm * m), ("x", sm * m), ("lu", sm * sm),
+                                             ("as", sm * sm), ("b", sm * sm), ("as32", sm * sm),
+                                             ("b32", sm * sm))} for _ in range(2))
+    flag = D(np.zeros(1, dtype=np.int32))
+    w = {k: b.ptr for k, b in want.items()}
+    assert lib.cacg_k_gram_fast(n, dQ.ptr, sm, sm, dAQ.ptr, sm, sm, dR.ptr, m, m, w["g1"], w["g2"],
+                                ws.ptr, None) == 0
+    assert lib.cacg_k_lu_solve(sm, w["g1"], m, w["g2"], w["x"], w["lu"], flag.ptr, 1, 0, None) == 0
+    assert lib.cacg_k_gram_fast(n, dAQ.ptr, sm, sm, dS.ptr, sm, sm, None, 1, 0, w["as"], None, ws.ptr,
+                                None) == 0
+    assert lib.cacg_k_lu_solve(sm, w["g1"], sm, w["as"], w["b"], w["lu"], flag.ptr, 1, 1, None) == 0
+    assert lib.cacg_k_gram_fast_f64f32(n, dAQ.ptr, sm, sm, dS32.ptr, sm, sm, None, 1, 0, w["as32"], None,
+                                       ws.ptr, None) == 0
+    assert lib.cacg_k_lu_solve(sm, w["g1"], sm, w["as32"], w["b32"], w["lu"], flag.ptr, 1, 1, None) == 0
+    g = {k: b.ptr for k, b in got.items()}
+    flag2 = D(np.zeros(1, dtype=np.int32))
+    assert lib.cacg_k_gram_alpha(n, sm, m, dQ.ptr, dAQ.ptr, dR.ptr, g["g1"], g["g2"], g["x"], g["lu"],
+                                 flag2.ptr, ws.ptr, None) == 0
+    assert lib.cacg_k_gram_beta(n, sm, dAQ.ptr, dS.ptr, None, g["as"], g["b"], g["lu"], ws.ptr, None) == 0
+    assert lib.cacg_k_gram_beta(n, sm, dAQ.ptr, None, dS32.ptr, g["as32"], g["b32"], g["lu"], ws.ptr,
+                                None) == 0
+    for k, b in got.items():
+        sz = (b.nbytes // 8,)
+        assert np.array_equal(b.download(sz), want[k].download(sz), equal_nan=True), k
+    assert flag2.download((1,), np.int32)[0] == flag.download((1,), np.int32)[0]
+
+
+@pytest.mark.parametrize("sm,m", [(9, 1), (8, 9), (0, 1), (4, 0)])
+def test_gram_with_solve_refuses_wider_blocks(gpu_lib, sm, m):
+    assert gpu_lib.lib().cacg_gram_solve_supported(sm, m) == 0
+    assert gpu_lib.lib().cacg_k_gram_alpha(10, sm, m, *([None] * 10)) != 0
