@@ -613,6 +613,116 @@ __global__ __launch_bounds__(64) void lu_back_ref_kernel(int N, const double *__
         x[e / kw * k + c0 + e % kw] = xs[e % kw * S + e / kw];
 }
 
+// The same for N <= 128, four columns to a wave: lane l holds entries l % 16, 16 +
+// l % 16, ... of column l / 16.  The products of 16 entries with a row of U are one
+// instruction, and sixteen v_fmac_f64 (x -1) take them in turn by DPP
+// (row_newbcast), each a subtraction rounded once, so a step of the chain costs the
+// wave one FP64 issue (8.5 cycles) instead of a product, a subtraction and their
+// operand reads.  U lies in LDS, its next row read while the current one runs.
+// Entries at or before i give zero products, which change nothing.
+// N = 128, the substitution alone: k = 16 164 -> about 30 us, k = 128 304 -> 32 us.
+constexpr int LB_W = 4;   // waves (of 4 columns) of a workgroup
+
+__device__ __forceinline__ void chain16_sub(double &acc, double v)
+{
+    const double minus = -1.0;
+    // s_nop: a DPP read comes two wait states after the write of its register
+#define CACG_LB(r) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #r " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" CACG_LB(0) CACG_LB(1) CACG_LB(2) CACG_LB(3) CACG_LB(4) CACG_LB(5) CACG_LB(6)
+            CACG_LB(7) CACG_LB(8) CACG_LB(9) CACG_LB(10) CACG_LB(11) CACG_LB(12) CACG_LB(13)
+                CACG_LB(14) CACG_LB(15)
+        : "+&v"(acc)
+        : "v"(v), "v"(minus));
+#undef CACG_LB
+}
+
+// rows 16 B + 15 .. 16 B of one column block, then the blocks before it; NB blocks
+// of 16 rows in all
+template <int NB, int B>
+__device__ __forceinline__ void back_block(double (&x)[NB], const double *us, const double *yc,
+                                           int S, int lane)
+{
+    double u[NB - B];
+    auto read = [&](double *w, int i) {
+#pragma unroll
+        for (int b = B; b < NB; b++)
+            w[b - B] = us[i * S + 16 * b + lane];
+    };
+    read(u, 16 * B + 15);
+    double y = yc[16 * B + 15];
+    for (int il = 15; il >= 0; il--) {
+        const int i = 16 * B + il, in = il > 0 ? i - 1 : i;
+        double un[NB - B];
+        read(un, in);
+        const double yn = yc[in];
+        double p[NB - B];
+#pragma unroll
+        for (int b = NB - 1; b > B; b--)
+            p[b - B] = mul_rn(x[b], u[b - B]);
+        p[0] = lane > il ? mul_rn(x[B], u[0]) : 0.0;
+        double acc = y;
+#pragma unroll
+        for (int b = B; b < NB; b++)
+            chain16_sub(acc, p[b - B]);
+        x[B] = lane == il ? acc : x[B];
+#pragma unroll
+        for (int b = 0; b < NB - B; b++)
+            u[b] = un[b];
+        y = yn;
+    }
+    if constexpr (B > 0)
+        back_block<NB, B - 1>(x, us, yc, S, lane);
+}
+
+// dynamic LDS: U (16 NB rows of 16 NB + 1, identity past N), then y of each column
+template <int NB>
+__global__ __launch_bounds__(LB_W * 64) void lu_back16_ref_kernel(int N,
+                                                                  const double *__restrict__ gw,
+                                                                  int k, double *__restrict__ x)
+{
+    extern __shared__ double us[];
+    constexpr int R = 16 * NB, S = R;
+    double *ys = us + R * S;   // entry i of column c at ys + c (R + 1) + i
+    const int t = threadIdx.x, c0 = blockIdx.x * LB_W * 4;
+    for (int e = t; e < R * R; e += LB_W * 64) {
+        const int i = e / R, q = e % R;
+        us[i * S + q] = i < N && q < N ? gw[(long)i * N + q] : 0.0;
+    }
+    for (int e = t; e < R * LB_W * 4; e += LB_W * 64) {
+        const int i = e / (LB_W * 4), c = e % (LB_W * 4);
+        ys[c * (R + 1) + i] = i < N && c0 + c < k ? x[(long)i * k + c0 + c] : 0.0;
+    }
+    __syncthreads();
+    const int lane = t & 15, c = t >> 4;
+    double v[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+        v[b] = 0.0;
+    back_block<NB, NB - 1>(v, us, ys + c * (R + 1), S, lane);
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+        ys[c * (R + 1) + 16 * b + lane] = v[b];
+    __syncthreads();
+    for (int e = t; e < N * LB_W * 4; e += LB_W * 64) {
+        const int i = e / (LB_W * 4), cc = e % (LB_W * 4);
+        if (c0 + cc < k)
+            x[(long)i * k + c0 + cc] = ys[cc * (R + 1) + i];
+    }
+}
+
+template <int NB>
+int launch_back16(int N, const double *gw, int k, double *x, hipStream_t st)
+{
+    constexpr int R = 16 * NB;
+    const size_t shm = ((size_t)R * R + LB_W * 4 * (R + 1)) * sizeof(double);
+    cacg_allow_lds(lu_back16_ref_kernel<NB>, shm);
+    hipLaunchKernelGGL(lu_back16_ref_kernel<NB>, dim3((k + LB_W * 4 - 1) / (LB_W * 4)),
+                       dim3(LB_W * 64), shm, st, N, gw, k, x);
+    CACG_LAUNCH_CHECK();
+    return 0;
+}
+
 // ---- batched ------------------------------------------------------------------------
 
 // workgroup b factors system items[b].x (N = sm <= 128, m <= 32): alpha = QtAQ^{-1} QtR
@@ -775,6 +885,18 @@ extern "C" int cacg_k_lu_solve(int N, const double *lhs, int k, const double *rh
             CACG_LAUNCH_CHECK();
         }
         LU_TRY(lu_blocked(N, k, rhs, x, d_work, d_flag, factor, fast, st));
+    }
+    if (!fast && N <= 128) {
+        switch ((N + 15) / 16) {
+        case 1: return launch_back16<1>(N, d_work, k, x, st);
+        case 2: return launch_back16<2>(N, d_work, k, x, st);
+        case 3: return launch_back16<3>(N, d_work, k, x, st);
+        case 4: return launch_back16<4>(N, d_work, k, x, st);
+        case 5: return launch_back16<5>(N, d_work, k, x, st);
+        case 6: return launch_back16<6>(N, d_work, k, x, st);
+        case 7: return launch_back16<7>(N, d_work, k, x, st);
+        default: return launch_back16<8>(N, d_work, k, x, st);
+        }
     }
     if (!fast) {
         // columns per workgroup: 16, fewer where N x 16 doubles exceed 128 KiB

@@ -263,3 +263,14 @@ def test_gram_with_solve_gives_the_bits_of_the_two_calls(gpu_lib, n, sm, m):
 def test_gram_with_solve_refuses_wider_blocks(gpu_lib, sm, m):
     assert gpu_lib.lib().cacg_gram_solve_supported(sm, m) == 0
     assert gpu_lib.lib().cacg_k_gram_alpha(10, sm, m, *([None] * 10)) != 0
+
+
+@pytest.mark.parametrize("N,k", [(1, 3), (2, 1), (15, 4), (16, 5), (17, 16), (32, 17), (47, 3), (60, 60),
+                                 (64, 1), (79, 10), (96, 33), (100, 20), (112, 7), (127, 16), (128, 130)])
+def test_lu_reference_edges_bitwise(gpu_lib, oracle_lib, N, k):
+    rng = np.random.default_rng(N + k)
+    M = rng.standard_normal((N, N))
+    A, rhs = M @ M.T + N * np.eye(N), rng.standard_normal((N, k))
+    print(f"reference solve N={N} k={k}", flush=True)
+    x, flag = gpu_lib.k_lu_solve(A, rhs, mode="reference")
+    assert flag == 0 and np.array_equal(x, oracle_lib.lu_solve(A, rhs))
