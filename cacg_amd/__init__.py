@@ -128,6 +128,7 @@ def lib() -> ctypes.CDLL:
         "cacg_k_cvt_f32_f64": ([c_long, _vp, _vp, _vp], c_int),
         "cacg_k_qupdate_zero": ([c_int, c_int, _vp, _vp, _vp], c_int),
         "cacg_tsqr_workspace": ([c_int], c_long),
+        "cacg_k_trimul_neg": ([c_int, c_int, _vp, c_long, _vp, _vp, _vp], c_int),
         "cacg_gram_solve_supported": ([c_int, c_int], c_int),
         "cacg_k_gram_alpha": ([c_int, c_int, c_int] + [_vp] * 10, c_int),
         "cacg_k_gram_beta": ([c_int, c_int] + [_vp] * 8, c_int),

@@ -732,7 +732,7 @@ __global__ __launch_bounds__(256) void xrupdate_mfma_kernel(int n, int m, const 
 // Q = S - Qin beta for any width sm <= SM (SM the next multiple of 16): the
 // scheme of qupdate_mfma_kernel with beta zero-padded to SM x SM in LDS and the
 // operand rows zero-padded in registers.  Qin (row stride ldi) may be Q itself:
-// a wave has read its 16 rows before it writes them.  S may be null (zero).
+// a wave has read its 16 rows before it writes them.
 // VEC 2: sm and ldi even, Qin 16-byte aligned (16-byte loads).
 // Bound by memory: three blocks of n sm values, and at n = 250,047, sm = 60 the
 // MFMAs take a fifth of that time.  Before, these widths took the
@@ -772,7 +772,7 @@ __global__ __launch_bounds__(256) void qupdate_pad_kernel(int n, int sm, const T
             for (int r = 0; r < 4; r++) {
                 const long i = i0 + lg + 4 * r;
                 const int c = j * 16 + lc;
-                sv[j][r] = S && i < n && c < sm ? S[i * sm + c] : (TS)0;
+                sv[j][r] = i < n && c < sm ? S[i * sm + c] : (TS)0;
             }
 #pragma unroll
         for (int j = 0; j < NTL; j++) {
@@ -967,6 +967,97 @@ int launch_xrupdate_mfma(int n, int m, const T *Q, const T *AQ, const double *al
         return 0;
     hipLaunchKernelGGL(colnorm2_final_kernel, dim3(m), dim3(256), 0, st, work, XR_BLOCKS,
                        m, d_norm2);
+    CACG_LAUNCH_CHECK();
+    return 0;
+}
+
+// Q = -A W for an upper triangular W (sm x sm, sm <= SM), A (row stride lda) may be Q
+// itself.  Of a wave's 16 rows lane (g, r) holds columns 8 p + 2 g, 8 p + 2 g + 1, so 8
+// contiguous columns of a row are one load and two MFMA steps, and column tile j takes
+// only the steps of rows k < 16 (j + 1) of W: 58% of them at SM = 96.  The next
+// tile's rows are loaded during the MFMAs.  Bound by memory (A read, Q written):
+// 300,000 x 96 146 -> 107 us (a copy of the same bytes takes 93).  W's rows lie 8 mod 16 doubles apart in LDS, which puts
+// the four lane groups (rows 2 g) of a read on two halves of the banks.
+template <int SM, int VEC>
+__global__ __launch_bounds__(256) void trimul_neg_kernel(int n, int sm, const double *A, long lda,
+                                                         double *Q, const double *__restrict__ W)
+{
+    constexpr int NP = SM / 8, NTL = SM / 16, LD = SM + 8;
+    extern __shared__ double bl[];
+    for (int e = threadIdx.x; e < SM * SM; e += 256) {
+        const int k = e / SM, c = e % SM;
+        bl[k * LD + c] = k < sm && c < sm ? W[k * sm + c] : 0.0;
+    }
+    __syncthreads();
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int lg = lane >> 4, lc = lane & 15;
+    const int ntiles = (n + 15) / 16, nw = gridDim.x * 4;
+    const int wid = xcd_remap(blockIdx.x, gridDim.x) * 4 + wave;
+    const int per = (ntiles + nw - 1) / nw;
+    const int tb = wid * per, te = tb + per < ntiles ? tb + per : ntiles;
+    double2 av[2][NP];
+    auto load = [&](int tile, int s) {
+        const long row = (long)tile * 16 + lc;
+        const double *a = A + (row < n ? row : n - 1) * lda + 2 * lg;
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            const int k = 8 * p + 2 * lg;
+            if constexpr (VEC == 2)
+                av[s][p] = k < sm ? *reinterpret_cast<const double2 *>(a + 8 * p) : double2{0.0, 0.0};
+            else
+                av[s][p] = double2{k < sm ? a[8 * p] : 0.0, k + 1 < sm ? a[8 * p + 1] : 0.0};
+        }
+    };
+    auto step = [&](int tile, int s) {
+        if (tile + 1 < te)
+            load(tile + 1, s ^ 1);
+#pragma unroll
+        for (int j = 0; j < NTL; j++) {
+            asm volatile("" ::: "memory");   // each tile's W reads after the last one's MFMAs
+            const double *w = bl + 2 * lg * LD + j * 16 + lc;
+            dbl4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int p = 0; p < 2 * (j + 1); p++) {
+                acc = mfma16x16x4(av[s][p].x, w[8 * p * LD], acc);
+                acc = mfma16x16x4(av[s][p].y, w[(8 * p + 1) * LD], acc);
+            }
+            const int c = j * 16 + lc;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const long i = (long)tile * 16 + lg + 4 * r;
+                if (i < n && c < sm)
+                    Q[i * sm + c] = -acc[r];
+            }
+        }
+    };
+    if (tb < te)
+        load(tb, 0);
+    for (int tile = tb; tile < te; tile += 2) {
+        step(tile, 0);
+        if (tile + 1 < te)
+            step(tile + 1, 1);
+    }
+}
+
+template <int SM>
+int launch_trimul(int n, int sm, const double *A, long lda, double *Q, const double *W, hipStream_t st)
+{
+    const size_t shm = (size_t)SM * (SM + 8) * sizeof(double);
+    const int perCU = SM <= 64 ? 4 : SM <= 96 ? 2 : 1;   // resident workgroups
+    int G = (n + 63) / 64;
+    if (G > 256 * perCU)
+        G = 256 * perCU;
+    if (G >= 8)
+        G &= ~7;
+    if (sm % 2 == 0 && lda % 2 == 0 && (uintptr_t)A % 16 == 0) {
+        cacg_allow_lds(trimul_neg_kernel<SM, 2>, shm);
+        hipLaunchKernelGGL((trimul_neg_kernel<SM, 2>), dim3(G), dim3(256), shm, st, n, sm, A, lda, Q,
+                           W);
+    } else {
+        cacg_allow_lds(trimul_neg_kernel<SM, 1>, shm);
+        hipLaunchKernelGGL((trimul_neg_kernel<SM, 1>), dim3(G), dim3(256), shm, st, n, sm, A, lda, Q,
+                           W);
+    }
     CACG_LAUNCH_CHECK();
     return 0;
 }
@@ -1373,14 +1464,23 @@ extern "C" int cacg_k_qupdate_zero(int n, int sm, double *Q, const double *beta,
     return qupdate<double, double>(n, sm, (const double *)nullptr, Q, beta, CACG_MODE_FAST, st);
 }
 
-extern "C" int cacg_k_rowmul_neg(int n, int sm, const double *A, long lda, double *Q,
-                                 const double *beta, hipStream_t st)
+extern "C" int cacg_k_trimul_neg(int n, int sm, const double *A, long lda, double *Q,
+                                 const double *W, hipStream_t st)
 {
     if (n < 0 || sm <= 0 || sm > 128 || lda < sm)
         return (int)hipErrorInvalidValue;
     if (n == 0)
         return 0;
-    return qupdate_pad<double>(n, sm, nullptr, A, lda, Q, beta, st);
+    switch ((sm + 15) / 16) {
+    case 1: return launch_trimul<16>(n, sm, A, lda, Q, W, st);
+    case 2: return launch_trimul<32>(n, sm, A, lda, Q, W, st);
+    case 3: return launch_trimul<48>(n, sm, A, lda, Q, W, st);
+    case 4: return launch_trimul<64>(n, sm, A, lda, Q, W, st);
+    case 5: return launch_trimul<80>(n, sm, A, lda, Q, W, st);
+    case 6: return launch_trimul<96>(n, sm, A, lda, Q, W, st);
+    case 7: return launch_trimul<112>(n, sm, A, lda, Q, W, st);
+    default: return launch_trimul<128>(n, sm, A, lda, Q, W, st);
+    }
 }
 
 extern "C" int cacg_k_qupdate_s32(int n, int sm, const float *S, double *Q, const double *beta,

@@ -248,7 +248,7 @@ extern "C" int cacg_k_tsqr(int n, int k, const double *A, long lda, double *Q, d
         hipLaunchKernelGGL(chol_inv_kernel, dim3(1), dim3(QT), 0, st, k, G, pass == 0 ? R1 : R2,
                            W, d_flag);
         CACG_LAUNCH_CHECK();
-        rc = cacg_k_rowmul_neg(n, k, in, ld, Q, W, st);   // Q = in (-W)
+        rc = cacg_k_trimul_neg(n, k, in, ld, Q, W, st);   // Q = in (-W)
         if (rc)
             return rc;
     }

@@ -195,8 +195,9 @@ int cacg_k_xrupdate_split(int n, int sm, int m, const double *Q, const double *A
                           double *d_work, int which, hipStream_t st);
 /* Q = -Q beta in place (S = 0; fast order), the tall-skinny product of the QR */
 int cacg_k_qupdate_zero(int n, int sm, double *Q, const double *beta, hipStream_t st);
-/* Q = -(A beta) for A n x sm with row stride lda (A may be Q itself with lda = sm), sm <= 128 */
-int cacg_k_rowmul_neg(int n, int sm, const double *A, long lda, double *Q, const double *beta,
+/* Q = -A W for an upper triangular W (sm x sm, sm <= 128; what lies below its
+ * diagonal is zero), A with row stride lda, possibly Q itself */
+int cacg_k_trimul_neg(int n, int sm, const double *A, long lda, double *Q, const double *W,
                       hipStream_t st);
 /* FP32 basis S, FP64 Q (the precision form's update): Q = S - Q beta in FP64. */
 int cacg_k_qupdate_s32(int n, int sm, const float *S, double *Q, const double *beta,

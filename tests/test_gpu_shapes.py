@@ -274,3 +274,19 @@ def test_lu_reference_edges_bitwise(gpu_lib, oracle_lib, N, k):
     print(f"reference solve N={N} k={k}", flush=True)
     x, flag = gpu_lib.k_lu_solve(A, rhs, mode="reference")
     assert flag == 0 and np.array_equal(x, oracle_lib.lu_solve(A, rhs))
+
+
+@pytest.mark.parametrize("n", [1, 16, 33, 5000, 40007])
+@pytest.mark.parametrize("k,lda", [(1, 1), (2, 5), (15, 15), (17, 20), (32, 32), (63, 64), (80, 80),
+                                   (97, 97), (112, 114), (128, 128)])
+def test_triangular_row_product_exact_on_integers(gpu_lib, n, k, lda):
+    lib, D, rng = gpu_lib.lib(), gpu_lib.DeviceBuffer.from_array, np.random.default_rng(n + k)
+    A = rng.integers(-8, 9, size=(n, lda)).astype(np.float64)
+    W = np.triu(rng.integers(-8, 9, size=(k, k))).astype(np.float64)
+    dA, dW, Q = D(A), D(W), gpu_lib.DeviceBuffer(8 * n * k)
+    print(f"triangular row product n={n} k={k} lda={lda}", flush=True)
+    assert lib.cacg_k_trimul_neg(n, k, dA.ptr, lda, Q.ptr, dW.ptr, None) == 0
+    assert np.array_equal(Q.download((n, k)), -(A[:, :k] @ W))
+    if lda == k:   # in place
+        assert lib.cacg_k_trimul_neg(n, k, dA.ptr, lda, dA.ptr, dW.ptr, None) == 0
+        assert np.array_equal(dA.download((n, k)), -(A @ W))
