@@ -526,7 +526,13 @@ __host__ __device__ inline int lds_row_stride(int k)
     return k + (48 - k % 32) % 32;
 }
 
-template <typename TL, typename T1, int NW, int MT, int NT, int SR, int LDG, int VPT>
+// FULL (FP64, every column of the tiles present: 128 x 128 and 128 x 144): the stage
+// loop without a bound, a select or an address computation beside one addition per
+// load; LDS strides and buffers are immediate offsets.  Every vector instruction
+// there is paid in matrix-core time (FP64 MFMAs leave the SIMD few issue slots: 60 more
+// of them a stage had cost 2 to 10%).  2,097,152 rows: 128 x 144 1390 -> 1246 us (62
+// TFLOP/s), 128 x 128 1249 -> 1110 us.
+template <typename TL, typename T1, int NW, int MT, int NT, int SR, int LDG, int VPT, bool FULL>
 __global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s,
                                                            double *__restrict__ part, int kl_pad,
                                                            int kr_pad, int chunk, int GN, int NG)
@@ -677,9 +683,66 @@ __global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s
     lstore(0, 0);
     gload(0, LDG);
     __syncthreads();
+    int first = 0;   // first stage of the general loop below
+    if constexpr (FULL) {
+        constexpr int P = 144, B = SR * 2 * P;   // LDS row stride of 128 and of 144 columns; a buffer
+        constexpr int VEC16 = SR * (128 + (NW == 12 ? 144 : 128)) / 2;   // vectors of a stage
+        static_assert(LDG == 2, "buffer and register slot go by the parity of the stage");
+        const int full = (r1 - r0) / SR;
+        const char *ptr[VPT];
+        long inc[VPT];
+        double *dst[VPT];
+        bool has[VPT];   // of the whole wave
+#pragma unroll
+        for (int u = 0; u < VPT; u++) {
+            ptr[u] = src[u] + (long)(r0 + (LDG + 1) * SR + max(srow[u], 0)) * ldb[u];
+            inc[u] = SR * ldb[u];
+            dst[u] = lds + loff[u];
+            has[u] = __builtin_amdgcn_readfirstlane(srow[u]) >= 0;
+        }
+        const double *const bl = lds + lr * P + ca0, *const br = lds + SR * P + lr * P + cb0;
+        double av[2][MT], bv[2][NT];
+        auto operands = [&](int buf, int ks, int p) {
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+                av[p][t] = bl[buf * B + ks * 4 * P + 16 * t];
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                bv[p][t] = br[buf * B + ks * 4 * P + 16 * t];
+        };
+        // loads reach LDG + 1 stages past the one computed
+        for (; first + 2 * LDG < full; first += 2) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                operands(q, 0, 0);
+#pragma unroll
+                for (int ks = 0; ks < SR / 4; ks++) {
+                    if (ks + 1 < SR / 4)
+                        operands(q, ks + 1, (ks + 1) & 1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+#pragma unroll
+                        for (int j = 0; j < NT; j++)
+                            acc[i][j] = mfma16x16x4(av[ks & 1][i], bv[ks & 1][j], acc[i][j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int u = 0; u < VPT; u++)
+                    if ((u + 1) * NTH <= VEC16 || has[u]) {
+                        double2 d;
+                        __builtin_memcpy(&d, &stg[q ^ 1][u], 16);
+                        *reinterpret_cast<double2 *>(dst[u] + (q ^ 1) * B) = d;
+                        stg[q ^ 1][u] = *reinterpret_cast<const uint4 *>(ptr[u]);
+                        ptr[u] += inc[u];
+                    }
+                __syncthreads();
+            }
+        }
+    }
     // stage st: computed from buffer st & 1; its successor st + 1 sits in
     // register slot (st + 1) % LDG and is stored to the other buffer
-    for (int st0 = 0; st0 < nstage; st0 += LDG) {
+    for (int st0 = first; st0 < nstage; st0 += LDG) {
 #pragma unroll
         for (int q = 0; q < LDG; q++) {
             const int st = st0 + q;
@@ -732,19 +795,36 @@ int launch_gram_wide(int n, const SrcT<TL, T1> &s, const GramPlan &p, double *wo
     if (!staged_ok || p.TM != 8 || p.chunk % SRW != 0 || (p.TN != 8 && p.TN != 9))
         return 0;
     const size_t shm = 2 * (size_t)SRW * (lds_row_stride(s.kl) + lds_row_stride(kr)) * sizeof(double);
+    // every column of the tiles present
+    const bool full = sizeof(TL) == 8 && sizeof(T1) == 8 && s.kl == 128 && kr == kr_pad;
+#define CACG_GW(NW, NT, VPT, FULL, GN)                                                            \
+    do {                                                                                          \
+        cacg_allow_lds(gram_lds_kernel<TL, T1, NW, 2, NT, SRW, 2, VPT, FULL>, shm);               \
+        hipLaunchKernelGGL((gram_lds_kernel<TL, T1, NW, 2, NT, SRW, 2, VPT, FULL>), dim3(p.gx, 1), \
+                           dim3(NW * 64), shm, st, n, s, work, kl_pad, kr_pad, p.chunk, GN, NW);  \
+    } while (0)
     if (p.TN == 9) {
         if (stage_vectors(s, SRW) > 12 * 64 * 3)
             return 0;
-        cacg_allow_lds(gram_lds_kernel<TL, T1, 12, 2, 3, SRW, 2, 3>, shm);
-        hipLaunchKernelGGL((gram_lds_kernel<TL, T1, 12, 2, 3, SRW, 2, 3>), dim3(p.gx, 1),
-                           dim3(12 * 64), shm, st, n, s, work, kl_pad, kr_pad, p.chunk, 3, 12);
+        if constexpr (sizeof(T1) == 8) {
+            if (full) {
+                CACG_GW(12, 3, 3, true, 3);
+                return 1;
+            }
+        }
+        CACG_GW(12, 3, 3, false, 3);
     } else {
         if (stage_vectors(s, SRW) > 16 * 64 * 2)
             return 0;
-        cacg_allow_lds(gram_lds_kernel<TL, T1, 16, 2, 2, SRW, 2, 2>, shm);
-        hipLaunchKernelGGL((gram_lds_kernel<TL, T1, 16, 2, 2, SRW, 2, 2>), dim3(p.gx, 1),
-                           dim3(16 * 64), shm, st, n, s, work, kl_pad, kr_pad, p.chunk, 4, 16);
+        if constexpr (sizeof(T1) == 8) {
+            if (full) {
+                CACG_GW(16, 2, 2, true, 4);
+                return 1;
+            }
+        }
+        CACG_GW(16, 2, 2, false, 4);
     }
+#undef CACG_GW
     return 1;
 }
 
