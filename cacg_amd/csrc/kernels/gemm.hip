@@ -486,17 +486,82 @@ __global__ __launch_bounds__(512) void qupdate_mfma_kernel(int n, const TS *__re
         }
     }
     __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // wave-uniform, so that tile addresses are scalar
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int lg = lane >> 4, lc = lane & 15;
     const int nw = gridDim.x * 8;
     const int wid = xcd_remap(blockIdx.x, gridDim.x) * 8 + wave;
     const int ntiles = (n + 15) / 16;
     // contiguous tile ranges per wave
     const int per = (ntiles + nw - 1) / nw;
-    const int tb = wid * per;
+    int tb = wid * per;
     int te = tb + per;
     if (te > ntiles)
         te = ntiles;
+    // Whole tiles (16 rows, FP64, a column tile inside one block of S): every address
+    // is a scalar tile address plus a lane offset that no tile changes, and nothing is
+    // tested.  FP64 MFMAs leave a SIMD few issue slots, and the row tests, 64-bit
+    // products and a division per column tile of the general form below took 600 vector
+    // instructions a tile of 288 MFMAs.  With the X update: 128 columns 2,097,152 rows 1598 ->
+    // 1590 us (a copy of the bytes takes 1407), 262,144 rows 235 -> 228 us; 96 columns
+    // 250,047 rows 151 -> 144 us; 64 columns 16,384 rows 12.4 -> 10.8 us.
+    if constexpr (sizeof(TS) == 8 && sizeof(T) == 8) {
+        const int rs = sbs ? sbw : SM;
+        if (S && (!sbs || sbw % 16 == 0)) {
+            unsigned so[4], qo[4], xo[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                so[r] = (unsigned)((lg + 4 * r) * rs + lc);
+                qo[r] = (unsigned)((lg + 4 * r) * SM + lc);
+                xo[r] = (unsigned)((lg + 4 * r) * m + lc);
+            }
+            const unsigned ao = (unsigned)(lc * SM + lg * KQ);
+            for (; tb < te && (long)tb * 16 + 16 <= n; tb++) {
+                const long i0 = (long)tb * 16;
+                double *const qt = reinterpret_cast<double *>(Q) + i0 * SM;
+                double av[KQ], xv[NA][4], sv[NTL][4];
+                load_row<double, KQ>(qt + ao, av);
+                if constexpr (NTX > 0) {
+#pragma unroll
+                    for (int j = 0; j < NA; j++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+                            xv[j][r] = 16 * j + lc < m ? (X + i0 * m + 16 * j)[xo[r]] : 0.0;
+                }
+#pragma unroll
+                for (int j = 0; j < NTL; j++) {
+                    const double *st = reinterpret_cast<const double *>(S) + i0 * rs +
+                                       (sbs ? 16 * j / sbw * sbs + 16 * j % sbw : 16 * j);
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        sv[j][r] = st[so[r]];
+                }
+#pragma unroll
+                for (int j = 0; j < NTL; j++) {
+                    asm volatile("" ::: "memory");
+                    const double *bcol = bl + (lg * KQ) * SM + j * 16 + lc;
+                    const dbl4 acc = mfma_chain_lds<KQ>(av, bcol, SM, dbl4{0.0, 0.0, 0.0, 0.0});
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        (qt + 16 * j)[qo[r]] = sv[j][r] - acc[r];
+                }
+                if constexpr (NTX > 0) {
+#pragma unroll
+                    for (int j = 0; j < NA; j++) {
+                        asm volatile("" ::: "memory");
+                        const double *acol = al + (lg * KQ) * (16 * NA) + j * 16 + lc;
+                        const dbl4 ax =
+                            mfma_chain_lds<KQ>(av, acol, 16 * NA, dbl4{0.0, 0.0, 0.0, 0.0});
+                        if (16 * j + lc < m) {
+#pragma unroll
+                            for (int r = 0; r < 4; r++)
+                                (X + i0 * m + 16 * j)[xo[r]] = xv[j][r] + ax[r];
+                        }
+                    }
+                }
+            }
+        }
+    }
     for (int tile = tb; tile < te; tile++) {
         const long i0 = (long)tile * 16;
         const long arow = i0 + lc;

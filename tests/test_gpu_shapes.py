@@ -290,3 +290,19 @@ def test_triangular_row_product_exact_on_integers(gpu_lib, n, k, lda):
     if lda == k:   # in place
         assert lib.cacg_k_trimul_neg(n, k, dA.ptr, lda, dA.ptr, dW.ptr, None) == 0
         assert np.array_equal(dA.download((n, k)), -(A @ W))
+
+
+@pytest.mark.parametrize("n,sm,m", [(16, 16, 4), (15, 32, 8), (17, 48, 12), (2048 * 16 + 5, 64, 16),
+                                    (4000, 96, 12), (4099, 112, 28), (33000, 128, 16), (5000, 128, 32),
+                                    (3000, 64, 32)])
+def test_q_update_whole_and_last_tiles_exact_on_integers(gpu_lib, n, sm, m):
+    rng = np.random.default_rng(n + sm)
+    S, Q = (rng.integers(-8, 9, size=(n, sm)).astype(np.float64) for _ in range(2))
+    beta, alpha = (rng.integers(-8, 9, size=(sm, k)).astype(np.float64) for k in (sm, m))
+    X = rng.integers(-8, 9, size=(n, m)).astype(np.float64)
+    print(f"q update n={n} sm={sm} m={m}", flush=True)
+    assert np.array_equal(gpu_lib.k_qupdate(S, Q, beta, mode="fast"), S - Q @ beta)
+    Qn, Xn = gpu_lib.k_qxupdate(S, Q, beta, alpha, X)
+    assert np.array_equal(Qn, S - Q @ beta) and np.array_equal(Xn, X + Q @ alpha)
+    Qb, Xb = gpu_lib.k_qxupdate_blk(S, Q, beta, alpha, X, 0)
+    assert np.array_equal(Qb, Qn) and np.array_equal(Xb, Xn)
