@@ -133,6 +133,7 @@ def lib() -> ctypes.CDLL:
         "cacg_k_gram_alpha": ([c_int, c_int, c_int] + [_vp] * 10, c_int),
         "cacg_k_gram_beta": ([c_int, c_int] + [_vp] * 8, c_int),
         "cacg_bgram_groups": ([c_int, c_int], c_int),
+        "cacg_kb_gram_class": ([_vp, _vp, c_int, c_int, c_int, c_int, c_int, _vp], c_int),
         "cacg_kb_gram": ([_vp, _vp, c_int, c_int, c_int, c_int, _vp], c_int),
         "cacg_kb_gram_reduce": ([_vp, _vp, c_int, c_int, _vp], c_int),
         "cacg_k_tsqr": ([c_int, c_int, _vp, c_long, _vp, _vp, _vp, _vp, _vp], c_int),

@@ -731,6 +731,17 @@ extern "C" int cacg_kb_gram(const cacg_bsys *d_sys, const int2 *d_chunks, int nc
     return 0;
 }
 
+// the systems of one tile class: tm = ceil(sm / 16), tn = ceil(kr / 16)
+extern "C" int cacg_kb_gram_class(const cacg_bsys *d_sys, const int2 *d_chunks, int nchunks,
+                                  int which, int f32, int tm, int tn, hipStream_t st)
+{
+    if (nchunks <= 0)
+        return 0;
+    if ((which != 0 && which != 1) || tm < 1 || tm > 8 || tn < tm || tn > tm + (which ? 2 : 0))
+        return (int)hipErrorInvalidValue;
+    return cacg_kb_gram(d_sys, d_chunks, nchunks, cacg_bgram_groups(16 * tm, 16 * tn), which, f32, st);
+}
+
 extern "C" int cacg_kb_gram_reduce(const cacg_bsys *d_sys, const int2 *d_blocks, int nblocks,
                                    int which, hipStream_t st)
 {

@@ -797,7 +797,7 @@ __global__ __launch_bounds__(256) void xrupdate_mfma_kernel(int n, int m, const 
 // Q = S - Qin beta for any width sm <= SM (SM the next multiple of 16): the
 // scheme of qupdate_mfma_kernel with beta zero-padded to SM x SM in LDS and the
 // operand rows zero-padded in registers.  Qin (row stride ldi) may be Q itself:
-// a wave has read its 16 rows before it writes them.
+// a wave has read its 16 rows before it writes them.  S may be null (zero).
 // VEC 2: sm and ldi even, Qin 16-byte aligned (16-byte loads).
 // Bound by memory: three blocks of n sm values, and at n = 250,047, sm = 60 the
 // MFMAs take a fifth of that time.  Before, these widths took the
@@ -837,7 +837,7 @@ __global__ __launch_bounds__(256) void qupdate_pad_kernel(int n, int sm, const T
             for (int r = 0; r < 4; r++) {
                 const long i = i0 + lg + 4 * r;
                 const int c = j * 16 + lc;
-                sv[j][r] = i < n && c < sm ? S[i * sm + c] : (TS)0;
+                sv[j][r] = S && i < n && c < sm ? S[i * sm + c] : (TS)0;
             }
 #pragma unroll
         for (int j = 0; j < NTL; j++) {

@@ -296,6 +296,10 @@ int cacg_kb_aq(const cacg_bsys *d_sys, const int2 *d_tiles, int count, hipStream
 int cacg_bgram_groups(int sm, int kr);
 int cacg_kb_gram(const cacg_bsys *d_sys, const int2 *d_chunks, int nchunks, int groups, int which,
                  int f32, hipStream_t st);
+/* the same for the systems of one tile class, tm = ceil(sm / 16) in 1 .. 8 and tn =
+ * ceil(kr / 16) in tm .. tm + 2 */
+int cacg_kb_gram_class(const cacg_bsys *d_sys, const int2 *d_chunks, int nchunks, int which,
+                       int f32, int tm, int tn, hipStream_t st);
 int cacg_kb_gram_reduce(const cacg_bsys *d_sys, const int2 *d_blocks, int nblocks, int which,
                         hipStream_t st);
 /* which 0: beta = QtAQ^{-1} QtAS (factor from the last which-1 call); which 1:

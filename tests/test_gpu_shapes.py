@@ -306,3 +306,20 @@ def test_q_update_whole_and_last_tiles_exact_on_integers(gpu_lib, n, sm, m):
     assert np.array_equal(Qn, S - Q @ beta) and np.array_equal(Xn, X + Q @ alpha)
     Qb, Xb = gpu_lib.k_qxupdate_blk(S, Q, beta, alpha, X, 0)
     assert np.array_equal(Qb, Qn) and np.array_equal(Xb, Xn)
+
+
+@pytest.mark.parametrize("sm", [4, 8, 12, 16, 20, 96, 100, 128])
+@pytest.mark.parametrize("n", [17, 5000])
+def test_q_update_without_s_exact_on_integers(gpu_lib, n, sm):
+    lib, D, rng = gpu_lib.lib(), gpu_lib.DeviceBuffer.from_array, np.random.default_rng(n + sm)
+    Q = rng.integers(-8, 9, size=(n, sm)).astype(np.float64)
+    beta = rng.integers(-8, 9, size=(sm, sm)).astype(np.float64)
+    dQ, db = D(Q), D(beta)
+    print(f"q update without S n={n} sm={sm}", flush=True)
+    assert lib.cacg_k_qupdate_zero(n, sm, dQ.ptr, db.ptr, None) == 0
+    assert np.array_equal(dQ.download((n, sm)), -(Q @ beta))
+
+
+@pytest.mark.parametrize("which,tm,tn", [(0, 1, 2), (1, 2, 1), (1, 1, 4), (2, 1, 1), (1, 9, 9), (0, 0, 0)])
+def test_batched_gram_class_refuses_what_is_no_class(gpu_lib, which, tm, tn):
+    assert gpu_lib.lib().cacg_kb_gram_class(None, None, 1, which, 0, tm, tn, None) != 0
