@@ -1051,7 +1051,49 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
     lstore(0, 0);
     gload(0, LDG);
     __syncthreads();
-    for (int st0 = 0; st0 < nstage; st0 += LDG) {
+    // whole stages without row tests or selects, as in gram_lds_kernel: an addition per
+    // load, and lanes without a vector load the start of L and store nothing.  Not where
+    // 16 waves' 128 registers would spill, nor for one or two tiles a wave, which are
+    // bound by memory (2,097,152 rows of 16 + 4 columns: 112 -> 118 us).  300,000 rows of 96
+    // columns 124 -> 113 us, 1,000,000 of 64 + 8 240 -> 222 us, 300,000 of 99 + 11 184 -> 168.
+    int first = 0;
+    const int full = (r1 - r0) / SR;
+    if (sizeof(T1) == 8 && VEC == 2 && MT * NT >= 3 && (W == 8 || MT * NT <= 4) && full > 2 * LDG) {
+        long inc[VPT];
+        V *dst[VPT];
+#pragma unroll
+        for (int u = 0; u < VPT; u++) {
+            const int kind = info[u] >> 10 & 3;
+            inc[u] = info[u] == ~0u ? 0 : kind == 0 ? incl : kind == 1 ? inc1 : inc2;
+            dst[u] = reinterpret_cast<V *>(lds + (info[u] >> 12));
+            if (info[u] == ~0u)
+                src[u] = reinterpret_cast<const char *>(s.L);
+        }
+        for (; first + 2 * LDG < full; first += 2) {
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                compute(q);
+                double *const b = lds + (q ^ 1) * BUF;
+                if constexpr (one) {
+                    if (t < SR && k2 > 0) {
+                        b[SR * LDP + t * RDP + k1] = stg1[q ^ 1];
+                        stg1[q ^ 1] = *src1;
+                    }
+                    src1 += SR * s.ld2;
+                }
+#pragma unroll
+                for (int u = 0; u < VPT; u++) {
+                    if (info[u] != ~0u)
+                        *reinterpret_cast<V *>(reinterpret_cast<double *>(dst[u]) + (q ^ 1) * BUF) =
+                            stg[q ^ 1][u];
+                    stg[q ^ 1][u] = *reinterpret_cast<const V *>(src[u]);
+                    src[u] += inc[u];
+                }
+                __syncthreads();
+            }
+        }
+    }
+    for (int st0 = first; st0 < nstage; st0 += LDG) {
 #pragma unroll
         for (int q = 0; q < LDG; q++) {
             const int st = st0 + q;
