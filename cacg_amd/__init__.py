@@ -234,7 +234,7 @@ class DeviceCSR:
         self.val = DeviceBuffer.from_array(np.asarray(A.val, dtype=np.float64))
         lm, ids = long_rows(A, long_min)
         self.n_long = len(ids)
-        self.long_min = lm if self.n_long else 0
+        self.long_min = lm   # with no long rows: looked for and not there
         self.lrows = DeviceBuffer.from_array(ids) if self.n_long else None
         lp = self.lrows.ptr if self.lrows else None
         self.s = DCsr(A.n, self.rowptr.ptr, self.col.ptr, self.val.ptr, lp, self.n_long,

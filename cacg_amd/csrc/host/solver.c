@@ -502,6 +502,7 @@ int cacg_solver_create(cacg_solver **out, long n, const long *row_start, const l
         /* rows far longer than the mean go to the row-split SpMM */
         const int lmin = cacg_csr_long_min(n, row_start);
         const long nl = cacg_csr_long_rows(n, row_start, lmin, NULL);
+        sv->A.long_min = lmin;   /* without long rows: looked for and not there */
         if (nl > 0) {
             int *ids = (int *)malloc(sizeof(int) * (size_t)nl);
             if (!ids || dalloc(sv, (void **)&sv->d_long_rows, nl * (long)sizeof(int)) != CACG_OK) {
@@ -518,7 +519,6 @@ int cacg_solver_create(cacg_solver **out, long n, const long *row_start, const l
             }
             sv->A.long_rows = sv->d_long_rows;
             sv->A.n_long = (int)nl;
-            sv->A.long_min = lmin;
         }
     }
     if (prec32) {

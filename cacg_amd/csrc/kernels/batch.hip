@@ -5,12 +5,15 @@
 // the SpMM kernels map lanes to the elements (row, column) of a 64-row tile:
 // lane e of the tile handles row e / k, column e % k, which keeps every lane
 // busy for any k.  The dense products (Gram blocks, Q = S - Q beta,
-// X += Q alpha) run on FP64 MFMA over 2048-row chunks, one launch per tile
-// class (the system's sm and m rounded up to 16-column tiles, zero-padded);
-// a second kernel sums the Gram chunk partials in chunk order.  Every sum of
-// a system runs in an order fixed by that system alone (its rows, tiles,
-// chunks and class), so a system's results are the same bits whatever else
-// shares the launch.
+// X += Q alpha) run on FP64 MFMA over 2048-row chunks: the Gram in one launch for
+// every width, a chunk's output tiles split over waves; the updates with one
+// launch per tile class (the system's sm and m rounded up to 16-column tiles,
+// zero-padded), a chunk's rows split until the launch fills the chip.  A second
+// kernel sums the Gram chunk partials in chunk order.  Every sum of a system runs
+// in an order fixed by that system alone (its rows, tiles, chunks and class), so a
+// system's results are the same bits whatever else shares the launch.
+// 64 systems, FP32 basis: 252 -> 116 ms; the Gram of a full round 1110 -> about 300
+// us, Q updates 830 -> 240, X updates 546 -> 118.
 #include <type_traits>
 
 #include "kcommon.hpp"

@@ -552,16 +552,18 @@ __global__ __launch_bounds__(LR_T) void spmm_long_kernel(
 // default is therefore as many workgroups as stay resident, in chunks: 3 per CU
 // and 2048 rows up to 16 columns (from 16 MB, where the order of the front starts
 // to count), 4 per CU and 1024 rows above 64 columns.  In between neither order
-// wins everywhere, and rows of very different lengths (a long-row list) need
-// the spare workgroups to balance.  128^3 Laplacian: k = 16 242 -> 224 us, k =
+// wins everywhere, and rows of very different lengths need the spare workgroups
+// to balance (1024^2 grid with 64 hub rows left to the lane groups: 5.2 -> 9.8 ms
+// at 16 columns), so it takes a matrix whose row lengths were looked at (long_min)
+// and held no long row.  128^3 Laplacian: k = 16 242 -> 224 us, k =
 // 128 1517 -> 1336 us (a copy of the same bytes takes 200 and 900); 96^3: 107 ->
 // 101, 673 -> 583; 1024^2: 109 -> 103, 667 -> 598; 64^3: 34 -> 33, 166 -> 147.
-inline cacg_spmm_sched default_sched(long n, int k, int lpr, int vw, bool ragged)
+inline cacg_spmm_sched default_sched(long n, int k, int lpr, int vw, bool even)
 {
     const long bytes = n * (long)k * 8;
-    if (!ragged && vw == 4 && lpr <= 4 && bytes >= 16L << 20)
+    if (even && vw == 4 && lpr <= 4 && bytes >= 16L << 20)
         return {768, 2048, 0};
-    if (!ragged && vw == 4 && k > 64 && bytes >= 256L << 20)
+    if (even && vw == 4 && k > 64 && bytes >= 256L << 20)
         return {1024, 1024, 0};
     return {0, 0, 0};
 }
@@ -574,7 +576,7 @@ int launch_spmm(int n, const int *rowptr, const int *col, const TV *val, int k, 
 {
     constexpr int RPG = LPR >= 16 ? 2 : 1;
     constexpr int TR = (256 / LPR) * RPG;
-    const cacg_spmm_sched def = default_sched(n, k, LPR, VW, n_long > 0);
+    const cacg_spmm_sched def = default_sched(n, k, LPR, VW, n_long == 0 && long_min > 0);
     if (!sc || (sc->grid == 0 && sc->chunk_rows == 0))
         sc = &def;
     const int gmax = sc->grid > 0 ? sc->grid : (LPR >= 16 ? 4096 : 8192);

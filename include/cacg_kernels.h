@@ -21,8 +21,9 @@ extern "C" {
  * Long rows: with long_min > 0, the SpMMs leave every row with at least
  * long_min nonzeros to a row-split kernel (one workgroup per row), and
  * long_rows (device, n_long ids) must list exactly those rows
- * (cacg_csr_long_rows builds it).  long_min = 0 (zero-initialised): every row
- * vector-per-row. */
+ * (cacg_csr_long_rows builds it).  long_min > 0 with no such row also says that
+ * the row lengths are even (the default launch order goes by it).  long_min = 0
+ * (zero-initialised): every row vector-per-row. */
 typedef struct {
     int n;
     const int *rowptr;
