@@ -17,6 +17,7 @@
 // independent of scheduling.
 #include <type_traits>
 
+#include "gram_plan.hpp"
 #include "kcommon.hpp"
 
 namespace {
@@ -274,54 +275,6 @@ __global__ __launch_bounds__(512) void gram_ref_kernel(int n, GrefSrc s, int nbb
 
 // ---- fast: split-K FP64 MFMA ------------------------------------------------
 
-struct GramPlan {
-    int TM, TN;      // 16x16 tiles in M (kl) and N (kr)
-    int MT, NT;      // tiles per wave
-    int GN, NG;      // tile groups along N, total groups
-    int WGG, KS;     // groups per workgroup, waves sharing one group (split K inside the workgroup)
-    int gy;          // workgroups along the tile-group dimension
-    int gx;          // row chunks (split K across workgroups)
-    int chunk;       // rows per chunk
-};
-
-GramPlan plan_gram(int n, int kl, int kr)
-{
-    GramPlan p;
-    p.TM = (kl + 15) / 16;
-    p.TN = (kr + 15) / 16;
-    p.NT = p.TN < 9 ? p.TN : 9;
-    p.GN = (p.TN + p.NT - 1) / p.NT;
-    p.MT = p.TM >= 8 ? 2 : 1;
-    const int GM = (p.TM + p.MT - 1) / p.MT;
-    p.NG = GM * p.GN;
-    if (p.NG >= 4) {
-        p.WGG = 4;
-        p.KS = 1;
-    } else {
-        p.WGG = p.NG;
-        p.KS = 4 / p.NG;
-    }
-    p.gy = (p.NG + p.WGG - 1) / p.WGG;
-    // about 2 workgroups per CU over 256 CUs, at least 64 rows per chunk; a
-    // function of n only, so the summation order does not depend on the device
-    int gx = 512 / p.gy;
-    if (gx < 1)
-        gx = 1;
-    const int step = 8 * p.KS;
-    long maxc = ((long)n + 63) / 64;
-    if (gx > maxc)
-        gx = (int)(maxc > 0 ? maxc : 1);
-    long chunk = ((long)n + gx - 1) / gx;
-    chunk = (chunk + step - 1) / step * step;
-    if (chunk < step)
-        chunk = step;
-    p.chunk = (int)chunk;
-    p.gx = (int)(((long)n + chunk - 1) / chunk);
-    if (p.gx < 1)
-        p.gx = 1;
-    return p;
-}
-
 // the shapes with a block-major R1, given the 16-byte vectors of a stage of 16
 // and of 8 rows: the wide kernels', or at most 5 vectors per lane of 256
 bool blk_shape(int n, const GramPlan &p, long vec16, long vec8)
@@ -516,16 +469,6 @@ __global__ __launch_bounds__(1024) void gram_solve_kernel(const double *__restri
 //   <12, 2, 3, 16, 2, 3>, <16, 2, 2, 16, 2, 2>: a 128-row G against 144 and
 //   128 columns, as 12 and 16 waves of 2 x 3 and 2 x 2 tiles (measured on
 //   gfx950: 58 and 56 TFLOP/s against 42 and 50 for the general shape).
-// LDS row stride (doubles) of a staged k-column block: k rounded up to 16
-// mod 32.  A wave reads 4 rows x 16 consecutive doubles per MFMA operand;
-// with a stride of 16 mod 32 doubles, rows 0, 1 (and 2, 3) fall into the two
-// disjoint halves of the 64 four-byte LDS banks, so a 64-lane read takes the
-// 2 cycles its 512 bytes need (a stride of k + 2 overlapped all four rows).
-__host__ __device__ inline int lds_row_stride(int k)
-{
-    return k + (48 - k % 32) % 32;
-}
-
 // FULL (FP64, every column of the tiles present: 128 x 128 and 128 x 144): the stage
 // loop without a bound, a select or an address computation beside one addition per
 // load; LDS strides and buffers are immediate offsets.  Every vector instruction
@@ -838,71 +781,10 @@ int launch_gram_wide(int n, const SrcT<TL, T1> &s, const GramPlan &p, double *wo
 // in flight, as wide ones.  Stages are loaded cooperatively two ahead (VEC
 // columns a load: 2, or 1 where a source has a single column) and read from one of two LDS buffers as in gram_lds_kernel.
 // Bound by memory up to about 64 columns, by the matrix cores above.
-struct GramTile {
-    int TMB, TNB;    // tiles of a block
-    int nbn;         // blocks along N
-    int GN, NG, KS;  // groups along N, groups, row shares
-    int MT, NT, VEC;
-    int W;           // waves the kernel is built for: 16, or 8 with twice the registers
-    size_t lds;
-};
-
-constexpr int GT_TM = 8, GT_TN = 10;
 
 // two columns, aligned as one
 typedef double pair64 __attribute__((ext_vector_type(2), aligned(8)));
 typedef float pair32 __attribute__((ext_vector_type(2), aligned(4)));
-
-// loads of a stage per lane
-__host__ __device__ constexpr int gt_loads(int W, int VEC)
-{
-    return W == 16 ? (VEC == 2 ? 3 : 5) : (VEC == 2 ? 5 : 9);
-}
-
-// the tile group and row shares of a block: the fewest MFMA slots per row on the
-// busiest SIMD (waves are dealt round-robin over 4), then the most waves; at
-// most 16 waves and 80 KiB of LDS (two workgroups a CU) while a single row share
-// allows it
-GramTile plan_tile(int TM, int TN, int VEC, int chunk)
-{
-    static const int shape[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 5}, {2, 2}, {2, 3}};
-    GramTile best{};
-    const int bm = (TM + GT_TM - 1) / GT_TM, bn = (TN + GT_TN - 1) / GT_TN;
-    best.TMB = (TM + bm - 1) / bm;
-    best.TNB = (TN + bn - 1) / bn;
-    best.nbn = (TN + best.TNB - 1) / best.TNB;
-    best.VEC = VEC;
-    double cost = 1e30;
-    const int cols = lds_row_stride(best.TMB * 16) + lds_row_stride(best.TNB * 16);
-    for (const auto &sh : shape) {
-        const int MT = sh[0], NT = sh[1];
-        const int GM = (best.TMB + MT - 1) / MT, GN = (best.TNB + NT - 1) / NT, NG = GM * GN;
-        // no more row shares than 16-row pieces in a chunk
-        for (int KS = 1; NG * KS <= 16 && (KS == 1 || 16 * KS <= chunk); KS++) {
-            const int W = NG * KS <= 8 ? 8 : 16;
-            // loads of a row: L, R1 and R2 may each end with an odd column
-            if (16 * (best.TMB + best.TNB) / VEC + VEC - 1 > 4 * gt_loads(W, VEC) * NG)
-                continue;
-            const size_t stage = 2 * (size_t)(16 * KS * cols + 32) * sizeof(double);
-            const size_t red = (size_t)(KS - 1) * NG * MT * NT * 256 * sizeof(double);
-            const size_t lds = stage > red ? stage : red;
-            if (lds > (KS == 1 ? 160 : 80) * 1024)
-                break;
-            const double c = (double)((NG * KS + 3) / 4) * MT * NT / KS - 1e-3 * NG * KS;
-            if (c < cost) {
-                cost = c;
-                best.GN = GN;
-                best.NG = NG;
-                best.KS = KS;
-                best.MT = MT;
-                best.NT = NT;
-                best.W = W;
-                best.lds = lds;
-            }
-        }
-    }
-    return best;
-}
 
 template <typename TL, typename T1, int MT, int NT, int VEC, int W, bool ONE>
 __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s,
@@ -918,8 +800,10 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
     const int krt = s.kr1 + s.kr2;
     const int kl = s.kl - ca < g.TMB * 16 ? s.kl - ca : g.TMB * 16;
     const int kr = krt - cb < g.TNB * 16 ? krt - cb : g.TNB * 16;
-    const int LDP = lds_row_stride(kl), RDP = lds_row_stride(kr);
-    const int SR = 16 * g.KS;
+    // R1's columns of the block, then R2's
+    const int k1 = s.kr1 - cb < 0 ? 0 : s.kr1 - cb < kr ? s.kr1 - cb : kr, k2 = kr - k1;
+    const GtStage<VEC, one> sv(16 * g.KS, kl, k1, k2);
+    const int SR = sv.SR, LDP = sv.LDP, RDP = sv.RDP;
     // a tile past the last column reads into the next row (past the last row: 32
     // doubles more); it feeds outputs of the padding only
     const int BUF = SR * (LDP + RDP) + 32;
@@ -927,41 +811,23 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
     const int wave = t >> 6, lane = t & 63, lr = lane >> 4, lc = lane & 15;
     const int gi = wave % g.NG, ks = wave / g.NG;
     const int tm = gi / g.GN * MT, tn = gi % g.GN * NT;
-    const int r0 = blockIdx.x * chunk, r1 = r0 + chunk < n ? r0 + chunk : n;
+    const int r0 = blockIdx.x * chunk, r1 = n - r0 < chunk ? n : r0 + chunk;
     const int nstage = (r1 - r0 + SR - 1) / SR;
 
-    // this lane's vectors of a stage: source address, and LDS offset, row and
-    // source (0 L, 1 R1, 2 R2) packed
+    // this lane's vectors of a stage: source address, and LDS offset, source and row packed
     const char *src[VPT];
     unsigned info[VPT];
-    // R1's columns of the block, then R2's; a last odd column's pair starts one
-    // column early, inside the row
-    const int k1 = s.kr1 - cb < 0 ? 0 : s.kr1 - cb < kr ? s.kr1 - cb : kr, k2 = kr - k1;
-    const int wl = (kl + VEC - 1) / VEC, w1 = (k1 + VEC - 1) / VEC;
-    const int wr = w1 + (one ? 0 : (k2 + VEC - 1) / VEC);
-    auto start = [](int q, int k) { return VEC * q + VEC <= k || VEC == 1 ? VEC * q : k - VEC; };
-    // v / w for v < 2^14, w <= 256: the error of the product is far below 0.5 / w
-    const float il = 1.0f / wl, ir = 1.0f / wr;
 #pragma unroll
     for (int u = 0; u < VPT; u++) {
-        int v = t + nth * u;
-        info[u] = ~0u;
+        int c;
+        info[u] = sv.vector(t + nth * u, c);
+        const long row = r0 + gt_row(info[u]);
         src[u] = reinterpret_cast<const char *>(s.L);
-        if (v < SR * wl) {
-            const int row = (int)((v + 0.5f) * il), c = start(v - row * wl, kl);
-            src[u] = reinterpret_cast<const char *>(s.L + (long)(r0 + row) * s.ldl + ca + c);
-            info[u] = (unsigned)(row * LDP + c) << 12 | row;
-        } else if ((v -= SR * wl) < SR * wr) {
-            const int row = (int)((v + 0.5f) * ir), q = v - row * wr;
-            const int c = q < w1 ? start(q, k1) : k1 + start(q - w1, k2);
-            if (q < w1)
-                src[u] = reinterpret_cast<const char *>(s.R1 + (long)(r0 + row) * s.ld1 +
-                                                        r1_col(s, cb + c));
-            else
-                src[u] = reinterpret_cast<const char *>(s.R2 + (long)(r0 + row) * s.ld2 + cb + c -
-                                                        s.kr1);
-            info[u] = (unsigned)(SR * LDP + row * RDP + c) << 12 | (q < w1 ? 1u : 2u) << 10 | row;
-        }
+        if (info[u] != ~0u)
+            src[u] = gt_kind(info[u]) == 0 ? reinterpret_cast<const char *>(s.L + row * s.ldl + ca + c)
+                     : gt_kind(info[u]) == 1
+                         ? reinterpret_cast<const char *>(s.R1 + row * s.ld1 + r1_col(s, cb + c))
+                         : reinterpret_cast<const char *>(s.R2 + row * s.ld2 + cb + c - s.kr1);
     }
     const long incl = (long)SR * s.ldl * sizeof(TL), inc1 = (long)SR * s.ld1 * sizeof(T1),
                inc2 = (long)SR * s.ld2 * sizeof(double);
@@ -970,16 +836,16 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
     double stg1[LDG];
     const double *src1 = s.R2 + (long)(r0 + t) * s.ld2;
     auto gload = [&](int slot, int st) {
-        const int left = st < nstage ? r1 - r0 - st * SR : 0;
+        const int left = gt_stage_rows(r1 - r0, SR, st);
         if constexpr (one) {
-            stg1[slot] = t < SR && t < left && k2 > 0 ? *src1 : 0.0;
+            stg1[slot] = t < left && k2 > 0 ? *src1 : 0.0;
             src1 += SR * s.ld2;
         }
 #pragma unroll
         for (int u = 0; u < VPT; u++) {
-            const int row = info[u] & 1023, kind = info[u] >> 10 & 3;
+            const int kind = gt_kind(info[u]);
             V w{};
-            if (row < left) {
+            if (gt_row(info[u]) < left) {
                 if (sizeof(T1) == 4 && kind == 1) {
                     const V4 f = *reinterpret_cast<const V4 *>(src[u]);
                     __builtin_memcpy(&w, &f, sizeof(f));
@@ -1002,7 +868,7 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
             if (info[u] == ~0u)
                 continue;
             V w = stg[slot][u];
-            if (sizeof(T1) == 4 && (info[u] >> 10 & 3) == 1) {
+            if (sizeof(T1) == 4 && gt_kind(info[u]) == 1) {
                 V4 f;
                 __builtin_memcpy(&f, &w, sizeof(f));
                 if constexpr (VEC == 2)
@@ -1063,7 +929,7 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
         V *dst[VPT];
 #pragma unroll
         for (int u = 0; u < VPT; u++) {
-            const int kind = info[u] >> 10 & 3;
+            const int kind = gt_kind(info[u]);
             inc[u] = info[u] == ~0u ? 0 : kind == 0 ? incl : kind == 1 ? inc1 : inc2;
             dst[u] = reinterpret_cast<V *>(lds + (info[u] >> 12));
             if (info[u] == ~0u)
@@ -1154,24 +1020,10 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
 template <typename TL, typename T1, int VEC>
 int launch_gram_tile(int n, const SrcT<TL, T1> &s, GramPlan &p, double *work, hipStream_t st)
 {
-    // from 8192 rows on at least 128 rows a chunk where a block's few tiles leave
-    // waves for more row shares: the same waves on half the partials (4 + 4 columns
-    // against 4, 20,000 rows: 14.0 -> 11.3 us; 100 columns: 28 -> 31 us, not taken)
-    if (n >= 8192 && p.chunk < 128 && p.TM * p.TN <= 24) {
-        p.chunk = 128;
-        p.gx = (n + 127) / 128;
-    }
+    tile_chunks(n, p);
     const GramTile g = plan_tile(p.TM, p.TN, VEC, p.chunk);
-    if (VEC == 2) {
-        // every source has two columns in every block it reaches, R2 one column in
-        // all; a block that holds a single one of a wider source cannot pair it
-        auto lone = [](int w, int k) { return k > 0 && k % w == 1; };
-        const int w = g.TNB * 16, e1 = s.kr1 % w;   // columns of R1 before R2 in their block
-        const int first2 = s.kr2 < w - e1 ? s.kr2 : w - e1;
-        const bool r2 = s.kr2 > 1 && (first2 == 1 || lone(w, s.kr2 - first2));
-        if (n < 2 || lone(g.TMB * 16, s.kl) || lone(w, s.kr1) || r2)
-            return (int)hipErrorInvalidValue;
-    }
+    if (VEC == 2 && !tile_pairs(n, s.kl, s.kr1, s.kr2, g))
+        return (int)hipErrorInvalidValue;
     const int kl_pad = p.TM * 16, kr_pad = p.TN * 16;
     const dim3 grid(p.gx, (p.TM + g.TMB - 1) / g.TMB * g.nbn), block(64 * g.NG * g.KS);
 #define CACG_GT(M, N, WV, ONE)                                                                    \

@@ -323,3 +323,19 @@ def test_q_update_without_s_exact_on_integers(gpu_lib, n, sm):
 @pytest.mark.parametrize("which,tm,tn", [(0, 1, 2), (1, 2, 1), (1, 1, 4), (2, 1, 1), (1, 9, 9), (0, 0, 0)])
 def test_batched_gram_class_refuses_what_is_no_class(gpu_lib, which, tm, tn):
     assert gpu_lib.lib().cacg_kb_gram_class(None, None, 1, which, 0, tm, tn, None) != 0
+
+
+@pytest.mark.parametrize("n,kl,kr1,kr2,ld2", [(130, 6, 6, 2, 9), (600011, 4, 4, 2, 16),
+                                              (600011, 2, 2, 1, 12), (530001, 3, 5, 3, 8)])
+def test_gram_fast_strided_second_block_exact_on_integers(gpu_lib, n, kl, kr1, kr2, ld2):
+    """R2 as columns of a wider block, with chunks of few rows and of more than 1023."""
+    lib, D, rng = gpu_lib.lib(), gpu_lib.DeviceBuffer.from_array, np.random.default_rng(n + kl)
+    L, R1, R2 = (rng.integers(-8, 9, size=(n, k)).astype(np.float64) for k in (kl, kr1, ld2))
+    dL, d1, d2 = D(L), D(R1), D(R2)
+    g1, g2 = gpu_lib.DeviceBuffer(8 * kl * kr1), gpu_lib.DeviceBuffer(8 * kl * kr2)
+    ws = gpu_lib.DeviceBuffer(8 * lib.cacg_gram_workspace(kl, kr1 + kr2))
+    print(f"gram n={n} {kl} x ({kr1} + {kr2} of {ld2})", flush=True)
+    assert lib.cacg_k_gram_fast(n, dL.ptr, kl, kl, d1.ptr, kr1, kr1, d2.ptr, ld2, kr2, g1.ptr, g2.ptr,
+                                ws.ptr, None) == 0
+    assert np.array_equal(g1.download((kl, kr1)), L.T @ R1)
+    assert np.array_equal(g2.download((kl, kr2)), L.T @ R2[:, :kr2])
