@@ -339,3 +339,11 @@ def test_gram_fast_strided_second_block_exact_on_integers(gpu_lib, n, kl, kr1, k
                                 ws.ptr, None) == 0
     assert np.array_equal(g1.download((kl, kr1)), L.T @ R1)
     assert np.array_equal(g2.download((kl, kr2)), L.T @ R2[:, :kr2])
+
+
+@pytest.mark.parametrize("n,kl,kr1,kr2", [(100003, 99, 99, 11), (150001, 61, 61, 7), (200003, 127, 127, 0),
+                                          (120001, 81, 81, 0)])
+def test_gram_many_stages_of_odd_widths_exact_on_integers(gpu_lib, n, kl, kr1, kr2):
+    """Chunks of 18 to 29 whole stages and a part of one, pairs that start a column early: 2 x 2,
+    1 x 4 and 1 x 3 tiles in 16 waves, 1 x 5 in 8."""
+    test_gram_fast_edges_exact_on_integers(gpu_lib, n, kl, kr1, kr2)
