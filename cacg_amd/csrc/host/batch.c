@@ -35,6 +35,7 @@
 #include "cacg.h"
 #include "cacg_batch.h"
 #include "cacg_kernels.h"
+#include "spmm_cand.h"
 
 enum { RQ_QUEUED = 0, RQ_ACTIVE = 1, RQ_DONE = 2 };
 
@@ -77,22 +78,17 @@ typedef struct {
     int s, f32, max_sm, pad_;
 } wlists;
 
-/* Online SpMM schedule tuning of a solo system: its first NCAND iterations each
+/* Online SpMM schedule tuning of a solo system: its first SPMM_CANDS iterations each
  * run their basis steps and A Q under one candidate schedule (tile order and
  * grid, cacg_spmm_sched), timed by events on the system's stream, and the
  * fastest of each shape is kept for the rest of the solve.  The timed launches
  * are the solve's own (a schedule changes no bit), so tuning costs no extra
  * work; the candidates are those of the single-system solver's offline tuner. */
-static const cacg_spmm_sched CAND[] = {
-    {0, 0, 0},       {4096, 0, 0},    {8192, 0, 0},    {0, 2048, 0},    {4096, 2048, 0},
-    {8192, 4096, 0}, {768, 2048, 0},  {1024, 1024, 0}, {16384, 512, 4}, {32768, 512, 4}};
-#define NCAND ((int)(sizeof(CAND) / sizeof(CAND[0])))
-
 typedef struct {
     hipEvent_t ev[4];          /* basis steps start / end, A Q start / end */
     int have_ev;
     int timing;                /* the candidate timed this round, -1: none */
-    int next;                  /* the next candidate; NCAND: done */
+    int next;                  /* the next candidate; SPMM_CANDS: done */
     float best_b, best_a;
     cacg_spmm_sched sb, sa;    /* in use: basis steps, A Q */
 } stune;
@@ -656,9 +652,9 @@ static int admit(cacg_batch *b, breq *r, int slot)
     b->slot[slot] = r;
     stune *t = &b->tune[slot];
     t->timing = -1;
-    t->next = b->o.tune ? 0 : NCAND;
+    t->next = b->o.tune ? 0 : SPMM_CANDS;
     t->best_b = t->best_a = -1.f;
-    t->sb = t->sa = CAND[0];
+    t->sb = t->sa = (cacg_spmm_sched){0, 0, 0};
     return 1;
 }
 
@@ -981,7 +977,7 @@ static int step_locked(cacg_batch *b, cacg_batch_stats *stats)
             if (r->joined && !r->verify) {
                 stune *t = &b->tune[i];
                 t->timing = -1;
-                if (t->next < NCAND && !t->have_ev) {
+                if (t->next < SPMM_CANDS && !t->have_ev) {
                     int e = 0;
                     while (e < 4 && hipEventCreate(&t->ev[e]) == hipSuccess)
                         e++;
@@ -989,16 +985,19 @@ static int step_locked(cacg_batch *b, cacg_batch_stats *stats)
                         (void)hipGetLastError();
                         while (e > 0)
                             hipEventDestroy(t->ev[--e]);
-                        t->next = NCAND;
+                        t->next = SPMM_CANDS;
                     } else {
                         t->have_ev = 1;
                     }
                 }
-                if (t->next < NCAND)
+                if (t->next < SPMM_CANDS)
                     t->timing = t->next;
-                const cacg_spmm_sched *sb = t->timing >= 0 ? &CAND[t->timing] : &t->sb;
-                const cacg_spmm_sched *sa = t->timing >= 0 ? &CAND[t->timing] : &t->sa;
-                rc = solo_iteration(&b->h_sys[i], r->fresh, s, f32, &rw->xpend, sb, sa,
+                cacg_spmm_sched sb = t->sb, sa = t->sa;
+                if (t->timing >= 0) {
+                    sb = spmm_cand(b->h_sys[i].m, t->timing);
+                    sa = spmm_cand(b->h_sys[i].sm, t->timing);
+                }
+                rc = solo_iteration(&b->h_sys[i], r->fresh, s, f32, &rw->xpend, &sb, &sa,
                                     t->timing >= 0 ? t->ev : NULL, ss);
             } else { /* admitted, or verifying: X complete, then the true residual */
                 rc = rw->xpend ? solo_flush_x(&b->h_sys[i], ss) : CACG_OK;
@@ -1271,11 +1270,11 @@ static int step_locked(cacg_batch *b, cacg_batch_stats *stats)
             (void)hipGetLastError();   /* an untimed candidate is skipped, not an error */
         if (eb == hipSuccess && (t->best_b < 0.f || tb < t->best_b)) {
             t->best_b = tb;
-            t->sb = CAND[t->timing];
+            t->sb = spmm_cand(b->h_sys[i].m, t->timing);
         }
         if (ea == hipSuccess && (t->best_a < 0.f || ta < t->best_a)) {
             t->best_a = ta;
-            t->sa = CAND[t->timing];
+            t->sa = spmm_cand(b->h_sys[i].sm, t->timing);
         }
         t->next = t->timing + 1;
         t->timing = -1;

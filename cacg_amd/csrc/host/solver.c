@@ -43,6 +43,7 @@
 
 #include "cacg_kernels.h"
 #include "cacg.h"
+#include "spmm_cand.h"
 
 #define NPHASE 12
 #define MAXEV 20
@@ -696,10 +697,6 @@ static unsigned long long pattern_key(long n, const long *row_start, const long 
  * them).  A schedule changes no result, so neither does the choice. */
 static int tune_spmm(cacg_solver *sv, int blk)
 {
-    static const cacg_spmm_sched cand[] = {
-        {0, 0, 0},       {4096, 0, 0},    {8192, 0, 0},   {0, 2048, 0},    {4096, 2048, 0},
-        {8192, 4096, 0}, {768, 2048, 0},  {1024, 1024, 0}, {16384, 512, 4}, {32768, 512, 4}};
-    const int nc = (int)(sizeof(cand) / sizeof(cand[0]));
     sv->tuned = 1;
     if (sv->n < TUNE_MIN_ROWS)
         return 0;
@@ -730,19 +727,20 @@ static int tune_spmm(cacg_solver *sv, int blk)
     const void *bp2 = f32 ? (const void *)(sv->f_S + (sm > m ? m : 0)) : (const void *)sv->d_AQ;
     void *by = f32 ? (void *)(sv->f_S + (sm > 2 * m ? 2 * m : 0)) : (void *)sv->d_Q;
     float best_b = -1.f, best_a = -1.f;
-    for (int c = 0; c < nc; c++) {
+    for (int c = 0; c < SPMM_CANDS; c++) {
+        const cacg_spmm_sched cb = spmm_cand(m, c), ca = spmm_cand(sm, c);
         /* the basis steps' leading dimension: m for a block-major basis */
         const float tb = time_spmm(sv, f32, m, blk ? m : sm, bx, by, bx, bp2, CACG_EPI_CHEB,
-                                   &cand[c], 2);
+                                   &cb, 2);
         if (tb >= 0.f && (best_b < 0.f || tb < best_b)) {
             best_b = tb;
-            sv->sch_basis = cand[c];
+            sv->sch_basis = cb;
         }
         const float ta = time_spmm(sv, 0, sm, sm, sv->d_Q, sv->d_AQ, NULL, NULL, CACG_EPI_NONE,
-                                   &cand[c], 2);
+                                   &ca, 2);
         if (ta >= 0.f && (best_a < 0.f || ta < best_a)) {
             best_a = ta;
-            sv->sch_aq = cand[c];
+            sv->sch_aq = ca;
         }
     }
     if (best_b < 0.f || best_a < 0.f)
