@@ -123,6 +123,7 @@ def lib() -> ctypes.CDLL:
                               c_double, c_double, _vp], c_int),
         "cacg_k_cvt_f64_f32": ([c_long, _vp, _vp, _vp], c_int),
         "cacg_csr_long_min": ([c_long, _vp], c_int),
+        "cacg_csr_even_bound": ([c_long, _vp], c_int),
         "cacg_csr_long_rows": ([c_long, _vp, c_int, _vp], c_long),
         "cacg_k_qupdate_s32": ([c_int, c_int, _vp, _vp, _vp, _vp], c_int),
         "cacg_k_cvt_f32_f64": ([c_long, _vp, _vp, _vp], c_int),
@@ -234,7 +235,11 @@ class DeviceCSR:
         self.val = DeviceBuffer.from_array(np.asarray(A.val, dtype=np.float64))
         lm, ids = long_rows(A, long_min)
         self.n_long = len(ids)
-        self.long_min = lm   # with no long rows: looked for and not there
+        if long_min is None and self.n_long == 0:
+            # no row is split; a bound on even rows is for the launch order
+            rp = np.ascontiguousarray(A.rowptr, dtype=np.int64)
+            lm = lib().cacg_csr_even_bound(A.n, rp.ctypes.data)
+        self.long_min = lm
         self.lrows = DeviceBuffer.from_array(ids) if self.n_long else None
         lp = self.lrows.ptr if self.lrows else None
         self.s = DCsr(A.n, self.rowptr.ptr, self.col.ptr, self.val.ptr, lp, self.n_long,

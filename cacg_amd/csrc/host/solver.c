@@ -503,7 +503,8 @@ int cacg_solver_create(cacg_solver **out, long n, const long *row_start, const l
         /* rows far longer than the mean go to the row-split SpMM */
         const int lmin = cacg_csr_long_min(n, row_start);
         const long nl = cacg_csr_long_rows(n, row_start, lmin, NULL);
-        sv->A.long_min = lmin;   /* without long rows: looked for and not there */
+        /* without long rows: what none of even rows reaches (the launch order) */
+        sv->A.long_min = nl > 0 ? lmin : cacg_csr_even_bound(n, row_start);
         if (nl > 0) {
             int *ids = (int *)malloc(sizeof(int) * (size_t)nl);
             if (!ids || dalloc(sv, (void **)&sv->d_long_rows, nl * (long)sizeof(int)) != CACG_OK) {
@@ -550,6 +551,16 @@ int cacg_csr_long_min(long n, const long *row_start)
     const long mean = (nnz + n - 1) / n;
     const long t = 16 * mean > 256 ? 16 * mean : 256;
     return t < 0x7fffffffL ? (int)t : 0x7fffffff;
+}
+
+int cacg_csr_even_bound(long n, const long *row_start)
+{
+    long longest = 0;
+    for (long i = 0; i < n; i++)
+        if (row_start[i + 1] - row_start[i] > longest)
+            longest = row_start[i + 1] - row_start[i];
+    const int even = n > 0 && 4.0 * n * (longest - 1) <= 5.0 * (row_start[n] - row_start[0]);
+    return even && longest < 0x7fffffffL ? (int)longest + 1 : 0;
 }
 
 long cacg_csr_long_rows(long n, const long *row_start, int long_min, int *out)

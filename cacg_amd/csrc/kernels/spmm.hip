@@ -548,23 +548,35 @@ __global__ __launch_bounds__(LR_T) void spmm_long_kernel(
 // and, unless the schedule names a grid, 32 and 16 workgroups per CU in bands.
 // A grid of more workgroups than run at once sweeps a band with gaps (the first
 // ones walk it to its end before the rest start), so the rows a front gathers
-// lie further apart.  For blocks that outgrow the 256 MB behind the L2s the
-// default is therefore as many workgroups as stay resident, in chunks: 3 per CU
-// and 2048 rows up to 16 columns (from 16 MB, where the order of the front starts
-// to count), 4 per CU and 1024 rows above 64 columns.  In between neither order
-// wins everywhere, and rows of very different lengths need the spare workgroups
-// to balance (1024^2 grid with 64 hub rows left to the lane groups: 5.2 -> 9.8 ms
-// at 16 columns), so it takes a matrix whose row lengths were looked at (long_min)
-// and held no long row.  128^3 Laplacian: k = 16 242 -> 224 us, k =
-// 128 1517 -> 1336 us (a copy of the same bytes takes 200 and 900); 96^3: 107 ->
-// 101, 673 -> 583; 1024^2: 109 -> 103, 667 -> 598; 64^3: 34 -> 33, 166 -> 147.
-inline cacg_spmm_sched default_sched(long n, int k, int lpr, int vw, bool even)
+// lie further apart.  For FP64 blocks that outgrow the caches the default is
+// therefore as many workgroups as stay resident, in chunks: 3 per CU and 2048
+// rows up to 16 columns, 4 per CU and 1024 rows above 64.  Fewer waves in flight
+// hide less latency, so this holds where a wave's rows are equally long and the
+// gather is what counts: for a matrix of even rows (`row`: the longest, 0 where
+// it is not known), and by epilogue and size.  us, bands -> chunks:
+//   Chebyshev step, 60 MB on: 128^3 Laplacian k = 16 308 -> 257, k = 8 168 -> 150; 1024^2 k =
+//   16 114 -> 110, k = 12 94 -> 95; below, 64^3 k = 8 22 -> 23.  First step, more than 4
+//   columns: 128^3 k = 16 324 -> 263, k = 8 174 -> 166, k = 4 101 -> 110.
+//   A x alone: 128^3 k = 16 198 -> 172, 160^3 k = 12 386 -> 337, but 1500^2 k = 16 176 -> 184 and
+//   96^3 k = 12 67 -> 72.
+//   Above 64 columns: 128^3 k = 128 1515 -> 1335, k = 96 1252 -> 1152, k = 72 977 -> 998; 160^3 k =
+//   72 2290 -> 2000; 64^3 k = 128 167 -> 148; 1024^2 k = 72 416 -> 460.
+//   27 points a row, 100^3: k = 4 326 -> 302, k = 16 444 -> 336, k = 72 1644 -> 1541.
+// Rows of 1 to 250 nonzeros: k = 16 537 -> 1081, k = 128 1863 -> 2193.  FP32 blocks: 1024^2
+// k = 16 55 -> 77, 128^3 123 -> 158.
+inline cacg_spmm_sched default_sched(long n, int k, int lpr, int vw, int epi, int row)
 {
-    const long bytes = n * (long)k * 8;
-    if (even && vw == 4 && lpr <= 4 && bytes >= 16L << 20)
-        return {768, 2048, 0};
-    if (even && vw == 4 && k > 64 && bytes >= 256L << 20)
+    const long mb = n * (long)k * 8 >> 20;
+    if (vw != 4 || row == 0)
+        return {0, 0, 0};
+    const bool dense = row > 16;
+    if (lpr <= 4) {
+        const bool cheb = epi == CACG_EPI_CHEB || (epi == CACG_EPI_CHEB1 && k > 4);
+        if (dense ? mb >= 30 : cheb ? mb >= 60 : epi != CACG_EPI_CHEB1 && k > 8 && row > 5 && mb >= 200)
+            return {768, 2048, 0};
+    } else if (k > 64 && mb >= (dense || k >= 96 ? 256 : 1280)) {
         return {1024, 1024, 0};
+    }
     return {0, 0, 0};
 }
 
@@ -576,7 +588,11 @@ int launch_spmm(int n, const int *rowptr, const int *col, const TV *val, int k, 
 {
     constexpr int RPG = LPR >= 16 ? 2 : 1;
     constexpr int TR = (256 / LPR) * RPG;
-    const cacg_spmm_sched def = default_sched(n, k, LPR, VW, n_long == 0 && long_min > 0);
+    // a row length that no row reaches, within what was measured: the rows are even
+    // (cacg_csr_even_bound gives none for others)
+    const bool even = sizeof(TV) == 8 && sizeof(TX) == 8 && sizeof(TY) == 8 && n_long == 0 &&
+                      long_min > 1 && long_min <= 32;
+    const cacg_spmm_sched def = default_sched(n, k, LPR, VW, epi, even ? long_min - 1 : 0);
     if (!sc || (sc->grid == 0 && sc->chunk_rows == 0))
         sc = &def;
     const int gmax = sc->grid > 0 ? sc->grid : (LPR >= 16 ? 4096 : 8192);

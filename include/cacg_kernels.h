@@ -21,9 +21,10 @@ extern "C" {
  * Long rows: with long_min > 0, the SpMMs leave every row with at least
  * long_min nonzeros to a row-split kernel (one workgroup per row), and
  * long_rows (device, n_long ids) must list exactly those rows
- * (cacg_csr_long_rows builds it).  long_min > 0 with no such row also says that
- * the row lengths are even (the default launch order goes by it).  long_min = 0
- * (zero-initialised): every row vector-per-row. */
+ * (cacg_csr_long_rows builds it).  A long_min of at most 32 with n_long = 0
+ * says that no row is as long, which the default launch order goes by: set it to
+ * cacg_csr_even_bound for rows of about one length.  long_min = 0
+ * (zero-initialised): every row vector-per-row, nothing known. */
 typedef struct {
     int n;
     const int *rowptr;
@@ -49,6 +50,9 @@ typedef struct {
  * kernel: max(256, 16 x the mean row length), so rows far above the mean.
  * Host-side, from the host row pointers (n + 1 of them, int64). */
 int cacg_csr_long_min(long n, const long *row_start);
+/* The longest row + 1 where no row is longer than 5/4 of the mean + 1 (host-side),
+ * else 0. */
+int cacg_csr_even_bound(long n, const long *row_start);
 /* The rows with at least long_min nonzeros, ascending, into out (host; may be
  * NULL to count).  Returns their number. */
 long cacg_csr_long_rows(long n, const long *row_start, int long_min, int *out);
