@@ -52,23 +52,79 @@ __device__ __forceinline__ void load_row(const T *p, double *out)
     }
 }
 
-// the first `have` of K consecutive values of a row, zeros after them; VEC 2:
-// 16-byte loads (p 16-byte aligned, `have` even)
-template <typename T, int K, int VEC>
-__device__ __forceinline__ void load_row_part(const T *p, int have, double *out)
+// two doubles, aligned as one
+typedef double pair64 __attribute__((ext_vector_type(2), aligned(8)));
+
+// the first `have` of K consecutive values of a row, zeros after them, in loads of
+//   ROW_PAIRS  two (p 16-byte aligned, `have` even)
+//   ROW_ONES   one
+//   ROW_MIXED  two wherever p lies, and a last odd one by itself: against ROW_ONES the X / R
+//              update of 127 + 1 columns 2,097,152 rows 2014 -> 1500 us, but the Q update of
+//              127 columns 1789 -> 2234
+// Vector instructions beside the loads are paid in matrix-core time: pairs chosen by a
+// select instead of a branch took 1.1 to 1.75 times as long.
+enum { ROW_PAIRS, ROW_ONES, ROW_MIXED };
+template <int K, int HOW>
+__device__ __forceinline__ void load_row_part(const double *p, int have, double *out)
 {
 #pragma unroll
-    for (int u = 0; u < K; u += VEC) {
-        if constexpr (VEC == 2) {
+    for (int u = 0; u < K; u += HOW == ROW_ONES ? 1 : 2) {
+        if constexpr (HOW == ROW_ONES) {
+            out[u] = u < have ? p[u] : 0.0;
+        } else if constexpr (HOW == ROW_PAIRS) {
             double2 w = {0.0, 0.0};
             if (u < have)
                 w = *reinterpret_cast<const double2 *>(p + u);
             out[u] = w.x;
             out[u + 1] = w.y;
         } else {
-            out[u] = u < have ? (double)p[u] : 0.0;
+            pair64 w = {0.0, 0.0};
+            if (u + 1 < have)
+                w = *reinterpret_cast<const pair64 *>(p + u);
+            else if (u < have)
+                w.x = p[u];
+            out[u] = w.x;
+            out[u + 1] = w.y;
         }
     }
+}
+
+// a rows x cols block (contiguous) into LDS, zero-padded to RP x CP with row stride LD,
+// by 256 lanes.  32 loads of a lane in flight, and no branch around any: a small
+// launch's time is otherwise this copy's, one memory latency per element of a lane
+// (20,000 rows, 100 + 20 columns: X / R update 47 -> 23 us, Q update 38 -> 28).
+template <int RP, int CP, int LD>
+__device__ __forceinline__ void stage_block(double *dst, const double *__restrict__ src, int rows,
+                                            int cols)
+{
+    constexpr int N = RP * CP / 256, B = N < 32 ? N : 32;
+#pragma unroll 1
+    for (int i0 = 0; i0 < N; i0 += B) {
+        double v[B];
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+            const int e = threadIdx.x + 256 * (i0 + u), k = e / CP, c = e % CP;
+            const bool in = k < rows && c < cols;
+            const double w = src[in ? k * cols + c : 0];
+            v[u] = in ? w : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+            const int e = threadIdx.x + 256 * (i0 + u);
+            if (N % B == 0 || i0 + u < N)
+                dst[e / CP * LD + e % CP] = v[u];
+        }
+    }
+}
+
+// the wave's share [tb, te) of the 16-row tiles: contiguous, and no two waves' differ by
+// more than one tile (with equal shares rounded up, some waves would have none: 140,000
+// rows of 15 columns, Q update 11.3 -> 9.3 us)
+__device__ __forceinline__ void tile_share(int ntiles, int wid, int nw, int &tb, int &te)
+{
+    const int q = ntiles / nw, r = ntiles % nw;
+    tb = wid * q + (wid < r ? wid : r);
+    te = tb + q + (wid < r ? 1 : 0);
 }
 
 // ---- reference order ----------------------------------------------------------
@@ -487,7 +543,9 @@ __global__ __launch_bounds__(512) void qupdate_mfma_kernel(int n, const TS *__re
     }
     __syncthreads();
     // wave-uniform, so that tile addresses are scalar
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int wave = sizeof(TS) == 8 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)
+                                     : (int)(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
     const int lg = lane >> 4, lc = lane & 15;
     const int nw = gridDim.x * 8;
     const int wid = xcd_remap(blockIdx.x, gridDim.x) * 8 + wave;
@@ -794,37 +852,33 @@ __global__ __launch_bounds__(256) void xrupdate_mfma_kernel(int n, int m, const 
     }
 }
 
-// Q = S - Qin beta for any width sm <= SM (SM the next multiple of 16): the
+// Q = S - Q beta for any width sm <= SM (SM the next multiple of 16): the
 // scheme of qupdate_mfma_kernel with beta zero-padded to SM x SM in LDS and the
-// operand rows zero-padded in registers.  Qin (row stride ldi) may be Q itself:
-// a wave has read its 16 rows before it writes them.  S may be null (zero).
-// VEC 2: sm and ldi even, Qin 16-byte aligned (16-byte loads).
+// operand rows zero-padded in registers.  A wave has read its 16 rows before it
+// writes them.  S may be null (zero).
 // Bound by memory: three blocks of n sm values, and at n = 250,047, sm = 60 the
 // MFMAs take a fifth of that time.  Before, these widths took the
 // reference-order kernel, whose every product reads LDS twice.
-template <typename TS, int SM, int VEC>
+template <typename TS, int SM, int HOW>
 __global__ __launch_bounds__(256) void qupdate_pad_kernel(int n, int sm, const TS *__restrict__ S,
-                                                          const double *Qin, long ldi, double *Q,
+                                                          double *Q,
                                                           const double *__restrict__ beta)
 {
     constexpr int KQ = SM / 4, NTL = SM / 16;
     extern __shared__ double bl[];
-    for (int e = threadIdx.x; e < SM * SM; e += 256) {
-        const int k = e / SM, c = e % SM;
-        bl[e] = k < sm && c < sm ? beta[k * sm + c] : 0.0;
-    }
+    stage_block<SM, SM, SM>(bl, beta, sm, sm);
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int lg = lane >> 4, lc = lane & 15;
     const int have = sm - lg * KQ;
     const int ntiles = (n + 15) / 16, nw = gridDim.x * 4;
     const int wid = xcd_remap(blockIdx.x, gridDim.x) * 4 + wave;
-    const int per = (ntiles + nw - 1) / nw;
-    const int tb = wid * per, te = tb + per < ntiles ? tb + per : ntiles;
+    int tb, te;
+    tile_share(ntiles, wid, nw, tb, te);
     double av[KQ];
     auto load = [&](int tile) {
         const long row = (long)tile * 16 + lc;
-        load_row_part<double, KQ, VEC>(Qin + (row < n ? row : n - 1) * ldi + lg * KQ, have, av);
+        load_row_part<KQ, HOW>(Q + (row < n ? row : n - 1) * sm + lg * KQ, have, av);
     };
     if (tb < te)
         load(tb);
@@ -859,7 +913,7 @@ __global__ __launch_bounds__(256) void qupdate_pad_kernel(int n, int sm, const T
 
 // X += Q alpha, R -= AQ alpha and the column norms of the new R for any width
 // sm <= SM, as xrupdate_mfma_kernel with zero-padded operands
-template <int SM, int NTM, int VEC>
+template <int SM, int NTM, int HOW>
 __global__ __launch_bounds__(256) void xrupdate_pad_kernel(int n, int sm, int m,
                                                            const double *__restrict__ Q,
                                                            const double *__restrict__ AQ,
@@ -873,10 +927,7 @@ __global__ __launch_bounds__(256) void xrupdate_pad_kernel(int n, int sm, int m,
     __shared__ double s_alf[SM][16 * NTM];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int lg = lane >> 4, lc = lane & 15;
-    for (int e = threadIdx.x; e < SM * 16 * NTM; e += 256) {
-        const int k = e / (16 * NTM), c = e % (16 * NTM);
-        s_alf[k][c] = k < sm && c < m ? alpha[(long)k * m + c] : 0.0;
-    }
+    stage_block<SM, 16 * NTM, 16 * NTM>(&s_alf[0][0], alpha, sm, m);
     __syncthreads();
     const int have = sm - lg * KQ;
     double nrm[NTM];
@@ -893,8 +944,8 @@ __global__ __launch_bounds__(256) void xrupdate_pad_kernel(int n, int sm, int m,
         const long i0 = (long)tile * 16;
         const long row = i0 + lc < n ? i0 + lc : (long)n - 1;
         double av[KQ], aq[KQ];
-        load_row_part<double, KQ, VEC>(Q + row * sm + lg * KQ, have, av);
-        load_row_part<double, KQ, VEC>(AQ + row * sm + lg * KQ, have, aq);
+        load_row_part<KQ, HOW>(Q + row * sm + lg * KQ, have, av);
+        load_row_part<KQ, HOW>(AQ + row * sm + lg * KQ, have, aq);
         double xo[NTM][4], ro[NTM][4];
 #pragma unroll
         for (int j = 0; j < NTM; j++) {
@@ -1049,17 +1100,14 @@ __global__ __launch_bounds__(256) void trimul_neg_kernel(int n, int sm, const do
 {
     constexpr int NP = SM / 8, NTL = SM / 16, LD = SM + 8;
     extern __shared__ double bl[];
-    for (int e = threadIdx.x; e < SM * SM; e += 256) {
-        const int k = e / SM, c = e % SM;
-        bl[k * LD + c] = k < sm && c < sm ? W[k * sm + c] : 0.0;
-    }
+    stage_block<SM, SM, LD>(bl, W, sm, sm);
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int lg = lane >> 4, lc = lane & 15;
     const int ntiles = (n + 15) / 16, nw = gridDim.x * 4;
     const int wid = xcd_remap(blockIdx.x, gridDim.x) * 4 + wave;
-    const int per = (ntiles + nw - 1) / nw;
-    const int tb = wid * per, te = tb + per < ntiles ? tb + per : ntiles;
+    int tb, te;
+    tile_share(ntiles, wid, nw, tb, te);
     double2 av[2][NP];
     auto load = [&](int tile, int s) {
         const long row = (long)tile * 16 + lc;
@@ -1104,16 +1152,20 @@ __global__ __launch_bounds__(256) void trimul_neg_kernel(int n, int sm, const do
     }
 }
 
+// workgroups of 4 waves: one tile a wave until `most`; rounded up to whole XCDs (down, a
+// wave of the last ones would take two tiles and half of them none)
+int pad_groups(int n, int most)
+{
+    const int G = (int)(((long)n + 63) / 64);
+    return G >= most ? most : G < 8 ? G : (G + 7) / 8 * 8;
+}
+
 template <int SM>
 int launch_trimul(int n, int sm, const double *A, long lda, double *Q, const double *W, hipStream_t st)
 {
     const size_t shm = (size_t)SM * (SM + 8) * sizeof(double);
     const int perCU = SM <= 64 ? 4 : SM <= 96 ? 2 : 1;   // resident workgroups
-    int G = (n + 63) / 64;
-    if (G > 256 * perCU)
-        G = 256 * perCU;
-    if (G >= 8)
-        G &= ~7;
+    const int G = pad_groups(n, 256 * perCU);
     if (sm % 2 == 0 && lda % 2 == 0 && (uintptr_t)A % 16 == 0) {
         cacg_allow_lds(trimul_neg_kernel<SM, 2>, shm);
         hipLaunchKernelGGL((trimul_neg_kernel<SM, 2>), dim3(G), dim3(256), shm, st, n, sm, A, lda, Q,
@@ -1130,43 +1182,36 @@ int launch_trimul(int n, int sm, const double *A, long lda, double *Q, const dou
 // workgroups of qupdate_pad_kernel: as many as are resident at once (4 waves each; LDS
 // holds beta once per workgroup)
 template <typename TS, int SM>
-int launch_qupdate_pad(int n, int sm, const TS *S, const double *Qin, long ldi, double *Q,
-                       const double *beta, hipStream_t st)
+int launch_qupdate_pad(int n, int sm, const TS *S, double *Q, const double *beta, hipStream_t st)
 {
     const size_t shm = (size_t)SM * SM * sizeof(double);
-    const int ntiles = (n + 15) / 16;
     const int perCU = SM <= 64 ? 4 : SM <= 96 ? 2 : 1;
-    int G = (ntiles + 3) / 4;
-    if (G > 256 * perCU)
-        G = 256 * perCU;
-    if (G >= 8)
-        G &= ~7;
-    if (sm % 2 == 0 && ldi % 2 == 0 && (uintptr_t)Qin % 16 == 0) {
-        cacg_allow_lds(qupdate_pad_kernel<TS, SM, 2>, shm);
-        hipLaunchKernelGGL((qupdate_pad_kernel<TS, SM, 2>), dim3(G), dim3(256), shm, st, n, sm, S,
-                           Qin, ldi, Q, beta);
+    const int G = pad_groups(n, 256 * perCU);
+    if (sm % 2 == 0 && (uintptr_t)Q % 16 == 0) {
+        cacg_allow_lds(qupdate_pad_kernel<TS, SM, ROW_PAIRS>, shm);
+        hipLaunchKernelGGL((qupdate_pad_kernel<TS, SM, ROW_PAIRS>), dim3(G), dim3(256), shm, st, n, sm,
+                           S, Q, beta);
     } else {
-        cacg_allow_lds(qupdate_pad_kernel<TS, SM, 1>, shm);
-        hipLaunchKernelGGL((qupdate_pad_kernel<TS, SM, 1>), dim3(G), dim3(256), shm, st, n, sm, S,
-                           Qin, ldi, Q, beta);
+        cacg_allow_lds(qupdate_pad_kernel<TS, SM, ROW_ONES>, shm);
+        hipLaunchKernelGGL((qupdate_pad_kernel<TS, SM, ROW_ONES>), dim3(G), dim3(256), shm, st, n, sm,
+                           S, Q, beta);
     }
     CACG_LAUNCH_CHECK();
     return 0;
 }
 
 template <typename TS>
-int qupdate_pad(int n, int sm, const TS *S, const double *Qin, long ldi, double *Q,
-                const double *beta, hipStream_t st)
+int qupdate_pad(int n, int sm, const TS *S, double *Q, const double *beta, hipStream_t st)
 {
     switch ((sm + 15) / 16) {
-    case 1: return launch_qupdate_pad<TS, 16>(n, sm, S, Qin, ldi, Q, beta, st);
-    case 2: return launch_qupdate_pad<TS, 32>(n, sm, S, Qin, ldi, Q, beta, st);
-    case 3: return launch_qupdate_pad<TS, 48>(n, sm, S, Qin, ldi, Q, beta, st);
-    case 4: return launch_qupdate_pad<TS, 64>(n, sm, S, Qin, ldi, Q, beta, st);
-    case 5: return launch_qupdate_pad<TS, 80>(n, sm, S, Qin, ldi, Q, beta, st);
-    case 6: return launch_qupdate_pad<TS, 96>(n, sm, S, Qin, ldi, Q, beta, st);
-    case 7: return launch_qupdate_pad<TS, 112>(n, sm, S, Qin, ldi, Q, beta, st);
-    case 8: return launch_qupdate_pad<TS, 128>(n, sm, S, Qin, ldi, Q, beta, st);
+    case 1: return launch_qupdate_pad<TS, 16>(n, sm, S, Q, beta, st);
+    case 2: return launch_qupdate_pad<TS, 32>(n, sm, S, Q, beta, st);
+    case 3: return launch_qupdate_pad<TS, 48>(n, sm, S, Q, beta, st);
+    case 4: return launch_qupdate_pad<TS, 64>(n, sm, S, Q, beta, st);
+    case 5: return launch_qupdate_pad<TS, 80>(n, sm, S, Q, beta, st);
+    case 6: return launch_qupdate_pad<TS, 96>(n, sm, S, Q, beta, st);
+    case 7: return launch_qupdate_pad<TS, 112>(n, sm, S, Q, beta, st);
+    case 8: return launch_qupdate_pad<TS, 128>(n, sm, S, Q, beta, st);
     default: return (int)hipErrorInvalidValue;
     }
 }
@@ -1176,14 +1221,15 @@ int launch_xrupdate_pad(int n, int sm, int m, const double *Q, const double *AQ,
                         const double *alpha, double *X, double *R, double *d_norm2, double *work,
                         hipStream_t st)
 {
+    const int G = pad_groups(n, XR_BLOCKS);   // the norm partials depend on n alone
     if (sm % 2 == 0 && ((uintptr_t)Q | (uintptr_t)AQ) % 16 == 0)
-        hipLaunchKernelGGL((xrupdate_pad_kernel<SM, NTM, 2>), dim3(XR_BLOCKS), dim3(256), 0, st, n,
-                           sm, m, Q, AQ, alpha, X, R, work);
+        hipLaunchKernelGGL((xrupdate_pad_kernel<SM, NTM, ROW_PAIRS>), dim3(G), dim3(256), 0, st, n, sm,
+                           m, Q, AQ, alpha, X, R, work);
     else
-        hipLaunchKernelGGL((xrupdate_pad_kernel<SM, NTM, 1>), dim3(XR_BLOCKS), dim3(256), 0, st, n,
-                           sm, m, Q, AQ, alpha, X, R, work);
+        hipLaunchKernelGGL((xrupdate_pad_kernel<SM, NTM, ROW_MIXED>), dim3(G), dim3(256), 0, st, n, sm,
+                           m, Q, AQ, alpha, X, R, work);
     CACG_LAUNCH_CHECK();
-    hipLaunchKernelGGL(colnorm2_final_kernel, dim3(m), dim3(256), 0, st, work, XR_BLOCKS, m,
+    hipLaunchKernelGGL(colnorm2_final_kernel, dim3(m), dim3(256), 0, st, work, G, m,
                        d_norm2);
     CACG_LAUNCH_CHECK();
     return 0;
@@ -1237,7 +1283,7 @@ int qupdate(int n, int sm, const TS *S, T *Q, const double *beta, int mode, hipS
         }
         // other widths up to 128: zero-padded to the next multiple of 16
         if (sm < 128 && !narrow_ref(n, sm))
-            return qupdate_pad<TS>(n, sm, S, Q, sm, Q, beta, st);
+            return qupdate_pad<TS>(n, sm, S, Q, beta, st);
     }
     // 512 lanes when sm is even, divides 512 and beta plus the tile fit in LDS
     if (sm % 2 == 0 && sm <= QR2_T && QR2_T % sm == 0 &&
