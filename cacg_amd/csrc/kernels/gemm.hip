@@ -1185,7 +1185,8 @@ template <typename TS, int SM>
 int launch_qupdate_pad(int n, int sm, const TS *S, double *Q, const double *beta, hipStream_t st)
 {
     const size_t shm = (size_t)SM * SM * sizeof(double);
-    const int perCU = SM <= 64 ? 4 : SM <= 96 ? 2 : 1;
+    // 8 at 16 columns, where a wave waits more than it works: 80,000 rows of 6 5.3 -> 4.3 us
+    const int perCU = SM == 16 ? 8 : SM <= 64 ? 4 : SM <= 96 ? 2 : 1;
     const int G = pad_groups(n, 256 * perCU);
     if (sm % 2 == 0 && (uintptr_t)Q % 16 == 0) {
         cacg_allow_lds(qupdate_pad_kernel<TS, SM, ROW_PAIRS>, shm);
@@ -1252,14 +1253,43 @@ extern "C" int cacg_k_colnorm2_ref(int n, int m, const double *R, long ldr, doub
 
 namespace {
 
-// widths of 4 and 8 over many rows stay on the reference-order kernels in the
-// fast order: an MFMA operand row would be 3/4 or 1/2 padding.  Q and X / R
-// updates at sm = 4 (8): 71 (136) us against 126 (177) at 2,097,152 rows, 21 (26)
-// against 24 (26) at 250,047, 16 (18) against 13 (14) at 20,000.
-bool narrow_ref(int n, int sm)
+// Where the reference-order kernels are the faster ones in the fast order too.  Times in
+// us, padded MFMA kernel / this one.
+//
+// Q update.  Up to 4 columns and at 8 an MFMA operand is mostly padding: 1 column
+// 2,097,152 rows 45 / 7, 250,047 7.6 / 3.7; 4 columns 49 / 30 and 8.6 / 5.0; 8 columns 63 / 59
+// and 9.4 / 8.5 (5 columns 51 / 56, and 7.1 / 6.1 at 140,000; 9 columns 73 / 136).  With an FP32 S up to 6: 71 / 63
+// (7 columns 71.5 / 74.8).  Above 32 columns a launch of few rows is one wave's chain of MFMAs
+// per 16 rows, so while all its workgroups (of 256 / sm rows) run at once this one is
+// shorter: 100 columns 1000 rows 14.3 / 10.7, 2000 rows 14.4 / 19.9; 72 columns 2000 rows
+// 8.4 / 7.8, 4000 rows 8.6 / 13.8; 120 columns 500 rows 15.6 / 12.8, 1000 rows 15.6 / 24.3.
+template <typename TS>
+bool qupdate_by_ref(int n, int sm)
 {
-    (void)n;
-    return sm <= 8 && sm % 4 == 0;
+    if (sm <= 4 || sm == 8 || (sm == 5 && n <= 1 << 18) || (sizeof(TS) == 4 && sm <= 6))
+        return true;
+    if (sm <= 32)
+        return false;
+    const int rb = 256 / sm, fit = 20480 / (sm * sm + rb * sm);   // rows, workgroups a CU by LDS
+    return ((long)n + rb - 1) / rb <= 256 * (fit < 3 ? fit : 3);
+}
+
+// X / R update, sm below 16.  One right-hand side, norms in the same launch: 4 + 1 columns
+// 2,097,152 rows 90 / 33, 20,000 7.7 / 7.5; 10 + 1 columns 1,048,576 rows 50 / 45, 2,097,152
+// 107 / 119.  Else a second pass forms the norms: up to 8 columns and 4 right-hand sides past
+// two tiles a wave, 6 + 2 columns at 196,608 rows 14.4 / 13.3 and 91 / 60 at 2,097,152, 4 + 4
+// columns 15.1 / 14.1 and 99 / 77, at 130,000 rows 12.0 / 12.1; 10 + 2 columns 1,048,576 rows 51 / 46; at 2,097,152
+// rows also 5 + 5 131 / 116, 8 + 8 202 / 188, 9 + 3 123 / 116, 12 + 4 149 / 140, 15 + 3 162 / 157, but
+// 6 + 6 137 / 145 and 15 + 5 180 / 195.
+bool xrupdate_by_ref(int n, int sm, int m)
+{
+    if (sm >= 16)
+        return false;
+    if (m == 1)
+        return sm <= 8 || n <= 1 << 20;
+    if (sm <= 8 ? m <= 4 : sm <= 10 && m == 2)
+        return n > 1 << 17;
+    return n >= 1 << 21 && (sm <= 5 || sm == 8 || (sm > 8 && m <= 4));
 }
 
 template <typename TS, typename T>
@@ -1282,7 +1312,7 @@ int qupdate(int n, int sm, const TS *S, T *Q, const double *beta, int mode, hipS
         default: break;
         }
         // other widths up to 128: zero-padded to the next multiple of 16
-        if (sm < 128 && !narrow_ref(n, sm))
+        if (sm < 128 && !qupdate_by_ref<TS>(n, sm))
             return qupdate_pad<TS>(n, sm, S, Q, beta, st);
     }
     // 512 lanes when sm is even, divides 512 and beta plus the tile fit in LDS
@@ -1376,7 +1406,7 @@ int xrupdate(int n, int sm, int m, const T *Q, const T *AQ, const double *alpha,
                        : launch_xrupdate_pad<SMV, 2>(n, sm, m, Q, AQ, alpha, X, R, d_norm2,       \
                                                      d_work, st);
         // other widths up to 128: zero-padded to the next multiple of 16
-        if (n > 0 && !narrow_ref(n, sm)) {
+        if (n > 0 && !xrupdate_by_ref(n, sm, m)) {
             switch ((sm + 15) / 16) {
                 CACG_XRP(16)
                 CACG_XRP(32)

@@ -43,3 +43,15 @@ def test_default_spmm_order_on_uneven_rows(gpu_lib, k):
     default, named = best_seconds(lambda: Y.download(1), lambda: run(None),
                                   lambda: run(ctypes.byref(bands)))
     assert default < 1.3 * named, (default, named)
+
+
+@pytest.mark.parametrize("sm", [1, 2, 3])
+def test_fast_order_q_update_of_few_columns(gpu_lib, sm):
+    """Against the reference order, whose kernel forms the same products one by one."""
+    n, B, lib = 1 << 20, gpu_lib.DeviceBuffer, gpu_lib.lib()
+    S, Q, beta = (B.from_array(np.ones(s)) for s in ((n, sm), (n, sm), (sm, sm)))
+    run = lambda mode: lib.cacg_k_qupdate(n, sm, S.ptr, Q.ptr, beta.ptr, mode, None)  # noqa: E731
+    print(f"q update sm={sm}", flush=True)
+    fast, ref = best_seconds(lambda: Q.download(1), lambda: run(gpu_lib.MODE["fast"]),
+                             lambda: run(gpu_lib.MODE["reference"]), launches=40)
+    assert fast < 1.5 * ref, (fast, ref)

@@ -347,3 +347,12 @@ def test_gram_many_stages_of_odd_widths_exact_on_integers(gpu_lib, n, kl, kr1, k
     """Chunks of 18 to 29 whole stages and a part of one, pairs that start a column early: 2 x 2,
     1 x 4 and 1 x 3 tiles in 16 waves, 1 x 5 in 8."""
     test_gram_fast_edges_exact_on_integers(gpu_lib, n, kl, kr1, kr2)
+
+
+@pytest.mark.parametrize("n,sm,m", [
+    (131072, 6, 2), (131073, 6, 2), (131073, 3, 3), (131073, 10, 2), (262144, 5, 5), (262145, 5, 5),
+    (1 << 20, 12, 1), ((1 << 20) + 1, 12, 1), (1 << 21, 9, 3), (1 << 21, 8, 8), (1024, 100, 20),
+    (1025, 100, 20), (2304, 72, 12), (2305, 72, 12), (512, 127, 1), (513, 127, 1)])
+def test_updates_at_the_lines_between_the_kernels_exact_on_integers(gpu_lib, n, sm, m):
+    """Row counts on both sides of the lines where another kernel takes over."""
+    test_padded_updates_exact_on_integers(gpu_lib, n, sm, m)
