@@ -802,7 +802,7 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
     const int kr = krt - cb < g.TNB * 16 ? krt - cb : g.TNB * 16;
     // R1's columns of the block, then R2's
     const int k1 = s.kr1 - cb < 0 ? 0 : s.kr1 - cb < kr ? s.kr1 - cb : kr, k2 = kr - k1;
-    const GtStage<VEC, one> sv(16 * g.KS, kl, k1, k2);
+    const GtStage<VEC, one, sizeof(T1) == 4> sv(16 * g.KS, kl, k1, k2);
     const int SR = sv.SR, LDP = sv.LDP, RDP = sv.RDP;
     // a tile past the last column reads into the next row (past the last row: 32
     // doubles more); it feeds outputs of the padding only
@@ -1021,7 +1021,7 @@ template <typename TL, typename T1, int VEC>
 int launch_gram_tile(int n, const SrcT<TL, T1> &s, GramPlan &p, double *work, hipStream_t st)
 {
     tile_chunks(n, p);
-    const GramTile g = plan_tile(p.TM, p.TN, VEC, p.chunk);
+    const GramTile g = plan_tile(p.TM, p.TN, VEC, p.chunk, sizeof(T1) == 4);
     if (VEC == 2 && !tile_pairs(n, s.kl, s.kr1, s.kr2, g))
         return (int)hipErrorInvalidValue;
     const int kl_pad = p.TM * 16, kr_pad = p.TN * 16;

@@ -105,8 +105,8 @@ inline void tile_chunks(int n, GramPlan &p)
 // the tile group and row shares of a block: the fewest MFMA slots per row on the
 // busiest SIMD (waves are dealt round-robin over 4), then the most waves; at
 // most 16 waves and 80 KiB of LDS (two workgroups a CU) while a single row share
-// allows it
-inline GramTile plan_tile(int TM, int TN, int VEC, int chunk)
+// allows it.  f32: R1 is FP32 and its vectors start at a wave's first lane.
+inline GramTile plan_tile(int TM, int TN, int VEC, int chunk, bool f32)
 {
     static const int shape[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 5}, {2, 2}, {2, 3}};
     GramTile best{};
@@ -124,7 +124,8 @@ inline GramTile plan_tile(int TM, int TN, int VEC, int chunk)
         for (int KS = 1; NG * KS <= 16 && (KS == 1 || 16 * KS <= chunk); KS++) {
             const int W = NG * KS <= 8 ? 8 : 16;
             // loads of a row: L, R1 and R2 may each end with an odd column
-            if (16 * (best.TMB + best.TNB) / VEC + VEC - 1 > 4 * gt_loads(W, VEC) * NG)
+            const int row = 16 * (best.TMB + best.TNB) / VEC + VEC - 1;
+            if (16 * KS * row + (f32 ? 63 : 0) > 64 * gt_loads(W, VEC) * NG * KS)
                 continue;
             const size_t stage = 2 * (size_t)(16 * KS * cols + 32) * sizeof(double);
             const size_t red = (size_t)(KS - 1) * NG * MT * NT * 256 * sizeof(double);
@@ -160,19 +161,25 @@ inline bool tile_pairs(int n, int kl, int kr1, int kr2, const GramTile &g)
 
 // The vectors of a stage of SR rows: VEC columns each, L's row by row, then those of
 // [R1 | R2] row by row, without R2's where it is a single column (ONE).  A last odd
-// column's pair starts one column early, inside the row.
-template <int VEC, bool ONE>
+// column's pair starts one column early, inside the row.  F32: R1 is FP32, and the
+// second part starts at a wave's first lane, so that no wave loads both types (it would
+// do so one after the other, and all waves wait for it at the stage's end: 2,097,152
+// rows of 60 columns 705 -> 517 us).
+template <int VEC, bool ONE, bool F32>
 struct GtStage {
     int SR, kl, k1, k2;   // columns of the block: L's, R1's, R2's
     int wl, w1, wr;       // vectors of a row of L, of R1, of [R1 | R2]
+    int second;           // first vector of [R1 | R2]
     int LDP, RDP;
     float il, ir;
     CACG_HD GtStage(int SR_, int kl_, int k1_, int k2_)
         : SR(SR_), kl(kl_), k1(k1_), k2(k2_), wl((kl_ + VEC - 1) / VEC), w1((k1_ + VEC - 1) / VEC),
-          wr((k1_ + VEC - 1) / VEC + (ONE ? 0 : (k2_ + VEC - 1) / VEC)), LDP(lds_row_stride(kl_)),
+          wr((k1_ + VEC - 1) / VEC + (ONE ? 0 : (k2_ + VEC - 1) / VEC)),
+          second(F32 ? (SR_ * wl + 63) / 64 * 64 : SR_ * wl), LDP(lds_row_stride(kl_)),
           RDP(lds_row_stride(k1_ + k2_)), il(1.0f / wl), ir(1.0f / wr)
     {
     }
+    CACG_HD int count() const { return second + SR * wr; }
     CACG_HD static int start(int q, int k) { return VEC * q + VEC <= k || VEC == 1 ? VEC * q : k - VEC; }
     // vector v's LDS offset, source (0 L, 1 R1, 2 R2) and row, packed; ~0u past the
     // last; col: its first column in L's or in [R1 | R2]'s part of the block.  The
@@ -186,7 +193,7 @@ struct GtStage {
             col = start(v - row * wl, kl);
             return (unsigned)(row * LDP + col) << 12 | row;
         }
-        if ((v -= SR * wl) < SR * wr) {
+        if ((v -= second) >= 0 && v < SR * wr) {
             const int row = (int)((v + 0.5f) * ir), q = v - row * wr;
             col = q < w1 ? start(q, k1) : k1 + start(q - w1, k2);
             return (unsigned)(SR * LDP + row * RDP + col) << 12 | (q < w1 ? 1u : 2u) << 10 | row;

@@ -356,3 +356,9 @@ def test_gram_many_stages_of_odd_widths_exact_on_integers(gpu_lib, n, kl, kr1, k
 def test_updates_at_the_lines_between_the_kernels_exact_on_integers(gpu_lib, n, sm, m):
     """Row counts on both sides of the lines where another kernel takes over."""
     test_padded_updates_exact_on_integers(gpu_lib, n, sm, m)
+
+
+@pytest.mark.parametrize("n,k", [(600011, 60), (70001, 47), (40003, 100), (5000, 128), (9001, 33)])
+def test_gram_f64f32_part_waves_exact_on_integers(gpu_lib, n, k):
+    """Rows of L that end inside a wave's lanes: R1's vectors start at the next wave."""
+    test_gram_f64f32_edges_exact_on_integers(gpu_lib, n, k)

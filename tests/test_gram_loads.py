@@ -22,15 +22,17 @@ static void fail(const char *what, int a, int b, int c)
 }
 
 // every lane, load and stage kind of one block over rows r0 .. r1 - 1
-template <int VEC, bool ONE>
+template <int VEC, bool ONE, bool F32>
 static void walk(const GramTile &g, int n, int kl_all, int kr1, int kr2, int r0, int r1, int by)
 {
     const int ca = by / g.nbn * g.TMB * 16, cb = by % g.nbn * g.TNB * 16, krt = kr1 + kr2;
     const int kl = kl_all - ca < g.TMB * 16 ? kl_all - ca : g.TMB * 16;
     const int kr = krt - cb < g.TNB * 16 ? krt - cb : g.TNB * 16;
     const int k1 = kr1 - cb < 0 ? 0 : kr1 - cb < kr ? kr1 - cb : kr, k2 = kr - k1;
-    const GtStage<VEC, ONE> sv(16 * g.KS, kl, k1, k2);
+    const GtStage<VEC, ONE, F32> sv(16 * g.KS, kl, k1, k2);
     const int SR = sv.SR, nth = 64 * g.NG * g.KS, vpt = gt_loads(g.W, VEC);
+    if (sv.count() > nth * vpt)
+        fail("more vectors than loads", sv.count(), nth, vpt);
     const int nstage = (r1 - r0 + SR - 1) / SR;
     const size_t buf = (size_t)SR * (sv.LDP + sv.RDP) + 32;
     if (2 * buf * sizeof(double) > g.lds)
@@ -67,15 +69,15 @@ static void walk(const GramTile &g, int n, int kl_all, int kr1, int kr2, int r0,
     }
 }
 
-int main(int argc, char **argv)
+template <bool F32>
+static int all(int n, int kl, int kr1, int kr2)
 {
-    const int n = atoi(argv[1]), kl = atoi(argv[2]), kr1 = atoi(argv[3]), kr2 = atoi(argv[4]);
     GramPlan p = plan_gram(n, kl, kr1 + kr2);
     tile_chunks(n, p);
-    GramTile g = plan_tile(p.TM, p.TN, 2, p.chunk);
-    const bool two = g.NG && tile_pairs(n, kl, kr1, kr2, g);
+    GramTile g = plan_tile(p.TM, p.TN, 2, p.chunk, F32);
+    const bool two = g.NG && tile_pairs(n, kl, kr1, kr2, g) && !(F32 && kr2 == 1);
     if (!two)
-        g = plan_tile(p.TM, p.TN, 1, p.chunk);
+        g = plan_tile(p.TM, p.TN, 1, p.chunk, F32);
     if (!g.NG)
         fail("no plan", n, kl, kr1 + kr2);
     const int gy = (p.TM + g.TMB - 1) / g.TMB * g.nbn;
@@ -83,13 +85,20 @@ int main(int argc, char **argv)
         for (int y = 0; y < gy; y++) {
             const int r0 = x * p.chunk, r1 = n - r0 < p.chunk ? n : r0 + p.chunk;
             if (!two)
-                walk<1, false>(g, n, kl, kr1, kr2, r0, r1, y);
+                walk<1, false, F32>(g, n, kl, kr1, kr2, r0, r1, y);
             else if (kr2 == 1)
-                walk<2, true>(g, n, kl, kr1, kr2, r0, r1, y);
+                walk<2, true, F32>(g, n, kl, kr1, kr2, r0, r1, y);
             else
-                walk<2, false>(g, n, kl, kr1, kr2, r0, r1, y);
+                walk<2, false, F32>(g, n, kl, kr1, kr2, r0, r1, y);
         }
-    std::printf("ok vec %d chunk %d\n", two ? 2 : 1, p.chunk);
+    return two ? 2 : 1;
+}
+
+int main(int argc, char **argv)
+{
+    const int n = atoi(argv[1]), kl = atoi(argv[2]), kr1 = atoi(argv[3]), kr2 = atoi(argv[4]);
+    std::printf("ok: %d columns a load, %d with an FP32 R1\n", all<false>(n, kl, kr1, kr2),
+                all<true>(n, kl, kr1, kr2));
     return 0;
 }
 """
