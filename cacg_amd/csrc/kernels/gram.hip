@@ -315,17 +315,18 @@ __device__ __forceinline__ long r1_col(const SrcT<TL, T1> &s, int c)
 
 // 64 consecutive outputs per block; wave w sums chunk partials x in
 // [w*gx/4, (w+1)*gx/4) in order, then the four wave sums are added in wave order.
-// 32 loads are in flight ahead of their additions: a wave's share is otherwise a
-// chain of memory latencies.
+// 32 loads (16 or 8 for what is left of them) are in flight ahead of their additions: a wave's
+// share is otherwise a chain of memory latencies.  2000 rows of 16 + 4 columns:
+// 3.1 -> 2.7 us with 8 instead of 32 where those do, and with scalar bounds.
 __global__ __launch_bounds__(256) void gram_reduce_kernel(const double *__restrict__ part, int gx,
                                                           int kl, int kr1, int kr2, int kl_pad,
                                                           int kr_pad, double *__restrict__ G1,
                                                           double *__restrict__ G2)
 {
-    constexpr int W = 4, LD = 32;
+    constexpr int W = 4;
     __shared__ double red[W][64];
     const int kr = kr1 + kr2;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const long e = (long)blockIdx.x * 64 + lane;
     const bool ok = e < (long)kl * kr;
     const int a = ok ? (int)(e / kr) : 0, b = ok ? (int)(e % kr) : 0;
@@ -334,17 +335,26 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(const double *__restri
     const int q = (gx + W - 1) / W;
     const int x0 = wave * q, x1 = (x0 + q) < gx ? (x0 + q) : gx;
     double acc = 0.0;
+    // past the share's end: its last partial is read again and not added
+    auto batch = [&](auto B, int x) {
+        constexpr int LD = decltype(B)::value;
+        double v[LD];
+#pragma unroll
+        for (int u = 0; u < LD; u++)
+            v[u] = p[(x + u < x1 ? x + u : x1 - 1) * stride];
+#pragma unroll
+        for (int u = 0; u < LD; u++)
+            if (x + u < x1)
+                acc += v[u];
+    };
     if (ok) {
-        for (int x = x0; x < x1; x += LD) {
-            double v[LD];
-#pragma unroll
-            for (int u = 0; u < LD; u++)
-                v[u] = x + u < x1 ? p[(x + u) * stride] : 0.0;
-#pragma unroll
-            for (int u = 0; u < LD; u++)
-                if (x + u < x1)
-                    acc += v[u];
-        }
+        int x = x0;
+        for (; x1 - x > 16; x += 32)
+            batch(std::integral_constant<int, 32>(), x);
+        if (x1 - x > 8)
+            batch(std::integral_constant<int, 16>(), x);
+        else if (x < x1)
+            batch(std::integral_constant<int, 8>(), x);
     }
     red[wave][lane] = acc;
     __syncthreads();
@@ -771,6 +781,129 @@ int launch_gram_wide(int n, const SrcT<TL, T1> &s, const GramPlan &p, double *wo
     return 1;
 }
 
+// ---- few rows of narrow blocks --------------------------------------------------
+//
+// At most 32 columns of L against 64: a chunk is a few MFMA steps, so a launch is latency
+// and what a stage costs beside its loads (the address setup, LDS, a barrier) is most of
+// it.  Waves feed the MFMAs from memory: wave (g, ks) forms tile row g against all NT
+// column tiles over every fourth step of 4 rows, 4 steps in flight, and the four partial
+// sums of a tile row are added in order.  Columns past the last are clamped to it (they
+// feed padding only), rows past the last are zeros.
+//
+// Up to 262,144 rows, 131,072 with an FP32 R1 (the tile kernel against this one, Gram in
+// us): 32 + 8 columns 2000 rows 7.8 / 7.1, 20,000 12.3 / 10.7, 250,047 39.5 / 39.0, 500,000
+// 65 / 74; 4 + 1 columns 20,000 8.6 / 7.0, 250,047 16.0 / 15.1, 500,000 19 / 21; 16 + 4 columns
+// 250,047 22.9 / 21.6, 1,000,000 52 / 59; 24 columns FP32 160,000 28.3 / 27.6, 250,047 35.5 / 37.0.
+constexpr int GD_TM = 2, GD_TN = 4;
+
+template <typename T1, int NT>
+__global__ __launch_bounds__(256 * GD_TM) void gram_direct_kernel(int n, SrcT<double, T1> s,
+                                                                  double *__restrict__ part,
+                                                                  int kr_pad, int chunk)
+{
+    constexpr int D = 4, PER = NT * 4;
+    __shared__ double red[GD_TM][3][PER][64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int lr = lane >> 4, lc = lane & 15, g = wave >> 2, ks = wave & 3;
+    const int r0 = blockIdx.x * chunk, rows = n - r0 < chunk ? n - r0 : chunk;
+    const int kr = s.kr1 + s.kr2;
+    const double *pa = s.L + (long)r0 * s.ldl + min(16 * g + lc, s.kl - 1);
+    const char *pb[NT];
+    long ib[NT];
+    bool f32[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const int b = min(16 * j + lc, kr - 1);
+        f32[j] = sizeof(T1) == 4 && b < s.kr1;
+        ib[j] = b < s.kr1 ? s.ld1 * (long)sizeof(T1) : s.ld2 * (long)sizeof(double);
+        pb[j] = b < s.kr1 ? reinterpret_cast<const char *>(s.R1 + r1_col(s, b))
+                          : reinterpret_cast<const char *>(s.R2 + (b - s.kr1));
+        pb[j] += r0 * ib[j];
+    }
+    dbl4 acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+        acc[j] = dbl4{0.0, 0.0, 0.0, 0.0};
+    double va[2][D], vb[2][D][NT];
+    auto load = [&](int p, int k0) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const int row = k0 + 16 * d + 4 * ks + lr;
+            const long i = row < rows ? row : rows - 1;
+            const double a = pa[i * s.ldl];
+            va[p][d] = row < rows ? a : 0.0;
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const char *q = pb[j] + i * ib[j];
+                const double b = f32[j] ? (double)*reinterpret_cast<const float *>(q)
+                                        : *reinterpret_cast<const double *>(q);
+                vb[p][d][j] = row < rows ? b : 0.0;
+            }
+        }
+    };
+    auto compute = [&](int p) {
+#pragma unroll
+        for (int d = 0; d < D; d++)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                acc[j] = mfma16x16x4(va[p][d], vb[p][d][j], acc[j]);
+    };
+    if (rows > 0)
+        load(0, 0);
+    for (int k0 = 0; k0 < rows; k0 += 32 * D) {
+        if (k0 + 16 * D < rows)
+            load(1, k0 + 16 * D);
+        compute(0);
+        if (k0 + 16 * D >= rows)
+            break;
+        if (k0 + 32 * D < rows)
+            load(0, k0 + 32 * D);
+        compute(1);
+    }
+    if (ks > 0) {
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                red[g][ks - 1][j * 4 + r][lane] = acc[j][r];
+    }
+    __syncthreads();
+    if (ks > 0)
+        return;
+    double *out = part + (long)blockIdx.x * (blockDim.x / 256 * 16) * kr_pad;
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            double v = acc[j][r];
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+                v += red[g][q][j * 4 + r][lane];
+            out[(long)(16 * g + lr + 4 * r) * kr_pad + 16 * j + lc] = v;
+        }
+}
+
+// launched: 1
+template <typename TL, typename T1>
+int launch_gram_direct(int n, const SrcT<TL, T1> &s, const GramPlan &p, double *work, hipStream_t st)
+{
+    if (n < 1 || n > (sizeof(T1) == 4 ? 1 << 17 : 1 << 18) || p.TM > GD_TM || p.TN > GD_TN)
+        return 0;
+#define CACG_GD(NT)                                                                               \
+    case NT:                                                                                      \
+        hipLaunchKernelGGL((gram_direct_kernel<T1, NT>), dim3(p.gx), dim3(256 * p.TM), 0, st, n,  \
+                           s, work, p.TN * 16, p.chunk);                                          \
+        return 1;
+    switch (p.TN) {
+        CACG_GD(1)
+        CACG_GD(2)
+        CACG_GD(3)
+        CACG_GD(4)
+    default: return 0;
+    }
+#undef CACG_GD
+}
+
 // ---- every other shape: waves share tiles out by group and by rows ----------------
 //
 // G is cut into blocks of at most 8 x 10 tiles of 16 x 16 (blockIdx.y); a workgroup
@@ -817,12 +950,21 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
     // this lane's vectors of a stage: source address, and LDS offset, source and row packed
     const char *src[VPT];
     unsigned info[VPT];
+    // narrow blocks (one or two tiles a wave, up to 8 waves) need few of the VPT loads: the
+    // rest is passed over by scalar branches (2,097,152 rows, 1 + 1 columns: 90 -> 41 us).
+    // Others need most, and the branches cost them 5%.
+    constexpr bool FEW = MT * NT <= 2 && (W == 8 || sizeof(T1) == 4);
+    const int nvec = sv.count();
+    auto none = [&](int u) { return FEW && nth * u >= nvec; };
 #pragma unroll
     for (int u = 0; u < VPT; u++) {
+        info[u] = ~0u;
+        src[u] = reinterpret_cast<const char *>(s.L);
+        if (none(u))
+            continue;
         int c;
         info[u] = sv.vector(t + nth * u, c);
         const long row = r0 + gt_row(info[u]);
-        src[u] = reinterpret_cast<const char *>(s.L);
         if (info[u] != ~0u)
             src[u] = gt_kind(info[u]) == 0 ? reinterpret_cast<const char *>(s.L + row * s.ldl + ca + c)
                      : gt_kind(info[u]) == 1
@@ -843,6 +985,8 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
         }
 #pragma unroll
         for (int u = 0; u < VPT; u++) {
+            if (none(u))
+                break;
             const int kind = gt_kind(info[u]);
             V w{};
             if (gt_row(info[u]) < left) {
@@ -865,6 +1009,8 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
         }
 #pragma unroll
         for (int u = 0; u < VPT; u++) {
+            if (none(u))
+                break;
             if (info[u] == ~0u)
                 continue;
             V w = stg[slot][u];
@@ -1018,12 +1164,9 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
 }
 
 template <typename TL, typename T1, int VEC>
-int launch_gram_tile(int n, const SrcT<TL, T1> &s, GramPlan &p, double *work, hipStream_t st)
+int launch_gram_tile(int n, const SrcT<TL, T1> &s, const GramPlan &p, const GramTile &g, double *work,
+                     hipStream_t st)
 {
-    tile_chunks(n, p);
-    const GramTile g = plan_tile(p.TM, p.TN, VEC, p.chunk, sizeof(T1) == 4);
-    if (VEC == 2 && !tile_pairs(n, s.kl, s.kr1, s.kr2, g))
-        return (int)hipErrorInvalidValue;
     const int kl_pad = p.TM * 16, kr_pad = p.TN * 16;
     const dim3 grid(p.gx, (p.TM + g.TMB - 1) / g.TMB * g.nbn), block(64 * g.NG * g.KS);
 #define CACG_GT(M, N, WV, ONE)                                                                    \
@@ -1033,15 +1176,15 @@ int launch_gram_tile(int n, const SrcT<TL, T1> &s, GramPlan &p, double *work, hi
                            st, n, s, work, kl_pad, kr_pad, p.chunk, g);                           \
         return 0;                                                                                 \
     }
-    if (VEC == 2 && s.kr2 == 1 && sizeof(T1) == 8) {
-        CACG_GT(1, 1, 8, true)
-        CACG_GT(1, 1, 16, true)
-        CACG_GT(1, 2, 8, true)
-        CACG_GT(1, 2, 16, true)
-        return (int)hipErrorInvalidValue;
+    if constexpr (VEC == 2 && sizeof(T1) == 8) {
+        if (s.kr2 == 1) {
+            CACG_GT(1, 1, 8, true)
+            CACG_GT(1, 1, 16, true)
+            CACG_GT(1, 2, 8, true)
+            CACG_GT(1, 2, 16, true)
+            return (int)hipErrorInvalidValue;
+        }
     }
-    if (VEC == 2 && s.kr2 == 1)
-        return (int)hipErrorInvalidValue;
 #define CACG_GTW(M, N) CACG_GT(M, N, 8, false) CACG_GT(M, N, 16, false)
     CACG_GTW(1, 1)
     CACG_GTW(1, 2)
@@ -1068,6 +1211,7 @@ int gram_fast(int n, const TL *L, long ldl, int kl, const T1 *R1, long ld1, int 
     if (n < 0 || kl <= 0 || kr1 < 0 || kr2 < 0 || kr1 + kr2 <= 0)
         return (int)hipErrorInvalidValue;
     GramPlan p = plan_gram(n, kl, kr1 + kr2);
+    tile_chunks(n, p);
     const SrcT<TL, T1> s = {L, ldl, kl, R1, ld1, kr1, R2, ld2, kr2, bs1};
     constexpr int EL = 16 / sizeof(TL), E1 = 16 / sizeof(T1);
     auto al16 = [](const void *q) { return ((uintptr_t)q & 15) == 0; };
@@ -1079,14 +1223,19 @@ int gram_fast(int n, const TL *L, long ldl, int kl, const T1 *R1, long ld1, int 
     // a block-major R1 is taken in the shapes cacg_gram_blk_supported names only
     if (bs1 && !(aligned && blk_shape(n, p, stage_vectors(s, 16), stage_vectors(s, 8))))
         return (int)hipErrorInvalidValue;
-    if (!launch_gram_wide(n, s, p, d_work, aligned, st)) {
+    if (!launch_gram_direct(n, s, p, d_work, st) &&
+        !launch_gram_wide(n, s, p, d_work, aligned, st)) {
         // pairs of columns (16-byte loads need no alignment beyond the element's), or
         // single ones where a source has only one
-        if (launch_gram_tile<TL, T1, 2>(n, s, p, d_work, st)) {
-            const int rc = launch_gram_tile<TL, T1, 1>(n, s, p, d_work, st);
-            if (rc)
-                return rc;
-        }
+        constexpr bool f32 = sizeof(T1) == 4;
+        GramTile g;
+        const int rc =
+            plan_pairs(n, kl, kr1, kr2, p, f32, g)
+                ? launch_gram_tile<TL, T1, 2>(n, s, p, g, d_work, st)
+                : launch_gram_tile<TL, T1, 1>(n, s, p, plan_tile(p.TM, p.TN, 1, p.chunk, p.gx, f32),
+                                              d_work, st);
+        if (rc)
+            return rc;
     }
     CACG_LAUNCH_CHECK();
     if (sol) {

@@ -6,6 +6,8 @@
 
 #include <stddef.h>
 
+#include <initializer_list>
+
 #ifdef __HIPCC__
 #include <hip/hip_runtime.h>
 
@@ -47,7 +49,8 @@ inline GramPlan plan_gram(int n, int kl, int kr)
     int gx = 512 / p.gy;
     if (gx < 1)
         gx = 1;
-    const int step = 8 * p.KS;
+    // whole stages of the 128-row kernels (16 rows), else of 8 rows a wave
+    const int step = p.TM == 8 ? 16 : 8 * p.KS;
     long maxc = ((long)n + 63) / 64;
     if (gx > maxc)
         gx = (int)(maxc > 0 ? maxc : 1);
@@ -91,12 +94,14 @@ CACG_HD constexpr int gt_loads(int W, int VEC)
     return W == 16 ? (VEC == 2 ? 3 : 5) : (VEC == 2 ? 5 : 9);
 }
 
-// from 8192 rows on at least 128 rows a chunk where a block's few tiles leave
-// waves for more row shares: the same waves on half the partials (4 + 4 columns
-// against 4, 20,000 rows: 14.0 -> 11.3 us; 100 columns: 28 -> 31 us, not taken)
+// at least 128 rows a chunk, half the partials: from 8192 rows on where a block's few
+// tiles leave waves for more row shares (4 + 4 columns against 4, 20,000 rows: 14.0 -> 11.3
+// us; 100 columns: 28 -> 31 us, not taken), and from 3072 to 8192 rows where a partial is
+// large (256 + 32 columns, 5000 rows: 46.5 -> 36.9 us; 10,000: 60 -> 64, not taken)
 inline void tile_chunks(int n, GramPlan &p)
 {
-    if (n >= 8192 && p.chunk < 128 && p.TM * p.TN <= 24) {
+    const int tiles = p.TM * p.TN;
+    if (p.chunk < 128 && (n >= 8192 ? tiles <= 24 : n >= 3072 && tiles >= 100)) {
         p.chunk = 128;
         p.gx = (n + 127) / 128;
     }
@@ -105,12 +110,24 @@ inline void tile_chunks(int n, GramPlan &p)
 // the tile group and row shares of a block: the fewest MFMA slots per row on the
 // busiest SIMD (waves are dealt round-robin over 4), then the most waves; at
 // most 16 waves and 80 KiB of LDS (two workgroups a CU) while a single row share
-// allows it.  f32: R1 is FP32 and its vectors start at a wave's first lane.
-inline GramTile plan_tile(int TM, int TN, int VEC, int chunk, bool f32)
+// allows it
+//
+// gx: row chunks.  With fewer workgroups than half the CUs the blocks are halved, the
+// longer side first, until there are: the chip is idle then, and a chunk's tiles take
+// the longer the more of them one CU forms (2000 rows, 112 + 16 columns: 19.4 ->
+// 10.8 us; 256 or 512 workgroups instead of 128: 14 to 16).
+// f32: R1 is FP32 and its vectors start at a wave's first lane.
+inline GramTile plan_tile(int TM, int TN, int VEC, int chunk, int gx, bool f32)
 {
     static const int shape[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 5}, {2, 2}, {2, 3}};
     GramTile best{};
-    const int bm = (TM + GT_TM - 1) / GT_TM, bn = (TN + GT_TN - 1) / GT_TN;
+    int bm = (TM + GT_TM - 1) / GT_TM, bn = (TN + GT_TN - 1) / GT_TN;
+    while (gx * bm * bn <= 128 && (bm < TM || bn < TN)) {
+        if ((TM + bm - 1) / bm >= (TN + bn - 1) / bn)
+            bm = 2 * bm < TM ? 2 * bm : TM;
+        else
+            bn = 2 * bn < TN ? 2 * bn : TN;
+    }
     best.TMB = (TM + bm - 1) / bm;
     best.TNB = (TN + bn - 1) / bn;
     best.nbn = (TN + best.TNB - 1) / best.TNB;
@@ -157,6 +174,20 @@ inline bool tile_pairs(int n, int kl, int kr1, int kr2, const GramTile &g)
     const int first2 = kr2 < w - e1 ? kr2 : w - e1;
     const bool r2 = kr2 > 1 && (first2 == 1 || lone(w, kr2 - first2));
     return !(n < 2 || lone(g.TMB * 16, kl) || lone(w, kr1) || r2);
+}
+
+// the plan with two columns a load, with the blocks halved for idle CUs or, where that
+// leaves a single column to a block, without; false: single columns
+inline bool plan_pairs(int n, int kl, int kr1, int kr2, const GramPlan &p, bool f32, GramTile &g)
+{
+    for (int gx : {p.gx, 129}) {
+        g = plan_tile(p.TM, p.TN, 2, p.chunk, gx, f32);
+        // a single column of R2 has a load of its own, in FP64 blocks of one or two tiles a wave
+        const bool one = kr2 == 1 && (f32 || g.MT * g.NT > 2);
+        if (g.NG && !one && tile_pairs(n, kl, kr1, kr2, g))
+            return true;
+    }
+    return false;
 }
 
 // The vectors of a stage of SR rows: VEC columns each, L's row by row, then those of

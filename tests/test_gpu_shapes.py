@@ -362,3 +362,19 @@ def test_updates_at_the_lines_between_the_kernels_exact_on_integers(gpu_lib, n, 
 def test_gram_f64f32_part_waves_exact_on_integers(gpu_lib, n, k):
     """Rows of L that end inside a wave's lanes: R1's vectors start at the next wave."""
     test_gram_f64f32_edges_exact_on_integers(gpu_lib, n, k)
+
+
+@pytest.mark.parametrize("n,kl,kr1,kr2", [
+    # the direct kernel and, past its rows, the tile kernel; several batches a wave, a ragged last chunk
+    (262144, 32, 32, 31), (262145, 32, 32, 31), (250001, 3, 2, 1), (100003, 17, 30, 3),
+    # few workgroups: halved blocks, some with a single column left over
+    (200, 112, 112, 16), (300, 33, 33, 3), (2000, 100, 100, 20), (1000, 160, 160, 32), (900, 97, 97, 1),
+    # chunks of 128 rows for large partials; whole 16-row stages a chunk at 128 columns
+    (3073, 256, 256, 32), (5000, 192, 192, 32), (140000, 128, 128, 16)])
+def test_gram_few_rows_exact_on_integers(gpu_lib, n, kl, kr1, kr2):
+    test_gram_fast_edges_exact_on_integers(gpu_lib, n, kl, kr1, kr2)
+
+
+@pytest.mark.parametrize("n,k", [(131072, 32), (131073, 32), (1000, 30), (64, 17), (2001, 25)])
+def test_gram_f64f32_few_rows_exact_on_integers(gpu_lib, n, k):
+    test_gram_f64f32_edges_exact_on_integers(gpu_lib, n, k)

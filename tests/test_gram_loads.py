@@ -74,10 +74,10 @@ static int all(int n, int kl, int kr1, int kr2)
 {
     GramPlan p = plan_gram(n, kl, kr1 + kr2);
     tile_chunks(n, p);
-    GramTile g = plan_tile(p.TM, p.TN, 2, p.chunk, F32);
-    const bool two = g.NG && tile_pairs(n, kl, kr1, kr2, g) && !(F32 && kr2 == 1);
+    GramTile g;
+    const bool two = plan_pairs(n, kl, kr1, kr2, p, F32, g);
     if (!two)
-        g = plan_tile(p.TM, p.TN, 1, p.chunk, F32);
+        g = plan_tile(p.TM, p.TN, 1, p.chunk, p.gx, F32);
     if (!g.NG)
         fail("no plan", n, kl, kr1 + kr2);
     const int gy = (p.TM + g.TMB - 1) / g.TMB * g.nbn;
