@@ -1276,20 +1276,24 @@ bool qupdate_by_ref(int n, int sm)
 
 // X / R update, sm below 16.  One right-hand side, norms in the same launch: 4 + 1 columns
 // 2,097,152 rows 90 / 33, 20,000 7.7 / 7.5; 10 + 1 columns 1,048,576 rows 50 / 45, 2,097,152
-// 107 / 119.  Else a second pass forms the norms: up to 8 columns and 4 right-hand sides past
-// two tiles a wave, 6 + 2 columns at 196,608 rows 14.4 / 13.3 and 91 / 60 at 2,097,152, 4 + 4
-// columns 15.1 / 14.1 and 99 / 77, at 130,000 rows 12.0 / 12.1; 10 + 2 columns 1,048,576 rows 51 / 46; at 2,097,152
-// rows also 5 + 5 131 / 116, 8 + 8 202 / 188, 9 + 3 123 / 116, 12 + 4 149 / 140, 15 + 3 162 / 157, but
-// 6 + 6 137 / 145 and 15 + 5 180 / 195.
+// 107 / 119.  Else a second pass forms the norms: up to 7 columns and 4 right-hand sides past
+// two tiles a wave, 6 + 2 columns at 196,608 rows 14.4 / 13.3 and 91 / 60 at 2,097,152, 3 + 3
+// columns at 250,047 17.4 / 16.0; 10 + 2 columns 1,048,576 rows 51 / 46; at 2,097,152 rows also
+// 5 + 5 131 / 116, 9 + 3 123 / 116, 12 + 4 149 / 140, 15 + 3 162 / 157, but 6 + 6 137 / 145 and 15 + 5
+// 180 / 195.  4 and 8 columns keep one order of sums, and so one rounding, over all row
+// counts: faster over many rows (4 + 4 columns 2,097,152 99 / 77), slower over few (8 + 2 columns
+// 20,000 7.2 / 11.4).
 bool xrupdate_by_ref(int n, int sm, int m)
 {
     if (sm >= 16)
         return false;
+    if (sm == 4 || sm == 8)
+        return true;
     if (m == 1)
         return sm <= 8 || n <= 1 << 20;
     if (sm <= 8 ? m <= 4 : sm <= 10 && m == 2)
         return n > 1 << 17;
-    return n >= 1 << 21 && (sm <= 5 || sm == 8 || (sm > 8 && m <= 4));
+    return n >= 1 << 21 && (sm <= 5 || (sm > 8 && m <= 4));
 }
 
 template <typename TS, typename T>
