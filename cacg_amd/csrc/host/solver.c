@@ -926,13 +926,14 @@ int cacg_solver_solve_device(cacg_solver *sv, const double *d_B, double *d_X, ca
     /* src/bcbcgKernel.c:113-115 */
     const double sa = 2.0 / (iv[1] - iv[0]);
     const double sb = -(iv[1] + iv[0]) / (iv[1] - iv[0]);
-    /* small blocks: the host needs longer to see the norms and launch again than a
-     * basis takes, so the next iteration's basis goes out before it waits for
-     * them (it reads R and writes S only; after the last iteration it is not
-     * used).  2^20 elements: a basis of about 10 us a step, the wait about 20 us;
-     * 16,384 x 1, s = 4: 11.9 -> 9.9 ms a solve together with the norms written
-     * to the host by the kernels and the cheaper marks */
-    const int ahead = sv->direct && s >= 2 && (long)n * m <= 1L << 20;
+    /* the next iteration's basis goes out before the host waits for the norms (it
+     * reads R and writes S only; after the last iteration it is not used), so the
+     * device works while the host sees them and launches again.  That is worth 10 to
+     * 13 us an iteration, nothing from 2^22 elements on.  us an iteration without / with
+     * it, s = 4: 128^2 m = 1 79 / 70, m = 4 93 / 84; 256^2 m = 4 115 / 106; 512^2 m = 4 215 / 203,
+     * m = 16 (2^22) 512 / 501; 1024^2 m = 2 357 / 345, m = 8 974 / 962; s = 8: 64^3 m = 16 (2^22)
+     * 1157 / 1156, 96^3 m = 16 3314 / 3323 */
+    const int ahead = sv->direct && s >= 2 && (long)n * m <= 1L << 22;
     int have = 0;   /* this iteration's basis is already enqueued */
 
     for (it = 0; it < o->maxiter; it++) {
