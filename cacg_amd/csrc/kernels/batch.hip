@@ -278,7 +278,7 @@ __global__ __launch_bounds__(256) void baq_kernel(const cacg_bsys *__restrict__ 
 // by splitting a chunk's output tiles, not its rows, over waves: a wave owns one
 // 16 x 16 tile (systems of up to BG_SMALL tiles) or 2 x 2 of them and feeds the
 // MFMAs straight from global memory, lane l loading L and [R1 | R2] at row
-// l / 16 of each step of 4 and its own columns, BG_D steps ahead in registers.
+// l / 16 of each step of 4 and its own columns, BgDepth steps ahead in registers.
 // No LDS, no barrier; the rows that the 4 waves of a workgroup share come from
 // L1, and grid.x is a multiple of 8, so a chunk's workgroups (grid.y) share an
 // L2.  One launch serves every width.  Per tile the k-steps run in row order

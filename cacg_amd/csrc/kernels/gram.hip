@@ -6,15 +6,16 @@
 // summation at one rank, bit for bit.  The chain bounds its time at n
 // dependent steps whatever the number of entries.
 //
-// Fast order: split-K.  Workgroup x owns a contiguous chunk of rows and a
-// group of 16x16 output tiles per wave; FP64 MFMA v_mfma_f64_16x16x4f64 with
-// the contraction index = row index, so both operands load straight from
-// row-major memory: the 16 lanes of a lane group read 16 consecutive doubles
-// (128 B) of one row and the 4 lane groups read 4 consecutive rows.  Loads for
-// the next 8 rows are issued before the MFMAs of the current 8 (register
-// double buffer).  Each chunk writes a kl_pad x kr_pad partial; a second
-// kernel sums the partials in chunk order, so the result is deterministic and
-// independent of scheduling.
+// Fast order: split-K.  Workgroup x owns a contiguous chunk of rows and forms its
+// partial of G with FP64 MFMA v_mfma_f64_16x16x4f64 (contraction index = row), kl_pad x
+// kr_pad, its sums in row order; a second kernel sums the partials in chunk order, so
+// the result is deterministic and independent of scheduling.  Three kernels share the
+// shapes out (gram_fast):
+//   gram_direct_kernel  up to 32 columns against 64 and not many rows: operands from
+//                       memory straight to the matrix cores;
+//   gram_lds_kernel     128 columns against 128 or 144: stages of 16 rows through LDS;
+//   gram_tile_kernel    every other shape, through LDS.
+// Either LDS kernel holds two stages in LDS and two more in registers.
 #include <type_traits>
 
 #include "gram_plan.hpp"
@@ -36,7 +37,7 @@ namespace {
 // alone, so loads stay in flight, and the chain lanes cross it with a batch in
 // registers.  With one chain wave, wave 4 does nothing else than the barriers:
 // it shares the chain's SIMD, and a producer there costs the chain 6%.
-// 262,144 rows, 128 x 144: 3.77 -> 1.86 ms (7.1 ns a row), 128 x 128 3.4 -> 1.63
+// 262,144 rows, 128 x 144: 3.77 -> 1.70 ms (6.5 ns a row), 128 x 128 3.4 -> 1.50
 // ms; the chain alone takes 3.7 ns a row, the producers alone 5.3 (products
 // through LDS and, with every CU at work, 13 TB/s out of the L2s).  Slower:
 // chain waves of 16 or 32 lanes (2.99, 2.53 ms), 9 producers, loads 2 or 8
@@ -275,26 +276,20 @@ __global__ __launch_bounds__(512) void gram_ref_kernel(int n, GrefSrc s, int nbb
 
 // ---- fast: split-K FP64 MFMA ------------------------------------------------
 
-// the shapes with a block-major R1, given the 16-byte vectors of a stage of 16
-// and of 8 rows: the wide kernels', or at most 5 vectors per lane of 256
-bool blk_shape(int n, const GramPlan &p, long vec16, long vec8)
-{
-    (void)n;
-    const bool wide = p.TM == 8 && p.chunk % 16 == 0 && (p.TN == 8 || p.TN == 9) &&
-                      vec16 <= (p.TN == 9 ? 12 * 64 * 3 : 16 * 64 * 2);
-    return wide || (vec8 <= 256 * 5 && p.chunk % 8 == 0);
-}
+// the shapes taken with a block-major R1: 49 columns on either side, 320 together at
+// most.  The kernels would read others; a narrower or wider basis stored block-major
+// has not been measured.
+bool blk_shape(const GramPlan &p, int kl, int kr1) { return p.KS == 1 && kl + kr1 <= 320; }
 
-// L and R1 are FP64 (the FP64 solver) or FP32 (the FP32 basis: Q, AQ, S);
-// R2 (the residual R) is always FP64.  Loaded values are widened to FP64 and
-// every product and sum is FP64.  R1 may be block-major (bs1 > 0): column c
-// of row i at R1[(c / ld1) * bs1 + i * ld1 + c % ld1], blocks of ld1 columns
-// bs1 elements apart (the basis S stored as its blocks S_0, S_1, ...); the
-// LDS-staged kernels read it (their 16-byte vectors stay inside a block),
-// the unstaged one does not.
-template <typename TL, typename T1>
+// L (Q, AQ) and R2 (the residual R) are FP64, R1 FP64 or FP32 (AQ; the basis S, FP32 in
+// the precision form).  Loaded values are widened to FP64 and every product and
+// sum is FP64.  R1 may be block-major (bs1 > 0): column c of row i at
+// R1[(c / ld1) * bs1 + i * ld1 + c % ld1], blocks of ld1 columns (an even number) bs1
+// elements apart (the basis S stored as its blocks S_0, S_1, ...), so a load of two
+// columns stays inside a block.
+template <typename T1>
 struct SrcT {
-    const TL *L;
+    const double *L;
     long ldl;
     int kl;
     const T1 *R1;
@@ -307,8 +302,8 @@ struct SrcT {
 };
 
 // offset of column c of R1 from its row start
-template <typename TL, typename T1>
-__device__ __forceinline__ long r1_col(const SrcT<TL, T1> &s, int c)
+template <typename T1>
+__device__ __forceinline__ long r1_col(const SrcT<T1> &s, int c)
 {
     return s.bs1 ? (long)(c / s.ld1) * s.bs1 + c % s.ld1 : (long)c;
 }
@@ -466,40 +461,32 @@ __global__ __launch_bounds__(1024) void gram_solve_kernel(const double *__restri
         x[(long)i * k + j - GS_N] = v;
 }
 
-// LDS-staged variant for the large case (even column counts, 16-byte aligned
-// rows).  A stage is SR rows of L and of [R1 | R2]; the NW * 64 lanes load it
-// cooperatively with 16-byte loads, LDG stages ahead, holding the data in
-// registers; the stage is then written to one of two LDS buffers and every
-// wave reads its MFMA operands from there.  Each row is read from HBM once per
-// workgroup.  Every wave owns one tile group (MT x NT tiles), so all tiles of
-// G are covered by one workgroup when NG <= NW.  Each tile accumulates its
-// k-steps of 4 rows in row order whatever SR, LDG, NW, MT and NT are, so the
-// partials depend on the row chunks only.
-//   <4, MT, NT, 8, 3, 5>: general large case (four tile groups per workgroup);
-//   <12, 2, 3, 16, 2, 3>, <16, 2, 2, 16, 2, 2>: a 128-row G against 144 and
-//   128 columns, as 12 and 16 waves of 2 x 3 and 2 x 2 tiles (measured on
-//   gfx950: 58 and 56 TFLOP/s against 42 and 50 for the general shape).
+// 128 columns of L against 128 or 144 of [R1 | R2] (even column counts, 16-byte aligned
+// rows).  A stage is 16 rows; the waves load it cooperatively with 16-byte loads, two
+// stages ahead, holding the data in registers; the stage is then written to one of
+// two LDS buffers and every wave reads its MFMA operands from there, so each row is
+// read from HBM once per workgroup.  12 waves of 2 x 3 tiles (144 columns) or 16 of 2 x
+// 2 (128) cover all of G; each tile takes its k-steps of 4 rows in row order.
+//
 // FULL (FP64, every column of the tiles present: 128 x 128 and 128 x 144): the stage
 // loop without a bound, a select or an address computation beside one addition per
 // load; LDS strides and buffers are immediate offsets.  Every vector instruction
 // there is paid in matrix-core time (FP64 MFMAs leave the SIMD few issue slots: 60 more
 // of them a stage had cost 2 to 10%).  2,097,152 rows: 128 x 144 1390 -> 1246 us (62
 // TFLOP/s), 128 x 128 1249 -> 1110 us.
-template <typename TL, typename T1, int NW, int MT, int NT, int SR, int LDG, int VPT, bool FULL>
-__global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s,
-                                                           double *__restrict__ part, int kl_pad,
-                                                           int kr_pad, int chunk, int GN, int NG)
+template <typename T1, int NW, bool FULL>
+__global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<T1> s,
+                                                           double *__restrict__ part, int chunk)
 {
-    constexpr int NTH = NW * 64;
+    constexpr int SR = 16, LDG = 2, MT = 2, NT = NW == 12 ? 3 : 2, GN = NW == 12 ? 3 : 4;
+    constexpr int VPT = NW == 12 ? 3 : 2, NTH = NW * 64, KR = NW == 12 ? 144 : 128;
     extern __shared__ double lds[];
     const int kr = s.kr1 + s.kr2;
     const int LDP = lds_row_stride(s.kl), RDP = lds_row_stride(kr);  // padded LDS row strides
     const int BUF = SR * (LDP + RDP);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int lr = lane >> 4, lc = lane & 15;
-    const int g = blockIdx.y * NW + wave;
-    const bool active = g < NG;
-    const int gm = active ? g / GN : 0, gn = active ? g % GN : 0;
+    const int gm = wave / GN, gn = wave % GN;
     const int ca0 = gm * MT * 16 + lc, cb0 = gn * NT * 16 + lc;
 
     const int r0 = blockIdx.x * chunk;
@@ -511,8 +498,8 @@ __global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s
     // this lane's share of a stage: 16-byte vector u -> (source row-0 address,
     // row stride in bytes, stage row, LDS offset, FP32 source); an FP32 vector
     // carries 4 columns and is widened into 4 doubles of LDS
-    constexpr int EL = 16 / sizeof(TL), E1 = 16 / sizeof(T1);
-    const int vl = SR * s.kl / EL, v1 = SR * s.kr1 / E1, v2 = SR * s.kr2 / 2;
+    constexpr int E1 = 16 / sizeof(T1);
+    const int vl = SR * s.kl / 2, v1 = SR * s.kr1 / E1, v2 = SR * s.kr2 / 2;
     const char *src[VPT];
     long ldb[VPT];
     int srow[VPT], loff[VPT];
@@ -526,12 +513,11 @@ __global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s
         loff[u] = 0;
         isf[u] = false;
         if (v < vl) {
-            const int row = v / (s.kl / EL), c = EL * (v % (s.kl / EL));
+            const int row = v / (s.kl / 2), c = 2 * (v % (s.kl / 2));
             src[u] = reinterpret_cast<const char *>(s.L + c);
-            ldb[u] = s.ldl * (long)sizeof(TL);
+            ldb[u] = s.ldl * (long)sizeof(double);
             srow[u] = row;
             loff[u] = row * LDP + c;
-            isf[u] = sizeof(TL) == 4;
         } else if ((v -= vl) < v1) {
             const int row = v / (s.kr1 / E1), c = E1 * (v % (s.kr1 / E1));
             src[u] = reinterpret_cast<const char *>(s.R1 + r1_col(s, c));
@@ -565,7 +551,7 @@ __global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s
             if (srow[u] < 0)
                 continue;
             const uint4 w = stg[slot][u];
-            if ((sizeof(TL) == 4 || sizeof(T1) == 4) && isf[u]) {
+            if (sizeof(T1) == 4 && isf[u]) {
                 float4 f;
                 __builtin_memcpy(&f, &w, 16);
                 *reinterpret_cast<double2 *>(b + loff[u]) = double2{(double)f.x, (double)f.y};
@@ -584,16 +570,13 @@ __global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s
 #pragma unroll
         for (int j = 0; j < NT; j++)
             acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
-    // the wide shapes (NW >= 12) read the operands of k-step ks + 1 while the
-    // MFMAs of ks run (two register sets; the scheduling barriers keep the
-    // reads ahead, which the compiler otherwise places just before their MFMAs
-    // and waits on); the general shape keeps one set (a second one would cost
-    // its 8-tile form a wave per SIMD)
-    constexpr bool PF = NW >= 12;
+    // the operands of k-step ks + 1 are read while the MFMAs of ks run (two register sets;
+    // the scheduling barriers keep the reads ahead, which the compiler otherwise places
+    // just before their MFMAs and waits on)
     auto compute = [&](int buf) {
         const double *bl = lds + buf * BUF;
         const double *br = bl + SR * LDP;
-        double av[PF ? 2 : 1][MT], bv[PF ? 2 : 1][NT];
+        double av[2][MT], bv[2][NT];
         auto operands = [&](int ks, int p) {
             const int row = ks * 4 + lr;
 #pragma unroll
@@ -607,25 +590,18 @@ __global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s
                 bv[p][t] = b < kr ? br[row * RDP + b] : 0.0;
             }
         };
-        if constexpr (PF)
-            operands(0, 0);
+        operands(0, 0);
 #pragma unroll
         for (int ks = 0; ks < SR / 4; ks++) {
-            const int p = PF ? ks & 1 : 0;
-            if constexpr (PF) {
-                if (ks + 1 < SR / 4)
-                    operands(ks + 1, (ks + 1) & 1);
-                __builtin_amdgcn_sched_barrier(0);
-            } else {
-                operands(ks, 0);
-            }
+            if (ks + 1 < SR / 4)
+                operands(ks + 1, (ks + 1) & 1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < MT; i++)
 #pragma unroll
                 for (int j = 0; j < NT; j++)
-                    acc[i][j] = mfma16x16x4(av[p][i], bv[p][j], acc[i][j]);
-            if constexpr (PF)
-                __builtin_amdgcn_sched_barrier(0);
+                    acc[i][j] = mfma16x16x4(av[ks & 1][i], bv[ks & 1][j], acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
 
@@ -639,8 +615,7 @@ __global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s
     int first = 0;   // first stage of the general loop below
     if constexpr (FULL) {
         constexpr int P = 144, B = SR * 2 * P;   // LDS row stride of 128 and of 144 columns; a buffer
-        constexpr int VEC16 = SR * (128 + (NW == 12 ? 144 : 128)) / 2;   // vectors of a stage
-        static_assert(LDG == 2, "buffer and register slot go by the parity of the stage");
+        constexpr int VEC16 = SR * (128 + KR) / 2;   // vectors of a stage
         const int full = (r1 - r0) / SR;
         const char *ptr[VPT];
         long inc[VPT];
@@ -700,8 +675,7 @@ __global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s
         for (int q = 0; q < LDG; q++) {
             const int st = st0 + q;
             if (st < nstage) {
-                if (active)
-                    compute(st & 1);
+                compute(st & 1);
                 const int nslot = (q + 1) % LDG;
                 lstore(nslot, (st + 1) & 1);
                 gload(nslot, st + 1 + LDG);
@@ -710,73 +684,46 @@ __global__ __launch_bounds__(NW * 64) void gram_lds_kernel(int n, SrcT<TL, T1> s
         }
     }
 
-    if (!active)
-        return;
-    double *out = part + (long)blockIdx.x * kl_pad * kr_pad;
+    double *out = part + (long)blockIdx.x * 128 * KR;
 #pragma unroll
-    for (int i = 0; i < MT; i++) {
-        const int tm = gm * MT + i;
-        if (tm * 16 >= kl_pad)
-            continue;
+    for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int j = 0; j < NT; j++) {
-            const int tn = gn * NT + j;
-            if (tn * 16 >= kr_pad)
-                continue;
+        for (int j = 0; j < NT; j++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                out[(long)(tm * 16 + lr + 4 * r) * kr_pad + tn * 16 + lc] = acc[i][j][r];
-        }
-    }
+                out[(long)((gm * MT + i) * 16 + lr + 4 * r) * KR + (gn * NT + j) * 16 + lc] = acc[i][j][r];
 }
 
-// 16-byte vectors of one stage of SR rows of L, R1 and R2
-template <typename TL, typename T1>
-long stage_vectors(const SrcT<TL, T1> &s, int SR)
-{
-    return (long)SR * (s.kl / (16 / (int)sizeof(TL)) + s.kr1 / (16 / (int)sizeof(T1)) + s.kr2 / 2);
-}
-
-// the 128-row shapes of the wide kernels: returns 1 when launched
-template <typename TL, typename T1>
-int launch_gram_wide(int n, const SrcT<TL, T1> &s, const GramPlan &p, double *work, bool staged_ok,
+// the shapes of gram_lds_kernel: returns 1 when launched
+template <typename T1>
+int launch_gram_wide(int n, const SrcT<T1> &s, const GramPlan &p, double *work, bool aligned,
                      hipStream_t st)
 {
-    constexpr int SRW = 16;
     const int kr = s.kr1 + s.kr2;
-    const int kl_pad = p.TM * 16, kr_pad = p.TN * 16;
-    if (!staged_ok || p.TM != 8 || p.chunk % SRW != 0 || (p.TN != 8 && p.TN != 9))
+    if (!aligned || p.TM != 8 || (p.TN != 8 && p.TN != 9))
         return 0;
-    const size_t shm = 2 * (size_t)SRW * (lds_row_stride(s.kl) + lds_row_stride(kr)) * sizeof(double);
+    const size_t shm = 2 * 16 * (size_t)(lds_row_stride(s.kl) + lds_row_stride(kr)) * sizeof(double);
     // every column of the tiles present
-    const bool full = sizeof(TL) == 8 && sizeof(T1) == 8 && s.kl == 128 && kr == kr_pad;
-#define CACG_GW(NW, NT, VPT, FULL, GN)                                                            \
+    const bool full = sizeof(T1) == 8 && s.kl == 128 && kr == p.TN * 16;
+#define CACG_GW(NW, FULL)                                                                         \
     do {                                                                                          \
-        cacg_allow_lds(gram_lds_kernel<TL, T1, NW, 2, NT, SRW, 2, VPT, FULL>, shm);               \
-        hipLaunchKernelGGL((gram_lds_kernel<TL, T1, NW, 2, NT, SRW, 2, VPT, FULL>), dim3(p.gx, 1), \
-                           dim3(NW * 64), shm, st, n, s, work, kl_pad, kr_pad, p.chunk, GN, NW);  \
+        cacg_allow_lds(gram_lds_kernel<T1, NW, FULL>, shm);                                       \
+        hipLaunchKernelGGL((gram_lds_kernel<T1, NW, FULL>), dim3(p.gx), dim3(NW * 64), shm, st, n, s, \
+                           work, p.chunk);                                                        \
     } while (0)
-    if (p.TN == 9) {
-        if (stage_vectors(s, SRW) > 12 * 64 * 3)
-            return 0;
-        if constexpr (sizeof(T1) == 8) {
-            if (full) {
-                CACG_GW(12, 3, 3, true, 3);
-                return 1;
-            }
+    if constexpr (sizeof(T1) == 8) {
+        if (full) {
+            if (p.TN == 9)
+                CACG_GW(12, true);
+            else
+                CACG_GW(16, true);
+            return 1;
         }
-        CACG_GW(12, 3, 3, false, 3);
-    } else {
-        if (stage_vectors(s, SRW) > 16 * 64 * 2)
-            return 0;
-        if constexpr (sizeof(T1) == 8) {
-            if (full) {
-                CACG_GW(16, 2, 2, true, 4);
-                return 1;
-            }
-        }
-        CACG_GW(16, 2, 2, false, 4);
     }
+    if (p.TN == 9)
+        CACG_GW(12, false);
+    else
+        CACG_GW(16, false);
 #undef CACG_GW
     return 1;
 }
@@ -797,7 +744,7 @@ int launch_gram_wide(int n, const SrcT<TL, T1> &s, const GramPlan &p, double *wo
 constexpr int GD_TM = 2, GD_TN = 4;
 
 template <typename T1, int NT>
-__global__ __launch_bounds__(256 * GD_TM) void gram_direct_kernel(int n, SrcT<double, T1> s,
+__global__ __launch_bounds__(256 * GD_TM) void gram_direct_kernel(int n, SrcT<T1> s,
                                                                   double *__restrict__ part,
                                                                   int kr_pad, int chunk)
 {
@@ -884,8 +831,8 @@ __global__ __launch_bounds__(256 * GD_TM) void gram_direct_kernel(int n, SrcT<do
 }
 
 // launched: 1
-template <typename TL, typename T1>
-int launch_gram_direct(int n, const SrcT<TL, T1> &s, const GramPlan &p, double *work, hipStream_t st)
+template <typename T1>
+int launch_gram_direct(int n, const SrcT<T1> &s, const GramPlan &p, double *work, hipStream_t st)
 {
     if (n < 1 || n > (sizeof(T1) == 4 ? 1 << 17 : 1 << 18) || p.TM > GD_TM || p.TN > GD_TN)
         return 0;
@@ -912,15 +859,16 @@ int launch_gram_direct(int n, const SrcT<TL, T1> &s, const GramPlan &p, double *
 // KS-th step of 4 rows of it for group g, and the KS partial sums are added in
 // order at the end.  Narrow blocks so get as many waves, and as many bytes
 // in flight, as wide ones.  Stages are loaded cooperatively two ahead (VEC
-// columns a load: 2, or 1 where a source has a single column) and read from one of two LDS buffers as in gram_lds_kernel.
+// columns a load: 2, or 1 where a source has a single column) and read from one of two
+// LDS buffers as in gram_lds_kernel.
 // Bound by memory up to about 64 columns, by the matrix cores above.
 
 // two columns, aligned as one
 typedef double pair64 __attribute__((ext_vector_type(2), aligned(8)));
 typedef float pair32 __attribute__((ext_vector_type(2), aligned(4)));
 
-template <typename TL, typename T1, int MT, int NT, int VEC, int W, bool ONE>
-__global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s,
+template <typename T1, int MT, int NT, int VEC, int W, bool ONE>
+__global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<T1> s,
                                                          double *__restrict__ part, int kl_pad,
                                                          int kr_pad, int chunk, GramTile g)
 {
@@ -971,7 +919,7 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
                          ? reinterpret_cast<const char *>(s.R1 + row * s.ld1 + r1_col(s, cb + c))
                          : reinterpret_cast<const char *>(s.R2 + row * s.ld2 + cb + c - s.kr1);
     }
-    const long incl = (long)SR * s.ldl * sizeof(TL), inc1 = (long)SR * s.ld1 * sizeof(T1),
+    const long incl = (long)SR * s.ldl * sizeof(double), inc1 = (long)SR * s.ld1 * sizeof(T1),
                inc2 = (long)SR * s.ld2 * sizeof(double);
     V stg[LDG][VPT];
     // a single column of R2 has a load of its own, row t of the stage
@@ -1085,14 +1033,6 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
 #pragma unroll
             for (int q = 0; q < 2; q++) {
                 compute(q);
-                double *const b = lds + (q ^ 1) * BUF;
-                if constexpr (one) {
-                    if (t < SR && k2 > 0) {
-                        b[SR * LDP + t * RDP + k1] = stg1[q ^ 1];
-                        stg1[q ^ 1] = *src1;
-                    }
-                    src1 += SR * s.ld2;
-                }
 #pragma unroll
                 for (int u = 0; u < VPT; u++) {
                     if (info[u] != ~0u)
@@ -1163,16 +1103,16 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<TL, T1> s
     }
 }
 
-template <typename TL, typename T1, int VEC>
-int launch_gram_tile(int n, const SrcT<TL, T1> &s, const GramPlan &p, const GramTile &g, double *work,
+template <typename T1, int VEC>
+int launch_gram_tile(int n, const SrcT<T1> &s, const GramPlan &p, const GramTile &g, double *work,
                      hipStream_t st)
 {
     const int kl_pad = p.TM * 16, kr_pad = p.TN * 16;
     const dim3 grid(p.gx, (p.TM + g.TMB - 1) / g.TMB * g.nbn), block(64 * g.NG * g.KS);
 #define CACG_GT(M, N, WV, ONE)                                                                    \
     if (g.MT == M && g.NT == N && g.W == WV) {                                                    \
-        cacg_allow_lds(gram_tile_kernel<TL, T1, M, N, VEC, WV, ONE>, g.lds);                      \
-        hipLaunchKernelGGL((gram_tile_kernel<TL, T1, M, N, VEC, WV, ONE>), grid, block, g.lds,    \
+        cacg_allow_lds(gram_tile_kernel<T1, M, N, VEC, WV, ONE>, g.lds);                      \
+        hipLaunchKernelGGL((gram_tile_kernel<T1, M, N, VEC, WV, ONE>), grid, block, g.lds,    \
                            st, n, s, work, kl_pad, kr_pad, p.chunk, g);                           \
         return 0;                                                                                 \
     }
@@ -1203,8 +1143,8 @@ struct GramSolve {
     int *flag, factor;
 };
 
-template <typename TL, typename T1>
-int gram_fast(int n, const TL *L, long ldl, int kl, const T1 *R1, long ld1, int kr1,
+template <typename T1>
+int gram_fast(int n, const double *L, long ldl, int kl, const T1 *R1, long ld1, int kr1,
               const double *R2, long ld2, int kr2, double *G1, double *G2, double *d_work,
               hipStream_t st, long bs1 = 0, const GramSolve *sol = nullptr)
 {
@@ -1212,16 +1152,16 @@ int gram_fast(int n, const TL *L, long ldl, int kl, const T1 *R1, long ld1, int 
         return (int)hipErrorInvalidValue;
     GramPlan p = plan_gram(n, kl, kr1 + kr2);
     tile_chunks(n, p);
-    const SrcT<TL, T1> s = {L, ldl, kl, R1, ld1, kr1, R2, ld2, kr2, bs1};
-    constexpr int EL = 16 / sizeof(TL), E1 = 16 / sizeof(T1);
+    const SrcT<T1> s = {L, ldl, kl, R1, ld1, kr1, R2, ld2, kr2, bs1};
+    constexpr int E1 = 16 / sizeof(T1);
     auto al16 = [](const void *q) { return ((uintptr_t)q & 15) == 0; };
     // 16-byte vectors: column counts and row strides in whole vectors, aligned rows
-    const bool aligned = p.KS == 1 && kl % EL == 0 && kr1 % E1 == 0 && kr2 % 2 == 0 &&
-                         ldl % EL == 0 && ld1 % E1 == 0 && bs1 % E1 == 0 &&
+    const bool aligned = p.KS == 1 && kl % 2 == 0 && kr1 % E1 == 0 && kr2 % 2 == 0 &&
+                         ldl % 2 == 0 && ld1 % E1 == 0 && bs1 % E1 == 0 &&
                          (kr2 == 0 || ld2 % 2 == 0) && al16(L) && al16(R1) &&
                          (kr2 == 0 || al16(R2));
     // a block-major R1 is taken in the shapes cacg_gram_blk_supported names only
-    if (bs1 && !(aligned && blk_shape(n, p, stage_vectors(s, 16), stage_vectors(s, 8))))
+    if (bs1 && !(aligned && blk_shape(p, kl, kr1)))
         return (int)hipErrorInvalidValue;
     if (!launch_gram_direct(n, s, p, d_work, st) &&
         !launch_gram_wide(n, s, p, d_work, aligned, st)) {
@@ -1231,8 +1171,8 @@ int gram_fast(int n, const TL *L, long ldl, int kl, const T1 *R1, long ld1, int 
         GramTile g;
         const int rc =
             plan_pairs(n, kl, kr1, kr2, p, f32, g)
-                ? launch_gram_tile<TL, T1, 2>(n, s, p, g, d_work, st)
-                : launch_gram_tile<TL, T1, 1>(n, s, p, plan_tile(p.TM, p.TN, 1, p.chunk, p.gx, f32),
+                ? launch_gram_tile<T1, 2>(n, s, p, g, d_work, st)
+                : launch_gram_tile<T1, 1>(n, s, p, plan_tile(p.TM, p.TN, 1, p.chunk, p.gx, f32),
                                               d_work, st);
         if (rc)
             return rc;
@@ -1287,7 +1227,8 @@ extern "C" int cacg_k_gram_ref(int n, const double *L, long ldl, int kl, const d
     const int kr = kr1 + kr2;
     const GrefSrc s = {L, ldl, kl, R1, ld1, kr1, R2, ld2, kr2};
     // the narrowest block whose grid gives no CU a second workgroup: 262,144 rows
-    // take 1.06, 1.24, 1.47, 1.86 ms with NJ = 1, 2, 4, 5
+    // of 28, 56, 112 and 128 against 144 columns take 1.30, 1.32, 1.50 and 1.70 ms with
+    // NJ = 1, 2, 4 and 5
     const int nbb = (kr + 15) / 16;
     const auto blocks = [&](int nj) { return (long)((kl + nj - 1) / nj) * nbb; };
 #define CACG_GREF(nj)                                                                             \
@@ -1319,8 +1260,7 @@ extern "C" int cacg_k_gram_fast(int n, const double *L, long ldl, int kl, const 
                                 long ld1, int kr1, const double *R2, long ld2, int kr2, double *G1,
                                 double *G2, double *d_work, hipStream_t st)
 {
-    return gram_fast<double, double>(n, L, ldl, kl, R1, ld1, kr1, R2, ld2, kr2, G1, G2, d_work,
-                                     st);
+    return gram_fast<double>(n, L, ldl, kl, R1, ld1, kr1, R2, ld2, kr2, G1, G2, d_work, st);
 }
 
 extern "C" int cacg_gram_blk_supported(int n, int kl, int kr1, int bw)
@@ -1328,9 +1268,7 @@ extern "C" int cacg_gram_blk_supported(int n, int kl, int kr1, int bw)
     if (n <= 0 || kl <= 0 || bw <= 0 || kr1 <= 0 || kr1 % bw != 0 || bw % 2 != 0 || kl % 2 != 0)
         return 0;
     // 16-byte aligned L, R1 and ldl = kl assumed
-    const GramPlan p = plan_gram(n, kl, kr1);
-    const SrcT<double, double> s = {nullptr, kl, kl, nullptr, bw, kr1, nullptr, 1, 0, (long)n * bw};
-    return p.KS == 1 && blk_shape(n, p, stage_vectors(s, 16), stage_vectors(s, 8)) ? 1 : 0;
+    return blk_shape(plan_gram(n, kl, kr1), kl, kr1) ? 1 : 0;
 }
 
 extern "C" int cacg_k_gram_fast_blk(int n, const double *L, long ldl, int kl, const double *R1,
@@ -1339,8 +1277,8 @@ extern "C" int cacg_k_gram_fast_blk(int n, const double *L, long ldl, int kl, co
 {
     if (bw <= 0 || bs < (long)n * bw || kr1 % bw != 0)
         return (int)hipErrorInvalidValue;
-    return gram_fast<double, double>(n, L, ldl, kl, R1, bw, kr1, nullptr, 1, 0, G1, nullptr,
-                                     d_work, st, bs);
+    return gram_fast<double>(n, L, ldl, kl, R1, bw, kr1, nullptr, 1, 0, G1, nullptr, d_work, st,
+                             bs);
 }
 
 extern "C" int cacg_gram_solve_supported(int sm, int m)
@@ -1355,8 +1293,7 @@ extern "C" int cacg_k_gram_alpha(int n, int sm, int m, const double *Q, const do
     if (n <= 0 || !cacg_gram_solve_supported(sm, m))
         return (int)hipErrorInvalidValue;
     const GramSolve sol = {lu, alpha, d_flag, 1};
-    return gram_fast<double, double>(n, Q, sm, sm, AQ, sm, sm, R, m, m, QtAQ, QtR, d_work, st, 0,
-                                     &sol);
+    return gram_fast<double>(n, Q, sm, sm, AQ, sm, sm, R, m, m, QtAQ, QtR, d_work, st, 0, &sol);
 }
 
 extern "C" int cacg_k_gram_beta(int n, int sm, const double *AQ, const double *S, const float *S32,
@@ -1367,16 +1304,15 @@ extern "C" int cacg_k_gram_beta(int n, int sm, const double *AQ, const double *S
         return (int)hipErrorInvalidValue;
     const GramSolve sol = {lu, beta, nullptr, 0};
     if (S32)
-        return gram_fast<double, float>(n, AQ, sm, sm, S32, sm, sm, nullptr, 1, 0, QtAS, nullptr,
-                                        d_work, st, 0, &sol);
-    return gram_fast<double, double>(n, AQ, sm, sm, S, sm, sm, nullptr, 1, 0, QtAS, nullptr, d_work,
-                                     st, 0, &sol);
+        return gram_fast<float>(n, AQ, sm, sm, S32, sm, sm, nullptr, 1, 0, QtAS, nullptr, d_work,
+                                st, 0, &sol);
+    return gram_fast<double>(n, AQ, sm, sm, S, sm, sm, nullptr, 1, 0, QtAS, nullptr, d_work, st, 0,
+                             &sol);
 }
 
 extern "C" int cacg_k_gram_fast_f64f32(int n, const double *L, long ldl, int kl, const float *R1,
                                        long ld1, int kr1, const double *R2, long ld2, int kr2,
                                        double *G1, double *G2, double *d_work, hipStream_t st)
 {
-    return gram_fast<double, float>(n, L, ldl, kl, R1, ld1, kr1, R2, ld2, kr2, G1, G2, d_work,
-                                    st);
+    return gram_fast<float>(n, L, ldl, kl, R1, ld1, kr1, R2, ld2, kr2, G1, G2, d_work, st);
 }

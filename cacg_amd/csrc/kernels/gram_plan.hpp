@@ -17,41 +17,29 @@
 #endif
 
 struct GramPlan {
-    int TM, TN;      // 16x16 tiles in M (kl) and N (kr)
-    int MT, NT;      // tiles per wave
-    int GN, NG;      // tile groups along N, total groups
-    int WGG, KS;     // groups per workgroup, waves sharing one group (split K inside the workgroup)
-    int gy;          // workgroups along the tile-group dimension
-    int gx;          // row chunks (split K across workgroups)
-    int chunk;       // rows per chunk
+    int TM, TN;   // 16x16 tiles in M (kl) and N (kr)
+    int KS;       // 1 from four groups of tiles on (see plan_gram), else more
+    int gx;       // row chunks (split K across workgroups)
+    int chunk;    // rows per chunk
 };
 
+// The chunks, and with them the order of the sums, are a function of n and the widths
+// only, not of the device: about 512 of them (2 workgroups a CU), fewer where a G is cut
+// into many groups of 2 x 9 (or 1 x 9) tiles, at least 64 rows each.
 inline GramPlan plan_gram(int n, int kl, int kr)
 {
     GramPlan p;
     p.TM = (kl + 15) / 16;
     p.TN = (kr + 15) / 16;
-    p.NT = p.TN < 9 ? p.TN : 9;
-    p.GN = (p.TN + p.NT - 1) / p.NT;
-    p.MT = p.TM >= 8 ? 2 : 1;
-    const int GM = (p.TM + p.MT - 1) / p.MT;
-    p.NG = GM * p.GN;
-    if (p.NG >= 4) {
-        p.WGG = 4;
-        p.KS = 1;
-    } else {
-        p.WGG = p.NG;
-        p.KS = 4 / p.NG;
-    }
-    p.gy = (p.NG + p.WGG - 1) / p.WGG;
-    // about 2 workgroups per CU over 256 CUs, at least 64 rows per chunk; a
-    // function of n only, so the summation order does not depend on the device
-    int gx = 512 / p.gy;
+    const int NT = p.TN < 9 ? p.TN : 9, MT = p.TM >= 8 ? 2 : 1;
+    const int NG = (p.TM + MT - 1) / MT * ((p.TN + NT - 1) / NT);
+    p.KS = NG >= 4 ? 1 : 4 / NG;
+    int gx = 512 / ((NG + 3) / 4);
     if (gx < 1)
         gx = 1;
-    // whole stages of the 128-row kernels (16 rows), else of 8 rows a wave
+    // whole stages of the 128-column kernels (16 rows), else of 8 rows a share
     const int step = p.TM == 8 ? 16 : 8 * p.KS;
-    long maxc = ((long)n + 63) / 64;
+    const long maxc = ((long)n + 63) / 64;
     if (gx > maxc)
         gx = (int)(maxc > 0 ? maxc : 1);
     long chunk = ((long)n + gx - 1) / gx;

@@ -52,6 +52,15 @@ __device__ __forceinline__ float sub_rn(float a, float b)
     return a - b;
 }
 
+// v of lane src (src the same on every lane of the wave)
+__device__ __forceinline__ double readlane_f64(double v, int src)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, src);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
 __device__ __forceinline__ dbl4 mfma16x16x4(double a, double b, dbl4 c)
 {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);

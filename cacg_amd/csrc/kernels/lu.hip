@@ -30,15 +30,6 @@ constexpr int LU_PS = 10;      // LDS row stride of a panel: 20 words, so 16 lan
 constexpr int LU_K = 32;       // right-hand sides that ride along with a factorisation
 constexpr int TRI_W = 8;       // waves of a triangular-solve workgroup
 
-// v of lane src (src the same on every lane of the wave)
-__device__ __forceinline__ double readlane_f64(double v, int src)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, src);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 // ---- substitutions of one vector by one wave -------------------------------------
 //
 // Lane l holds entries l (y0) and 64 + l (y1) of a vector of nb <= 128.  Step q
@@ -208,7 +199,8 @@ __host__ __device__ inline int lu_factor_lds(int N, int k, bool back)
 //      of the whole panel are ready without a barrier inside it;
 //   2. every lane applies the 8 rank-1 updates to its elements, in order, and
 //      the owners of the next panel put it into LDS.
-// Two barriers per 8 pivots.  What bounds it is the chain of pivots: one
+// Three barriers per 8 pivots (panel factored, panel's readers done, next panel in
+// place).  What bounds it is the chain of pivots: one
 // reciprocal, one product and one subtraction each, about 200 cycles; a barrier
 // and a broadcast through LDS for every pivot had taken 1870.
 __device__ __forceinline__ void lu_factor_body(int N, const double *lhs, long ldl, double *gw,
@@ -674,7 +666,7 @@ __device__ __forceinline__ void back_block(double (&x)[NB], const double *us, co
         back_block<NB, B - 1>(x, us, yc, S, lane);
 }
 
-// dynamic LDS: U (16 NB rows of 16 NB + 1, identity past N), then y of each column
+// dynamic LDS: U (16 NB x 16 NB, zeros past N), then y of each column
 template <int NB>
 __global__ __launch_bounds__(LB_W * 64) void lu_back16_ref_kernel(int N,
                                                                   const double *__restrict__ gw,

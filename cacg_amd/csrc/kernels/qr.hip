@@ -23,14 +23,6 @@ constexpr int QT = 1024;
 constexpr int QP = 8;      // pivots of a panel
 constexpr int QS = 10;     // LDS stride of a panel column (16-byte reads, all 64 banks)
 
-__device__ __forceinline__ double readlane_f64(double v, int src)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, src);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 // G (N x N, row-major, symmetric positive definite, N <= 128) -> R (upper, the
 // lower triangle written as zeros) and W = -R^{-1} (upper, zeros below).
 //

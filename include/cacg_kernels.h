@@ -93,15 +93,15 @@ int cacg_k_cheb1_f32(const cacg_scsr *A, int k, const double *r, long ldr, float
                      float *s0, long ld0, double a, double b, hipStream_t st);
 
 /* Launch schedule of the SpMMs above (no effect on any result: each output is
- * summed by one lane group in CSR order).  grid: workgroups (0: 8192 for
- * k <= 32, 4096 above); chunk_rows: 0 deals each XCD a contiguous band of row
+ * summed by one lane group in CSR order).  grid: workgroups (0: 8192
+ * where at most 8 lanes serve a row, 4096 above); chunk_rows: 0 deals each XCD a contiguous band of row
  * tiles, > 0 deals chunks of that many rows round-robin over the XCDs (an XCD
  * then owns a slice of every grid plane of a stencil matrix); passes (with
  * chunk_rows > 0; 0 or 1: one): each XCD sweeps its chunks in that many passes,
  * pass h taking its chunks h, h + passes, ... (a narrow column of the grid,
  * plane by plane; taken for k > 32, ignored for k = 4..32, whose kernel
  * sweeps one pass).  The _x forms take one (NULL or all zeros: the default for
- * the block's size); the forms above use the default. */
+ * the block's size and the matrix: see long_min above); the forms above use the default. */
 typedef struct {
     int grid;
     int chunk_rows;
