@@ -276,9 +276,9 @@ __global__ __launch_bounds__(512) void gram_ref_kernel(int n, GrefSrc s, int nbb
 
 // ---- fast: split-K FP64 MFMA ------------------------------------------------
 
-// the shapes taken with a block-major R1: 49 columns on either side, 320 together at
-// most.  The kernels would read others; a narrower or wider basis stored block-major
-// has not been measured.
+// the shapes taken with a block-major R1: from four groups of tiles on (49 columns of
+// L, or fewer against more than 144), at most 320 columns together.  The kernels would
+// read others; a narrower or wider basis stored block-major has not been measured.
 bool blk_shape(const GramPlan &p, int kl, int kr1) { return p.KS == 1 && kl + kr1 <= 320; }
 
 // L (Q, AQ) and R2 (the residual R) are FP64, R1 FP64 or FP32 (AQ; the basis S, FP32 in
@@ -1013,7 +1013,8 @@ __global__ __launch_bounds__(64 * W) void gram_tile_kernel(int n, SrcT<T1> s,
     __syncthreads();
     // whole stages without row tests or selects, as in gram_lds_kernel: an addition per
     // load, and lanes without a vector load the start of L and store nothing.  Not where
-    // 16 waves' 128 registers would spill, nor for one or two tiles a wave, which are
+    // 16 waves' 128 registers would spill more (2 x 3, 1 x 4 and 1 x 5 tiles keep a few
+    // registers in scratch as they are), nor for one or two tiles a wave, which are
     // bound by memory (2,097,152 rows of 16 + 4 columns: 112 -> 118 us).  300,000 rows of 96
     // columns 124 -> 113 us, 1,000,000 of 64 + 8 240 -> 222 us, 300,000 of 99 + 11 184 -> 168.
     int first = 0;
@@ -1111,9 +1112,9 @@ int launch_gram_tile(int n, const SrcT<T1> &s, const GramPlan &p, const GramTile
     const dim3 grid(p.gx, (p.TM + g.TMB - 1) / g.TMB * g.nbn), block(64 * g.NG * g.KS);
 #define CACG_GT(M, N, WV, ONE)                                                                    \
     if (g.MT == M && g.NT == N && g.W == WV) {                                                    \
-        cacg_allow_lds(gram_tile_kernel<T1, M, N, VEC, WV, ONE>, g.lds);                      \
-        hipLaunchKernelGGL((gram_tile_kernel<T1, M, N, VEC, WV, ONE>), grid, block, g.lds,    \
-                           st, n, s, work, kl_pad, kr_pad, p.chunk, g);                           \
+        cacg_allow_lds(gram_tile_kernel<T1, M, N, VEC, WV, ONE>, g.lds);                          \
+        hipLaunchKernelGGL((gram_tile_kernel<T1, M, N, VEC, WV, ONE>), grid, block, g.lds, st, n, \
+                           s, work, kl_pad, kr_pad, p.chunk, g);                                  \
         return 0;                                                                                 \
     }
     if constexpr (VEC == 2 && sizeof(T1) == 8) {
